@@ -14,12 +14,13 @@
 // IQ3_S repacks onto the IQ4_XS planes under its own format id (the kernels differ in the
 // codebook).  Q5_1 is an expert-tensor format only (rein_ingest_expert_format), as in the
 // reference, where a dense Q5_1 tensor stays in its on-disk layout.
+#include <algorithm>
 #include <cstring>
 #include <string>
-#include <vector>
 
 #include "../../../include/rein.h"
 #include "hip_api.h"
+#include "repack.h"
 
 namespace {
 
@@ -35,35 +36,61 @@ inline int q3k_scale(const uint8_t* scales, int k)
     return lo | (hi << 4);
 }
 
-// stored 3-bit quant of weight y (0..255): low two bits from qs, third bit from hmask.
 // The weight is d * (sc - 32) * (q3 - 4): hmask bit set means "no -4".
-inline int q3k_quant(const uint8_t* hmask, const uint8_t* qs, int y)
-{
-    const int n = y >> 7, s = (y >> 5) & 3, l = y & 31;
-    const int lo = (qs[32 * n + l] >> (2 * s)) & 3;
-    const int hi = (hmask[l] >> (4 * n + s)) & 1;
-    return lo | (hi << 2);
-}
-
+// Weight y = 128 n + 32 s + l: low bits at 2s of qs[32n + l], third bit at 4n + s of hmask[l]; as a Q6_K quant it goes to half n,
+// group s, lane l (src/quant/q6_k.rs:31-69): low nibble in ql[64n + 32(s & 1) + l] at 4(s >> 1), bits 4-5 in qh[32n + l] at 2s.
+// Eight lanes at a time: q6 = q3 + 28 <= 35 stays inside its byte.
 void q3k_block_to_q6k(const uint8_t* src, uint8_t* dst)
 {
-    const uint8_t* hmask = src;
-    const uint8_t* qs = src + 32;
-    const uint8_t* scales = src + 96;
-    uint8_t* ql = dst;
-    uint8_t* qh = dst + 128;
-    int8_t* sc6 = reinterpret_cast<int8_t*>(dst + 192);
-    std::memset(dst, 0, 192);
-    for (int k = 0; k < 16; k++) sc6[k] = (int8_t)(q3k_scale(scales, k) - 32);
-    for (int y = 0; y < 256; y++) {
-        const int q6 = q3k_quant(hmask, qs, y) + 28;
-        // Q6_K placement of weight y (src/quant/q6_k.rs:31-69): half n, group g of 32, lane l
-        const int n = y >> 7, g = (y >> 5) & 3, l = y & 31;
-        ql[64 * n + 32 * (g & 1) + l] |= (uint8_t)((q6 & 0x0F) << (4 * (g >> 1)));
-        qh[32 * n + l] |= (uint8_t)((q6 >> 4) << (2 * g));
-    }
+    constexpr uint64_t k1 = 0x0101010101010101ull;
+    const uint8_t *hmask = src, *qs = src + 32, *scales = src + 96;
+    for (int n = 0; n < 2; n++)
+        for (int l = 0; l < 32; l += 8) {
+            uint64_t q, h, ql[2] = {0, 0}, qh = 0;
+            std::memcpy(&q, qs + 32 * n + l, 8);
+            std::memcpy(&h, hmask + l, 8);
+            for (int s = 0; s < 4; s++) {
+                const uint64_t q6 = ((q >> (2 * s)) & (3 * k1)) + (((h >> (4 * n + s)) & k1) << 2) + 28 * k1;
+                ql[s & 1] |= (q6 & (15 * k1)) << (4 * (s >> 1));
+                qh |= ((q6 >> 4) & (3 * k1)) << (2 * s);
+            }
+            std::memcpy(dst + 64 * n + l, &ql[0], 8);
+            std::memcpy(dst + 64 * n + 32 + l, &ql[1], 8);
+            std::memcpy(dst + 128 + 32 * n + l, &qh, 8);
+        }
+    for (int k = 0; k < 16; k++) dst[192 + k] = (uint8_t)(q3k_scale(scales, k) - 32);
     dst[208] = src[108];
     dst[209] = src[109];
+}
+
+// Rows of the two types that are converted on the way, into the staging row of the thread that repacks them: no
+// converted copy of the tensor, and the conversion runs on every thread.
+struct Rows { const uint8_t* src; size_t in_dim; };
+
+const uint8_t* q3k_row(const void* ctx, size_t row, uint8_t* staging)
+{
+    const Rows* r = static_cast<const Rows*>(ctx);
+    const size_t n_super = r->in_dim / 256;
+    for (size_t b = 0; b < n_super; b++) q3k_block_to_q6k(r->src + (row * n_super + b) * kQ3kBytes, staging + b * kQ6kBytes);
+    return staging;
+}
+
+const uint8_t* bf16_row(const void* ctx, size_t row, uint8_t* staging)
+{
+    const Rows* r = static_cast<const Rows*>(ctx);
+    const uint8_t* p = r->src + row * r->in_dim * 2;
+    constexpr size_t kAt = 256;                            // values converted at a time (in_dim is a multiple of 32)
+    for (size_t i = 0; i < r->in_dim; i += kAt) {
+        const size_t n = std::min(kAt, r->in_dim - i);
+        uint16_t h[kAt];
+        uint32_t f[kAt];
+        std::memcpy(h, p + 2 * i, 2 * n);
+        for (size_t k = 0; k < n; k++) f[k] = (uint32_t)h[k] << 16;
+        float v[kAt];
+        std::memcpy(v, f, 4 * n);
+        rein::quantize_q8_0_blocks(v, n / 32, staging + i / 32 * 34);
+    }
+    return staging;
 }
 
 int label_of(int ggml_type)
@@ -131,21 +158,15 @@ extern "C" int rein_ingest_for_matvec(int ggml_type, const uint8_t* src, size_t 
         return rein_repack_for_matvec(REIN_TYPE_Q4_0, src, in_dim, out_dim, dst);
     case REIN_GGML_Q3_K: {
         if (in_dim % 256) return rein::fail(REIN_E_BAD_SHAPE, std::string(who) + ": Q3_K in_dim must be a multiple of 256");
-        std::vector<uint8_t> q6(in_dim * out_dim / 256 * kQ6kBytes);
-        if (int rc = rein_transcode_q3_k_to_q6_k(src, in_dim * out_dim, q6.data())) return rc;
-        return rein_repack_for_matvec(REIN_TYPE_Q6_K, q6.data(), in_dim, out_dim, dst);
+        const Rows rows = {src, in_dim};
+        rein::repack_parallel(REIN_TYPE_Q6_K, in_dim, out_dim, dst, q3k_row, &rows, true);
+        return 0;
     }
     case REIN_GGML_BF16: {
         if (in_dim % 32) return rein::fail(REIN_E_BAD_SHAPE, std::string(who) + ": BF16 in_dim must be a multiple of 32");
-        const size_t n = in_dim * out_dim;
-        std::vector<float> f(n);
-        for (size_t i = 0; i < n; i++) {
-            const uint32_t bits = (uint32_t)(src[2 * i] | (src[2 * i + 1] << 8)) << 16;
-            std::memcpy(&f[i], &bits, 4);
-        }
-        std::vector<uint8_t> q8(n / 32 * 34);
-        if (int rc = rein_quantize_weights(REIN_TYPE_Q8_0, f.data(), n, q8.data())) return rc;
-        return rein_repack_for_matvec(REIN_TYPE_Q8_0, q8.data(), in_dim, out_dim, dst);
+        const Rows rows = {src, in_dim};
+        rein::repack_parallel(REIN_TYPE_Q8_0, in_dim, out_dim, dst, bf16_row, &rows, true);
+        return 0;
     }
     default: return rein::fail(REIN_E_BAD_FORMAT, std::string(who) + ": unreachable");
     }

@@ -1,8 +1,7 @@
 // Host-side mirror of the reference's src/quant layout contract: repacked_len,
 // repacked_n_sub_padded and repack_for_matvec for the six formats.  Load-time
-// code (runs once per weight, host to host), written destination-first: for
-// every 32-weight sub-block of the output it pulls that sub-block's fields out
-// of the on-disk block and emits the planes.  Rows are split over threads.
+// code (runs once per weight, host to host): a row of on-disk blocks at a time, eight bytes of
+// a plane per step.  Rows are split over threads.
 #include <algorithm>
 #include <cstring>
 #include <thread>
@@ -11,6 +10,7 @@
 #include "../../../include/rein.h"
 #include "hip_api.h"
 #include "iq3s_grid.h"
+#include "repack.h"
 
 namespace {
 
@@ -81,160 +81,227 @@ uint16_t float_to_half(float f)
     return h;
 }
 
-// 6-bit (scale, min) of sub-block j from the 12 packed bytes (q4_k.rs:40-48).
-inline void scale_min_k4(const uint8_t* q, int j, uint8_t* sc, uint8_t* mn)
-{
-    if (j < 4) {
-        *sc = q[j] & 63;
-        *mn = q[4 + j] & 63;
-    } else {
-        *sc = (uint8_t)((q[4 + j] & 15) | ((q[j - 4] >> 6) << 4));
-        *mn = (uint8_t)((q[4 + j] >> 4) | ((q[j] >> 6) << 4));
+// nibbles 8 + l of the four weights of a codebook entry, one to a byte
+struct Iq3sNibbles {
+    uint32_t at[512];
+    constexpr Iq3sNibbles() : at()
+    {
+        for (unsigned e = 0; e < 512; e++)
+            for (unsigned j = 0; j < 4; j++) at[e] |= (uint32_t)((rein::iq3s_magnitude(e, j) + 15) / 2) << (8 * j);
     }
+    constexpr uint32_t operator[](unsigned e) const { return at[e]; }
+};
+constexpr Iq3sNibbles kIq3sNibbles;
+// bits 0-3 -> 0xFF in bytes 0-3
+inline uint32_t spread4(uint32_t v) { return (((v & 15u) * 0x00204081u) & 0x01010101u) * 0xFFu; }
+
+// ---- eight bytes at a time.  Every nibble plane byte j of a sub-block is weight j in the low half and weight 16 + j in
+// the high half (q4_k.rs:158-165), so it comes from two runs of source bytes by a mask and a shift.
+constexpr uint64_t kLow = 0x0F0F0F0F0F0F0F0Full, kHigh = ~kLow;
+inline uint64_t load64(const uint8_t* p) { uint64_t v; std::memcpy(&v, p, 8); return v; }
+inline uint32_t load32(const uint8_t* p) { uint32_t v; std::memcpy(&v, p, 4); return v; }
+inline void store64(uint8_t* p, uint64_t v) { std::memcpy(p, &v, 8); }
+inline void store32(uint8_t* p, uint32_t v) { std::memcpy(p, &v, 4); }
+// low nibbles (high nibbles) of 32 bytes -> one 16-byte plane entry
+inline void low_entry(const uint8_t* q, uint8_t* o)
+{
+    for (int j = 0; j < 16; j += 8) store64(o + j, (load64(q + j) & kLow) | ((load64(q + 16 + j) & kLow) << 4));
+}
+inline void high_entry(const uint8_t* q, uint8_t* o)
+{
+    for (int j = 0; j < 16; j += 8) store64(o + j, ((load64(q + j) >> 4) & kLow) | (load64(q + 16 + j) & kHigh));
+}
+// bit 0 of four bytes -> four bits, two bits of four bytes -> one byte: the partial products of the
+// multiplication do not overlap
+inline uint32_t gather1(uint32_t v) { return ((v & 0x01010101u) * 0x01020408u) >> 24 & 15u; }
+inline uint32_t gather2(uint32_t v) { return ((v & 0x03030303u) * 0x01041040u) >> 24; }
+static_assert(0x01041040u == ((1u << 24) | (1u << 18) | (1u << 12) | (1u << 6)), "byte i of the word moves to bit 24 + 2 i");
+
+// (scale, min) pairs of the eight sub-blocks from the 12 packed bytes (q4_k.rs:40-48), interleaved
+inline void scales_k4(const uint8_t* q, uint8_t* o)
+{
+    const uint32_t a = load32(q), b = load32(q + 4), c = load32(q + 8);
+    const uint32_t sc[2] = {a & 0x3F3F3F3Fu, (c & 0x0F0F0F0Fu) | ((a >> 2) & 0x30303030u)};
+    const uint32_t mn[2] = {b & 0x3F3F3F3Fu, ((c >> 4) & 0x0F0F0F0Fu) | ((b >> 2) & 0x30303030u)};
+    for (int h = 0; h < 2; h++)
+        for (int i = 0; i < 4; i++) {
+            o[8 * h + 2 * i]     = (uint8_t)(sc[h] >> (8 * i));
+            o[8 * h + 2 * i + 1] = (uint8_t)(mn[h] >> (8 * i));
+        }
 }
 
-// One 32-weight sub-block in dot order: element k pairs with activation quant k.
-struct SubBlock {
-    uint8_t lo4[32];     // low four bits of every weight
-    uint8_t ext[32];     // Q5_K: bit 4; Q6_K: bits 4-5
-    uint8_t sm[2];       // per-sub-block scale bytes
+// One output row's place in the planes of a slab: byte offsets of its first entry, in plane order (at most four planes
+// of one entry per sub-block, then one entry per superblock).
+struct Layout {
+    size_t n_sub, nsp, n_super, n_rows;
+    size_t entry[4];                   // bytes per sub-block of each plane (0: no such plane)
+    size_t super;                      // bytes per superblock
 };
 
-// nibble plane: byte 4j+b = lo4[4j+b] | lo4[16+4j+b] << 4 (q4_k.rs:158-165); the
-// two halves of the sub-block end up in the low / high nibbles of 16 bytes.
-inline void emit_nibbles(const SubBlock& s, uint8_t* dst)
+Layout layout_of(int fmt, const Geometry& g, size_t in_dim, size_t out_dim)
 {
-    for (int k = 0; k < 16; k++) dst[k] = (uint8_t)(s.lo4[k] | (s.lo4[16 + k] << 4));
-}
-
-// qh word of the Q5_K kernels: bit 4g+b = 5th bit of weight b of dot group g; group 2j is
-// weights 4j.., group 2j+1 weights 16+4j.. (q5_k.rs:122-141, q5_1.rs:70-73)
-inline uint32_t fifth_bits(const SubBlock& w)
-{
-    uint32_t qh = 0;
-    for (int k = 0; k < 16; k++) {
-        qh |= (uint32_t)(w.ext[k] & 1) << (8 * (k / 4) + (k % 4));
-        qh |= (uint32_t)(w.ext[16 + k] & 1) << (8 * (k / 4) + 4 + (k % 4));
+    Layout l = {in_dim / 32, rein_repacked_n_sub_padded(in_dim), in_dim / 256, out_dim, {16, 0, 0, 0}, g.per_super};
+    switch (fmt) {
+    case REIN_TYPE_Q8_0: l.entry[1] = 16; l.entry[2] = 2; break;      // quants 16-31; fp16 d
+    case REIN_TYPE_Q5_K: l.entry[1] = 4; l.entry[2] = 2; break;       // fifth bits; scale, min
+    case REIN_TYPE_Q5_1: l.entry[1] = 4; l.entry[2] = 4; break;       // fifth bits; fp16 d, m
+    case REIN_TYPE_Q6_K: l.entry[1] = 8; l.entry[2] = 2; break;       // bits 4-5; two int8 scales
+    default:             l.entry[1] = 2; break;                       // scale, min (Q4_K) or fp16 scale
     }
-    return qh;
+    return l;
 }
 
-void repack_rows(int fmt, const Geometry& g, const uint8_t* src, size_t in_dim, size_t out_dim,
-                 uint8_t* dst, size_t row_begin, size_t row_end)
+// One row: `b` its on-disk blocks; p[i] its first entry of plane i, ps its first superblock entry.
+template <int FMT>
+void repack_row(const uint8_t* b, size_t n_sub, uint8_t* const p[4], uint8_t* ps)
 {
-    const size_t n_sub   = in_dim / 32;
-    const size_t nsp     = rein_repacked_n_sub_padded(in_dim);
-    const size_t n_super = in_dim / 256;
-    const size_t n       = out_dim * nsp;
-    uint8_t* const nib = dst;
-
-    for (size_t row = row_begin; row < row_end; row++) {
-        for (size_t sb = 0; sb < n_sub; sb++) {
-            const size_t i = row * nsp + sb;
-            switch (fmt) {
-            case REIN_TYPE_Q4_0: {     // q4_0.rs:86-104: nibble bytes verbatim, fp16 d split out
-                const uint8_t* b = src + (row * n_sub + sb) * 18;
-                std::memcpy(nib + i * 16, b + 2, 16);
-                std::memcpy(dst + n * 16 + i * 2, b, 2);
-                break;
-            }
-            case REIN_TYPE_Q8_0: {     // q8_0.rs:93-119: quants 0-15 | quants 16-31 | fp16 d
-                const uint8_t* b = src + (row * n_sub + sb) * 34;
-                std::memcpy(nib + i * 16, b + 2, 16);
-                std::memcpy(dst + n * 16 + i * 16, b + 18, 16);
-                std::memcpy(dst + n * 32 + i * 2, b, 2);
-                break;
-            }
-            case REIN_TYPE_IQ4_XS: {   // iq4_xs.rs:106-136: nibbles verbatim, fp16(d*(ls-32))
-                const uint8_t* b = src + (row * n_super + sb / 8) * 136;
-                const int ib = (int)(sb % 8);
-                const int ls = ((b[4 + ib / 2] >> (4 * (ib & 1))) & 15) | (((load16(b + 2) >> (2 * ib)) & 3) << 4);
-                std::memcpy(nib + i * 16, b + 8 + ib * 16, 16);
-                store16(dst + n * 16 + i * 2, float_to_half(half_to_float(load16(b)) * (float)(ls - 32)));
-                break;
-            }
-            case REIN_TYPE_Q5_1: {     // q5_1.rs:82-104: nibbles verbatim, qh in dot-group order, raw fp16 d | m
-                const uint8_t* b = src + (row * n_sub + sb) * 24;
-                std::memcpy(nib + i * 16, b + 8, 16);
-                const uint32_t bits = (uint32_t)b[4] | ((uint32_t)b[5] << 8) | ((uint32_t)b[6] << 16) | ((uint32_t)b[7] << 24);
-                SubBlock w;
-                for (int k = 0; k < 32; k++) w.ext[k] = (uint8_t)((bits >> k) & 1);   // on disk bit k is weight k
-                const uint32_t qh = fifth_bits(w);
-                std::memcpy(dst + n * 16 + i * 4, &qh, 4);
-                std::memcpy(dst + n * 20 + i * 4, b, 4);
-                break;
-            }
-            case REIN_TYPE_IQ3_S: {    // iq3_s.rs:186-207: signed odd values -> nibble (v + 15) / 2, fp16(d * (1 + 2*scale))
-                const uint8_t* b = src + (row * n_super + sb / 8) * 110;
-                const int s = (int)(sb % 8);
-                const uint8_t* index = b + 2 + 8 * s;                // eight grid indices, low 8 bits
-                const unsigned high = b[66 + s];                     // their 9th bits
-                const uint8_t* sign = b + 74 + 4 * s;                // one bit per weight
-                const int scale = (b[106 + s / 2] >> (4 * (s & 1))) & 15;
-                SubBlock w;
-                for (int k = 0; k < 32; k++) {
-                    const unsigned entry = index[k / 4] | (((high >> (k / 4)) & 1u) << 8);
-                    const int mag = rein::iq3s_magnitude(entry, (unsigned)k % 4);
-                    const int v = ((sign[k / 8] >> (k % 8)) & 1) ? -mag : mag;
-                    w.lo4[k] = (uint8_t)((v + 15) / 2);
+    uint8_t *nib = p[0], *p1 = p[1], *p2 = p[2];
+    if constexpr (FMT == REIN_TYPE_Q4_0) {             // q4_0.rs:86-104: nibble bytes verbatim, fp16 d split out
+        for (size_t i = 0; i < n_sub; i++, b += 18) {
+            std::memcpy(nib + i * 16, b + 2, 16);
+            std::memcpy(p1 + i * 2, b, 2);
+        }
+    } else if constexpr (FMT == REIN_TYPE_Q8_0) {      // q8_0.rs:93-119: quants 0-15 | quants 16-31 | fp16 d
+        for (size_t i = 0; i < n_sub; i++, b += 34) {
+            std::memcpy(nib + i * 16, b + 2, 16);
+            std::memcpy(p1 + i * 16, b + 18, 16);
+            std::memcpy(p2 + i * 2, b, 2);
+        }
+    } else if constexpr (FMT == REIN_TYPE_Q5_1) {      // q5_1.rs:82-104: nibbles verbatim, qh in dot-group order, raw fp16 d | m
+        for (size_t i = 0; i < n_sub; i++, b += 24) {
+            std::memcpy(nib + i * 16, b + 8, 16);
+            // on disk bit k is weight k; in the plane byte j holds weights 4j.. and 16 + 4j..
+            const uint32_t bits = load32(b + 4);
+            uint32_t qh = 0;
+            for (int j = 0; j < 4; j++) qh |= (((bits >> (4 * j)) & 15u) | (((bits >> (16 + 4 * j)) & 15u) << 4)) << (8 * j);
+            store32(p1 + i * 4, qh);
+            std::memcpy(p2 + i * 4, b, 4);
+        }
+    } else {
+        for (size_t sb = 0; sb < n_sub; sb += 8) {
+            uint8_t* n0 = nib + sb * 16;
+            if constexpr (FMT == REIN_TYPE_IQ4_XS) {   // iq4_xs.rs:106-136: nibbles verbatim, fp16(d*(ls-32))
+                std::memcpy(n0, b + 8, 128);
+                const float d = half_to_float(load16(b));
+                const unsigned high = load16(b + 2);
+                for (int s = 0; s < 8; s++) {
+                    const int ls = ((b[4 + s / 2] >> (4 * (s & 1))) & 15) | (((high >> (2 * s)) & 3) << 4);
+                    store16(p1 + (sb + s) * 2, float_to_half(d * (float)(ls - 32)));
                 }
-                emit_nibbles(w, nib + i * 16);
-                store16(dst + n * 16 + i * 2, float_to_half(half_to_float(load16(b)) * (1.0f + 2.0f * (float)scale)));
-                break;
-            }
-            case REIN_TYPE_Q4_K:       // q4_k.rs:126-176
-            case REIN_TYPE_Q5_K: {     // q5_k.rs:97-151
-                const bool q5 = fmt == REIN_TYPE_Q5_K;
-                const uint8_t* b = src + (row * n_super + sb / 8) * (size_t)g.bytes;
-                const int s = (int)(sb % 8);
-                const uint8_t* qs = b + (q5 ? 48 : 16) + (s / 2) * 32;
-                SubBlock w;
-                for (int k = 0; k < 32; k++) {
-                    w.lo4[k] = (s & 1) ? (uint8_t)(qs[k] >> 4) : (uint8_t)(qs[k] & 15);
-                    w.ext[k] = q5 ? (uint8_t)((b[16 + k] >> s) & 1) : (uint8_t)0;
+                b += 136;
+            } else if constexpr (FMT == REIN_TYPE_IQ3_S) {   // iq3_s.rs:186-207: signed odd values -> nibble (v + 15) / 2, fp16(d * (1 + 2*scale))
+                const float d = half_to_float(load16(b));
+                for (int s = 0; s < 8; s++) {
+                    const uint8_t* index = b + 2 + 8 * s;                // eight grid indices, low 8 bits
+                    const unsigned high = b[66 + s];                     // their 9th bits
+                    const uint32_t sign = load32(b + 74 + 4 * s);        // one bit per weight
+                    uint32_t half[2][4];                                 // nibbles of weights 0-15, 16-31, four to a word
+                    for (int q = 0; q < 8; q++) {
+                        const uint32_t mag = kIq3sNibbles[index[q] | (((high >> q) & 1u) << 8)];
+                        // (15 - mag) / 2 for a negative weight is 7 - l, and (15 + mag) / 2 is 8 + l: the complement of 8 + l in four bits
+                        half[q / 4][q % 4] = mag ^ (0x0F0F0F0Fu & spread4(sign >> (4 * q)));
+                    }
+                    for (int j = 0; j < 4; j++) store32(n0 + s * 16 + 4 * j, half[0][j] | (half[1][j] << 4));
+                    const int scale = (b[106 + s / 2] >> (4 * (s & 1))) & 15;
+                    store16(p1 + (sb + s) * 2, float_to_half(d * (1.0f + 2.0f * (float)scale)));
                 }
-                scale_min_k4(b + 4, s, &w.sm[0], &w.sm[1]);
-                emit_nibbles(w, nib + i * 16);
-                size_t off = n * 16;
-                if (q5) {
-                    const uint32_t qh = fifth_bits(w);
-                    std::memcpy(dst + off + i * 4, &qh, 4);
-                    off += n * 4;
+                b += 110;
+            } else if constexpr (FMT == REIN_TYPE_Q4_K || FMT == REIN_TYPE_Q5_K) {   // q4_k.rs:126-176, q5_k.rs:97-151
+                constexpr bool q5 = FMT == REIN_TYPE_Q5_K;
+                const uint8_t* qs = b + (q5 ? 48 : 16);
+                for (int s = 0; s < 8; s += 2, qs += 32) {
+                    low_entry(qs, n0 + s * 16);
+                    high_entry(qs, n0 + s * 16 + 16);
                 }
-                dst[off + i * 2]     = w.sm[0];
-                dst[off + i * 2 + 1] = w.sm[1];
-                if (s == 0) std::memcpy(dst + off + n * 2 + (row * n_super + sb / 8) * 4, b, 4);
-                break;
-            }
-            case REIN_TYPE_Q6_K: {     // q6_k.rs:86-148
-                const uint8_t* b = src + (row * n_super + sb / 8) * 210;
-                const int s = (int)(sb % 8), chunk = s / 4, quad = s % 4;
-                const uint8_t* ql = b + chunk * 64 + (quad & 1) * 32;
-                const uint8_t* qh = b + 128 + chunk * 32;
-                SubBlock w;
-                for (int k = 0; k < 32; k++) {
-                    w.lo4[k] = (quad & 2) ? (uint8_t)(ql[k] >> 4) : (uint8_t)(ql[k] & 15);
-                    w.ext[k] = (uint8_t)((qh[k] >> (2 * quad)) & 3);
+                if constexpr (q5) {                    // byte j: fifth bits of weights 4j.. and 16 + 4j.. (q5_k.rs:122-141)
+                    for (int s = 0; s < 8; s++) {
+                        uint32_t qh = 0;
+                        for (int j = 0; j < 4; j++)
+                            qh |= (gather1(load32(b + 16 + 4 * j) >> s) | (gather1(load32(b + 32 + 4 * j) >> s) << 4)) << (8 * j);
+                        store32(p1 + (sb + s) * 4, qh);
+                    }
                 }
-                emit_nibbles(w, nib + i * 16);
-                // byte g = the four 2-bit fields of dot group g (q6_k.rs:128-138)
-                uint8_t h2[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-                for (int k = 0; k < 16; k++) {
-                    h2[2 * (k / 4)]     |= (uint8_t)(w.ext[k] << (2 * (k % 4)));
-                    h2[2 * (k / 4) + 1] |= (uint8_t)(w.ext[16 + k] << (2 * (k % 4)));
+                scales_k4(b + 4, (q5 ? p2 : p1) + sb * 2);
+                std::memcpy(ps + sb / 8 * 4, b, 4);
+                b += q5 ? 176 : 144;
+            } else {                                   // Q6_K (q6_k.rs:86-148)
+                for (int chunk = 0; chunk < 2; chunk++) {
+                    const uint8_t *ql = b + chunk * 64, *qh = b + 128 + chunk * 32;
+                    uint8_t* o = n0 + chunk * 64;
+                    low_entry(ql, o);
+                    low_entry(ql + 32, o + 16);
+                    high_entry(ql, o + 32);
+                    high_entry(ql + 32, o + 48);
+                    // byte g = the four 2-bit fields of dot group g (q6_k.rs:128-138)
+                    for (int quad = 0; quad < 4; quad++) {
+                        uint8_t* h2 = p1 + (sb + chunk * 4 + quad) * 8;
+                        for (int j = 0; j < 4; j++) {
+                            h2[2 * j]     = (uint8_t)gather2(load32(qh + 4 * j) >> (2 * quad));
+                            h2[2 * j + 1] = (uint8_t)gather2(load32(qh + 16 + 4 * j) >> (2 * quad));
+                        }
+                    }
                 }
-                std::memcpy(dst + n * 16 + i * 8, h2, 8);
-                dst[n * 24 + i * 2]     = b[192 + chunk * 8 + quad * 2];
-                dst[n * 24 + i * 2 + 1] = b[192 + chunk * 8 + quad * 2 + 1];
-                if (s == 0) std::memcpy(dst + n * 26 + (row * n_super + sb / 8) * 2, b + 208, 2);
-                break;
-            }
+                std::memcpy(p2 + sb * 2, b + 192, 16);
+                std::memcpy(ps + sb / 8 * 2, b + 208, 2);
+                b += 210;
             }
         }
     }
 }
 
+using RowFn = void (*)(const uint8_t*, size_t, uint8_t* const*, uint8_t*);
+RowFn row_fn(int fmt)
+{
+    switch (fmt) {
+    case REIN_TYPE_Q4_0:   return repack_row<REIN_TYPE_Q4_0>;
+    case REIN_TYPE_Q8_0:   return repack_row<REIN_TYPE_Q8_0>;
+    case REIN_TYPE_Q4_K:   return repack_row<REIN_TYPE_Q4_K>;
+    case REIN_TYPE_Q5_K:   return repack_row<REIN_TYPE_Q5_K>;
+    case REIN_TYPE_Q6_K:   return repack_row<REIN_TYPE_Q6_K>;
+    case REIN_TYPE_IQ4_XS: return repack_row<REIN_TYPE_IQ4_XS>;
+    case REIN_TYPE_Q5_1:   return repack_row<REIN_TYPE_Q5_1>;
+    default:               return repack_row<REIN_TYPE_IQ3_S>;
+    }
+}
+
+void repack_range(int fmt, const Layout& l, size_t row_bytes, uint8_t* dst, rein::RowSource source, const void* ctx, bool staged,
+                  size_t row_begin, size_t row_end)
+{
+    const RowFn fn = row_fn(fmt);
+    std::vector<uint8_t> staging(staged ? row_bytes : 0);
+    for (size_t row = row_begin; row < row_end; row++) {
+        uint8_t *p[4], *at = dst;
+        for (int i = 0; i < 4; i++) {
+            p[i] = at + row * l.nsp * l.entry[i];
+            at += l.n_rows * l.nsp * l.entry[i];
+        }
+        fn(source(ctx, row, staging.data()), l.n_sub, p, at + row * l.n_super * l.super);
+        for (int i = 0; i < 4 && l.nsp > l.n_sub; i++) std::memset(p[i] + l.n_sub * l.entry[i], 0, l.entry[i]);
+    }
+}
+
 }  // namespace
+
+// The output is the larger part of the traffic and, in a buffer that a loader has just allocated, is touched here for the
+// first time: each thread writes its rows (and zeroes their padding) itself, so the kernel hands out and clears the pages
+// of all threads at once.  A pass that zeroed the slab before the threads started was most of the call (Q4_K 5120 x 17408,
+// 50 MB in and out, sixteen threads of the GPU host: 9.7 ms with it and a byte at a time, 1.1 ms now).  A thread is worth
+// its start from about a million weights on.
+void rein::repack_parallel(int fmt, size_t in_dim, size_t out_dim, uint8_t* dst, RowSource source, const void* ctx, bool staged)
+{
+    Geometry g;
+    geometry(fmt, &g);
+    const Layout l = layout_of(fmt, g, in_dim, out_dim);
+    const size_t row_bytes = in_dim / (size_t)g.block * (size_t)g.bytes;
+    size_t n_threads = std::min<size_t>(std::max(1u, std::thread::hardware_concurrency()), 16);
+    n_threads = std::max<size_t>(1, std::min({n_threads, in_dim * out_dim >> 20, out_dim}));
+    std::vector<std::thread> pool;
+    const size_t step = (out_dim + n_threads - 1) / n_threads;
+    for (size_t a = step; a < out_dim; a += step)
+        pool.emplace_back(repack_range, fmt, std::cref(l), row_bytes, dst, source, ctx, staged, a, std::min(out_dim, a + step));
+    repack_range(fmt, l, row_bytes, dst, source, ctx, staged, 0, std::min(out_dim, step));
+    for (auto& th : pool) th.join();
+}
 
 extern "C" {
 
@@ -270,23 +337,12 @@ int rein_repack_for_matvec(int fmt, const uint8_t* src, size_t in_dim, size_t ou
     if (in_dim == 0 || in_dim % (size_t)g.block != 0)
         return rein::fail(REIN_E_BAD_SHAPE, "rein_repack_for_matvec: in_dim must be a non-zero multiple of " + std::to_string(g.block));
     if (!src || !dst) return rein::fail(REIN_E_BAD_POINTER, "rein_repack_for_matvec: null pointer");
-    std::memset(dst, 0, rein_repacked_len(fmt, in_dim, out_dim));
-
-    size_t n_threads = std::min<size_t>(std::max(1u, std::thread::hardware_concurrency()), 16);
-    if (in_dim * out_dim < ((size_t)1 << 22)) n_threads = 1;
-    n_threads = std::min(n_threads, std::max<size_t>(out_dim, 1));
-    if (n_threads <= 1) {
-        repack_rows(fmt, g, src, in_dim, out_dim, dst, 0, out_dim);
-        return 0;
-    }
-    std::vector<std::thread> pool;
-    const size_t step = (out_dim + n_threads - 1) / n_threads;
-    for (size_t t = 0; t < n_threads; t++) {
-        const size_t a = t * step, b = std::min(out_dim, a + step);
-        if (a >= b) break;
-        pool.emplace_back(repack_rows, fmt, std::cref(g), src, in_dim, out_dim, dst, a, b);
-    }
-    for (auto& th : pool) th.join();
+    const struct { const uint8_t* src; size_t row_bytes; } rows = {src, in_dim / (size_t)g.block * (size_t)g.bytes};
+    rein::repack_parallel(fmt, in_dim, out_dim, dst,
+                          [](const void* ctx, size_t row, uint8_t*) {
+                              const auto* r = static_cast<const decltype(rows)*>(ctx);
+                              return r->src + row * r->row_bytes;
+                          }, &rows, false);
     return 0;
 }
 

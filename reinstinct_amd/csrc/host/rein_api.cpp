@@ -785,7 +785,7 @@ int rein_init(const char* hsaco_path)
 {
     std::lock_guard<std::mutex> lock(g_init_mu);
     if (g_rt.loaded) return 0;
-    const HipApi* api;
+    const HipApi* api = nullptr;
     if (int rc = need_api(&api)) return rc;
     const std::string path = hsaco_path && *hsaco_path ? hsaco_path : default_hsaco_path();
     hipModule_t m = nullptr;
@@ -799,7 +799,7 @@ int rein_init(const char* hsaco_path)
 
 int rein_is_loaded(void) { return g_rt.loaded ? 1 : 0; }
 
-#define API_OR_RETURN() const HipApi* api; if (int rc_ = need_api(&api)) return rc_
+#define API_OR_RETURN() const HipApi* api = nullptr; if (int rc_ = need_api(&api)) return rc_
 
 int rein_device_count(int* n) { API_OR_RETURN(); return check_hip(api, api->GetDeviceCount(n), "hipGetDeviceCount"); }
 int rein_set_device(int d) { API_OR_RETURN(); return check_hip(api, api->SetDevice(d), "hipSetDevice"); }
