@@ -172,8 +172,12 @@ def load():
 
 
 class _Lazy:
+    """The library's functions as attributes; each is looked up once and then an attribute of the object itself."""
+
     def __getattr__(self, name):
-        return getattr(load(), name)
+        fn = getattr(load(), name)
+        setattr(self, name, fn)
+        return fn
 
 
 lib = _Lazy()

@@ -27,7 +27,7 @@ struct Runtime {
     const HipApi* api = nullptr;
     hipModule_t   module = nullptr;
     std::mutex    mu;
-    std::unordered_map<std::string, hipFunction_t> fns;
+    uint32_t      n_fns = 0;              // entries of g_fns, under mu
     bool loaded = false;
 };
 
@@ -61,33 +61,85 @@ int need_runtime()
     return 0;
 }
 
-int get_fn(const std::string& name, hipFunction_t* f)
+// A kernel's name, put together from texts and numbers without allocating, and its hash
+struct KName {
+    char text[56];
+    uint32_t len = 0;
+    template <class... P>
+    KName(const P&... parts)
+    {
+        (add(parts), ...);
+        text[len] = 0;
+    }
+    void add(const char* t)
+    {
+        while (*t && len + 1 < sizeof text) text[len++] = *t++;
+    }
+    void add(unsigned v)
+    {
+        char d[10];
+        int n = 0;
+        do { d[n++] = (char)('0' + v % 10); v /= 10; } while (v);
+        while (n && len + 1 < sizeof text) text[len++] = d[--n];
+    }
+    uint32_t hash() const
+    {
+        uint32_t h = 2166136261u;
+        for (uint32_t i = 0; i < len; i++) h = (h ^ (uint8_t)text[i]) * 16777619u;
+        return h ^ (h >> 15);
+    }
+};
+
+// The kernels looked up so far.  A launch is a few microseconds of a decode step, so the lookup takes no lock and
+// allocates nothing once a kernel is known: open addressing over entries that never move or go away (the code object
+// holds a few hundred kernels), each published with one release store.  (Per launch in a run of small eager calls:
+// strings, a mutex and a message for the error that did not happen cost 0.4-0.8 us beside the 2.5 of hipModuleLaunchKernel.)
+struct KEntry { KName name; hipFunction_t fn; };
+constexpr uint32_t kFnSlots = 2048;
+std::atomic<const KEntry*> g_fns[kFnSlots];
+
+int get_fn(const KName& name, hipFunction_t* f)
 {
+    const uint32_t h = name.hash();
+    const auto find = [&](uint32_t* at) {
+        for (uint32_t i = h % kFnSlots;; i = (i + 1) % kFnSlots) {
+            const KEntry* e = g_fns[i].load(std::memory_order_acquire);
+            *at = i;
+            if (!e || (e->name.len == name.len && std::memcmp(e->name.text, name.text, name.len) == 0)) return e;
+        }
+    };
+    uint32_t at;
+    if (const KEntry* e = find(&at)) {
+        *f = e->fn;
+        return 0;
+    }
     if (int rc = need_runtime()) return rc;
     std::lock_guard<std::mutex> lock(g_rt.mu);
-    auto it = g_rt.fns.find(name);
-    if (it != g_rt.fns.end()) {
-        *f = it->second;
+    if (const KEntry* e = find(&at)) {
+        *f = e->fn;
         return 0;
     }
     hipFunction_t fn = nullptr;
-    const hipError_t e = g_rt.api->ModuleGetFunction(&fn, g_rt.module, name.c_str());
+    const hipError_t e = g_rt.api->ModuleGetFunction(&fn, g_rt.module, name.text);
     if (e != 0) {
-        check_hip(g_rt.api, e, ("hipModuleGetFunction(" + name + ")").c_str());
+        check_hip(g_rt.api, e, (std::string("hipModuleGetFunction(") + name.text + ")").c_str());
         return REIN_E_NO_KERNEL;
     }
-    g_rt.fns.emplace(name, fn);
+    if (g_rt.n_fns < kFnSlots / 2) {                 // never full: find() ends at a free slot
+        g_fns[at].store(new KEntry{name, fn}, std::memory_order_release);
+        g_rt.n_fns++;
+    }
     *f = fn;
     return 0;
 }
 
-int launch(const std::string& name, unsigned gx, unsigned gy, unsigned gz, unsigned bx, unsigned shmem,
+int launch(const KName& name, unsigned gx, unsigned gy, unsigned gz, unsigned bx, unsigned shmem,
            rein_stream_t s, void** args)
 {
     hipFunction_t f;
     if (int rc = get_fn(name, &f)) return rc;
-    return check_hip(g_rt.api, g_rt.api->ModuleLaunchKernel(f, gx, gy, gz, bx, 1, 1, shmem, s, args, nullptr),
-                     ("hipModuleLaunchKernel(" + name + ")").c_str());
+    const hipError_t e = g_rt.api->ModuleLaunchKernel(f, gx, gy, gz, bx, 1, 1, shmem, s, args, nullptr);
+    return e == 0 ? 0 : check_hip(g_rt.api, e, (std::string("hipModuleLaunchKernel(") + name.text + ")").c_str());
 }
 
 const char* fmt_tag(int fmt)
@@ -260,7 +312,7 @@ int launch_skinny(int fmt, const void* w, const void* xq, float* y, unsigned in_
     if (occ == 2 && nv == 4 && tiles >= 1024 && ks < 4 && ks_max >= 4) ks = 4;
     const unsigned forced = opt_u(O_SKINNY_KS, 0);
     if (forced >= 1 && forced <= ks_max) ks = forced;
-    const std::string name = std::string("rein_mmqs_") + fmt_tag(fmt) + "_v" + std::to_string(nv);
+    const KName name("rein_mmqs_", fmt_tag(fmt), "_v", nv);
     void* args[] = {(void*)&w, (void*)&xq, (void*)&y, (void*)&in_dim, (void*)&out_dim, (void*)&n_rows};
     return launch(name, (out_dim + 31) / 32, (n_rows + tok - 1) / tok, 1, ks * 64, ks * lds_per_wave, s, args);
 }
@@ -451,7 +503,7 @@ int launch_matvec_lds(int fmt, const void* w, const void* xq, float* y, unsigned
     unsigned r, wpb, grid;
     mvl_geometry(fmt, in_dim, out_dim, n_rows, &r, &wpb, &grid);
     const unsigned b = n_rows <= 2 ? 2 : 4;
-    const std::string name = std::string("rein_mvl_") + fmt_tag(fmt) + "_r" + std::to_string(r) + "_b" + std::to_string(b);
+    const KName name("rein_mvl_", fmt_tag(fmt), "_r", r, "_b", b);
     void* args[] = {(void*)&w, (void*)&xq, (void*)&y, (void*)&in_dim, (void*)&out_dim, (void*)&n_rows};
     return launch(name, grid, 1, 1, wpb * 64, (unsigned)mvl_lds_bytes(in_dim, n_rows), s, args);
 }
@@ -602,7 +654,7 @@ int launch_quad_lds(int fmt, const void* w, const void* xq, float* y, unsigned i
                     unsigned n_rows, rein_stream_t s)
 {
     const QuadLdsGeometry g = mvql_geometry(fmt, in_dim, out_dim, n_rows);
-    const std::string name = std::string("rein_mvql_") + fmt_tag(fmt) + (n_rows <= 4 ? "_t4" : n_rows <= 8 ? "_t8" : n_rows <= 16 ? "_t16" :
+    const KName name("rein_mvql_", fmt_tag(fmt), n_rows <= 4 ? "_t4" : n_rows <= 8 ? "_t8" : n_rows <= 16 ? "_t16" :
                                                                          mvql_wide32(fmt) ? "_t32w" : "_t32");
     // Trips of weights in flight per wavefront where wavefronts stride over row groups or own a whole one (no slices,
     // no phases): two for the formats with little arithmetic per sub-block at 3-4 rows -- two register sets taking
@@ -681,7 +733,7 @@ int launch_matvec(const char* who, int fmt, const void* w, const void* xq, float
     if (family == MvFamily::Dot4Lds) return launch_matvec_lds(fmt, w, xq, y, in_dim, out_dim, n_rows, s);
     if (family == MvFamily::Quad) {
         // four output rows per wavefront, four wavefronts per workgroup
-        const std::string name = std::string("rein_mvq_") + fmt_tag(fmt) + (n_rows <= 4 ? "_t4" : "_t8");
+        const KName name("rein_mvq_", fmt_tag(fmt), n_rows <= 4 ? "_t4" : "_t8");
         void* args[] = {(void*)&w, (void*)&xq, (void*)&y, (void*)&in_dim, (void*)&out_dim, (void*)&n_rows};
         return launch(name, ((out_dim + 3) / 4 + 3) / 4, 1, 1, 256, 0, s, args);
     }
@@ -691,7 +743,7 @@ int launch_matvec(const char* who, int fmt, const void* w, const void* xq, float
     const unsigned groups = (out_dim + r - 1) / r;
     const unsigned wpb = pick_wpb(fmt, groups, b);
     const unsigned grid = (groups + wpb - 1) / wpb;
-    const std::string name = std::string("rein_mv_") + fmt_tag(fmt) + "_r" + std::to_string(r) + "_b" + std::to_string(b);
+    const KName name("rein_mv_", fmt_tag(fmt), "_r", r, "_b", b);
     void* args[] = {(void*)&w, (void*)&xq, (void*)&y, (void*)&in_dim, (void*)&out_dim, (void*)&n_rows};
     return launch(name, grid, 1, 1, wpb * 64, 0, s, args);
 }
@@ -714,9 +766,9 @@ int launch_grouped(int fmt, const void* slab0, const void* slab1, unsigned bytes
         float* o1 = y1 ? y1 : y0;
         void* a[] = {(void*)&slab0, (void*)&s1, (void*)&bytes_per_expert, (void*)&expert_off, (void*)&tile_off,
                      (void*)&n_expert, (void*)&xq, (void*)&y0, (void*)&o1, (void*)&in_dim, (void*)&out_dim, (void*)&n_slab};
-        return launch(std::string("rein_mmq_") + fmt_tag(fmt) + "_grouped_t32", (unsigned)grid, 1, 1, 256, 0, s, a);
+        return launch(KName("rein_mmq_", fmt_tag(fmt), "_grouped_t32"), (unsigned)grid, 1, 1, 256, 0, s, a);
     }
-    const std::string name = std::string("mmq_gemm_") + fmt_tag(fmt) + "_grouped_f32";
+    const KName name("mmq_gemm_", fmt_tag(fmt), "_grouped_f32");
     for (int z = 0; z < (slab1 ? 2 : 1); z++) {
         const void* slab = z ? slab1 : slab0;
         float* y = z ? y1 : y0;
@@ -1047,7 +1099,7 @@ int rein_matvec_multi_xq8(unsigned n_mat, const int* fmts, const void* const* ws
     for (unsigned i = n_mat; i < kMax; i++) a.m[i] = a.m[n_mat - 1];
     const unsigned wpb = pick_wpb(lead, groups, b);
     void* args[] = {(void*)&a, (void*)&xq, (void*)&in_dim, (void*)&n_mat, (void*)&n_rows};
-    return launch("rein_mv_multi_r" + std::to_string(r) + "_b" + std::to_string(b), (groups + wpb - 1) / wpb, 1, 1, wpb * 64, 0, s, args);
+    return launch(KName("rein_mv_multi_r", r, "_b", b), (groups + wpb - 1) / wpb, 1, 1, wpb * 64, 0, s, args);
 }
 
 int rein_matvec_kernel_name(int fmt, unsigned in_dim, unsigned out_dim, unsigned n_rows, char* name, size_t name_len)
@@ -1192,7 +1244,7 @@ int rein_mmq_xq8(int fmt, const void* w, const void* xq, float* y, unsigned in_d
         const unsigned long long g = 8ull * ((n_rb + 7) / 8) * ((p_rows + 63) / 64);
         if (g > 0x7FFFFFFFull) return fail(REIN_E_TOO_LARGE, "rein_mmq_xq8: too many tiles for one launch");
         void* a[] = {(void*)&w, (void*)&xq, (void*)&y, (void*)&in_dim, (void*)&out_dim, (void*)&p_rows};
-        return launch(std::string("rein_mmq_") + fmt_tag(fmt) + "_t64", (unsigned)g, 1, 1, 256, 0, s, a);
+        return launch(KName("rein_mmq_", fmt_tag(fmt), "_t64"), (unsigned)g, 1, 1, 256, 0, s, a);
     }
     // 1-D grids; workgroup i runs on XCD i % 8 and the kernels map it to (row block, token
     // tile) so that one weight block stays on one XCD
@@ -1201,12 +1253,12 @@ int rein_mmq_xq8(int fmt, const void* w, const void* xq, float* y, unsigned in_d
         const unsigned long long g = 8ull * ((n_rb + 7) / 8) * (n64 + n32);
         if (g > 0x7FFFFFFFull) return fail(REIN_E_TOO_LARGE, "rein_mmq_xq8: too many tiles for one launch");
         void* a[] = {(void*)&w, (void*)&xq, (void*)&y, (void*)&in_dim, (void*)&out_dim, (void*)&p_rows, (void*)&n64};
-        return launch(std::string("rein_mmq_") + fmt_tag(fmt) + "_mix", (unsigned)g, 1, 1, 256, 0, s, a);
+        return launch(KName("rein_mmq_", fmt_tag(fmt), "_mix"), (unsigned)g, 1, 1, 256, 0, s, a);
     }
     const unsigned long long grid = 8ull * ((n_rb + 7) / 8) * ((p_rows + 31) / 32);
     if (grid > 0x7FFFFFFFull) return fail(REIN_E_TOO_LARGE, "rein_mmq_xq8: too many tiles for one launch");
     void* args[] = {(void*)&w, (void*)&xq, (void*)&y, (void*)&in_dim, (void*)&out_dim, (void*)&p_rows};
-    return launch(std::string("rein_mmq_") + fmt_tag(fmt) + "_t32", (unsigned)grid, 1, 1, 256, 0, s, args);
+    return launch(KName("rein_mmq_", fmt_tag(fmt), "_t32"), (unsigned)grid, 1, 1, 256, 0, s, args);
 }
 
 // ---- Q4_K on the block-scaled fp6 matrix instruction (kernels/mmq_fp6.h)
@@ -1553,7 +1605,7 @@ int rein_mmq_xq8_ws(int fmt, const void* w, const void* xq, float* y, unsigned i
         if (int rc = check_ptr(who, workspace, 16, "workspace")) return rc;
         const unsigned first = sk8.n_unit - sk8.n_tail, n_chunk = (in_dim / 32 + 7) / 8, split = sk8.split;
         void* a[] = {(void*)&w, (void*)&xq, (void*)&y, (void*)&workspace, (void*)&in_dim, (void*)&out_dim, (void*)&p_rows, (void*)&split};
-        if (int rc = launch(std::string("rein_mmq_") + fmt_tag(fmt) + (sk8.tm == 32 ? "_sk32" : "_sk"), sk8.g, 1, 1, 256, 0, s, a)) return rc;
+        if (int rc = launch(KName("rein_mmq_", fmt_tag(fmt), sk8.tm == 32 ? "_sk32" : "_sk"), sk8.g, 1, 1, 256, 0, s, a)) return rc;
         if (sk8.n_tail == 0 || split == 1) return 0;
         void* b[] = {(void*)&workspace, (void*)&y, (void*)&n_chunk, (void*)&out_dim, (void*)&p_rows, (void*)&first, (void*)&split};
         return launch(sk8.tm == 32 ? "rein_mmq_tail_sum_t32" : "rein_mmq_tail_sum_t64", sk8.n_tail, sk8.tm / 32, 4, 256, 0, s, b);
@@ -1638,7 +1690,7 @@ int rein_noalloc_prepare(void)
     for (int fmt : fmts) {
         for (const char* form : forms) {
             hipFunction_t f;
-            if (int rc = get_fn(std::string("rein_mmq_") + fmt_tag(fmt) + form, &f)) return rc;
+            if (int rc = get_fn(KName("rein_mmq_", fmt_tag(fmt), form), &f)) return rc;
         }
         for (const char* pattern : few) {
             char name[64];
@@ -1650,9 +1702,9 @@ int rein_noalloc_prepare(void)
             for (unsigned b = 1; b <= 8; b *= 2) {
                 hipFunction_t f;
                 if (r * b <= 16)
-                    if (int rc = get_fn(std::string("rein_mv_") + fmt_tag(fmt) + "_r" + std::to_string(r) + "_b" + std::to_string(b), &f)) return rc;
+                    if (int rc = get_fn(KName("rein_mv_", fmt_tag(fmt), "_r", r, "_b", b), &f)) return rc;
                 if (b == 2 || b == 4)
-                    if (int rc = get_fn(std::string("rein_mvl_") + fmt_tag(fmt) + "_r" + std::to_string(r) + "_b" + std::to_string(b), &f)) return rc;
+                    if (int rc = get_fn(KName("rein_mvl_", fmt_tag(fmt), "_r", r, "_b", b), &f)) return rc;
             }
     }
     return 0;
@@ -1777,11 +1829,11 @@ int rein_block_dots(int fmt, const void* w, const void* xq, int32_t* out, unsign
     if (n_rows > 65535) return fail(REIN_E_TOO_LARGE, "rein_block_dots: at most 65535 rows");
     if (via_mfma) {
         if (int rc = check_dense_fmt(who, fmt)) return rc;
-        const std::string name = std::string("rein_mmq_dots_") + fmt_tag(fmt);
+        const KName name("rein_mmq_dots_", fmt_tag(fmt));
         void* args[] = {(void*)&w, (void*)&xq, (void*)&out, (void*)&in_dim, (void*)&out_dim, (void*)&n_rows};
         return launch(name, (out_dim + 127) / 128, (n_rows + 31) / 32, 1, 256, 0, s, args);
     }
-    const std::string name = std::string("rein_block_dots_") + fmt_tag(fmt);
+    const KName name("rein_block_dots_", fmt_tag(fmt));
     void* args[] = {(void*)&w, (void*)&xq, (void*)&out, (void*)&in_dim, (void*)&out_dim};
     return launch(name, out_dim < 4096 ? out_dim : 4096, n_rows, 1, 64, 0, s, args);
 }
@@ -1940,11 +1992,11 @@ int rein_moe_grouped_swiglu_q8(int fmt, const void* gate_slab, const void* up_sl
     if (grid > 0x7FFFFFFFull) return fail(REIN_E_TOO_LARGE, std::string(who) + ": more than 2^31 workgroup tiles");
     void* a[] = {(void*)&gate_slab, (void*)&up_slab, (void*)&bytes_per_expert, (void*)&expert_off, (void*)&tile_off,
                  (void*)&n_expert, (void*)&xq, (void*)&xq_out, (void*)&in_dim, (void*)&out_dim};
-    return launch(std::string("rein_mmq_") + fmt_tag(fmt) + "_grouped_swiglu_q8", (unsigned)grid, 1, 1, 256, 0, s, a);
+    return launch(KName("rein_mmq_", fmt_tag(fmt), "_grouped_swiglu_q8"), (unsigned)grid, 1, 1, 256, 0, s, a);
 }
 
 namespace {
-int moe_mv_launch(const char* who, const std::string& kernel, unsigned rows_per_block, int fmt, const void* slab0,
+int moe_mv_launch(const char* who, const KName& kernel, unsigned rows_per_block, int fmt, const void* slab0,
                   const void* slab1, const int32_t* ids, const void* xq, float* y, unsigned in_dim, unsigned out_dim,
                   unsigned bytes_per_expert, unsigned xq_tok_stride, unsigned xq_slot_stride, unsigned n_used,
                   unsigned n_tok, rein_stream_t s)
@@ -1980,7 +2032,7 @@ int rein_moe_expert_matvec(int fmt, const void* slab, const int32_t* ids, const 
     const char* who = "rein_moe_expert_matvec";
     if (!moe_mv_fmt(fmt)) return fail(REIN_E_BAD_FORMAT, std::string(who) + ": formats are Q4_K, Q5_K, Q6_K, Q8_0, Q5_1");
     // 4 wavefronts x 2 rows per 256-thread workgroup (the reference's grid, qwen35.rs:3086)
-    return moe_mv_launch(who, std::string("moe_matvec_") + fmt_tag(fmt) + "_repacked_f32", 8, fmt, slab, nullptr, ids, xq,
+    return moe_mv_launch(who, KName("moe_matvec_", fmt_tag(fmt), "_repacked_f32"), 8, fmt, slab, nullptr, ids, xq,
                          y, in_dim, out_dim, bytes_per_expert, xq_tok_stride, xq_slot_stride, n_used, n_tok, s);
 }
 
@@ -1993,9 +2045,9 @@ int rein_moe_down(int fmt, const void* slab, const int32_t* ids, const void* xq,
     if (in_dim / 32 > 32)       // long contraction: the full-wavefront mapping wastes nothing
         return rein_moe_expert_matvec(fmt, slab, ids, xq, y, in_dim, out_dim, bytes_per_expert, xq_tok_stride,
                                       xq_slot_stride, n_used, n_tok, s);
-    const std::string kernel = fmt == REIN_TYPE_Q4_K   ? "rein_moe_matvec_q4k_down_f32"
-                               : fmt == REIN_TYPE_Q8_0 ? "moe_matvec_q8_0_repacked_down_f32"
-                                                       : std::string("moe_matvec_") + fmt_tag(fmt) + "_down_f32";
+    const KName kernel = fmt == REIN_TYPE_Q4_K   ? KName("rein_moe_matvec_q4k_down_f32")
+                         : fmt == REIN_TYPE_Q8_0 ? KName("moe_matvec_q8_0_repacked_down_f32")
+                                                 : KName("moe_matvec_", fmt_tag(fmt), "_down_f32");
     // 8 half-wavefronts x 2 rows per workgroup
     return moe_mv_launch(who, kernel, 16, fmt, slab, nullptr, ids, xq, y, in_dim, out_dim, bytes_per_expert,
                          xq_tok_stride, xq_slot_stride, n_used, n_tok, s);
@@ -2039,7 +2091,7 @@ int rein_moe_gate_up_swiglu_q8(int fmt, const void* gate_slab, const void* up_sl
     // 4 / 8 / 16 tokens 32.9 / 51.9 / 88.4 us per FFN against 34.1 / 55.9 / 99.3, one token 16.9 against 15.9
     const unsigned gu_rows = opt_u(O_MOE_GU_ROWS, 0);
     const bool r4 = gu_rows == 4 || (gu_rows != 2 && (unsigned long long)(out_dim / 32) * n_used * n_tok >= 2ull * kCUs);
-    return launch(std::string("rein_moe_gate_up_swiglu_q8_") + fmt_tag(fmt) + (r4 ? "_r4" : ""), out_dim / 32, n_used, n_tok, r4 ? 512 : 1024, 0, s, a);
+    return launch(KName("rein_moe_gate_up_swiglu_q8_", fmt_tag(fmt), r4 ? "_r4" : ""), out_dim / 32, n_used, n_tok, r4 ? 512 : 1024, 0, s, a);
 }
 
 int rein_moe_down_combine(int fmt, const void* slab, const int32_t* ids, const float* weights, const float* down_exps_s,
@@ -2074,7 +2126,7 @@ int rein_moe_down_combine(int fmt, const void* slab, const int32_t* ids, const f
     }
     void* a[] = {(void*)&slab, (void*)&ids, (void*)&weights, (void*)&down_exps_s, (void*)&xq, (void*)&out, (void*)&in_dim,
                  (void*)&out_dim, (void*)&bytes_per_expert, (void*)&xq_tok_stride, (void*)&xq_slot_stride, (void*)&n_used};
-    return launch(std::string("rein_moe_down_combine_") + fmt_tag(fmt) + (half ? "_h" : "") + (rows == 2 ? "" : rows == 4 ? "_r4" : "_r8"),
+    return launch(KName("rein_moe_down_combine_", fmt_tag(fmt), half ? "_h" : "", rows == 2 ? "" : rows == 4 ? "_r4" : "_r8"),
                   (out_dim + rows - 1) / rows, 1, n_tok, threads, 0, s, a);
 }
 
@@ -2198,7 +2250,7 @@ int rein_moe_ffn(const rein_moe_shape* shp, const float* x, const float* logits,
                          (void*)&sh.hidden, (void*)&sh.expert_ff, (void*)&bpe, (void*)&sh.n_expert, (void*)&sh.n_used};
             const unsigned gu_rows = opt_u(O_MOE_GU_ROWS, 0);
             const bool r4 = gu_rows == 4 || (gu_rows != 2 && (unsigned long long)(sh.expert_ff / 32) * sh.n_used * sh.n_tok >= 2ull * kCUs);
-            if (int rc = launch(std::string("rein_moe_route_gate_up_swiglu_q8_") + fmt_tag(sh.gate_up_fmt) + (r4 ? "_r4" : ""), sh.expert_ff / 32,
+            if (int rc = launch(KName("rein_moe_route_gate_up_swiglu_q8_", fmt_tag(sh.gate_up_fmt), r4 ? "_r4" : ""), sh.expert_ff / 32,
                                 sh.n_used, sh.n_tok, r4 ? 512 : 1024, ns_h * 40u, s, a)) return rc;
         } else {
             if (wave) {

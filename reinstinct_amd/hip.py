@@ -42,6 +42,11 @@ class DeviceBuf:
         check(lib.rein_malloc(C.byref(p), max(self.nbytes, 1)))
         self.ptr = p.value
 
+    @property
+    def _as_parameter_(self):
+        """what ctypes passes for a pointer argument"""
+        return self.ptr
+
     @classmethod
     def from_host(cls, arr):
         arr = np.ascontiguousarray(arr)
@@ -81,7 +86,7 @@ class Stream:
     def __init__(self):
         p = C.c_void_p(0)
         check(lib.rein_stream_create(C.byref(p)))
-        self.raw = p.value
+        self.raw = self._as_parameter_ = p.value
 
     def synchronize(self):
         check(lib.rein_stream_synchronize(self.raw))
