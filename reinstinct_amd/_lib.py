@@ -154,14 +154,19 @@ SIGNATURES = {
 _lib = None
 
 
+def need_built(name):
+    path = os.path.join(_HERE, name)
+    if not os.path.exists(path):
+        raise ReinError(-1, f"{path} is not built: run `make -C reinstinct_amd/csrc` "
+                            "(or __graft_entry__.build()); there is no fallback path")
+
+
 def load():
     """dlopen librein.so and type every entry point (no GPU needed for this)."""
     global _lib
     if _lib is not None:
         return _lib
-    if not os.path.exists(SO_PATH):
-        raise ReinError(-1, f"{SO_PATH} is not built: run `make -C reinstinct_amd/csrc` "
-                            "(or __graft_entry__.build()); there is no fallback path")
+    need_built("librein.so")
     handle = C.CDLL(SO_PATH)
     for name, (res, args) in SIGNATURES.items():
         fn = getattr(handle, name)
