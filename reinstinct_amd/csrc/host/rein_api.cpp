@@ -1125,9 +1125,19 @@ int rein_matvec_ondisk_xq8(int fmt, const void* w_blocks, const void* xq, float*
     if (int rc = check_ptr(who, w_blocks, 16, "w_blocks")) return rc;
     if (int rc = check_ptr(who, xq, 8, "xq")) return rc;
     if (int rc = check_ptr(who, y, 4, "y")) return rc;
+    void* a[] = {(void*)&w_blocks, (void*)&xq, (void*)&y, (void*)&in_dim, (void*)&out_dim};
+    // rein_mvd_<fmt> pairs sub-blocks and keeps the activations in LDS: every shape but a Q8_0 row of an odd number of blocks
+    // (which starts at 2-byte alignment) and a contraction whose activations do not fit, about 100 000 values.  Grids: the comment at
+    // the kernel.
+    const unsigned n_sub = in_dim / 32, n_pad = (n_sub + 7) & ~7u;
+    const unsigned pad = fmt == REIN_TYPE_Q6_K ? 32 : 16, words = fmt == REIN_TYPE_Q6_K ? 3 : fmt == REIN_TYPE_Q8_0 ? 1 : 2;
+    const size_t lds = (size_t)n_pad / 8 * (256 + pad) + (size_t)n_pad * 4 * words;
+    if (n_sub % 2 == 0 && lds <= kLdsPerCu) {
+        const unsigned most = fmt == REIN_TYPE_Q6_K || fmt == REIN_TYPE_Q8_0 ? 2 * kCUs : 4 * kCUs;
+        return launch(KName("rein_mvd_", fmt_tag(fmt)), std::min((out_dim + 15) / 16, most), 1, 1, 256, (unsigned)lds, s, a);
+    }
     // 4 wavefronts x 2 rows per workgroup; the kernel strides, so cap the grid at a few waves per SIMD
     const unsigned gx = std::min((out_dim + 7) / 8, kCUs * 16);
-    void* a[] = {(void*)&w_blocks, (void*)&xq, (void*)&y, (void*)&in_dim, (void*)&out_dim};
     return launch(name, gx, 1, 1, 256, 0, s, a);
 }
 

@@ -9,6 +9,9 @@
 //     tiny out_dim (kernels/matvec_q8_0_repacked.cpp:117-176): partial sums go to
 //     y[blockIdx.y][out_dim], the consumer adds them.
 //
+// The library launches rein_mvd_<fmt> (matvec_disk.hip) instead of the dp4a kernels wherever a row is an even number of
+// sub-blocks whose activations fit in LDS; these keep the reference's geometry and take the rest.
+//
 // Lane l of a wavefront walks sub-blocks l, l+64, ... of R rows exactly as the
 // repacked matvec does; only the address arithmetic differs (a sub-block's bytes sit
 // inside its 256-weight block), and the per-sub-block math is Fmt<FMT>::term.  Any
