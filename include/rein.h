@@ -106,9 +106,10 @@ int rein_is_loaded(void);
  * REIN_MMQ6_SK_GRID, REIN_MMQ6_SK_SPLIT (Q4_K fp6 launch: 0 off, first row count, token groups
  * of four / two tiles per row block, split-tail 0 off / 2 forced, its grid and ranges),
  * REIN_MMQ16 (1: the fp16 formulation where the code object holds it), REIN_TOPK_WAVE,
- * REIN_MOE_SORT_SPLIT, REIN_MOE_CHAIN, REIN_MOE_FUSED, REIN_MOE_GU_ROWS, REIN_MOE_DC_ROWS (MoE
- * glue: 0 = the workgroup router, 1 = the four-launch sort, 0 = no decode chain for few
- * tokens, 0 = unfused gate/up, rows per workgroup of the two decode launches).
+ * REIN_MOE_SORT_SPLIT, REIN_MOE_CHAIN, REIN_MOE_FUSED, REIN_MOE_FEW, REIN_MOE_GU_ROWS, REIN_MOE_DC_ROWS
+ * (MoE glue: 0 = the workgroup router, 1 = the four-launch sort, 0 = no decode chain for few
+ * tokens, 0 = unfused gate/up, 0 never / 1 wherever the shape allows the launches that read every touched
+ * expert once, rows per workgroup of the two decode launches).
  * Unknown name: REIN_E_NOT_FOUND; a value that is not an unsigned 32-bit decimal:
  * REIN_E_BAD_SHAPE. */
 int rein_set_option(const char *name, const char *value);   /* value NULL or "": unset */
@@ -548,11 +549,12 @@ size_t rein_moe_workspace_bytes(const rein_moe_shape *shape);
  * kernels instead (top-k -> quantize -> rein_moe_gate_up_swiglu_q8 -> rein_moe_down_combine, the
  * launches of qwen35.rs:3071-3167 fused in pairs): no sort, one expert read per entry; for one
  * and two tokens the gate / up launch also routes and quantizes, so the FFN is two launches.
- * The two forms add a token's eight expert rows, and the terms inside each row, in different
- * orders (slot order in the decode form, expert-sorted tiles in the pipeline): the fp32 bits
- * of a token's output row therefore depend on how many tokens share the call (25 against 26
- * at 128 experts top-8), within the path's 1e-3 / 1e-4 tolerance of either order.  The option
- * REIN_MOE_CHAIN = 0 keeps every call on the pipeline. */
+ * From about 0.8 to 5.5 entries per expert a third form reads every expert that the router touched once
+ * for all of its tokens (four launches: router + quantizer, gate + up, down, combine); it needs hidden and
+ * expert_ff to be multiples of 64.
+ * The forms add the terms inside an expert's row in different orders: the fp32 bits of a token's output row
+ * therefore depend on how many tokens share the call, within the path's 1e-3 / 1e-4 tolerance of any
+ * order.  The option REIN_MOE_CHAIN = 0 (with REIN_MOE_FEW unset) keeps every call on the pipeline. */
 int rein_moe_ffn(const rein_moe_shape *shape, const float *x, const float *logits,
                  const void *gate_exps, const void *up_exps, const void *down_exps,
                  const float *down_exps_s, void *workspace, float *out, rein_stream_t s);

@@ -192,8 +192,8 @@ int check_ptr(const char* who, const void* p, size_t align, const char* what)
 // rein_set_option changes an entry, so the launch an entry point chooses depends on its arguments
 // and on this table alone.  Entries are single atomic words: setting one while another thread
 // launches is safe, the launch sees the old or the new value.
-enum Opt : int { O_MV_ROWS, O_MV_WPB, O_MV_LDS, O_QUAD_LDS, O_QUAD_SLICES, O_QUAD_DEPTH, O_QUAD_WIDE32, O_SKINNY_KS, O_SKINNY_FROM, O_QUAD_FROM, O_GROUPED_STRIDED, O_MMQ_TM, O_MMQ_N64, O_MMQ6, O_MMQ6_N4, O_MMQ6_N2, O_MMQ6_SK_GRID, O_MMQ6_SK_SPLIT, O_MMQ6_SK, O_MMQ6_FROM, O_MMQ_SK, O_MMQ_SK_GRID, O_MMQ_SK_SPLIT, O_MMQ_SK_TM, O_MMQ16, O_TOPK_WAVE, O_MOE_SORT_SPLIT, O_MOE_GU_ROWS, O_MOE_DC_ROWS, O_MOE_CHAIN, O_MOE_FUSED, O_COUNT };
-const char* const kOptNames[O_COUNT] = {"REIN_MV_ROWS", "REIN_MV_WPB", "REIN_MV_LDS", "REIN_QUAD_LDS", "REIN_QUAD_SLICES", "REIN_QUAD_DEPTH", "REIN_QUAD_WIDE32", "REIN_SKINNY_KS", "REIN_SKINNY_FROM", "REIN_QUAD_FROM", "REIN_GROUPED_STRIDED", "REIN_MMQ_TM", "REIN_MMQ_N64", "REIN_MMQ6", "REIN_MMQ6_N4", "REIN_MMQ6_N2", "REIN_MMQ6_SK_GRID", "REIN_MMQ6_SK_SPLIT", "REIN_MMQ6_SK", "REIN_MMQ6_FROM", "REIN_MMQ_SK", "REIN_MMQ_SK_GRID", "REIN_MMQ_SK_SPLIT", "REIN_MMQ_SK_TM", "REIN_MMQ16", "REIN_TOPK_WAVE", "REIN_MOE_SORT_SPLIT", "REIN_MOE_GU_ROWS", "REIN_MOE_DC_ROWS", "REIN_MOE_CHAIN", "REIN_MOE_FUSED"};
+enum Opt : int { O_MV_ROWS, O_MV_WPB, O_MV_LDS, O_QUAD_LDS, O_QUAD_SLICES, O_QUAD_DEPTH, O_QUAD_WIDE32, O_SKINNY_KS, O_SKINNY_FROM, O_QUAD_FROM, O_GROUPED_STRIDED, O_MMQ_TM, O_MMQ_N64, O_MMQ6, O_MMQ6_N4, O_MMQ6_N2, O_MMQ6_SK_GRID, O_MMQ6_SK_SPLIT, O_MMQ6_SK, O_MMQ6_FROM, O_MMQ_SK, O_MMQ_SK_GRID, O_MMQ_SK_SPLIT, O_MMQ_SK_TM, O_MMQ16, O_TOPK_WAVE, O_MOE_SORT_SPLIT, O_MOE_GU_ROWS, O_MOE_DC_ROWS, O_MOE_CHAIN, O_MOE_FUSED, O_MOE_FEW, O_COUNT };
+const char* const kOptNames[O_COUNT] = {"REIN_MV_ROWS", "REIN_MV_WPB", "REIN_MV_LDS", "REIN_QUAD_LDS", "REIN_QUAD_SLICES", "REIN_QUAD_DEPTH", "REIN_QUAD_WIDE32", "REIN_SKINNY_KS", "REIN_SKINNY_FROM", "REIN_QUAD_FROM", "REIN_GROUPED_STRIDED", "REIN_MMQ_TM", "REIN_MMQ_N64", "REIN_MMQ6", "REIN_MMQ6_N4", "REIN_MMQ6_N2", "REIN_MMQ6_SK_GRID", "REIN_MMQ6_SK_SPLIT", "REIN_MMQ6_SK", "REIN_MMQ6_FROM", "REIN_MMQ_SK", "REIN_MMQ_SK_GRID", "REIN_MMQ_SK_SPLIT", "REIN_MMQ_SK_TM", "REIN_MMQ16", "REIN_TOPK_WAVE", "REIN_MOE_SORT_SPLIT", "REIN_MOE_GU_ROWS", "REIN_MOE_DC_ROWS", "REIN_MOE_CHAIN", "REIN_MOE_FUSED", "REIN_MOE_FEW"};
 constexpr uint64_t kOptSet = 1ull << 63;
 std::atomic<uint64_t> g_opts[O_COUNT];          // zero = unset
 std::once_flag g_opts_env_once;
@@ -2195,6 +2195,50 @@ MoeWs moe_ws(const rein_moe_shape& sh)
 }
 }  // namespace
 
+namespace {
+// Lanes to a row of rein_moe_few_* (kernels/moe_few.hip): 16, 8 or 4, the least of trips x lanes (idle lanes count) times what
+// the narrower groups lose to their shorter runs of bytes.  gate + up of 2048 -> 768 (no idle lanes at any width), 48
+// tokens: 52.5 / 56.5 / 70.7 us; down 768 -> 2048 (a quarter of 16 or 8 lanes idle): 54.1 / 52.3 / 43.4.
+unsigned moe_few_lanes(unsigned in_dim, bool two_slabs)
+{
+    const unsigned n_unit = in_dim / 64;
+    unsigned best = 16;
+    double least = 1e30;
+    for (unsigned g : {16u, 8u, 4u}) {
+        const double cost = (n_unit + g - 1) / g * g * (g == 16 ? 1.0 : g == 8 ? (two_slabs ? 1.08 : 1.0) : (two_slabs ? 1.35 : 1.07));
+        if (cost < least) { least = cost; best = g; }
+    }
+    return best;
+}
+unsigned moe_few_lds(int fmt, unsigned in_dim, unsigned lanes)
+{
+    return 8 * (fmt == REIN_TYPE_Q6_K ? 96 : 80) * ((in_dim / 64 + lanes - 1) / lanes * lanes);
+}
+// their shapes: contractions of whole pairs of sub-blocks, eight entries of each in LDS beside the kernel's own arrays, at most
+// one entry of an expert per token and 1024 of those
+bool moe_few_fits(const rein_moe_shape& sh)
+{
+    return sh.hidden % 64 == 0 && sh.expert_ff % 64 == 0 && sh.n_tok <= 1024 && (unsigned long long)sh.n_tok * sh.n_used <= 65535ull &&
+           moe_few_lds(REIN_TYPE_Q6_K, std::max(sh.hidden, sh.expert_ff), 16) <= 128u * 1024u;
+}
+// Where they pay, from eight expert shapes x 4 .. 192 tokens against the decode launches and the pipeline.  Below: the decode launches read
+// an expert again for every entry, which costs nothing while the entries meet different experts, and are one launch fewer -- from
+// 0.8 entries per expert (Q8_0, whose decode launch runs at 5.6 TB/s, 0.95), or once 160 MB are read twice (us, decode / these: 128
+// experts top-8, 2048 x 768, 12 / 16 / 24 tokens 68 / 71, 87 / 77, 122 / 88; 256 top-6, 1280 x 1280, 16 / 64 tokens 107 / 88, 393 / 160).
+// Above: every further entry costs its dots, while a 32-token tile costs the same until it is full -- up to 5.5 entries per expert
+// (48 / 64 / 96 / 128 tokens of the first shape: pipeline 149-154, these 106 / 121 / 150 / 180), 4 where the experts are small and the tiles
+// few (64 top-6, 1792 x 512, 32 / 48 tokens 60 / 51, 61 / 64).
+bool moe_few_pays(const rein_moe_shape& sh)
+{
+    const double entries = (double)sh.n_tok * sh.n_used, per_expert = entries / sh.n_expert;
+    const double bytes = 2.0 * rein_repacked_len(sh.gate_up_fmt, sh.hidden, sh.expert_ff) + (double)rein_repacked_len(sh.down_fmt, sh.expert_ff, sh.hidden);
+    if (per_expert > (bytes * sh.n_expert < 134e6 ? 4.0 : 5.5)) return false;
+    if (per_expert >= (sh.gate_up_fmt == REIN_TYPE_Q8_0 ? 0.95 : 0.8)) return true;
+    const double touched = sh.n_expert * (1.0 - std::pow(1.0 - (double)sh.n_used / sh.n_expert, (double)sh.n_tok));
+    return (entries - touched) * bytes >= 160e6;
+}
+}  // namespace
+
 size_t rein_moe_workspace_bytes(const rein_moe_shape* sh)
 {
     if (!sh) return 0;
@@ -2245,13 +2289,43 @@ int rein_moe_ffn(const rein_moe_shape* shp, const float* x, const float* logits,
     // mostly empty tile pays its full matrix work -- and are ahead up to 1.6 entries per expert: 128 experts top-8
     // at 1 / 4 / 16 / 24 tokens 16 / 33 / 89 / 125 us against 48 / 61 / 126 / 141 for the pipeline below, at 28
     // tokens 141 against 143, at 32 tokens 160 against 145.  Same integer dots, fp32 sums in the decode kernels' order.
+    const bool wave = sh.n_expert <= 256 && sh.n_used <= 64 && sh.n_used <= sh.n_expert && opt_u(O_TOPK_WAVE, 1) != 0;
+    const auto route_quantize = [&]() -> int {       // router and quantizer as one small launch
+        int n_e = (int)sh.n_expert, n_u = (int)sh.n_used, n_t = (int)sh.n_tok;
+        void* xq = base + w.xq_in;
+        unsigned q_per_tok = (sh.hidden + 511) / 512;
+        void* a[] = {(void*)&logits, (void*)&n_e, (void*)&n_u, (void*)&ids, (void*)&weights, (void*)&n_t,
+                     (void*)&x, (void*)&xq, (void*)&sh.hidden, (void*)&q_per_tok};
+        return launch("rein_moe_route_quantize", (sh.n_tok + 3) / 4 + sh.n_tok * q_per_tok, 1, 1, 256, 0, s, a);
+    };
+    // A few tokens per expert: every touched expert read once for all of them (kernels/moe_few.hip), four launches.  (An option
+    // that pins one of the other forms keeps it.)
+    const bool few = opt_is_set(O_MOE_FEW) ? opt_u(O_MOE_FEW, 0) != 0
+                                           : !opt_is_set(O_MOE_CHAIN) && !opt_is_set(O_MOE_FUSED) && !opt_is_set(O_GROUPED_STRIDED) && moe_few_pays(sh);
+    if (few && wave && moe_few_fits(sh) && ((uintptr_t)out & 15) == 0) {
+        const unsigned bpe_g = (unsigned)bpe_gu, bpe_d = (unsigned)bpe_dn;
+        void* xq = base + w.xq_in;
+        void* h = base + w.xq_exp;
+        void* rows = base + w.g_out;
+        if (int rc = route_quantize()) return rc;
+        void* a[] = {(void*)&gate_exps, (void*)&up_exps, (void*)&ids, (void*)&xq, (void*)&h, (void*)&bpe_g, (void*)&sh.hidden,
+                     (void*)&sh.expert_ff, (void*)&sh.n_used, (void*)&ne};
+        const unsigned g = moe_few_lanes(sh.hidden, true), gd = moe_few_lanes(sh.expert_ff, false);
+        if (int rc = launch(KName("rein_moe_few_gate_up_", fmt_tag(sh.gate_up_fmt), "_g", g), (sh.expert_ff + 63) / 64, sh.n_expert, 1, 256,
+                            moe_few_lds(sh.gate_up_fmt, sh.hidden, g), s, a)) return rc;
+        void* b[] = {(void*)&down_exps, (void*)&ids, (void*)&h, (void*)&rows, (void*)&bpe_d, (void*)&sh.expert_ff, (void*)&sh.hidden, (void*)&ne};
+        if (int rc = launch(KName("rein_moe_few_down_", fmt_tag(sh.down_fmt), "_g", gd), (sh.hidden + 127) / 128, sh.n_expert, 1, 128,
+                            moe_few_lds(sh.down_fmt, sh.expert_ff, gd), s, b)) return rc;
+        void* c[] = {(void*)&rows, (void*)&ids, (void*)&weights, (void*)&down_exps_s, (void*)&out, (void*)&sh.hidden, (void*)&sh.n_used,
+                     (void*)&sh.n_expert};
+        return launch("rein_moe_combine_rows4_f32", (sh.hidden / 4 + 127) / 128, sh.n_tok, 1, 128, 0, s, c);
+    }
     const bool chain = 5ull * ne <= 8ull * sh.n_expert && sh.expert_ff % 32 == 0 && opt_u(O_MOE_CHAIN, 1) != 0;
     if (chain) {
         const unsigned ns_h = sh.hidden / 32, ns_f = sh.expert_ff / 32;
         // Where the one-wavefront router applies it shares a launch: for one or two tokens the gate / up launch
         // routes and quantizes its token itself (every workgroup again: 15.9 / 23.8 us against 17.3 / 25.4), beyond
         // that router and quantizer run as one small launch in front (16 tokens: 105 us against 111)
-        const bool wave = sh.n_expert <= 256 && sh.n_used <= 64 && sh.n_used <= sh.n_expert && opt_u(O_TOPK_WAVE, 1) != 0;
         const bool routed = wave && sh.n_tok <= 2 && ns_h * 40u <= 48u * 1024u;
         if (routed) {
             void* xq_exp = base + w.xq_exp;
@@ -2264,12 +2338,7 @@ int rein_moe_ffn(const rein_moe_shape* shp, const float* x, const float* logits,
                                 sh.n_used, sh.n_tok, r4 ? 512 : 1024, ns_h * 40u, s, a)) return rc;
         } else {
             if (wave) {
-                int n_e = (int)sh.n_expert, n_u = (int)sh.n_used, n_t = (int)sh.n_tok;
-                void* xq = base + w.xq_in;
-                unsigned q_per_tok = (sh.hidden + 511) / 512;
-                void* a[] = {(void*)&logits, (void*)&n_e, (void*)&n_u, (void*)&ids, (void*)&weights, (void*)&n_t,
-                             (void*)&x, (void*)&xq, (void*)&sh.hidden, (void*)&q_per_tok};
-                if (int rc = launch("rein_moe_route_quantize", (sh.n_tok + 3) / 4 + sh.n_tok * q_per_tok, 1, 1, 256, 0, s, a)) return rc;
+                if (int rc = route_quantize()) return rc;
             } else {
                 if (int rc = rein_moe_topk(logits, sh.n_tok, sh.n_expert, sh.n_used, ids, weights, s)) return rc;
                 if (int rc = rein_quantize_q8(x, base + w.xq_in, sh.hidden, sh.n_tok, s)) return rc;

@@ -81,3 +81,29 @@ void rein_moe_combine_sorted4_f32(const float* __restrict__ sorted, const int* _
     }
 }
 
+// The same over expert outputs in routing order (row tok * n_used + j), for launches that leave out the rows of ids beyond n_expert
+extern "C" __global__ __launch_bounds__(256)
+void rein_moe_combine_rows4_f32(const float* __restrict__ rows, const int* __restrict__ ids, const float* __restrict__ weights,
+                                const float* __restrict__ down_exps_s, float* __restrict__ out, unsigned int hidden,
+                                unsigned int n_used, unsigned int n_expert)
+{
+#pragma clang fp contract(off)
+    const size_t tok = blockIdx.y;
+    rows    += tok * n_used * hidden;
+    ids     += tok * n_used;
+    weights += tok * n_used;
+    out     += tok * hidden;
+    const unsigned h4 = hidden >> 2;
+    for (unsigned i = blockIdx.x * blockDim.x + threadIdx.x; i < h4; i += gridDim.x * blockDim.x) {
+        float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll 8
+        for (unsigned j = 0; j < n_used; j++) {
+            const unsigned e = (unsigned)ids[j];
+            if (e >= n_expert) continue;
+            const float s = weights[j] * down_exps_s[e];
+            const float4 v = *reinterpret_cast<const float4*>(rows + (size_t)j * hidden + 4u * i);
+            acc.x += s * v.x; acc.y += s * v.y; acc.z += s * v.z; acc.w += s * v.w;
+        }
+        *reinterpret_cast<float4*>(out + 4u * i) = acc;
+    }
+}
