@@ -382,6 +382,26 @@ bool small_for_matrix_cores(int fmt, unsigned in_dim, unsigned out_dim, unsigned
     return out_dim <= 2048 || (!quad_family && weights <= (1ull << 24) && out_dim < 8192);
 }
 
+// Which build of a few-row kernel a launch takes, by how it loads its `bytes` of weights (rein_formats.h): "" all planes
+// nontemporal, "_m" the 16- and 8-byte planes only, "_p" plain.  Where the lines lie (each kernel built all three ways, 17
+// shapes x Q4_K, Q5_K, Q6_K, Q8_0, matrices rotating through 600 MB; against all nontemporal):
+//   below 6.5 MB   plain 4-16 % faster at 1-4 rows (5120 -> 1024 Q4_K 3.75 -> 3.30 us, Q6_K 4.25 -> 3.70), level to +7 % at more
+//   5 rows up      mix level to +8 % at every larger size
+//   3-4 rows       mix from 14 MB: +1-8 % up to 28 MB, +2-17 % beyond (5120 -> 34816 Q4_K 24.8 -> 23.0, Q5_K 30.0 -> 26.7);
+//                  under 14 MB it goes either way (6144 -> 2048 Q8_0 -5 %, 2560 -> 6144 Q4_K +7 %)
+//   1-2 rows       mix from 28 MB: +1-9 % (5120 -> 34816 Q4_K 19.5 -> 18.5, 8192 -> 8192 Q5_K 11.9 -> 10.9); from 6.5 to
+//                  28 MB it costs 1-6 % and plain 2-8 %
+//   Q8_0 with padded rows (a power of two of sub-blocks: 16-byte-aligned rows share their first and last lines with the
+//   neighbours in both wide planes), 3 rows up, from 25 MB: plain (4096 -> 14336 17.2 -> 15.0, mix 16.3; 4096 -> 6144 +11 %
+//   against mix +3 %)
+const char* load_tag(int fmt, unsigned in_dim, unsigned long long bytes, unsigned n_rows)
+{
+    const unsigned long long kib = bytes >> 10;
+    if (kib < 6500) return "_p";
+    if (n_rows >= 3 && fmt == REIN_TYPE_Q8_0 && kib >= 25000 && rein_repacked_n_sub_padded(in_dim) != in_dim / 32) return "_p";
+    return kib >= (n_rows >= 5 ? 6500u : n_rows >= 3 ? 14000u : 28000u) ? "_m" : "";
+}
+
 // LDS-staged dot4 matvec (rein_mvl_*, kernels/matvec_lds.h), 2..4 activation rows: the rows of a
 // workgroup's activations live in LDS, B x (in_dim / 32) x 40 bytes of it.
 constexpr size_t kLdsPerCu = 160u * 1024u;
@@ -503,7 +523,7 @@ int launch_matvec_lds(int fmt, const void* w, const void* xq, float* y, unsigned
     unsigned r, wpb, grid;
     mvl_geometry(fmt, in_dim, out_dim, n_rows, &r, &wpb, &grid);
     const unsigned b = n_rows <= 2 ? 2 : 4;
-    const KName name("rein_mvl_", fmt_tag(fmt), "_r", r, "_b", b);
+    const KName name("rein_mvl_", fmt_tag(fmt), "_r", r, "_b", b, load_tag(fmt, in_dim, rein_repacked_len(fmt, in_dim, out_dim), n_rows));
     void* args[] = {(void*)&w, (void*)&xq, (void*)&y, (void*)&in_dim, (void*)&out_dim, (void*)&n_rows};
     return launch(name, grid, 1, 1, wpb * 64, (unsigned)mvl_lds_bytes(in_dim, n_rows), s, args);
 }
@@ -655,7 +675,8 @@ int launch_quad_lds(int fmt, const void* w, const void* xq, float* y, unsigned i
 {
     const QuadLdsGeometry g = mvql_geometry(fmt, in_dim, out_dim, n_rows);
     const KName name("rein_mvql_", fmt_tag(fmt), n_rows <= 4 ? "_t4" : n_rows <= 8 ? "_t8" : n_rows <= 16 ? "_t16" :
-                                                                         mvql_wide32(fmt) ? "_t32w" : "_t32");
+                                                                         mvql_wide32(fmt) ? "_t32w" : "_t32",
+                     n_rows <= 16 ? load_tag(fmt, in_dim, rein_repacked_len(fmt, in_dim, out_dim), n_rows) : "");
     // Trips of weights in flight per wavefront where wavefronts stride over row groups or own a whole one (no slices,
     // no phases): two for the formats with little arithmetic per sub-block at 3-4 rows -- two register sets taking
     // turns -- (us, 5120 -> 34816 / 5120 -> 17408 / 3584 -> 18944 at 4 rows, one -> two: Q4_K 28.3 -> 26.0, 18.8 -> 17.3,
@@ -692,7 +713,7 @@ MvFamily matvec_family(int fmt, unsigned in_dim, unsigned out_dim, unsigned n_ro
     return MvFamily::Dot4;
 }
 
-// The kernel a few-row product launches: 1..8 rows as rein_matvec_batched_xq8 dispatches them, 9..32 rows the few-row
+// The kernel a few-row product launches (without the suffix of load_tag): 1..8 rows as rein_matvec_batched_xq8 dispatches them, 9..32 rows the few-row
 // kernels behind rein_mmq_xq8 ("" where that entry point launches token tiles).
 std::string matvec_kernel_name(int fmt, unsigned in_dim, unsigned out_dim, unsigned n_rows)
 {
@@ -743,7 +764,7 @@ int launch_matvec(const char* who, int fmt, const void* w, const void* xq, float
     const unsigned groups = (out_dim + r - 1) / r;
     const unsigned wpb = pick_wpb(fmt, groups, b);
     const unsigned grid = (groups + wpb - 1) / wpb;
-    const KName name("rein_mv_", fmt_tag(fmt), "_r", r, "_b", b);
+    const KName name("rein_mv_", fmt_tag(fmt), "_r", r, "_b", b, b <= 4 ? load_tag(fmt, in_dim, rein_repacked_len(fmt, in_dim, out_dim), n_rows) : "");
     void* args[] = {(void*)&w, (void*)&xq, (void*)&y, (void*)&in_dim, (void*)&out_dim, (void*)&n_rows};
     return launch(name, grid, 1, 1, wpb * 64, 0, s, args);
 }
@@ -1055,7 +1076,7 @@ int rein_matvec_multi_xq8(unsigned n_mat, const int* fmts, const void* const* ws
     if (n_rows > 4) return fail(REIN_E_TOO_LARGE, std::string(who) + ": at most 4 activation rows");
     if (!fmts || !ws || !ys || !out_dims) return fail(REIN_E_BAD_POINTER, std::string(who) + ": a NULL table");
     if (int rc = check_ptr(who, xq, 8, "xq")) return rc;
-    unsigned long long total = 0;
+    unsigned long long total = 0, bytes = 0;
     unsigned widest = 0;
     for (unsigned i = 0; i < n_mat; i++) {
         if (int rc = check_shape(who, fmts[i], in_dim, out_dims[i], n_rows)) return rc;
@@ -1063,6 +1084,7 @@ int rein_matvec_multi_xq8(unsigned n_mat, const int* fmts, const void* const* ws
         if (int rc = check_ptr(who, ws[i], 16, "w")) return rc;
         if (int rc = check_ptr(who, ys[i], 4, "y")) return rc;
         total += out_dims[i];
+        bytes += rein_repacked_len(fmts[i], in_dim, out_dims[i]);
         if (out_dims[i] > out_dims[widest]) widest = i;
     }
     if (total > 0x3FFFFFFFull) return fail(REIN_E_TOO_LARGE, std::string(who) + ": too many rows for one launch");
@@ -1099,7 +1121,7 @@ int rein_matvec_multi_xq8(unsigned n_mat, const int* fmts, const void* const* ws
     for (unsigned i = n_mat; i < kMax; i++) a.m[i] = a.m[n_mat - 1];
     const unsigned wpb = pick_wpb(lead, groups, b);
     void* args[] = {(void*)&a, (void*)&xq, (void*)&in_dim, (void*)&n_mat, (void*)&n_rows};
-    return launch(KName("rein_mv_multi_r", r, "_b", b), (groups + wpb - 1) / wpb, 1, 1, wpb * 64, 0, s, args);
+    return launch(KName("rein_mv_multi_r", r, "_b", b, load_tag(lead, in_dim, bytes, n_rows)), (groups + wpb - 1) / wpb, 1, 1, wpb * 64, 0, s, args);
 }
 
 int rein_matvec_kernel_name(int fmt, unsigned in_dim, unsigned out_dim, unsigned n_rows, char* name, size_t name_len)
@@ -1696,7 +1718,8 @@ int rein_noalloc_prepare(void)
     // (up to 32 rows the entry point launches the few-row kernels: skinny MMQ, both 4x4x4 kernels, and from eight rows
     // down the decode matvecs in every rows-per-wavefront x batch-slot instantiation there is)
     static const char* const few[] = {"rein_mmqs_%s_v1", "rein_mmqs_%s_v2", "rein_mmqs_%s_v4", "rein_mmqs_%s_v8", "rein_mvql_%s_t4", "rein_mvql_%s_t8",
-                                      "rein_mvql_%s_t16", "rein_mvql_%s_t32", "rein_mvql_%s_t32w", "rein_mvq_%s_t4", "rein_mvq_%s_t8"};
+                                      "rein_mvql_%s_t16", "rein_mvql_%s_t4_m", "rein_mvql_%s_t8_m", "rein_mvql_%s_t16_m", "rein_mvql_%s_t4_p",
+                                      "rein_mvql_%s_t8_p", "rein_mvql_%s_t16_p", "rein_mvql_%s_t32", "rein_mvql_%s_t32w", "rein_mvq_%s_t4", "rein_mvq_%s_t8"};
     for (int fmt : fmts) {
         for (const char* form : forms) {
             hipFunction_t f;
@@ -1711,10 +1734,12 @@ int rein_noalloc_prepare(void)
         for (unsigned r = 1; r <= 4; r *= 2)
             for (unsigned b = 1; b <= 8; b *= 2) {
                 hipFunction_t f;
-                if (r * b <= 16)
-                    if (int rc = get_fn(KName("rein_mv_", fmt_tag(fmt), "_r", r, "_b", b), &f)) return rc;
-                if (b == 2 || b == 4)
-                    if (int rc = get_fn(KName("rein_mvl_", fmt_tag(fmt), "_r", r, "_b", b), &f)) return rc;
+                for (const char* loads : {"", "_m", "_p"}) {
+                    if (r * b <= 16 && (b <= 4 || !*loads))
+                        if (int rc = get_fn(KName("rein_mv_", fmt_tag(fmt), "_r", r, "_b", b, loads), &f)) return rc;
+                    if (b == 2 || b == 4)
+                        if (int rc = get_fn(KName("rein_mvl_", fmt_tag(fmt), "_r", r, "_b", b, loads), &f)) return rc;
+                }
             }
     }
     return 0;

@@ -27,7 +27,7 @@
 
 #include "matvec_repacked.h"
 
-template <int FMT, int R, int B>
+template <int FMT, int R, int B, int POL>
 __device__ __forceinline__ void rein_matvec_lds_body(const uint8_t* __restrict__ w, const BlockQ8* __restrict__ xq,
                                                      float* __restrict__ y, unsigned in_dim, unsigned out_dim,
                                                      unsigned n_rows)
@@ -63,7 +63,7 @@ __device__ __forceinline__ void rein_matvec_lds_body(const uint8_t* __restrict__
         const unsigned row0 = min(p.g, n_groups - 1) * R;
         const unsigned sb = p.sb0 + lane < n_sub ? p.sb0 + lane : n_sub - 1;
 #pragma unroll
-        for (int rr = 0; rr < R; rr++) r[rr] = fmt.load(min(row0 + rr, rmax), sb);
+        for (int rr = 0; rr < R; rr++) r[rr] = fmt.template load<POL>(min(row0 + rr, rmax), sb);
     };
     Pos p, q;
     p.g = g; p.sb0 = 0u;
@@ -136,9 +136,14 @@ __device__ __forceinline__ void rein_matvec_lds_body(const uint8_t* __restrict__
     }
 }
 
-// name(w, xq[n_rows][n_sub], y[n_rows][out_dim], in_dim, out_dim, n_rows), n_rows <= B
-#define REIN_DEFINE_MATVEC_LDS(name, FMT, R, B)                                                   \
+// name(w, xq[n_rows][n_sub], y[n_rows][out_dim], in_dim, out_dim, n_rows), n_rows <= B; name_m and name_p are the same
+// with the other loads of the weights (rein_formats.h)
+#define REIN_DEFINE_MATVEC_LDS_LD(name, FMT, R, B, POL)                                           \
     extern "C" __global__ __launch_bounds__(1024) void name(REIN_MATVEC_ARGS, unsigned int n_rows) \
     {                                                                                             \
-        rein_matvec_lds_body<FMT, R, B>(w, xq, y, in_dim, out_dim, n_rows);                       \
+        rein_matvec_lds_body<FMT, R, B, POL>(w, xq, y, in_dim, out_dim, n_rows);                  \
     }
+#define REIN_DEFINE_MATVEC_LDS(name, FMT, R, B)                                                   \
+    REIN_DEFINE_MATVEC_LDS_LD(name, FMT, R, B, REIN_LD_STREAM)                                    \
+    REIN_DEFINE_MATVEC_LDS_LD(name##_m, FMT, R, B, REIN_LD_MIX)                                   \
+    REIN_DEFINE_MATVEC_LDS_LD(name##_p, FMT, R, B, REIN_LD_PLAIN)

@@ -26,7 +26,7 @@ struct ReinMultiArgs {
     ReinMultiMat m[REIN_MULTI_MAX];
 };
 
-template <int R, int B>
+template <int R, int B, int POL>
 __device__ __forceinline__ void rein_matvec_multi_body(const ReinMultiArgs& a, const BlockQ8* __restrict__ xq,
                                                        unsigned in_dim, unsigned n_mat, unsigned n_rows)
 {
@@ -47,24 +47,29 @@ __device__ __forceinline__ void rein_matvec_multi_body(const ReinMultiArgs& a, c
     // one row group per wavefront: first = g, and a step that ends the walk after it
     const unsigned step = 0x40000000u;
     switch (fmt) {
-    case REIN_Q4_K:   rein_matvec_span<REIN_Q4_K, R, B>(w, xq, y, in_dim, out_dim, n_rows, g, step); break;
-    case REIN_Q6_K:   rein_matvec_span<REIN_Q6_K, R, B>(w, xq, y, in_dim, out_dim, n_rows, g, step); break;
-    case REIN_Q5_K:   rein_matvec_span<REIN_Q5_K, R, B>(w, xq, y, in_dim, out_dim, n_rows, g, step); break;
-    case REIN_Q8_0:   rein_matvec_span<REIN_Q8_0, R, B>(w, xq, y, in_dim, out_dim, n_rows, g, step); break;
-    case REIN_Q4_0:   rein_matvec_span<REIN_Q4_0, R, B>(w, xq, y, in_dim, out_dim, n_rows, g, step); break;
-    case REIN_IQ4_XS: rein_matvec_span<REIN_IQ4_XS, R, B>(w, xq, y, in_dim, out_dim, n_rows, g, step); break;
-    case REIN_IQ3_S:  rein_matvec_span<REIN_IQ3_S, R, B>(w, xq, y, in_dim, out_dim, n_rows, g, step); break;
+    case REIN_Q4_K:   rein_matvec_span<REIN_Q4_K, R, B, 1, POL>(w, xq, y, in_dim, out_dim, n_rows, g, step); break;
+    case REIN_Q6_K:   rein_matvec_span<REIN_Q6_K, R, B, 1, POL>(w, xq, y, in_dim, out_dim, n_rows, g, step); break;
+    case REIN_Q5_K:   rein_matvec_span<REIN_Q5_K, R, B, 1, POL>(w, xq, y, in_dim, out_dim, n_rows, g, step); break;
+    case REIN_Q8_0:   rein_matvec_span<REIN_Q8_0, R, B, 1, POL>(w, xq, y, in_dim, out_dim, n_rows, g, step); break;
+    case REIN_Q4_0:   rein_matvec_span<REIN_Q4_0, R, B, 1, POL>(w, xq, y, in_dim, out_dim, n_rows, g, step); break;
+    case REIN_IQ4_XS: rein_matvec_span<REIN_IQ4_XS, R, B, 1, POL>(w, xq, y, in_dim, out_dim, n_rows, g, step); break;
+    case REIN_IQ3_S:  rein_matvec_span<REIN_IQ3_S, R, B, 1, POL>(w, xq, y, in_dim, out_dim, n_rows, g, step); break;
     default: break;
     }
 }
 
 // name(table, xq[n_rows][in_dim / 32], in_dim, n_mat, n_rows): n_rows <= B; y of matrix i is [n_rows][out_dim i]
+// (name_m and name_p: the same with the other loads of the weights, rein_formats.h)
 #define REIN_DEFINE_MATVEC_MULTI(name, R, B)                                                                 \
+    REIN_DEFINE_MATVEC_MULTI_LD(name, R, B, REIN_LD_STREAM)                                                  \
+    REIN_DEFINE_MATVEC_MULTI_LD(name##_m, R, B, REIN_LD_MIX)                                                 \
+    REIN_DEFINE_MATVEC_MULTI_LD(name##_p, R, B, REIN_LD_PLAIN)
+#define REIN_DEFINE_MATVEC_MULTI_LD(name, R, B, POL)                                                         \
     extern "C" __global__ __launch_bounds__(256) void name(ReinMultiArgs a, const BlockQ8* __restrict__ xq,   \
                                                            unsigned int in_dim, unsigned int n_mat,           \
                                                            unsigned int n_rows)                               \
     {                                                                                                        \
-        rein_matvec_multi_body<R, B>(a, xq, in_dim, n_mat, n_rows);                                          \
+        rein_matvec_multi_body<R, B, POL>(a, xq, in_dim, n_mat, n_rows);                                          \
     }
 
 REIN_DEFINE_MATVEC_MULTI(rein_mv_multi_r1_b1, 1, 1)

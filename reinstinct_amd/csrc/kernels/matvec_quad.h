@@ -259,7 +259,7 @@ __device__ __forceinline__ void rein_matvec_quad_body(const uint8_t* __restrict_
 // Launch: block = 64 x W threads (W <= 16, a multiple of S), dynamic shared memory =
 //   4*NT * stride * 40 + W * kParts * 76 * 16 bytes, stride = n + ((20 - n % 16) % 16) for
 //   n = min(in_dim / 32, phase_sub); grid >= ceil(row groups / (W / S)) unless single-phase with S = 1.
-template <int FMT, int NT>
+template <int FMT, int NT, int POL>
 __device__ __forceinline__ void rein_matvec_quad_lds_body(const uint8_t* __restrict__ w, const BlockQ8* __restrict__ xq,
                                                           float* __restrict__ y, unsigned in_dim, unsigned out_dim,
                                                           unsigned n_rows, unsigned phase_sub, unsigned slices, unsigned depth)
@@ -315,7 +315,7 @@ __device__ __forceinline__ void rein_matvec_quad_lds_body(const uint8_t* __restr
         __builtin_amdgcn_sched_barrier(0);
         {
             const unsigned nrow = min(min(png, n_groups - 1u) * 4u + lr, out_dim - 1u);
-            rqx = fmt.load(nrow, min(psb + ls, n_sub - 1u));
+            rqx = fmt.template load<POL>(nrow, min(psb + ls, n_sub - 1u));
         }
         __builtin_amdgcn_sched_barrier(0);
         QuadRawBits<FMT> mine;
@@ -392,7 +392,7 @@ __device__ __forceinline__ void rein_matvec_quad_lds_body(const uint8_t* __restr
         unsigned g = blockIdx.x * wpb + wave;
         {   // the first trip's weights are on their way while the activations are staged
             const unsigned row = min(min(g, n_groups - 1u) * 4u + lr, out_dim - 1u);
-            rq = fmt.load(row, min(ls, n_sub - 1u));
+            rq = fmt.template load<POL>(row, min(ls, n_sub - 1u));
         }
         if (kTwoSets && depth >= 2u) {
             // two trips of weights in flight per wavefront: two register sets take turns, each refilled with the trip
@@ -404,7 +404,7 @@ __device__ __forceinline__ void rein_matvec_quad_lds_body(const uint8_t* __restr
             Raw rq2;
             {
                 const unsigned row = min(min(q.g, n_groups - 1u) * 4u + lr, out_dim - 1u);
-                rq2 = fmt.load(row, min(q.sb0 + ls, n_sub - 1u));
+                rq2 = fmt.template load<POL>(row, min(q.sb0 + ls, n_sub - 1u));
             }
             stage_x(0u, n_sub);
             __syncthreads();
@@ -448,8 +448,8 @@ __device__ __forceinline__ void rein_matvec_quad_lds_body(const uint8_t* __restr
         Raw rq2;
         {
             const unsigned row = min(min(g, n_groups - 1u) * 4u + lr, out_dim - 1u);
-            rq = fmt.load(row, min(16u * slice + ls, n_sub - 1u));
-            if (two) rq2 = fmt.load(row, min(16u * slice + ahead + ls, n_sub - 1u));
+            rq = fmt.template load<POL>(row, min(16u * slice + ls, n_sub - 1u));
+            if (two) rq2 = fmt.template load<POL>(row, min(16u * slice + ahead + ls, n_sub - 1u));
         }
         bool odd = false;
         for (unsigned ph0 = 0; ph0 < n_sub; ph0 += phase_sub) {
@@ -502,13 +502,19 @@ __device__ __forceinline__ void rein_matvec_quad_lds_body(const uint8_t* __restr
 // (32 rows: by default for eight wavefronts per workgroup at most, so that the 32 partial sums and the eight activation
 // tiles of a trip stay in registers; REIN_DEFINE_MATVEC_QUAD_LDS_BOUND builds it for sixteen wavefronts' 128 registers as
 // well, where the heavier formats spill)
+// (name_m and name_p: the same with the other loads of the weights, rein_formats.h)
 #define REIN_DEFINE_MATVEC_QUAD_LDS(name, FMT, NT) REIN_DEFINE_MATVEC_QUAD_LDS_BOUND(name, FMT, NT, (NT >= 8 ? 512 : 1024))
-#define REIN_DEFINE_MATVEC_QUAD_LDS_BOUND(name, FMT, NT, BOUND)                                   \
+#define REIN_DEFINE_MATVEC_QUAD_LDS_BOUND(name, FMT, NT, BOUND) REIN_DEFINE_MATVEC_QUAD_LDS_LD(name, FMT, NT, BOUND, REIN_LD_STREAM)
+#define REIN_DEFINE_MATVEC_QUAD_LDS_LOADS(name, FMT, NT)                                          \
+    REIN_DEFINE_MATVEC_QUAD_LDS(name, FMT, NT)                                                    \
+    REIN_DEFINE_MATVEC_QUAD_LDS_LD(name##_m, FMT, NT, 1024, REIN_LD_MIX)                          \
+    REIN_DEFINE_MATVEC_QUAD_LDS_LD(name##_p, FMT, NT, 1024, REIN_LD_PLAIN)
+#define REIN_DEFINE_MATVEC_QUAD_LDS_LD(name, FMT, NT, BOUND, POL)                                 \
     extern "C" __global__ __launch_bounds__(BOUND) void name(                                     \
         const uint8_t* __restrict__ w, const BlockQ8* __restrict__ xq, float* __restrict__ y,    \
         unsigned int in_dim, unsigned int out_dim, unsigned int n_rows, unsigned int phase_sub,   \
         unsigned int slices, unsigned int depth)                                                  \
     {                                                                                             \
-        rein_matvec_quad_lds_body<FMT, NT>(w, xq, y, in_dim, out_dim, n_rows, phase_sub, slices,  \
-                                           depth);                                                \
+        rein_matvec_quad_lds_body<FMT, NT, POL>(w, xq, y, in_dim, out_dim, n_rows, phase_sub,     \
+                                                slices, depth);                                   \
     }

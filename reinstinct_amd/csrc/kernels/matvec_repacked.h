@@ -30,7 +30,7 @@ struct XBlocks {
 };
 
 // The row groups first, first + step, ... of one matrix, walked by the calling wavefront.
-template <int FMT, int R, int B, int U = 1>
+template <int FMT, int R, int B, int U = 1, int POL = REIN_LD_STREAM>
 __device__ __forceinline__ void rein_matvec_span(const uint8_t* __restrict__ w,
                                                  const BlockQ8* __restrict__ xq,
                                                  float* __restrict__ y,
@@ -68,7 +68,7 @@ __device__ __forceinline__ void rein_matvec_span(const uint8_t* __restrict__ w,
                 live[u] = sb0 + 64 * u + lane < n_sub;
                 sb[u]   = live[u] ? sb0 + 64 * u + lane : n_sub - 1;
 #pragma unroll
-                for (int r = 0; r < R; r++) raw[u][r] = fmt.load(min(row0 + r, rmax), sb[u]);
+                for (int r = 0; r < R; r++) raw[u][r] = fmt.template load<POL>(min(row0 + r, rmax), sb[u]);
             }
 #pragma unroll
             for (int u = 0; u < U; u++)
@@ -120,14 +120,14 @@ __device__ __forceinline__ void rein_matvec_span(const uint8_t* __restrict__ w,
 }
 
 // Every wavefront of the launch takes the row groups of its own index, striding by the launch's wavefront count.
-template <int FMT, int R, int B, int U = 1>
+template <int FMT, int R, int B, int U = 1, int POL = REIN_LD_STREAM>
 __device__ __forceinline__ void rein_matvec_body(const uint8_t* __restrict__ w,
                                                  const BlockQ8* __restrict__ xq,
                                                  float* __restrict__ y,
                                                  unsigned in_dim, unsigned out_dim, unsigned n_rows)
 {
     const unsigned wpb = blockDim.x >> 6;
-    rein_matvec_span<FMT, R, B, U>(w, xq, y, in_dim, out_dim, n_rows, blockIdx.x * wpb + (threadIdx.x >> 6), gridDim.x * wpb);
+    rein_matvec_span<FMT, R, B, U, POL>(w, xq, y, in_dim, out_dim, n_rows, blockIdx.x * wpb + (threadIdx.x >> 6), gridDim.x * wpb);
 }
 
 // Per-block integer dots exactly as the matvec forms them, for the bit-exact
@@ -182,6 +182,17 @@ __device__ __forceinline__ void rein_block_dots_body(const uint8_t* __restrict__
     {                                                                                             \
         rein_matvec_body<FMT, R, B>(w, xq, y, in_dim, out_dim, n_rows);                           \
     }
+
+// the same three times, by the way it loads the weights: name (streaming), name_m (mixed), name_p (plain)
+#define REIN_DEFINE_MATVEC_LD(name, FMT, R, B, POL)                                               \
+    extern "C" __global__ __launch_bounds__(256) void name(REIN_MATVEC_ARGS, unsigned int n_rows) \
+    {                                                                                             \
+        rein_matvec_body<FMT, R, B, 1, POL>(w, xq, y, in_dim, out_dim, n_rows);                   \
+    }
+#define REIN_DEFINE_MATVEC_LOADS(name, FMT, R, B)                                                 \
+    REIN_DEFINE_MATVEC_LD(name, FMT, R, B, REIN_LD_STREAM)                                        \
+    REIN_DEFINE_MATVEC_LD(name##_m, FMT, R, B, REIN_LD_MIX)                                       \
+    REIN_DEFINE_MATVEC_LD(name##_p, FMT, R, B, REIN_LD_PLAIN)
 
 // tuned variant with U trips of loads in flight per iteration
 #define REIN_DEFINE_MATVEC_TUNED(name, FMT, R, B, U)                                              \

@@ -104,22 +104,39 @@ template <int FMT> __device__ __forceinline__ int rein_codebook4(uint32_t w, uns
     }
 }
 
-// Streaming (nontemporal) loads for the matvec weight planes: every weight byte is
-// read exactly once per launch, so it should not displace the activations in L2.
+// Loads of the weight planes.  Every weight byte is read once per launch, but what the nontemporal hint does for it depends
+// on how much of the matrix the launch streams (measured per shape and format with the matrices rotating through 0.06, 0.6
+// and 4 GB; the host's load_tag picks the kernel built for one or the other):
+//   REIN_LD_PLAIN   no hint
+//   REIN_LD_STREAM  all planes nontemporal
+//   REIN_LD_MIX     the 16- and 8-byte planes nontemporal, the 4- and 2-byte planes (scales, 5th bits) plain: a wavefront's
+//                   burst of scales covers part of a 128-byte line whose rest the neighbouring rows want, so these lines
+//                   should stay
 typedef uint32_t rein_u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t rein_u32x2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ uint4 rein_ldw(const uint4* p)
+#define REIN_LD_PLAIN  0
+#define REIN_LD_MIX    1
+#define REIN_LD_STREAM 2
+template <int POL = REIN_LD_STREAM> __device__ __forceinline__ uint4 rein_ldw(const uint4* p)
 {
+    if (POL == REIN_LD_PLAIN) return *p;
     const rein_u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const rein_u32x4*>(p));
     return make_uint4(v.x, v.y, v.z, v.w);
 }
-__device__ __forceinline__ uint2 rein_ldw(const uint2* p)
+template <int POL = REIN_LD_STREAM> __device__ __forceinline__ uint2 rein_ldw(const uint2* p)
 {
+    if (POL == REIN_LD_PLAIN) return *p;
     const rein_u32x2 v = __builtin_nontemporal_load(reinterpret_cast<const rein_u32x2*>(p));
     return make_uint2(v.x, v.y);
 }
-__device__ __forceinline__ uint32_t rein_ldw(const uint32_t* p) { return __builtin_nontemporal_load(p); }
-__device__ __forceinline__ uint16_t rein_ldw(const uint16_t* p) { return __builtin_nontemporal_load(p); }
+template <int POL = REIN_LD_STREAM> __device__ __forceinline__ uint32_t rein_ldw(const uint32_t* p)
+{
+    return POL == REIN_LD_STREAM ? __builtin_nontemporal_load(p) : *p;
+}
+template <int POL = REIN_LD_STREAM> __device__ __forceinline__ uint16_t rein_ldw(const uint16_t* p)
+{
+    return POL == REIN_LD_STREAM ? __builtin_nontemporal_load(p) : *p;
+}
 
 template <int FMT> struct Fmt;
 
@@ -140,13 +157,13 @@ template <> struct Fmt<REIN_Q4_K> {
         smp = reinterpret_cast<const uint16_t*>(w + n * 16);
         ddp = reinterpret_cast<const uint32_t*>(w + n * 18);
     }
-    __device__ __forceinline__ Raw load(unsigned row, unsigned sb) const
+    template <int POL = REIN_LD_STREAM> __device__ __forceinline__ Raw load(unsigned row, unsigned sb) const
     {
         const size_t i = (size_t)row * nsp + sb;
         Raw r;
-        r.q  = rein_ldw(&nib[i]);
-        r.sm = rein_ldw(&smp[i]);
-        r.dd = rein_ldw(&ddp[(size_t)row * n_super + (sb >> 3)]);
+        r.q  = rein_ldw<POL>(&nib[i]);
+        r.sm = rein_ldw<POL>(&smp[i]);
+        r.dd = rein_ldw<POL>(&ddp[(size_t)row * n_super + (sb >> 3)]);
         return r;
     }
     static __device__ __forceinline__ void unpack(const Raw& r, SubW& s)
@@ -188,14 +205,14 @@ template <> struct Fmt<REIN_Q5_K> {
         smp = reinterpret_cast<const uint16_t*>(w + n * 20);
         ddp = reinterpret_cast<const uint32_t*>(w + n * 22);
     }
-    __device__ __forceinline__ Raw load(unsigned row, unsigned sb) const
+    template <int POL = REIN_LD_STREAM> __device__ __forceinline__ Raw load(unsigned row, unsigned sb) const
     {
         const size_t i = (size_t)row * nsp + sb;
         Raw r;
-        r.q  = rein_ldw(&nib[i]);
-        r.qh = rein_ldw(&qhp[i]);
-        r.sm = rein_ldw(&smp[i]);
-        r.dd = rein_ldw(&ddp[(size_t)row * n_super + (sb >> 3)]);
+        r.q  = rein_ldw<POL>(&nib[i]);
+        r.qh = rein_ldw<POL>(&qhp[i]);
+        r.sm = rein_ldw<POL>(&smp[i]);
+        r.dd = rein_ldw<POL>(&ddp[(size_t)row * n_super + (sb >> 3)]);
         return r;
     }
     static __device__ __forceinline__ void unpack(const Raw& r, SubW& s)
@@ -239,14 +256,14 @@ template <> struct Fmt<REIN_Q6_K> {
         smp = reinterpret_cast<const uint16_t*>(w + n * 24);
         dp  = reinterpret_cast<const uint16_t*>(w + n * 26);
     }
-    __device__ __forceinline__ Raw load(unsigned row, unsigned sb) const
+    template <int POL = REIN_LD_STREAM> __device__ __forceinline__ Raw load(unsigned row, unsigned sb) const
     {
         const size_t i = (size_t)row * nsp + sb;
         Raw r;
-        r.q  = rein_ldw(&nib[i]);
-        r.h2 = rein_ldw(&h2p[i]);
-        r.sm = rein_ldw(&smp[i]);
-        r.d  = rein_ldw(&dp[(size_t)row * n_super + (sb >> 3)]);
+        r.q  = rein_ldw<POL>(&nib[i]);
+        r.h2 = rein_ldw<POL>(&h2p[i]);
+        r.sm = rein_ldw<POL>(&smp[i]);
+        r.d  = rein_ldw<POL>(&dp[(size_t)row * n_super + (sb >> 3)]);
         return r;
     }
     static __device__ __forceinline__ void unpack(const Raw& r, SubW& s)
@@ -294,13 +311,13 @@ template <> struct Fmt<REIN_Q8_0> {
         hip_ = reinterpret_cast<const uint4*>(w + n * 16);
         dp   = reinterpret_cast<const uint16_t*>(w + n * 32);
     }
-    __device__ __forceinline__ Raw load(unsigned row, unsigned sb) const
+    template <int POL = REIN_LD_STREAM> __device__ __forceinline__ Raw load(unsigned row, unsigned sb) const
     {
         const size_t i = (size_t)row * nsp + sb;
         Raw r;
-        r.lo = rein_ldw(&lop[i]);
-        r.hi = rein_ldw(&hip_[i]);
-        r.d  = rein_ldw(&dp[i]);
+        r.lo = rein_ldw<POL>(&lop[i]);
+        r.hi = rein_ldw<POL>(&hip_[i]);
+        r.d  = rein_ldw<POL>(&dp[i]);
         return r;
     }
     static __device__ __forceinline__ void unpack(const Raw& r, SubW& s)
@@ -333,12 +350,12 @@ template <> struct Fmt<REIN_Q4_0> {
         nib = reinterpret_cast<const uint4*>(w);
         dp  = reinterpret_cast<const uint16_t*>(w + n * 16);
     }
-    __device__ __forceinline__ Raw load(unsigned row, unsigned sb) const
+    template <int POL = REIN_LD_STREAM> __device__ __forceinline__ Raw load(unsigned row, unsigned sb) const
     {
         const size_t i = (size_t)row * nsp + sb;
         Raw r;
-        r.q = rein_ldw(&nib[i]);
-        r.d = rein_ldw(&dp[i]);
+        r.q = rein_ldw<POL>(&nib[i]);
+        r.d = rein_ldw<POL>(&dp[i]);
         return r;
     }
     static __device__ __forceinline__ void unpack(const Raw& r, SubW& s)
@@ -381,12 +398,12 @@ template <int FMT> struct FmtCodebook16 {
         nib = reinterpret_cast<const uint4*>(w);
         dp  = reinterpret_cast<const uint16_t*>(w + n * 16);
     }
-    __device__ __forceinline__ Raw load(unsigned row, unsigned sb) const
+    template <int POL = REIN_LD_STREAM> __device__ __forceinline__ Raw load(unsigned row, unsigned sb) const
     {
         const size_t i = (size_t)row * nsp + sb;
         Raw r;
-        r.q = rein_ldw(&nib[i]);
-        r.d = rein_ldw(&dp[i]);
+        r.q = rein_ldw<POL>(&nib[i]);
+        r.d = rein_ldw<POL>(&dp[i]);
         return r;
     }
     static __device__ __forceinline__ void unpack(const Raw& r, SubW& s)
@@ -430,13 +447,13 @@ template <> struct Fmt<REIN_Q5_1> {
         qhp = reinterpret_cast<const uint32_t*>(w + n * 16);
         dmp = reinterpret_cast<const uint32_t*>(w + n * 20);
     }
-    __device__ __forceinline__ Raw load(unsigned row, unsigned sb) const
+    template <int POL = REIN_LD_STREAM> __device__ __forceinline__ Raw load(unsigned row, unsigned sb) const
     {
         const size_t i = (size_t)row * nsp + sb;
         Raw r;
-        r.q  = rein_ldw(&nib[i]);
-        r.qh = rein_ldw(&qhp[i]);
-        r.dm = rein_ldw(&dmp[i]);
+        r.q  = rein_ldw<POL>(&nib[i]);
+        r.qh = rein_ldw<POL>(&qhp[i]);
+        r.dm = rein_ldw<POL>(&dmp[i]);
         return r;
     }
     static __device__ __forceinline__ void unpack(const Raw& r, SubW& s)
