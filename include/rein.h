@@ -105,7 +105,8 @@ int rein_is_loaded(void);
  * width), REIN_MMQ6, REIN_MMQ6_FROM, REIN_MMQ6_N4, REIN_MMQ6_N2, REIN_MMQ6_SK,
  * REIN_MMQ6_SK_GRID, REIN_MMQ6_SK_SPLIT (Q4_K fp6 launch: 0 off, first row count, token groups
  * of four / two tiles per row block, split-tail 0 off / 2 forced, its grid and ranges),
- * REIN_MMQ16 (1: the fp16 formulation where the code object holds it), REIN_TOPK_WAVE,
+ * REIN_MMQ16 (1: the fp16 formulation where the code object holds it), REIN_MMQXH (0 / 2: the exact-dot fp16
+ * GEMM of rein_matmul_ws off / wherever it can run), REIN_MMQXH_SPLIT (its ranges per unit), REIN_TOPK_WAVE,
  * REIN_MOE_SORT_SPLIT, REIN_MOE_CHAIN, REIN_MOE_FUSED, REIN_MOE_FEW, REIN_MOE_GU_ROWS, REIN_MOE_DC_ROWS
  * (MoE glue: 0 = the workgroup router, 1 = the four-launch sort, 0 = no decode chain for few
  * tokens, 0 = unfused gate/up, 0 never / 1 wherever the shape allows the launches that read every touched
@@ -409,7 +410,10 @@ int rein_matmul(int fmt, const void *w, const float *x, float *y, unsigned in_di
                 unsigned out_dim, unsigned n_rows, void *xq_scratch, rein_stream_t s);
 /* rein_matmul with one scratch buffer of rein_matmul_scratch_bytes(fmt, in_dim, n_rows) bytes
  * (16-byte aligned) that holds the quantized activations and, for the MMQ path, the workspace
- * of rein_mmq_xq8_ws.  A scratch that only holds the activations runs rein_matmul. */
+ * of rein_mmq_xq8_ws.  A scratch that only holds the activations runs rein_matmul.
+ * Q4_K, Q5_K and Q6_K from 65 rows: a scratch of the full size runs the fp16-instruction GEMM with exact block
+ * dots where it is the faster one (activation image and up to 64 MiB of partial tiles in the scratch; three
+ * launches, no allocation); a smaller one runs what rein_mmq_xq8_ws takes for it. */
 size_t rein_matmul_scratch_bytes(int fmt, unsigned in_dim, unsigned n_rows);
 int rein_matmul_ws(int fmt, const void *w, const float *x, float *y, unsigned in_dim,
                    unsigned out_dim, unsigned n_rows, void *scratch, size_t scratch_bytes,

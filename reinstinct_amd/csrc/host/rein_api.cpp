@@ -192,8 +192,8 @@ int check_ptr(const char* who, const void* p, size_t align, const char* what)
 // rein_set_option changes an entry, so the launch an entry point chooses depends on its arguments
 // and on this table alone.  Entries are single atomic words: setting one while another thread
 // launches is safe, the launch sees the old or the new value.
-enum Opt : int { O_MV_ROWS, O_MV_WPB, O_MV_LDS, O_QUAD_LDS, O_QUAD_SLICES, O_QUAD_DEPTH, O_QUAD_WIDE32, O_SKINNY_KS, O_SKINNY_FROM, O_QUAD_FROM, O_GROUPED_STRIDED, O_MMQ_TM, O_MMQ_N64, O_MMQ6, O_MMQ6_N4, O_MMQ6_N2, O_MMQ6_SK_GRID, O_MMQ6_SK_SPLIT, O_MMQ6_SK, O_MMQ6_FROM, O_MMQ_SK, O_MMQ_SK_GRID, O_MMQ_SK_SPLIT, O_MMQ_SK_TM, O_MMQ16, O_TOPK_WAVE, O_MOE_SORT_SPLIT, O_MOE_GU_ROWS, O_MOE_DC_ROWS, O_MOE_CHAIN, O_MOE_FUSED, O_MOE_FEW, O_COUNT };
-const char* const kOptNames[O_COUNT] = {"REIN_MV_ROWS", "REIN_MV_WPB", "REIN_MV_LDS", "REIN_QUAD_LDS", "REIN_QUAD_SLICES", "REIN_QUAD_DEPTH", "REIN_QUAD_WIDE32", "REIN_SKINNY_KS", "REIN_SKINNY_FROM", "REIN_QUAD_FROM", "REIN_GROUPED_STRIDED", "REIN_MMQ_TM", "REIN_MMQ_N64", "REIN_MMQ6", "REIN_MMQ6_N4", "REIN_MMQ6_N2", "REIN_MMQ6_SK_GRID", "REIN_MMQ6_SK_SPLIT", "REIN_MMQ6_SK", "REIN_MMQ6_FROM", "REIN_MMQ_SK", "REIN_MMQ_SK_GRID", "REIN_MMQ_SK_SPLIT", "REIN_MMQ_SK_TM", "REIN_MMQ16", "REIN_TOPK_WAVE", "REIN_MOE_SORT_SPLIT", "REIN_MOE_GU_ROWS", "REIN_MOE_DC_ROWS", "REIN_MOE_CHAIN", "REIN_MOE_FUSED", "REIN_MOE_FEW"};
+enum Opt : int { O_MV_ROWS, O_MV_WPB, O_MV_LDS, O_QUAD_LDS, O_QUAD_SLICES, O_QUAD_DEPTH, O_QUAD_WIDE32, O_SKINNY_KS, O_SKINNY_FROM, O_QUAD_FROM, O_GROUPED_STRIDED, O_MMQ_TM, O_MMQ_N64, O_MMQ6, O_MMQ6_N4, O_MMQ6_N2, O_MMQ6_SK_GRID, O_MMQ6_SK_SPLIT, O_MMQ6_SK, O_MMQ6_FROM, O_MMQ_SK, O_MMQ_SK_GRID, O_MMQ_SK_SPLIT, O_MMQ_SK_TM, O_MMQ16, O_MMQXH, O_MMQXH_SPLIT, O_TOPK_WAVE, O_MOE_SORT_SPLIT, O_MOE_GU_ROWS, O_MOE_DC_ROWS, O_MOE_CHAIN, O_MOE_FUSED, O_MOE_FEW, O_COUNT };
+const char* const kOptNames[O_COUNT] = {"REIN_MV_ROWS", "REIN_MV_WPB", "REIN_MV_LDS", "REIN_QUAD_LDS", "REIN_QUAD_SLICES", "REIN_QUAD_DEPTH", "REIN_QUAD_WIDE32", "REIN_SKINNY_KS", "REIN_SKINNY_FROM", "REIN_QUAD_FROM", "REIN_GROUPED_STRIDED", "REIN_MMQ_TM", "REIN_MMQ_N64", "REIN_MMQ6", "REIN_MMQ6_N4", "REIN_MMQ6_N2", "REIN_MMQ6_SK_GRID", "REIN_MMQ6_SK_SPLIT", "REIN_MMQ6_SK", "REIN_MMQ6_FROM", "REIN_MMQ_SK", "REIN_MMQ_SK_GRID", "REIN_MMQ_SK_SPLIT", "REIN_MMQ_SK_TM", "REIN_MMQ16", "REIN_MMQXH", "REIN_MMQXH_SPLIT", "REIN_TOPK_WAVE", "REIN_MOE_SORT_SPLIT", "REIN_MOE_GU_ROWS", "REIN_MOE_DC_ROWS", "REIN_MOE_CHAIN", "REIN_MOE_FUSED", "REIN_MOE_FEW"};
 constexpr uint64_t kOptSet = 1ull << 63;
 std::atomic<uint64_t> g_opts[O_COUNT];          // zero = unset
 std::once_flag g_opts_env_once;
@@ -1826,11 +1826,80 @@ int rein_matmul(int fmt, const void* w, const float* x, float* y, unsigned in_di
     }
 }
 
+namespace {
+// ---- Q4_K / Q5_K / Q6_K prefill with exact block dots on the fp16 instruction (kernels/mmq_exact16.h), out of rein_matmul_ws
+struct XhPlan {
+    unsigned n_grp, n_unit, n_whole, split;
+    size_t image;                                    // bytes of the activation image, partial tiles behind it
+};
+constexpr size_t kXhPart = (size_t)4 * 16 * 256 * 4;
+constexpr size_t kXhParts = (size_t)64 << 20;        // room for partial tiles: 1024
+bool xh_format(int fmt) { return fmt == REIN_TYPE_Q4_K || fmt == REIN_TYPE_Q5_K || fmt == REIN_TYPE_Q6_K; }
+bool xh_has_min(int fmt) { return fmt != REIN_TYPE_Q6_K; }
+size_t xh_image_bytes(int fmt, unsigned in_dim, unsigned p_rows)
+{
+    const size_t n_tt = ((size_t)p_rows + 31) / 32;
+    return (in_dim / 64) * n_tt * 4352 + (xh_has_min(fmt) ? (in_dim / 256) * n_tt * 2048 : 0);
+}
+unsigned xh_lds_bytes(int fmt) { return 2 * 17408 + 4 * 4096 + 4 * 3584 + (xh_has_min(fmt) ? 8192 : 0); }     // rein_xh_lds_bytes
+bool xh_shape(int fmt, unsigned in_dim, unsigned p_rows)
+{
+    const unsigned mode = opt_u(O_MMQXH, 1);
+    if (mode == 0 || !xh_format(fmt) || in_dim == 0 || in_dim % 256 != 0) return false;
+    return p_rows > 64u;                               // from three token tiles on a group has at least two (rein_xh_group)
+}
+// Units of 128 rows x 96..128 tokens, 512 resident workgroups.  Whole rounds run unsplit; what is left over is cut into the
+// cheapest number of ranges, counted in superblocks of a workgroup that shares its CU: a range costs its superblocks and one
+// and a half for its start; a last round of at most one workgroup per CU takes 0.6 of one with two; a partial tile is
+// written and read once.  Q6_K, us at 1 / 2 / 3 / 4 / 6 ranges: 17408 -> 5120, 777 rows (280 units) 475 / 409 / 382 / 382 /
+// 382, 512 rows (160 units) 349 / 290 / 228 / 249 / 240; 5120 -> 17408, 512 rows (a round and 32) 274 / 228 / 214 / 208 / 208.
+XhPlan xh_plan(int fmt, unsigned in_dim, unsigned out_dim, unsigned p_rows)
+{
+    XhPlan p{};
+    p.n_grp = (p_rows + 127) / 128;
+    p.n_unit = (out_dim + 127) / 128 * p.n_grp;
+    p.n_whole = p.n_unit / 512 * 512;
+    p.split = 1;
+    p.image = (xh_image_bytes(fmt, in_dim, p_rows) + 255) & ~(size_t)255;
+    const unsigned tail = p.n_unit - p.n_whole, chunks = in_dim / 256;
+    if (tail == 0) return p;
+    const unsigned most = std::min<unsigned>(std::min(16u, chunks), (unsigned)(kXhParts / kXhPart / tail));
+    double best = 0.0;
+    for (unsigned k = 1; k <= std::max(1u, most); k++) {
+        const unsigned wg = tail * k, rem = wg % 512;
+        const double rounds = wg / 512 + (rem == 0 ? 0.0 : rem <= kCUs ? 0.6 : 1.0);
+        const double cost = rounds * (chunks / (double)k + 1.5) + (k > 1 ? 0.4 + wg * 0.0012 : 0.0);
+        if (k == 1 || cost < best) { best = cost; p.split = k; }
+    }
+    const unsigned forced = opt_u(O_MMQXH_SPLIT, 0);
+    if (forced) p.split = std::max(1u, std::min(forced, most));
+    return p;
+}
+// Where it is taken, from a sweep of 11 model shapes (hidden 1024-18432 against 1024-18944) x 16 row counts 72-2048 through
+// rein_matmul_ws, every cell beside the launches of rein_mmq_xq8_ws (their time / this one's):
+//   Q6_K  0.99-2.1 in all 110 cells (17408 -> 5120, 512 rows 444 / 216 us; 5120 -> 17408 307 / 208): everywhere from three token
+//         tiles; below 5e8 operations a call is a few launches either way and nothing was measured.
+//   Q4_K  contractions of 3584 and more 0.96-1.25, median 1.06 (17408 -> 5120, 512 rows 166 / 152); 2048 and less 0.59-1.09: a
+//         range of few superblocks does not pay back its start and the image.  The line is between them.
+//   Q5_K  the same contractions from 384 rows 0.97-1.46, median 1.11 (5120 -> 17408, 512 rows 190 / 167); below, groups of two
+//         and three tiles share the unpack of its fifth bits too little (72-320 rows 0.75-1.8, median 0.98).
+bool xh_take(int fmt, unsigned in_dim, unsigned out_dim, unsigned p_rows)
+{
+    if (!xh_shape(fmt, in_dim, p_rows)) return false;
+    if (opt_u(O_MMQXH, 1) == 2) return true;
+    if (fmt == REIN_TYPE_Q6_K) return 2.0 * p_rows * (double)out_dim * in_dim >= 5.0e8;
+    return in_dim >= 3072 && p_rows >= (fmt == REIN_TYPE_Q4_K ? 96u : 384u);
+}
+}  // namespace
+
 size_t rein_matmul_scratch_bytes(int fmt, unsigned in_dim, unsigned n_rows)
 {
     if (!rein_block_size(fmt) || in_dim == 0 || in_dim % 32 != 0 || n_rows == 0) return 0;
     const size_t xq = ((size_t)n_rows * (in_dim / 32) * 40 + 255) & ~(size_t)255;
-    return xq + (rein_matmul_path(fmt, n_rows) == 2 ? rein_mmq_workspace_bytes(fmt, in_dim, n_rows) : 0);
+    size_t behind = rein_matmul_path(fmt, n_rows) == 2 ? rein_mmq_workspace_bytes(fmt, in_dim, n_rows) : 0;
+    if (rein_matmul_path(fmt, n_rows) == 2 && xh_shape(fmt, in_dim, n_rows))
+        behind = std::max(behind, ((xh_image_bytes(fmt, in_dim, n_rows) + 255) & ~(size_t)255) + kXhParts);
+    return xq + behind;
 }
 
 int rein_matmul_ws(int fmt, const void* w, const float* x, float* y, unsigned in_dim, unsigned out_dim,
@@ -1847,6 +1916,25 @@ int rein_matmul_ws(int fmt, const void* w, const float* x, float* y, unsigned in
     if (rein_matmul_path(fmt, n_rows) != 2 || rein_mmq_workspace_bytes(fmt, in_dim, n_rows) == 0 ||
         scratch_bytes < xq + std::max<size_t>(least, 16))
         return rein_matmul(fmt, w, x, y, in_dim, out_dim, n_rows, scratch, s);
+    if (n_rows <= 65535 && xh_take(fmt, in_dim, out_dim, n_rows) && scratch_bytes >= rein_matmul_scratch_bytes(fmt, in_dim, n_rows)) {
+        if (int rc = check_ptr("rein_matmul_ws", x, 4, "x")) return rc;
+        if (int rc = check_ptr("rein_matmul_ws", w, 16, "w")) return rc;
+        if (int rc = check_ptr("rein_matmul_ws", y, 4, "y")) return rc;
+        const XhPlan p = xh_plan(fmt, in_dim, out_dim, n_rows);
+        char* const img = static_cast<char*>(scratch) + xq;
+        char* const parts = img + p.image;
+        const unsigned tail = p.n_unit - p.n_whole, with_xsum = xh_has_min(fmt);
+        const unsigned long long grid = p.n_whole + 8ull * (((unsigned long long)tail * p.split + 7) / 8);
+        if (grid <= 0x7FFFFFFFull && in_dim / 256 <= 65535) {
+            void* pa[] = {(void*)&x, (void*)&img, (void*)&in_dim, (void*)&n_rows, (void*)&with_xsum};
+            if (int rc = launch("rein_xh_quantize", (n_rows + 31) / 32, in_dim / 256, 1, 256, 0, s, pa)) return rc;
+            void* a[] = {(void*)&w, (void*)&img, (void*)&y, (void*)&parts, (void*)&in_dim, (void*)&out_dim, (void*)&n_rows, (void*)&p.n_whole, (void*)&p.split};
+            if (int rc = launch(KName("rein_xh_", fmt_tag(fmt), ""), (unsigned)grid, 1, 1, 256, xh_lds_bytes(fmt), s, a)) return rc;
+            if (p.split == 1) return 0;
+            void* b[] = {(void*)&parts, (void*)&y, (void*)&out_dim, (void*)&n_rows, (void*)&p.n_whole, (void*)&p.split};
+            return launch("rein_xh_sum", tail, 16, 1, 256, 0, s, b);
+        }
+    }
     if (int rc = rein_quantize_q8(x, scratch, in_dim, n_rows, s)) return rc;
     return rein_mmq_xq8_ws(fmt, w, scratch, y, in_dim, out_dim, n_rows, static_cast<char*>(scratch) + xq, scratch_bytes - xq, s);
 }

@@ -1,0 +1,542 @@
+// Prefill GEMM for Q4_K, Q5_K and Q6_K on the fp16 matrix instruction with exact block dots.
+//
+// The int8 tile (mmq_gemm.h) leaves a conversion, a scale outer product and a multiply-add per output element and 32-weight
+// sub-block on the vector ALU, and for Q6_K a second matrix instruction per sub-block with half of its operand zeroed plus an
+// integer combine.  Here the integer scale of a sub-block goes into the weight operand and stays exact:
+//   Q4_K  q * sc               4 + 6 bits, at most 945: one fp16 number
+//   Q5_K  q * sc               5 + 6 bits, at most 1953: one
+//   Q6_K  (q - 32) * sc / 4  = n * sc / 4  +  4 * (c - 2) * sc     n the nibble, c the two high bits, q = n + 16 c: both
+//                              terms are integers of at most 11 bits times a power of two, so each is one fp16 number, and
+//                              the two are two operands of the same accumulation
+// and the activations are their int8 quants as fp16.  v_mfma_f32_32x32x16_f16 multiplies exactly and every partial sum is an
+// integer (times 1/4) below 2^24, so the fp32 result IS the integer dot of the sub-block with its scale: no rounding, nothing
+// to convert.  With the weights as rows of the tile (register = weight row, lane = token) the activation scale is one number
+// per lane: per sub-block and element the vector ALU does s1 += dx * dot, per 256 weights acc += d * s1 -- the products and
+// sums that the int8 tile makes in fp32, fewer of them.  The minimum term of Q4_K and Q5_K is the int8 tile's: bf16 instructions on
+// the three-way bf16 split of xsum (24 bits) against the integer minimums, scaled by -dmin.
+//
+// A wavefront owns 32 weight rows x 32 NT tokens, NT up to 4 (the unpack of a weight is shared by NT tiles), a workgroup of
+// four 128 rows x 32 NT tokens; two workgroups per CU.
+//
+// Bound: matrix unit (2 / 4 fp16 instructions of 32 cycles per tile and sub-block, Q4_K and Q5_K / Q6_K) plus the 16
+// multiply-adds and the share of the unpack, which issue between them.  Measured per tile and sub-block and SIMD at 2048 x 5120 x
+// 17408: 104 / 122 / 150 ns, the launches before it (fp6, int8, int8) 108 / 139 / 211.  Whole calls of rein_matmul_ws, us before
+// and now: Q6_K 777 x 17408 -> 5120 523 / 379, 512 x 5120 -> 17408 307 / 208; Q5_K the same 190 / 167; Q4_K 147 / 145, 512 x
+// 17408 -> 5120 166 / 152.
+//
+// Replaces, from 65 rows, kernels/mmq_gemm_{q4k,q5k,q6k}_repacked.cpp of the reference behind rein_matmul_ws.
+#pragma once
+
+#include "mmq_fp6.h"
+
+typedef _Float16 rein_h2 __attribute__((ext_vector_type(2)));
+typedef _Float16 rein_v8h __attribute__((ext_vector_type(8)));
+
+// HBM -> LDS transfers of a dword / a 16-bit word per lane (which lands as a dword, zero-extended), scalar base + lane offset
+__device__ __forceinline__ void rein_xh_dma_u32(unsigned voff, const void* sbase, unsigned lds_base)
+{
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" : : "v"(voff), "s"(sbase), "s"(lds_base) : "memory", "m0");
+}
+__device__ __forceinline__ void rein_xh_dma_u16(unsigned voff, const void* sbase, unsigned lds_base)
+{
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_ushort %0, %1" : : "v"(voff), "s"(sbase), "s"(lds_base) : "memory", "m0");
+}
+
+// ---- operand slot order ---------------------------------------------------------------
+// An instruction contracts 16 slots; lane half h holds slots 8h .. 8h+7 of both operands.  The two instructions kh = 0, 1 of
+// a sub-block take word 2h + kh of its 16-byte nibble entry (low nibble of byte f: weight 4 (2h + kh) + f, high nibble 16 more),
+// in the order in which the masks below produce them.
+__host__ __device__ constexpr int rein_xh_slot_weight(int kh, int h, int e)
+{
+    constexpr int t[8] = {0, 2, 16, 18, 1, 3, 17, 19};
+    return 4 * (2 * h + kh) + t[e];
+}
+
+// ---- activation image -----------------------------------------------------------------
+//   records  [sub-block pair][32-token tile] of 4352 bytes:
+//              [q: sub-block of the pair][kh][lane = 32 h + token][8 x fp16], then dx [q][32] fp32
+//   xsum     [superblock][32-token tile] of 2048 bytes: [op][lane][8 x bf16]: lane halves 0 / 1 of op 0 the first and second
+//            bf16 of the 8 sub-blocks' xsum, half 0 of op 1 the third, half 1 zeros
+#define REIN_XH_X   4096u
+#define REIN_XH_REC 4352u
+#define REIN_XH_XS  2048u
+
+// x [p_rows][in_dim] fp32 -> image, with the numbers that quantize_q8_f32 gives: the same sum tree (halves of 16, 8, 4, 2, 1),
+// divisions and rounding, by one thread for a block of 32.  blockIdx.x = token tile, blockIdx.y = superblock, 256 threads:
+// thread 8 j + s handles token j, sub-block s: eight threads read a kilobyte of a row and write runs of 128 bytes.
+// Bound by memory: 4 bytes in, 2.1 out per value (777 x 17408: 54 + 29 MB).
+__device__ __forceinline__ void rein_xh_quantize_body(const float* __restrict__ x, uint8_t* __restrict__ img, unsigned in_dim, unsigned p_rows, unsigned with_xsum)
+{
+#pragma clang fp contract(off)
+    __shared__ float xsum[8][33];
+    const unsigned n_tt = (p_rows + 31u) / 32u, n_sub = in_dim >> 5, tt = blockIdx.x, c = blockIdx.y;
+    const unsigned j = threadIdx.x >> 3, s = threadIdx.x & 7u, tok = tt * 32u + j, sb = c * 8u + s;
+
+    float v[32];
+    float d = 0.0f, inv = 0.0f, sum = 0.0f;
+    if (tok < p_rows) {
+        const float* p = x + (size_t)tok * in_dim + sb * 32u;
+        if (((size_t)x & 15u) == 0u) {
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                const float4 f = reinterpret_cast<const float4*>(p)[i];
+                v[4 * i] = f.x; v[4 * i + 1] = f.y; v[4 * i + 2] = f.z; v[4 * i + 3] = f.w;
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < 32; i++) v[i] = p[i];
+        }
+        float amax = 0.0f, t[16];
+#pragma unroll
+        for (int i = 0; i < 32; i++) amax = fmaxf(amax, fabsf(v[i]));
+#pragma unroll
+        for (int i = 0; i < 16; i++) t[i] = v[i] + v[i + 16];
+#pragma unroll
+        for (int m = 8; m >= 1; m >>= 1)
+#pragma unroll
+            for (int i = 0; i < m; i++) t[i] = t[i] + t[i + m];
+        sum = t[0];
+        d   = amax > 0.0f ? amax / 127.0f : 1.0f;
+        inv = amax > 0.0f ? 127.0f / amax : 0.0f;
+    } else {
+#pragma unroll
+        for (int i = 0; i < 32; i++) v[i] = 0.0f;
+    }
+    uint8_t* rec = img + ((size_t)(sb >> 1) * n_tt + tt) * REIN_XH_REC;
+    reinterpret_cast<float*>(rec + REIN_XH_X)[(sb & 1u) * 32u + j] = d;
+#pragma unroll
+    for (int kh = 0; kh < 2; kh++)
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            rein_v8h o;
+#pragma unroll
+            for (int e = 0; e < 8; e++) o[e] = (_Float16)max(-127, min(127, (int)rintf(v[rein_xh_slot_weight(kh, h, e)] * inv)));
+            *reinterpret_cast<rein_v8h*>(rec + (sb & 1u) * 2048u + kh * 1024u + (32u * h + j) * 16u) = o;
+        }
+    if (!with_xsum) return;                          // the image of a format without minimums has no xsum part
+    xsum[s][j] = sum;
+    __syncthreads();
+    if (threadIdx.x < 128u) {                        // op = threadIdx.x / 64, lane = threadIdx.x % 64
+        const unsigned op = threadIdx.x >> 6, h = (threadIdx.x >> 5) & 1u;
+        uint32_t o[4] = {0u, 0u, 0u, 0u};
+        if (op == 0u || h == 0u) {
+#pragma unroll
+            for (int k = 0; k < 8; k++) {
+                uint16_t p3[3];
+                rein_mmq_split_xsum(xsum[k][threadIdx.x & 31u], p3);
+                const uint32_t b = op ? p3[2] : (h ? p3[1] : p3[0]);
+                o[k >> 1] |= b << (16 * (k & 1));
+            }
+        }
+        uint8_t* dst = img + (size_t)(n_sub >> 1) * n_tt * REIN_XH_REC + ((size_t)c * n_tt + tt) * REIN_XH_XS;
+        *reinterpret_cast<uint4*>(dst + threadIdx.x * 16u) = make_uint4(o[0], o[1], o[2], o[3]);
+    }
+}
+
+// Token tiles are dealt evenly over ceil(tiles / 4) groups: 25 tiles are four groups of 4 and three of 3, not six of 4 and
+// one of 1.  From three tiles on every group has at least two.
+struct XhGroup { unsigned tile, n; };
+__device__ __forceinline__ XhGroup rein_xh_group(unsigned p_rows, unsigned g)
+{
+    const unsigned n_tt = (p_rows + 31u) >> 5, n_grp = (n_tt + 3u) >> 2, base = n_tt / n_grp, more = n_tt - base * n_grp;
+    return XhGroup{g * base + min(g, more), base + (g < more ? 1u : 0u)};
+}
+
+// ---- weight operands ------------------------------------------------------------------
+// A nibble or-ed into the mantissa of 1024 (low nibble) or 64 (high nibble, which sits four bits up) is 1024 + n or 64 + n;
+// one packed fma with the scale takes the offset out again, exactly: (1024 + n) sc - 1024 sc.
+// (v & mask) | base as one instruction, which takes one constant out of a scalar register and needs the other in a vector one
+struct XhMasks {
+    uint32_t lo, hi, two;                            // low nibbles, high nibbles, bits 8, 9 of both halves
+    __device__ __forceinline__ XhMasks() : lo(0x000F000Fu), hi(0x00F000F0u), two(0x03000300u)
+    {
+        asm volatile("" : "+v"(lo), "+v"(hi), "+v"(two));
+    }
+};
+__device__ __forceinline__ uint32_t rein_xh_or(uint32_t v, uint32_t mask, uint32_t base) { return (v & mask) | base; }
+__device__ __forceinline__ rein_h2 rein_xh_fma(uint32_t v, rein_h2 sc, rein_h2 c) { return __builtin_elementwise_fma(__builtin_bit_cast(rein_h2, v), sc, c); }
+__device__ __forceinline__ rein_h2 rein_xh_splat(float v) { return rein_h2{(_Float16)v, (_Float16)v}; }
+__device__ __forceinline__ rein_v8h rein_xh_join(rein_h2 a, rein_h2 b, rein_h2 c, rein_h2 d)
+{
+    return rein_v8h{a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
+}
+
+template <int FMT> struct XhWeights;
+
+template <> struct XhWeights<REIN_Q4_K> {
+    static constexpr int kOps = 1;                   // operands per instruction position
+    static constexpr bool kHasMin = true;
+    static constexpr float kUnit = 1.0f;             // what the operands were divided by
+    // plane of extra bits: bytes per sub-block (0: none) and the lane half's word in them; plane of the superblocks' scales
+    static constexpr unsigned kHiBytes = 0, kHiHalf = 0, kDBytes = 4;
+    static __device__ __forceinline__ const char* hi(const Fmt<REIN_Q4_K>&) { return nullptr; }
+    static __device__ __forceinline__ const char* d(const Fmt<REIN_Q4_K>& f) { return reinterpret_cast<const char*>(f.ddp); }
+    static __device__ __forceinline__ float scale(uint32_t dd) { return rein_h2f((uint16_t)(dd & 0xFFFFu)); }
+    static __device__ __forceinline__ float min_scale(uint32_t dd) { return -rein_h2f((uint16_t)(dd >> 16)); }
+    // words 2h, 2h + 1 of a sub-block's nibbles and its (sc, m)
+    static __device__ __forceinline__ void unpack(rein_v8h (&o)[2][kOps], uint2 w2, uint32_t, uint32_t sm, unsigned, const XhMasks& mk)
+    {
+        const float scf = (float)(sm & 0xFFu);
+        const rein_h2 sc = rein_xh_splat(scf), c1024 = rein_xh_splat(scf * -1024.0f), c64 = rein_xh_splat(scf * -64.0f);
+#pragma unroll
+        for (int kh = 0; kh < 2; kh++) {
+            const uint32_t w = kh ? w2.y : w2.x, w8 = w >> 8;
+            o[kh][0] = rein_xh_join(rein_xh_fma(rein_xh_or(w, mk.lo, 0x64006400u), sc, c1024), rein_xh_fma(rein_xh_or(w, mk.hi, 0x54005400u), sc, c64),
+                                    rein_xh_fma(rein_xh_or(w8, mk.lo, 0x64006400u), sc, c1024), rein_xh_fma(rein_xh_or(w8, mk.hi, 0x54005400u), sc, c64));
+        }
+    }
+};
+
+template <> struct XhWeights<REIN_Q5_K> {
+    static constexpr int kOps = 1;
+    static constexpr bool kHasMin = true;
+    static constexpr float kUnit = 1.0f;
+    static constexpr unsigned kHiBytes = 4, kHiHalf = 0, kDBytes = 4;
+    static __device__ __forceinline__ const char* hi(const Fmt<REIN_Q5_K>& f) { return reinterpret_cast<const char*>(f.qhp); }
+    static __device__ __forceinline__ const char* d(const Fmt<REIN_Q5_K>& f) { return reinterpret_cast<const char*>(f.ddp); }
+    static __device__ __forceinline__ float scale(uint32_t dd) { return rein_h2f((uint16_t)(dd & 0xFFFFu)); }
+    static __device__ __forceinline__ float min_scale(uint32_t dd) { return -rein_h2f((uint16_t)(dd >> 16)); }
+    // words 2h, 2h + 1 of a sub-block's nibbles, its fifth bits and (sc, m)
+    static __device__ __forceinline__ void unpack(rein_v8h (&o)[2][kOps], uint2 w2, uint32_t qh, uint32_t sm, unsigned h, const XhMasks& mk)
+    {
+        const float scf = (float)(sm & 0xFFu);
+        const rein_h2 sc = rein_xh_splat(scf), c1024 = rein_xh_splat(scf * -1024.0f), c64 = rein_xh_splat(scf * -64.0f);
+        const uint32_t q = qh >> (16u * h), q2 = q >> 2;      // bits f of byte kh: weights f of the low nibbles, bits 4 + f: of the high
+#pragma unroll
+        for (int kh = 0; kh < 2; kh++) {
+            const uint32_t w = kh ? w2.y : w2.x, w8 = w >> 8;
+            // byte kh with elements 0, 1 in the low half, elements 2, 3 in the high half
+            const uint32_t p = __builtin_amdgcn_perm(q2, q, kh ? 0x0C050C01u : 0x0C040C00u), p4 = p << 4, p3 = p << 3;
+            const uint32_t r0 = rein_xh_or(p4, 0x00100010u, rein_xh_or(w, mk.lo, 0x64006400u));
+            const uint32_t r1 = rein_xh_or(p4, 0x01000100u, rein_xh_or(w, mk.hi, 0x54005400u));
+            const uint32_t r2 = rein_xh_or(p3, 0x00100010u, rein_xh_or(w8, mk.lo, 0x64006400u));
+            const uint32_t r3 = rein_xh_or(p3, 0x01000100u, rein_xh_or(w8, mk.hi, 0x54005400u));
+            o[kh][0] = rein_xh_join(rein_xh_fma(r0, sc, c1024), rein_xh_fma(r1, sc, c64), rein_xh_fma(r2, sc, c1024), rein_xh_fma(r3, sc, c64));
+        }
+    }
+};
+
+template <> struct XhWeights<REIN_Q6_K> {
+    static constexpr int kOps = 2;
+    static constexpr bool kHasMin = false;
+    static constexpr float kUnit = 4.0f;
+    static constexpr unsigned kHiBytes = 8, kHiHalf = 4, kDBytes = 2;
+    static __device__ __forceinline__ const char* hi(const Fmt<REIN_Q6_K>& f) { return reinterpret_cast<const char*>(f.h2p); }
+    static __device__ __forceinline__ const char* d(const Fmt<REIN_Q6_K>& f) { return reinterpret_cast<const char*>(f.dp); }
+    static __device__ __forceinline__ float scale(uint32_t dd) { return rein_h2f((uint16_t)dd) * kUnit; }
+    static __device__ __forceinline__ float min_scale(uint32_t) { return 0.0f; }
+    // Words 2h, 2h + 1 of a sub-block's nibbles, the word of two-bit fields that goes with them, both group scales.  Low nibbles
+    // are weights 0..15 (first scale), high ones 16..31 (second).  A two-bit field at bits 8, 9 of 4.0 is 4 + c:
+    // (4 + c) 4 sc - 24 sc = 4 (c - 2) sc; 4 sc is at most 512, 24 sc has 9 bits: exact.  The nibble term is held as a quarter,
+    // so that 1024 * sc / 4 stays inside fp16.
+    static __device__ __forceinline__ void unpack(rein_v8h (&o)[2][kOps], uint2 w2, uint32_t hw, uint32_t sm, unsigned, const XhMasks& mk)
+    {
+        const float a = (float)(int)(int8_t)(sm & 0xFFu), b = (float)(int)(int8_t)((sm >> 8) & 0xFFu);
+        const rein_h2 na = rein_xh_splat(a * 0.25f), nb = rein_xh_splat(b * 0.25f), ca = rein_xh_splat(a * -256.0f), cb = rein_xh_splat(b * -16.0f);
+        const rein_h2 ha = rein_xh_splat(a * 4.0f), hb = rein_xh_splat(b * 4.0f), ga = rein_xh_splat(a * -24.0f), gb = rein_xh_splat(b * -24.0f);
+        const uint32_t hw4 = hw >> 4;
+#pragma unroll
+        for (int kh = 0; kh < 2; kh++) {
+            const uint32_t w = kh ? w2.y : w2.x, w8 = w >> 8;
+            o[kh][0] = rein_xh_join(rein_xh_fma(rein_xh_or(w, mk.lo, 0x64006400u), na, ca), rein_xh_fma(rein_xh_or(w, mk.hi, 0x54005400u), nb, cb),
+                                    rein_xh_fma(rein_xh_or(w8, mk.lo, 0x64006400u), na, ca), rein_xh_fma(rein_xh_or(w8, mk.hi, 0x54005400u), nb, cb));
+            // byte 2 kh (weights of the low nibbles) / 2 kh + 1 (of the high ones): elements 0, 1 to bits 8..11, 2, 3 to bits 24..27
+            const uint32_t pa = __builtin_amdgcn_perm(hw4, hw, kh ? 0x060C020Cu : 0x040C000Cu), pa2 = pa >> 2;
+            const uint32_t pb = __builtin_amdgcn_perm(hw4, hw, kh ? 0x070C030Cu : 0x050C010Cu), pb2 = pb >> 2;
+            o[kh][1] = rein_xh_join(rein_xh_fma(rein_xh_or(pa, mk.two, 0x44004400u), ha, ga), rein_xh_fma(rein_xh_or(pb, mk.two, 0x44004400u), hb, gb),
+                                    rein_xh_fma(rein_xh_or(pa2, mk.two, 0x44004400u), ha, ga), rein_xh_fma(rein_xh_or(pb2, mk.two, 0x44004400u), hb, gb));
+        }
+    }
+};
+
+// Sums tied to this point of the program: instruction selection otherwise moves them past the scheduling fences
+__device__ __forceinline__ void rein_xh_pin(float (&s)[16])
+{
+    asm volatile("" : "+v"(s[0]), "+v"(s[1]), "+v"(s[2]), "+v"(s[3]), "+v"(s[4]), "+v"(s[5]), "+v"(s[6]), "+v"(s[7]));
+    asm volatile("" : "+v"(s[8]), "+v"(s[9]), "+v"(s[10]), "+v"(s[11]), "+v"(s[12]), "+v"(s[13]), "+v"(s[14]), "+v"(s[15]));
+}
+
+// ---- the tile -------------------------------------------------------------------------
+// LDS of one workgroup:
+//   acts  2 x 4 x 4352     records of two consecutive sub-block pairs
+//   ring  4 x 2 x 2048     per wavefront: two slots of 4 sub-blocks x 32 rows x 16 B
+//   small 4 x 3584         per wavefront: extra bits of a superblock [sub-block][lane], (sc, m) or both group scales
+//                          [row][sub-block], each in a dword, and the scale words of two superblocks [row]
+//   xs    4 x 2048             xsum operands of a superblock (formats with minimums)
+template <int FMT> constexpr unsigned rein_xh_lds_bytes()
+{
+    return 8u * REIN_XH_REC + 4u * 2u * 2048u + 4u * 3584u + (XhWeights<FMT>::kHasMin ? 4u * REIN_XH_XS : 0u);
+}
+
+// Superblocks [c0, c1) of rows 128 rb .. and the NT token tiles from `tile` on, into acc.  One barrier per sub-block
+// pair: at its top everything in flight has landed (it was issued a whole pair earlier: 8 NT or 16 NT matrix instructions per
+// wavefront), behind it the next pair's transfers go out.
+template <int FMT, int NT>
+__device__ __forceinline__ void rein_xh_acc(const uint8_t* __restrict__ w, const uint8_t* __restrict__ img, unsigned in_dim, unsigned out_dim,
+                                            unsigned n_tt, unsigned rb, unsigned tile, unsigned c0, unsigned c1, unsigned char* const raw, float (&acc)[NT][16])
+{
+    using W = XhWeights<FMT>;
+    typedef __attribute__((address_space(3))) const void* lptr_t;
+    constexpr unsigned kRing = 8u * REIN_XH_REC, kSmall = kRing + 4u * 4096u, kXs = kSmall + 4u * 3584u;
+    const unsigned lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), j = lane & 31u, h = lane >> 5;
+    const unsigned n_sub = in_dim >> 5;
+    const Fmt<FMT> fmt(w, n_sub, out_dim);
+    const unsigned row_base = rb * 128u + wave * 32u, first = min(row_base, out_dim - 1u);
+    // rows past the matrix read its last one; offsets from the wavefront's first row
+    const unsigned row = min(row_base + j, out_dim - 1u) - first;
+    const unsigned hi_off = row * fmt.nsp * W::kHiBytes + h * W::kHiHalf, d_off = row * fmt.n_super * W::kDBytes;
+    unsigned sm_off[4];
+#pragma unroll
+    for (unsigned k = 0; k < 4; k++) sm_off[k] = ((min(row_base + 8u * k + (lane >> 3), out_dim - 1u) - first) * fmt.nsp + (lane & 7u)) * 2u;
+
+    const uint4* const ring = reinterpret_cast<const uint4*>(raw + kRing + wave * 4096u);
+    const uint32_t* const small = reinterpret_cast<const uint32_t*>(raw + kSmall + wave * 3584u);
+    const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(lptr_t)raw);
+    MmqWSrc<FMT> wsrc;
+    wsrc.init(*reinterpret_cast<const MmqWLds<FMT>*>(ring), fmt, row_base, out_dim, lane);
+    const uint8_t* const xsimg = img + (size_t)(n_sub >> 1) * n_tt * REIN_XH_REC;
+
+    auto issue_acts = [&](unsigned pair) {
+        const uint8_t* src = img + ((size_t)pair * n_tt + tile) * REIN_XH_REC;
+        const unsigned buf = lds0 + (pair & 1u) * (4u * REIN_XH_REC);
+#pragma unroll
+        for (unsigned t = 0; t < (unsigned)NT; t++) {
+            const unsigned off = t * REIN_XH_REC + wave * 1024u;
+            rein_lds_dma16_s(lane * 16u, src + off, buf + off);
+        }
+        if (wave < (unsigned)NT) rein_xh_dma_u32(lane * 4u, src + wave * REIN_XH_REC + REIN_XH_X, buf + wave * REIN_XH_REC + REIN_XH_X);
+    };
+    auto issue_xs = [&](unsigned c) {
+        if constexpr (W::kHasMin) {
+            const uint8_t* src = xsimg + ((size_t)c * n_tt + tile) * REIN_XH_XS;
+#pragma unroll
+            for (unsigned k = 0; k < 2; k++) {
+                const unsigned off = (k * 4u + wave) * 1024u;
+                if (k * 4u + wave < 2u * NT) rein_lds_dma16_s(lane * 16u, src + off, lds0 + kXs + off);
+            }
+        }
+    };
+    auto issue_small = [&](unsigned c) {
+        const unsigned dst = lds0 + kSmall + wave * 3584u;
+        if constexpr (W::kHiBytes != 0) {
+            const char* hp = W::hi(fmt) + ((size_t)first * fmt.nsp + c * 8u) * W::kHiBytes;
+#pragma unroll
+            for (unsigned k = 0; k < 8; k++) rein_xh_dma_u32(hi_off, hp + k * W::kHiBytes, dst + k * 256u);
+        }
+        const char* sp = reinterpret_cast<const char*>(fmt.smp) + ((size_t)first * fmt.nsp + c * 8u) * 2u;
+#pragma unroll
+        for (unsigned k = 0; k < 4; k++) rein_xh_dma_u16(sm_off[k], sp, dst + 2048u + k * 256u);
+        const char* dp = W::d(fmt) + ((size_t)first * fmt.n_super + c) * W::kDBytes;
+        if constexpr (W::kDBytes == 4) rein_xh_dma_u32(d_off, dp, dst + 3072u + (c & 1u) * 256u);
+        else rein_xh_dma_u16(d_off, dp, dst + 3072u + (c & 1u) * 256u);
+    };
+    rein_v16f dot[2], z16;
+    float s1[NT][16];
+    float dx[2] = {0.0f, 0.0f};
+#pragma unroll
+    for (int v = 0; v < 16; v++) z16[v] = 0.0f;
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) acc[t][v] = s1[t][v] = 0.0f;
+    dot[0] = dot[1] = z16;
+
+    __syncthreads();                                 // the LDS may still be read by the caller's previous tile
+    issue_acts(c0 * 4u);
+    issue_small(c0);
+    rein_mmq_wload<FMT>(wsrc, 0u, fmt, c0 * 8u, n_sub);
+    const unsigned rot = j >> 1;
+    const XhMasks mk;
+
+    for (unsigned c = c0; c < c1; c++) {
+        uint32_t mpk[4];                             // the superblock's minimums as bf16
+#pragma unroll
+        for (unsigned u = 0; u < 4; u++) {
+            const unsigned pair = c * 4u + u;
+            const bool last = c + 1u == c1;
+            REIN_WAIT_VMCNT(0);
+            __syncthreads();
+            const uint2 sm2 = *reinterpret_cast<const uint2*>(small + 512u + j * 8u + 2u * u);
+            const uint32_t hi2[2] = {small[2u * u * 64u + lane], small[(2u * u + 1u) * 64u + lane]};
+            if (u < 3u || !last) issue_acts(pair + 1u);
+            if (u == 0u) rein_mmq_wload<FMT>(wsrc, 1u, fmt, c * 8u + 4u, n_sub);
+            if (u == 1u) issue_xs(c);                // read at the superblock's end; the barrier of u = 0 freed it
+            if (u == 2u && !last) rein_mmq_wload<FMT>(wsrc, 0u, fmt, c * 8u + 8u, n_sub);
+            if (u == 3u && !last) {
+                __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the reads above have left the buffer
+                issue_small(c + 1u);
+            }
+            const unsigned char* const act = raw + (pair & 1u) * (4u * REIN_XH_REC);
+#pragma unroll
+            for (unsigned q = 0; q < 2; q++) {
+                const unsigned sb = 2u * u + q, s4 = sb & 3u;
+                const uint2 w2 = reinterpret_cast<const uint2*>(ring + (u >> 1) * 128u + 4u * j + ((s4 + rot) & 3u))[h];
+                rein_v8h a[2][W::kOps];
+                const uint32_t sm = q ? sm2.y : sm2.x;
+                W::unpack(a, w2, hi2[q], sm, h, mk);
+                if constexpr (W::kHasMin) {
+                    const uint32_t m = rein_bf16_of_u8(sm >> 8);
+                    if (q == 0u) mpk[u] = m; else mpk[u] |= m << 16;
+                }
+                const float* const dxp = reinterpret_cast<const float*>(act + REIN_XH_X) + q * 32u + j;
+                const unsigned char* const x = act + q * 2048u + lane * 16u;
+                rein_v8h xa[2][2];
+                xa[0][0] = *reinterpret_cast<const rein_v8h*>(x);
+                xa[0][1] = *reinterpret_cast<const rein_v8h*>(x + 1024u);
+                __builtin_amdgcn_sched_barrier(0);
+                // Stage t: tile t's dots in the matrix unit, the multiply-adds of the tile before (the last tile of the
+                // previous sub-block for t = 0) under them, the next tile's operand reads.  The fences keep the stages as
+                // written: left alone, the scheduler starts all tiles at once and spills.
+#pragma unroll
+                for (int t = 0; t < NT; t++) {
+                    const int now = (int)(sb * NT + t) & 1;
+                    if (t + 1 < NT) {
+                        xa[(t + 1) & 1][0] = *reinterpret_cast<const rein_v8h*>(x + (t + 1) * REIN_XH_REC);
+                        xa[(t + 1) & 1][1] = *reinterpret_cast<const rein_v8h*>(x + (t + 1) * REIN_XH_REC + 1024u);
+                    }
+                    dot[now] = z16;
+#pragma unroll
+                    for (int k = 0; k < W::kOps; k++) {
+                        dot[now] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[0][k], xa[t & 1][0], dot[now], 0, 0, 0);
+                        dot[now] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[1][k], xa[t & 1][1], dot[now], 0, 0, 0);
+                    }
+                    dx[now] = dxp[t * (REIN_XH_REC / 4u)];
+                    if (sb * NT + t > 0u) {
+                        const int tp = (t + NT - 1) % NT;
+                        const bool first = sb * NT + t <= (unsigned)NT;              // the sums' first term of this superblock
+#pragma unroll
+                        for (int v = 0; v < 16; v++) s1[tp][v] = first ? dx[now ^ 1] * dot[now ^ 1][v] : fmaf(dx[now ^ 1], dot[now ^ 1][v], s1[tp][v]);
+                        rein_xh_pin(s1[tp]);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+        }
+        {
+            constexpr int end = (8 * NT - 1) & 1;
+#pragma unroll
+            for (int v = 0; v < 16; v++) s1[NT - 1][v] = fmaf(dx[end], dot[end][v], s1[NT - 1][v]);
+        }
+        // acc += d s1 - dmin (m . xsum): register v is weight row 8 (v / 4) + 4 h + v % 4
+        const unsigned char* const xb = raw + kXs + lane * 16u;
+        float dv[16], nv[16];
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            const uint4 d4 = *reinterpret_cast<const uint4*>(small + 768u + (c & 1u) * 64u + 8 * g + 4u * h);
+            const uint32_t dw[4] = {d4.x, d4.y, d4.z, d4.w};
+#pragma unroll
+            for (int v = 0; v < 4; v++) { dv[4 * g + v] = W::scale(dw[v]); nv[4 * g + v] = W::min_scale(dw[v]); }
+        }
+#pragma unroll
+        for (int t = 0; t < NT; t++) {
+#pragma unroll
+            for (int v = 0; v < 16; v++) acc[t][v] = fmaf(dv[v], s1[t][v], acc[t][v]);
+            if constexpr (W::kHasMin) {
+                const rein_v8bf m = __builtin_bit_cast(rein_v8bf, make_uint4(mpk[0], mpk[1], mpk[2], mpk[3]));
+                rein_v16f s2 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(m, *reinterpret_cast<const rein_v8bf*>(xb + t * 2048u), z16, 0, 0, 0);
+                s2 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(m, *reinterpret_cast<const rein_v8bf*>(xb + t * 2048u + 1024u), s2, 0, 0, 0);
+#pragma unroll
+                for (int v = 0; v < 16; v++) acc[t][v] = fmaf(nv[v], s2[v], acc[t][v]);
+            }
+        }
+    }
+    REIN_WAIT_VMCNT(0);
+}
+
+// One piece of the launch: superblocks [c0, c1) of unit (rb, grp), to y or (part not null) to a partial tile
+// [t][v / 4][thread] of float4.
+template <int FMT, int NT>
+__device__ __forceinline__ void rein_xh_piece(const uint8_t* __restrict__ w, const uint8_t* __restrict__ img, float* __restrict__ y, float* __restrict__ part,
+                                              unsigned in_dim, unsigned out_dim, unsigned p_rows, unsigned rb, unsigned tile, unsigned c0, unsigned c1,
+                                              unsigned char* raw)
+{
+    float acc[NT][16];
+    rein_xh_acc<FMT, NT>(w, img, in_dim, out_dim, (p_rows + 31u) / 32u, rb, tile, c0, c1, raw, acc);
+    const unsigned lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, j = lane & 31u, h = lane >> 5;
+    if (part) {
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+#pragma unroll
+            for (int g = 0; g < 4; g++)
+                reinterpret_cast<float4*>(part)[(t * 4 + g) * 256 + threadIdx.x] = make_float4(acc[t][4 * g], acc[t][4 * g + 1], acc[t][4 * g + 2], acc[t][4 * g + 3]);
+        return;
+    }
+    const bool wide = (out_dim & 3u) == 0u && ((size_t)y & 15u) == 0u;
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+        const unsigned tok = (tile + t) * 32u + j;
+        if (tok >= p_rows) continue;
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            const unsigned row = rb * 128u + wave * 32u + 8u * g + 4u * h;
+            float* o = y + (size_t)tok * out_dim + row;
+            if (wide) {
+                if (row < out_dim) *reinterpret_cast<float4*>(o) = make_float4(acc[t][4 * g], acc[t][4 * g + 1], acc[t][4 * g + 2], acc[t][4 * g + 3]);
+            } else {
+#pragma unroll
+                for (unsigned v = 0; v < 4; v++)
+                    if (row + v < out_dim) o[v] = acc[t][4 * g + v];
+            }
+        }
+    }
+}
+
+// Units u = (128-row block u / n_grp, token group u % n_grp).  The first n_whole (whole rounds of 512 workgroups, two per
+// CU) are one workgroup each; the others are cut into `split` ranges of superblocks, a workgroup each, whose partial tiles
+// rein_xh_sum_body adds in range order.  Workgroup i runs on XCD i % 8: neighbouring units and ranges go to one XCD, so the
+// token groups of a row block meet its weights in one L2.  Grid: n_whole + 8 ceil((units - n_whole) split / 8).
+__device__ __forceinline__ unsigned rein_xh_deal(unsigned i, unsigned n)
+{
+    const unsigned per = (n + 7u) >> 3, k = i >> 3;
+    return k < per ? (i & 7u) * per + k : 0xFFFFFFFFu;
+}
+template <int FMT>
+__device__ __forceinline__ void rein_xh_dense(const uint8_t* __restrict__ w, const uint8_t* __restrict__ img, float* __restrict__ y, float* __restrict__ parts,
+                                              unsigned in_dim, unsigned out_dim, unsigned p_rows, unsigned n_whole, unsigned split)
+{
+    extern __shared__ __attribute__((aligned(16))) unsigned char rein_xh_lds[];
+    const unsigned n_grp = (p_rows + 127u) / 128u, n_unit = ((out_dim + 127u) / 128u) * n_grp, n_chunk = in_dim >> 8;
+    unsigned u, c0 = 0u, c1 = n_chunk;
+    float* part = nullptr;
+    if (blockIdx.x < n_whole) {
+        u = (blockIdx.x & ~511u) + rein_xh_deal(blockIdx.x & 511u, 512u);
+    } else {
+        const unsigned n_seg = (n_unit - n_whole) * split, seg = rein_xh_deal(blockIdx.x - n_whole, n_seg);
+        if (seg >= n_seg) return;
+        const unsigned tu = seg / split, k = seg - tu * split;
+        u = n_whole + tu;
+        c0 = n_chunk * k / split; c1 = n_chunk * (k + 1u) / split;       // split <= n_chunk: no range is empty
+        if (split > 1u) part = parts + (size_t)seg * (4u * 16u * 256u);
+    }
+    if (u >= n_unit) return;
+    const unsigned rb = u / n_grp;
+    const XhGroup g = rein_xh_group(p_rows, u - rb * n_grp);
+    if (g.n == 4u) rein_xh_piece<FMT, 4>(w, img, y, part, in_dim, out_dim, p_rows, rb, g.tile, c0, c1, rein_xh_lds);
+    else if (g.n == 3u) rein_xh_piece<FMT, 3>(w, img, y, part, in_dim, out_dim, p_rows, rb, g.tile, c0, c1, rein_xh_lds);
+    else if (g.n == 2u) rein_xh_piece<FMT, 2>(w, img, y, part, in_dim, out_dim, p_rows, rb, g.tile, c0, c1, rein_xh_lds);
+}
+
+// y of the split units.  Grid (units - n_whole, 16): blockIdx.y = 4 t + v / 4, 256 threads as in the GEMM.
+__device__ __forceinline__ void rein_xh_sum_body(const float* __restrict__ parts, float* __restrict__ y, unsigned out_dim, unsigned p_rows, unsigned n_whole, unsigned split)
+{
+    const unsigned n_grp = (p_rows + 127u) / 128u, u = n_whole + blockIdx.x, rb = u / n_grp;
+    const XhGroup grp = rein_xh_group(p_rows, u - rb * n_grp);
+    const unsigned lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, j = lane & 31u, h = lane >> 5, t = blockIdx.y >> 2, g = blockIdx.y & 3u;
+    const unsigned tok = (grp.tile + t) * 32u + j, row = rb * 128u + wave * 32u + 8u * g + 4u * h;
+    if (t >= grp.n || tok >= p_rows) return;
+    float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    const float4* src = reinterpret_cast<const float4*>(parts + (size_t)blockIdx.x * split * (4u * 16u * 256u)) + blockIdx.y * 256u + threadIdx.x;
+#pragma unroll 4
+    for (unsigned k = 0; k < split; k++) {
+        const float4 p = src[(size_t)k * (4u * 4u * 256u)];
+        s[0] += p.x; s[1] += p.y; s[2] += p.z; s[3] += p.w;
+    }
+    float* o = y + (size_t)tok * out_dim + row;
+    if ((out_dim & 3u) == 0u && ((size_t)y & 15u) == 0u) {
+        if (row < out_dim) *reinterpret_cast<float4*>(o) = make_float4(s[0], s[1], s[2], s[3]);
+        return;
+    }
+#pragma unroll
+    for (unsigned v = 0; v < 4; v++)
+        if (row + v < out_dim) o[v] = s[v];
+}

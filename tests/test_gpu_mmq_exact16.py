@@ -1,0 +1,106 @@
+"""The Q4_K / Q5_K / Q6_K prefill GEMM with exact block dots on the fp16 instruction (kernels/mmq_exact16.h, taken by rein_matmul_ws),
+at the edges of its tiles, against the CPU oracle, and its distance from 64-bit sums beside the int8 tile's."""
+import numpy as np
+import pytest
+
+import reinstinct_amd as rein
+from oracle import orc
+from reinstinct_amd import hip, quant, runtime
+from reinstinct_amd._lib import init, set_option
+from tests.helpers import assert_close_f32
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True)
+def _options():
+    init()
+    hip.set_device(0)
+    yield
+    for name in ("REIN_MMQXH", "REIN_MMQXH_SPLIT"):
+        set_option(name, None)
+
+
+def matmul(fmt, packed, x, out_dim, mode, split=None):
+    rows, in_dim = x.shape
+    set_option("REIN_MMQXH", str(mode))
+    set_option("REIN_MMQXH_SPLIT", split and str(split))
+    size = runtime.matmul_scratch_bytes(fmt, in_dim, rows)
+    dw, dx, scratch = hip.DeviceBuf.from_host(packed), hip.DeviceBuf.from_host(x), hip.DeviceBuf(size)
+    guard = 64                                        # words behind the output that must stay as they are
+    dy = hip.DeviceBuf.from_host(np.full(rows * out_dim + guard, 12345.0, np.float32))
+    print(f"fmt {fmt} rows {rows} in {in_dim} out {out_dim} mode {mode} split {split}", flush=True)
+    runtime.matmul_ws(fmt, dw, dx, dy, in_dim, out_dim, rows, scratch, size)
+    hip.synchronize()
+    y = dy.to_host(np.float32)
+    assert (y[rows * out_dim:] == 12345.0).all()
+    return y[:rows * out_dim].reshape(rows, out_dim)
+
+
+def weights(fmt, in_dim, out_dim, seed):
+    w = np.random.default_rng(seed).standard_normal((out_dim, in_dim)).astype(np.float32) * 0.02
+    return quant.repack_for_matvec(fmt, quant.quantize_weights(fmt, w), in_dim, out_dim)
+
+
+@pytest.mark.parametrize("fmt", [rein.Q4_K, rein.Q5_K, rein.Q6_K])
+@pytest.mark.parametrize("rows, in_dim, out_dim, split", [
+    (65, 256, 5, None),          # three token tiles, one superblock, a row block almost empty, scalar stores
+    (128, 512, 128, None),       # one whole unit; padded weight rows (16 sub-blocks)
+    (90, 768, 130, 3),           # a range per superblock
+    (128, 2048, 264, 1),
+    (129, 1280, 127, 2),         # groups of three and two tiles
+    (300, 2304, 257, 4),         # uneven ranges of nine superblocks
+    (777, 512, 96, None),
+])
+def test_against_the_oracle(fmt, rows, in_dim, out_dim, split):
+    packed = weights(fmt, in_dim, out_dim, rows)
+    x = np.random.default_rng(in_dim).standard_normal((rows, in_dim)).astype(np.float32)
+    x[0] *= 1e-20
+    x[rows // 2] = 0.0
+    x[rows - 1] *= 1e20
+    got = matmul(fmt, packed, x, out_dim, 2, split)
+    want = orc.matvec_q8(fmt, packed, in_dim, out_dim, orc.quantize_q8(x), rows)
+    scale = np.abs(x).max(axis=1, keepdims=True) + (np.abs(x).max(axis=1, keepdims=True) == 0)
+    assert_close_f32(got / scale, want / scale, what=f"fmt {fmt}")
+
+
+@pytest.mark.parametrize("fmt", [rein.Q4_K, rein.Q5_K, rein.Q6_K])
+def test_no_further_from_64_bits_than_the_int8_tile(fmt):
+    rows, in_dim, out_dim = 160, 4352, 256
+    w = quant.quantize_weights(fmt, np.random.default_rng(1).standard_normal((out_dim, in_dim)).astype(np.float32) * 0.02)
+    packed = quant.repack_for_matvec(fmt, w, in_dim, out_dim)
+    x = np.random.default_rng(2).standard_normal((rows, in_dim)).astype(np.float32)
+    q = orc.quantize_q8(x).reshape(-1, 40)
+    xd = (q[:, 8:].view(np.int8) * q[:, :4].copy().view(np.float32).astype(np.float64)).reshape(rows, in_dim)
+    if fmt == rein.Q6_K:
+        exact = xd @ orc.dequantize_to_f32(fmt, w, out_dim * in_dim).astype(np.float64).reshape(out_dim, in_dim).T
+    else:                                            # the minimum term goes with the blocks' xsum, not with their quants
+        blocks = w.reshape(out_dim * in_dim // 256, -1)
+        no_min, only_min = blocks.copy(), blocks.copy()
+        no_min[:, 2:4] = 0
+        only_min[:, 16:] = 0
+        part = [orc.dequantize_to_f32(fmt, b.reshape(-1), out_dim * in_dim).astype(np.float64).reshape(out_dim, in_dim) for b in (no_min, only_min)]
+        xsum = q[:, 4:8].copy().view(np.float32).astype(np.float64).reshape(rows, in_dim // 32)
+        exact = xd @ part[0].T + xsum @ part[1][:, ::32].T
+    err = [np.linalg.norm(matmul(fmt, packed, x, out_dim, mode) - exact) / np.linalg.norm(exact) for mode in (2, 0)]
+    print("relative error: exact dots", err[0], "int8 tile", err[1], flush=True)
+    assert err[0] <= 1.05 * err[1]
+
+
+def test_all_scales_and_quants_are_exact():
+    """every scale byte of Q6_K, -128 and 127 among them, against every quant: integers through and through"""
+    in_dim, out_dim, rows = 256, 256, 65
+    rng = np.random.default_rng(3)
+    blocks = np.zeros((out_dim, 210), np.uint8)
+    blocks[:, :192] = rng.integers(0, 256, (out_dim, 192))
+    blocks[:, 192:208] = (np.arange(out_dim)[:, None] + 16 * np.arange(16)[None, :]).astype(np.uint8)
+    blocks[:, 208:] = np.array([1.0], np.float16).view(np.uint8)
+    packed = quant.repack_for_matvec(rein.Q6_K, blocks.reshape(-1), in_dim, out_dim)
+    x = rng.integers(-15, 16, (rows, in_dim)).astype(np.float32)
+    x.reshape(rows, -1, 32)[:, :, 0] = 127.0         # activation scale 1
+    got = matmul(rein.Q6_K, packed, x, out_dim, 2)
+    w = orc.dequantize_to_f32(rein.Q6_K, blocks.reshape(-1), in_dim * out_dim).reshape(out_dim, in_dim).astype(np.int64)
+    want = x.astype(np.int64) @ w.T
+    exact = np.abs(want) < 1 << 22
+    assert exact.mean() > 0.5
+    assert (got.astype(np.int64) == want)[exact].all()
