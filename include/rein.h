@@ -411,7 +411,7 @@ int rein_matmul(int fmt, const void *w, const float *x, float *y, unsigned in_di
 /* rein_matmul with one scratch buffer of rein_matmul_scratch_bytes(fmt, in_dim, n_rows) bytes
  * (16-byte aligned) that holds the quantized activations and, for the MMQ path, the workspace
  * of rein_mmq_xq8_ws.  A scratch that only holds the activations runs rein_matmul.
- * Q4_K, Q5_K and Q6_K from 65 rows: a scratch of the full size runs the fp16-instruction GEMM with exact block
+ * Q4_K, Q5_K and Q6_K from 33 rows: a scratch of the full size runs the fp16-instruction GEMM with exact block
  * dots where it is the faster one (activation image and up to 64 MiB of partial tiles in the scratch; three
  * launches, no allocation); a smaller one runs what rein_mmq_xq8_ws takes for it. */
 size_t rein_matmul_scratch_bytes(int fmt, unsigned in_dim, unsigned n_rows);

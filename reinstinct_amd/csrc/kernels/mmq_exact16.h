@@ -24,7 +24,7 @@
 // and now: Q6_K 777 x 17408 -> 5120 523 / 379, 512 x 5120 -> 17408 307 / 208; Q5_K the same 190 / 167; Q4_K 147 / 145, 512 x
 // 17408 -> 5120 166 / 152.
 //
-// Replaces, from 65 rows, kernels/mmq_gemm_{q4k,q5k,q6k}_repacked.cpp of the reference behind rein_matmul_ws.
+// Replaces, from 33 rows, kernels/mmq_gemm_{q4k,q5k,q6k}_repacked.cpp of the reference behind rein_matmul_ws.
 #pragma once
 
 #include "mmq_fp6.h"
@@ -134,7 +134,7 @@ __device__ __forceinline__ void rein_xh_quantize_body(const float* __restrict__ 
 }
 
 // Token tiles are dealt evenly over ceil(tiles / 4) groups: 25 tiles are four groups of 4 and three of 3, not six of 4 and
-// one of 1.  From three tiles on every group has at least two.
+// one of 1.  From two tiles on every group has at least two.
 struct XhGroup { unsigned tile, n; };
 __device__ __forceinline__ XhGroup rein_xh_group(unsigned p_rows, unsigned g)
 {

@@ -44,8 +44,9 @@ def weights(fmt, in_dim, out_dim, seed):
 
 @pytest.mark.parametrize("fmt", [rein.Q4_K, rein.Q5_K, rein.Q6_K])
 @pytest.mark.parametrize("rows, in_dim, out_dim, split", [
-    (65, 256, 5, None),          # three token tiles, one superblock, a row block almost empty, scalar stores
+    (33, 256, 5, None),          # two token tiles, one superblock, a row block almost empty, scalar stores
     (128, 512, 128, None),       # one whole unit; padded weight rows (16 sub-blocks)
+    (64, 1024, 200, 2),
     (90, 768, 130, 3),           # a range per superblock
     (128, 2048, 264, 1),
     (129, 1280, 127, 2),         # groups of three and two tiles
