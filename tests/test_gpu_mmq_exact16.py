@@ -105,3 +105,33 @@ def test_all_scales_and_quants_are_exact():
     exact = np.abs(want) < 1 << 22
     assert exact.mean() > 0.5
     assert (got.astype(np.int64) == want)[exact].all()
+
+
+def test_smaller_scratch_and_capture():
+    """a scratch without the room runs the launches of rein_mmq_xq8_ws, bit for bit; a captured call replays to the eager bits"""
+    fmt, rows, in_dim, out_dim = rein.Q6_K, 200, 4096, 640
+    packed = weights(fmt, in_dim, out_dim, 5)
+    x = np.random.default_rng(6).standard_normal((rows, in_dim)).astype(np.float32)
+    size = runtime.matmul_scratch_bytes(fmt, in_dim, rows)
+    dw, dx, scratch, dy = hip.DeviceBuf.from_host(packed), hip.DeviceBuf.from_host(x), hip.DeviceBuf(size), hip.DeviceBuf(rows * out_dim * 4)
+
+    def call(n, stream=None):
+        runtime.matmul_ws(fmt, dw, dx, dy, in_dim, out_dim, rows, scratch, n, stream)
+
+    call(size)
+    hip.synchronize()
+    eager = dy.to_host(np.uint32)
+    call(size - 1)
+    hip.synchronize()
+    assert np.array_equal(dy.to_host(np.uint32).reshape(rows, out_dim), matmul(fmt, packed, x, out_dim, 0).view(np.uint32))
+    set_option("REIN_MMQXH", None)
+    stream = hip.Stream()
+    stream.begin_capture()
+    call(size, stream)
+    graph = stream.end_capture().instantiate()
+    for _ in range(3):
+        runtime.quantize_q8(dx, scratch, in_dim, rows)          # the program's own work on the same scratch between replays
+        hip.synchronize()
+        graph.launch(stream)
+        stream.synchronize()
+        assert np.array_equal(dy.to_host(np.uint32), eager)
