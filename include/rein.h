@@ -317,7 +317,8 @@ int rein_matvec_multi_xq8(unsigned n_mat, const int *fmts, const void *const *ws
 /* Which kernel a product of few activation rows launches, given the shape and the option table
  * (host logic only, nothing is launched): 1..8 rows as rein_matvec_xq8 / rein_matvec_batched_xq8
  * dispatch them, 9..32 rows the few-row kernels behind rein_mmq_xq8, "" where that entry point
- * launches token tiles.  The reference picks its kernels in qwen35.rs:2232-2280 by format alone;
+ * launches token tiles.  The name is the symbol of the code object, the suffix of a build included
+ * (_m, _p: how the kernel loads its weights).  The reference picks its kernels in qwen35.rs:2232-2280 by format alone;
  * here the choice also depends on the shape, and this call makes it visible. */
 int rein_matvec_kernel_name(int fmt, unsigned in_dim, unsigned out_dim, unsigned n_rows, char *name,
                             size_t name_len);

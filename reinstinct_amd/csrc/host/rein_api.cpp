@@ -269,6 +269,11 @@ unsigned pick_wpb(int fmt, unsigned groups, unsigned b)
     return wpb;
 }
 
+// The kernel names of the few-row families are put together in one place each: the launchers and rein_matvec_kernel_name
+// ask the same functions (skinny_name, mvl_name, mvql_name, mvq_name, mv_name).
+unsigned skinny_nv(unsigned n_rows) { return n_rows <= 2 ? 1 : n_rows <= 4 ? 2 : n_rows <= 8 ? 4 : 8; }
+KName skinny_name(int fmt, unsigned n_rows) { return KName("rein_mmqs_", fmt_tag(fmt), "_v", skinny_nv(n_rows)); }
+
 // Skinny MMQ launch: grid.x = 32-row tiles, grid.y = token groups, block = KS
 // wavefronts that split the contraction of one tile.  The kernels keep several
 // chunks of weights in flight in registers, which leaves room for two or three
@@ -281,7 +286,7 @@ unsigned pick_wpb(int fmt, unsigned groups, unsigned b)
 int launch_skinny(int fmt, const void* w, const void* xq, float* y, unsigned in_dim, unsigned out_dim,
                   unsigned n_rows, rein_stream_t s)
 {
-    const unsigned nv = n_rows <= 2 ? 1 : n_rows <= 4 ? 2 : n_rows <= 8 ? 4 : 8, tok = 2 * nv;
+    const unsigned nv = skinny_nv(n_rows), tok = 2 * nv;
     const unsigned tiles = ((out_dim + 31) / 32) * ((n_rows + tok - 1) / tok);
     const unsigned n_chunks = (in_dim / 32 + 7) / 8;
     const unsigned planes = fmt == REIN_TYPE_Q8_0 ? 2 : 1;
@@ -312,9 +317,8 @@ int launch_skinny(int fmt, const void* w, const void* xq, float* y, unsigned in_
     if (occ == 2 && nv == 4 && tiles >= 1024 && ks < 4 && ks_max >= 4) ks = 4;
     const unsigned forced = opt_u(O_SKINNY_KS, 0);
     if (forced >= 1 && forced <= ks_max) ks = forced;
-    const KName name("rein_mmqs_", fmt_tag(fmt), "_v", nv);
     void* args[] = {(void*)&w, (void*)&xq, (void*)&y, (void*)&in_dim, (void*)&out_dim, (void*)&n_rows};
-    return launch(name, (out_dim + 31) / 32, (n_rows + tok - 1) / tok, 1, ks * 64, ks * lds_per_wave, s, args);
+    return launch(skinny_name(fmt, n_rows), (out_dim + 31) / 32, (n_rows + tok - 1) / tok, 1, ks * 64, ks * lds_per_wave, s, args);
 }
 
 // Activation rows from which the batched decode leaves the dot4 kernels for the
@@ -517,15 +521,17 @@ bool use_mvl(int fmt, unsigned in_dim, unsigned out_dim, unsigned n_rows)
     return out_dim >= 7168 && (fmt == REIN_TYPE_Q4_K || fmt == REIN_TYPE_Q4_0 || fmt == REIN_TYPE_Q5_K || fmt == REIN_TYPE_IQ3_S);
 }
 
+KName mvl_name(int fmt, unsigned in_dim, unsigned out_dim, unsigned n_rows, unsigned r)
+{
+    return KName("rein_mvl_", fmt_tag(fmt), "_r", r, "_b", n_rows <= 2 ? 2u : 4u, load_tag(fmt, in_dim, rein_repacked_len(fmt, in_dim, out_dim), n_rows));
+}
 int launch_matvec_lds(int fmt, const void* w, const void* xq, float* y, unsigned in_dim, unsigned out_dim,
                       unsigned n_rows, rein_stream_t s)
 {
     unsigned r, wpb, grid;
     mvl_geometry(fmt, in_dim, out_dim, n_rows, &r, &wpb, &grid);
-    const unsigned b = n_rows <= 2 ? 2 : 4;
-    const KName name("rein_mvl_", fmt_tag(fmt), "_r", r, "_b", b, load_tag(fmt, in_dim, rein_repacked_len(fmt, in_dim, out_dim), n_rows));
     void* args[] = {(void*)&w, (void*)&xq, (void*)&y, (void*)&in_dim, (void*)&out_dim, (void*)&n_rows};
-    return launch(name, grid, 1, 1, wpb * 64, (unsigned)mvl_lds_bytes(in_dim, n_rows), s, args);
+    return launch(mvl_name(fmt, in_dim, out_dim, n_rows, r), grid, 1, 1, wpb * 64, (unsigned)mvl_lds_bytes(in_dim, n_rows), s, args);
 }
 
 // The 4x4x4 kernel with the activation rows staged in LDS (rein_mvql_*, kernels/matvec_quad.h), 3..8 rows.
@@ -670,13 +676,16 @@ bool use_mvql(int fmt, unsigned in_dim, unsigned out_dim, unsigned n_rows)
     return mvql_few_rows(fmt, in_dim, out_dim);
 }
 
+KName mvql_name(int fmt, unsigned in_dim, unsigned out_dim, unsigned n_rows)
+{
+    if (n_rows > 16) return KName("rein_mvql_", fmt_tag(fmt), mvql_wide32(fmt) ? "_t32w" : "_t32");
+    return KName("rein_mvql_", fmt_tag(fmt), n_rows <= 4 ? "_t4" : n_rows <= 8 ? "_t8" : "_t16",
+                 load_tag(fmt, in_dim, rein_repacked_len(fmt, in_dim, out_dim), n_rows));
+}
 int launch_quad_lds(int fmt, const void* w, const void* xq, float* y, unsigned in_dim, unsigned out_dim,
                     unsigned n_rows, rein_stream_t s)
 {
     const QuadLdsGeometry g = mvql_geometry(fmt, in_dim, out_dim, n_rows);
-    const KName name("rein_mvql_", fmt_tag(fmt), n_rows <= 4 ? "_t4" : n_rows <= 8 ? "_t8" : n_rows <= 16 ? "_t16" :
-                                                                         mvql_wide32(fmt) ? "_t32w" : "_t32",
-                     n_rows <= 16 ? load_tag(fmt, in_dim, rein_repacked_len(fmt, in_dim, out_dim), n_rows) : "");
     // Trips of weights in flight per wavefront where wavefronts stride over row groups or own a whole one (no slices,
     // no phases): two for the formats with little arithmetic per sub-block at 3-4 rows -- two register sets taking
     // turns -- (us, 5120 -> 34816 / 5120 -> 17408 / 3584 -> 18944 at 4 rows, one -> two: Q4_K 28.3 -> 26.0, 18.8 -> 17.3,
@@ -694,7 +703,7 @@ int launch_quad_lds(int fmt, const void* w, const void* xq, float* y, unsigned i
     depth = opt_u(O_QUAD_DEPTH, depth);
     void* args[] = {(void*)&w, (void*)&xq, (void*)&y, (void*)&in_dim, (void*)&out_dim, (void*)&n_rows, (void*)&g.phase_sub, (void*)&g.slices,
                     (void*)&depth};
-    return launch(name, g.grid, 1, 1, g.wpb * 64, (unsigned)g.lds, s, args);
+    return launch(mvql_name(fmt, in_dim, out_dim, n_rows), g.grid, 1, 1, g.wpb * 64, (unsigned)g.lds, s, args);
 }
 
 // Which kernel family a decode of 1..8 activation rows runs on.
@@ -713,30 +722,33 @@ MvFamily matvec_family(int fmt, unsigned in_dim, unsigned out_dim, unsigned n_ro
     return MvFamily::Dot4;
 }
 
-// The kernel a few-row product launches (without the suffix of load_tag): 1..8 rows as rein_matvec_batched_xq8 dispatches them, 9..32 rows the few-row
-// kernels behind rein_mmq_xq8 ("" where that entry point launches token tiles).
-std::string matvec_kernel_name(int fmt, unsigned in_dim, unsigned out_dim, unsigned n_rows)
+KName mvq_name(int fmt, unsigned n_rows) { return KName("rein_mvq_", fmt_tag(fmt), n_rows <= 4 ? "_t4" : "_t8"); }
+KName mv_name(int fmt, unsigned in_dim, unsigned out_dim, unsigned n_rows)
 {
-    const std::string tag = fmt_tag(fmt);
-    const std::string t = n_rows <= 4 ? "_t4" : n_rows <= 8 ? "_t8" : n_rows <= 16 ? "_t16" : mvql_wide32(fmt) ? "_t32w" : "_t32";
+    const unsigned b = batch_slot(n_rows);
+    return KName("rein_mv_", fmt_tag(fmt), "_r", pick_rows_per_wave(fmt, out_dim, b), "_b", b,
+                 b <= 4 ? load_tag(fmt, in_dim, rein_repacked_len(fmt, in_dim, out_dim), n_rows) : "");
+}
+
+// The kernel a few-row product launches: 1..8 rows as rein_matvec_batched_xq8 dispatches them, 9..32 rows the few-row
+// kernels behind rein_mmq_xq8 ("" where that entry point launches token tiles).
+KName matvec_kernel_name(int fmt, unsigned in_dim, unsigned out_dim, unsigned n_rows)
+{
     if (n_rows > 8) {
-        if (n_rows <= 32 && use_mvql(fmt, in_dim, out_dim, n_rows)) return "rein_mvql_" + tag + t;
-        if (n_rows <= 16 && in_dim >= 256 && skinny_from_rows(fmt) <= 16) return "rein_mmqs_" + tag + "_v8";
-        return "";
+        if (n_rows <= 32 && use_mvql(fmt, in_dim, out_dim, n_rows)) return mvql_name(fmt, in_dim, out_dim, n_rows);
+        if (n_rows <= 16 && in_dim >= 256 && skinny_from_rows(fmt) <= 16) return skinny_name(fmt, n_rows);
+        return KName("");
     }
     switch (matvec_family(fmt, in_dim, out_dim, n_rows)) {
-    case MvFamily::QuadLds: return "rein_mvql_" + tag + t;
-    case MvFamily::Quad:    return "rein_mvq_" + tag + t;
-    case MvFamily::Skinny:  return "rein_mmqs_" + tag + "_v" + std::to_string(n_rows <= 2 ? 1 : n_rows <= 4 ? 2 : 4);
+    case MvFamily::QuadLds: return mvql_name(fmt, in_dim, out_dim, n_rows);
+    case MvFamily::Quad:    return mvq_name(fmt, n_rows);
+    case MvFamily::Skinny:  return skinny_name(fmt, n_rows);
     case MvFamily::Dot4Lds: {
         unsigned r, wpb, grid;
         mvl_geometry(fmt, in_dim, out_dim, n_rows, &r, &wpb, &grid);
-        return "rein_mvl_" + tag + "_r" + std::to_string(r) + "_b" + std::to_string(n_rows <= 2 ? 2 : 4);
+        return mvl_name(fmt, in_dim, out_dim, n_rows, r);
     }
-    default: {
-        const unsigned b = batch_slot(n_rows);
-        return "rein_mv_" + tag + "_r" + std::to_string(pick_rows_per_wave(fmt, out_dim, b)) + "_b" + std::to_string(b);
-    }
+    default: return mv_name(fmt, in_dim, out_dim, n_rows);
     }
 }
 
@@ -754,9 +766,8 @@ int launch_matvec(const char* who, int fmt, const void* w, const void* xq, float
     if (family == MvFamily::Dot4Lds) return launch_matvec_lds(fmt, w, xq, y, in_dim, out_dim, n_rows, s);
     if (family == MvFamily::Quad) {
         // four output rows per wavefront, four wavefronts per workgroup
-        const KName name("rein_mvq_", fmt_tag(fmt), n_rows <= 4 ? "_t4" : "_t8");
         void* args[] = {(void*)&w, (void*)&xq, (void*)&y, (void*)&in_dim, (void*)&out_dim, (void*)&n_rows};
-        return launch(name, ((out_dim + 3) / 4 + 3) / 4, 1, 1, 256, 0, s, args);
+        return launch(mvq_name(fmt, n_rows), ((out_dim + 3) / 4 + 3) / 4, 1, 1, 256, 0, s, args);
     }
     if (family == MvFamily::Skinny) return launch_skinny(fmt, w, xq, y, in_dim, out_dim, n_rows, s);
     const unsigned b = batch_slot(n_rows);
@@ -764,9 +775,8 @@ int launch_matvec(const char* who, int fmt, const void* w, const void* xq, float
     const unsigned groups = (out_dim + r - 1) / r;
     const unsigned wpb = pick_wpb(fmt, groups, b);
     const unsigned grid = (groups + wpb - 1) / wpb;
-    const KName name("rein_mv_", fmt_tag(fmt), "_r", r, "_b", b, b <= 4 ? load_tag(fmt, in_dim, rein_repacked_len(fmt, in_dim, out_dim), n_rows) : "");
     void* args[] = {(void*)&w, (void*)&xq, (void*)&y, (void*)&in_dim, (void*)&out_dim, (void*)&n_rows};
-    return launch(name, grid, 1, 1, wpb * 64, 0, s, args);
+    return launch(mv_name(fmt, in_dim, out_dim, n_rows), grid, 1, 1, wpb * 64, 0, s, args);
 }
 
 // Grouped GEMM launch.  The tile count lives on the device; the grid covers its upper bound
@@ -1130,9 +1140,9 @@ int rein_matvec_kernel_name(int fmt, unsigned in_dim, unsigned out_dim, unsigned
     if (!name || name_len == 0) return fail(REIN_E_BAD_POINTER, std::string(who) + ": no room for the name");
     if (int rc = check_shape(who, fmt, in_dim, out_dim, n_rows)) return rc;
     if (int rc = check_dense_fmt(who, fmt)) return rc;
-    const std::string k = matvec_kernel_name(fmt, in_dim, out_dim, n_rows);
-    if (k.size() + 1 > name_len) return fail(REIN_E_TOO_LARGE, std::string(who) + ": the name needs " + std::to_string(k.size() + 1) + " bytes");
-    std::memcpy(name, k.c_str(), k.size() + 1);
+    const KName k = matvec_kernel_name(fmt, in_dim, out_dim, n_rows);
+    if (k.len + 1 > name_len) return fail(REIN_E_TOO_LARGE, std::string(who) + ": the name needs " + std::to_string(k.len + 1) + " bytes");
+    std::memcpy(name, k.text, k.len + 1);
     return 0;
 }
 
