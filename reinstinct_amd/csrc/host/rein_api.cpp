@@ -387,7 +387,7 @@ bool small_for_matrix_cores(int fmt, unsigned in_dim, unsigned out_dim, unsigned
 }
 
 // Which build of a few-row kernel a launch takes, by how it loads its `bytes` of weights (rein_formats.h): "" all planes
-// nontemporal, "_m" the 16- and 8-byte planes only, "_p" plain.  Where the lines lie (each kernel built all three ways, 17
+// nontemporal (not built for five rows and more), "_m" the 16- and 8-byte planes only, "_p" plain.  Where the lines lie (each kernel built all three ways, 17
 // shapes x Q4_K, Q5_K, Q6_K, Q8_0, matrices rotating through 600 MB; against all nontemporal):
 //   below 6.5 MB   plain 4-16 % faster at 1-4 rows (5120 -> 1024 Q4_K 3.75 -> 3.30 us, Q6_K 4.25 -> 3.70), level to +7 % at more
 //   5 rows up      mix level to +8 % at every larger size
@@ -1727,8 +1727,8 @@ int rein_noalloc_prepare(void)
     static const char* const forms[] = {"_t32", "_t64", "_mix", "_sk", "_sk32"};
     // (up to 32 rows the entry point launches the few-row kernels: skinny MMQ, both 4x4x4 kernels, and from eight rows
     // down the decode matvecs in every rows-per-wavefront x batch-slot instantiation there is)
-    static const char* const few[] = {"rein_mmqs_%s_v1", "rein_mmqs_%s_v2", "rein_mmqs_%s_v4", "rein_mmqs_%s_v8", "rein_mvql_%s_t4", "rein_mvql_%s_t8",
-                                      "rein_mvql_%s_t16", "rein_mvql_%s_t4_m", "rein_mvql_%s_t8_m", "rein_mvql_%s_t16_m", "rein_mvql_%s_t4_p",
+    static const char* const few[] = {"rein_mmqs_%s_v1", "rein_mmqs_%s_v2", "rein_mmqs_%s_v4", "rein_mmqs_%s_v8", "rein_mvql_%s_t4",
+                                      "rein_mvql_%s_t4_m", "rein_mvql_%s_t8_m", "rein_mvql_%s_t16_m", "rein_mvql_%s_t4_p",
                                       "rein_mvql_%s_t8_p", "rein_mvql_%s_t16_p", "rein_mvql_%s_t32", "rein_mvql_%s_t32w", "rein_mvq_%s_t4", "rein_mvq_%s_t8"};
     for (int fmt : fmts) {
         for (const char* form : forms) {

@@ -502,13 +502,16 @@ __device__ __forceinline__ void rein_matvec_quad_lds_body(const uint8_t* __restr
 // (32 rows: by default for eight wavefronts per workgroup at most, so that the 32 partial sums and the eight activation
 // tiles of a trip stay in registers; REIN_DEFINE_MATVEC_QUAD_LDS_BOUND builds it for sixteen wavefronts' 128 registers as
 // well, where the heavier formats spill)
-// (name_m and name_p: the same with the other loads of the weights, rein_formats.h)
+// (name_m and name_p: the same with the other loads of the weights, rein_formats.h; from five rows up only these two, the host
+// never takes the all-nontemporal build there)
 #define REIN_DEFINE_MATVEC_QUAD_LDS(name, FMT, NT) REIN_DEFINE_MATVEC_QUAD_LDS_BOUND(name, FMT, NT, (NT >= 8 ? 512 : 1024))
 #define REIN_DEFINE_MATVEC_QUAD_LDS_BOUND(name, FMT, NT, BOUND) REIN_DEFINE_MATVEC_QUAD_LDS_LD(name, FMT, NT, BOUND, REIN_LD_STREAM)
-#define REIN_DEFINE_MATVEC_QUAD_LDS_LOADS(name, FMT, NT)                                          \
-    REIN_DEFINE_MATVEC_QUAD_LDS(name, FMT, NT)                                                    \
+#define REIN_DEFINE_MATVEC_QUAD_LDS_MP(name, FMT, NT)                                             \
     REIN_DEFINE_MATVEC_QUAD_LDS_LD(name##_m, FMT, NT, 1024, REIN_LD_MIX)                          \
     REIN_DEFINE_MATVEC_QUAD_LDS_LD(name##_p, FMT, NT, 1024, REIN_LD_PLAIN)
+#define REIN_DEFINE_MATVEC_QUAD_LDS_LOADS(name, FMT, NT)                                          \
+    REIN_DEFINE_MATVEC_QUAD_LDS(name, FMT, NT)                                                    \
+    REIN_DEFINE_MATVEC_QUAD_LDS_MP(name, FMT, NT)
 #define REIN_DEFINE_MATVEC_QUAD_LDS_LD(name, FMT, NT, BOUND, POL)                                 \
     extern "C" __global__ __launch_bounds__(BOUND) void name(                                     \
         const uint8_t* __restrict__ w, const BlockQ8* __restrict__ xq, float* __restrict__ y,    \

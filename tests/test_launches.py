@@ -1,7 +1,9 @@
 """Which kernels the entry points launch (CPU: tests/launches.py records the launches instead of making them)."""
 import random
+import re
 
 import reinstinct_amd as rein
+from reinstinct_amd._lib import HSACO_PATH
 from launches import P, record
 
 DENSE = (rein.Q4_0, rein.Q4_K, rein.Q5_K, rein.Q6_K, rein.Q8_0, rein.IQ4_XS, rein.IQ3_S)
@@ -35,3 +37,26 @@ def test_the_reported_name_is_the_kernel_that_is_launched(tmp_path):
         else:
             assert args[3] > 8 and launched[0].startswith("rein_mmq_"), args
     assert {"m", "p", "b1", "t4", "t32", "t32w", "v4"} <= builds
+
+
+def test_every_few_row_kernel_of_the_code_object_can_be_launched(tmp_path):
+    """no build of the decode matvecs is compiled for nothing: products of every size class, with each choice pinned in turn,
+    reach every rein_mv* symbol"""
+    code = open(HSACO_PATH, "rb").read()
+    there = {m.decode() for m in re.findall(rb"\0(rein_mv[a-z0-9_]+)\.kd(?=\0)", code)}
+    shapes = [(1024, 1024), (2560, 3712), (4096, 3072), (5120, 5120), (5120, 8192), (4096, 14336), (5120, 34816)]
+    calls = []
+    for pin in ([], [("REIN_QUAD_LDS", 1)], [("REIN_QUAD_LDS", 1), ("REIN_QUAD_WIDE32", 0)], [("REIN_QUAD_LDS", 1), ("REIN_QUAD_WIDE32", 1)],
+                [("REIN_QUAD_FROM", 1)], *([("REIN_MV_LDS", 1), ("REIN_MV_ROWS", r)] for r in (1, 2, 4)),
+                *([("REIN_MV_LDS", 0), ("REIN_QUAD_LDS", 0), ("REIN_SKINNY_FROM", 99), ("REIN_QUAD_FROM", 99), ("REIN_MV_ROWS", r)] for r in (1, 2, 4))):
+        calls += [("option", [n, v]) for n, v in pin]
+        for k, n in shapes:
+            for rows in (1, 2, 3, 8, 16, 32):
+                calls += [("mmq_xq8", [fmt, P, P, P, k, n, rows]) for fmt in DENSE]
+                if rows <= 4:
+                    calls.append(("matvec_multi_xq8", [[rein.Q4_K, rein.Q6_K], [P, P], [P, P], [n, 8], P, k, rows]))
+        calls += [("option", [n, None]) for n, _ in pin]
+    calls += [("matvec_ondisk_xq8", [fmt, P, P, P, 2048, 8192]) for fmt in (rein.Q4_K, rein.Q5_K, rein.Q6_K, rein.Q8_0)]
+    reached = {r[0] for d in record(calls, tmp_path) for r in d["launches"]}
+    assert len(there) > 100
+    assert there - reached == set()
