@@ -410,7 +410,8 @@ int rein_mmq_tile_plan_ws(int fmt, unsigned out_dim, unsigned p_rows, unsigned *
 int rein_matmul(int fmt, const void *w, const float *x, float *y, unsigned in_dim,
                 unsigned out_dim, unsigned n_rows, void *xq_scratch, rein_stream_t s);
 /* rein_matmul with one scratch buffer of rein_matmul_scratch_bytes(fmt, in_dim, n_rows) bytes
- * (16-byte aligned) that holds the quantized activations and, for the MMQ path, the workspace
+ * (16-byte aligned) that holds the quantized activations -- its first n_rows*in_dim/32*40 bytes, as
+ * rein_quantize_q8 writes them, whichever launch is taken -- and, for the MMQ path, the workspace
  * of rein_mmq_xq8_ws.  A scratch that only holds the activations runs rein_matmul.
  * Q4_K, Q5_K and Q6_K from 33 rows: a scratch of the full size runs the fp16-instruction GEMM with exact block
  * dots where it is the faster one (activation image and up to 64 MiB of partial tiles in the scratch; three

@@ -1939,7 +1939,7 @@ int rein_matmul_ws(int fmt, const void* w, const float* x, float* y, unsigned in
         const unsigned tail = p.n_unit - p.n_whole, with_xsum = xh_has_min(fmt);
         const unsigned long long grid = p.n_whole + 8ull * (((unsigned long long)tail * p.split + 7) / 8);
         if (grid <= 0x7FFFFFFFull && in_dim / 256 <= 65535) {
-            void* pa[] = {(void*)&x, (void*)&img, (void*)&in_dim, (void*)&n_rows, (void*)&with_xsum};
+            void* pa[] = {(void*)&x, (void*)&img, (void*)&scratch, (void*)&in_dim, (void*)&n_rows, (void*)&with_xsum};
             if (int rc = launch("rein_xh_quantize", (n_rows + 31) / 32, in_dim / 256, 1, 256, 0, s, pa)) return rc;
             void* a[] = {(void*)&w, (void*)&img, (void*)&y, (void*)&parts, (void*)&in_dim, (void*)&out_dim, (void*)&n_rows, (void*)&p.n_whole, (void*)&p.split};
             if (int rc = launch(KName("rein_xh_", fmt_tag(fmt), ""), (unsigned)grid, 1, 1, 256, xh_lds_bytes(fmt), s, a)) return rc;

@@ -61,11 +61,13 @@ __host__ __device__ constexpr int rein_xh_slot_weight(int kh, int h, int e)
 #define REIN_XH_REC 4352u
 #define REIN_XH_XS  2048u
 
-// x [p_rows][in_dim] fp32 -> image, with the numbers that quantize_q8_f32 gives: the same sum tree (halves of 16, 8, 4, 2, 1),
-// divisions and rounding, by one thread for a block of 32.  blockIdx.x = token tile, blockIdx.y = superblock, 256 threads:
-// thread 8 j + s handles token j, sub-block s: eight threads read a kilobyte of a row and write runs of 128 bytes.
-// Bound by memory: 4 bytes in, 2.1 out per value (777 x 17408: 54 + 29 MB).
-__device__ __forceinline__ void rein_xh_quantize_body(const float* __restrict__ x, uint8_t* __restrict__ img, unsigned in_dim, unsigned p_rows, unsigned with_xsum)
+// x [p_rows][in_dim] fp32 -> image, and the blocks themselves to xq [p_rows][in_dim / 32] (the caller of rein_matmul_ws may read
+// them there), with the numbers that quantize_q8_f32 gives: the same sum tree (halves of 16, 8, 4, 2, 1), divisions and rounding,
+// by one thread for a block of 32.  blockIdx.x = token tile, blockIdx.y = superblock, 256 threads: thread 8 j + s handles token j,
+// sub-block s: eight threads read a kilobyte of a row and write runs of 128 bytes to the image and 320 to xq.
+// Bound by memory: 4 bytes in, 3.4 out per value (777 x 17408: 54 + 46 MB).
+__device__ __forceinline__ void rein_xh_quantize_body(const float* __restrict__ x, uint8_t* __restrict__ img, BlockQ8* __restrict__ xq, unsigned in_dim,
+                                                      unsigned p_rows, unsigned with_xsum)
 {
 #pragma clang fp contract(off)
     __shared__ float xsum[8][33];
@@ -102,6 +104,17 @@ __device__ __forceinline__ void rein_xh_quantize_body(const float* __restrict__ 
 #pragma unroll
         for (int i = 0; i < 32; i++) v[i] = 0.0f;
     }
+    int q[32];
+#pragma unroll
+    for (int i = 0; i < 32; i++) q[i] = max(-127, min(127, (int)rintf(v[i] * inv)));
+    if (tok < p_rows) {
+        BlockQ8 b;
+        b.d = d;
+        b.xsum = sum;
+#pragma unroll
+        for (int i = 0; i < 8; i++) b.qs[i] = (q[4 * i] & 0xFF) | (q[4 * i + 1] & 0xFF) << 8 | (q[4 * i + 2] & 0xFF) << 16 | q[4 * i + 3] << 24;
+        xq[(size_t)tok * n_sub + sb] = b;
+    }
     uint8_t* rec = img + ((size_t)(sb >> 1) * n_tt + tt) * REIN_XH_REC;
     reinterpret_cast<float*>(rec + REIN_XH_X)[(sb & 1u) * 32u + j] = d;
 #pragma unroll
@@ -110,7 +123,7 @@ __device__ __forceinline__ void rein_xh_quantize_body(const float* __restrict__ 
         for (int h = 0; h < 2; h++) {
             rein_v8h o;
 #pragma unroll
-            for (int e = 0; e < 8; e++) o[e] = (_Float16)max(-127, min(127, (int)rintf(v[rein_xh_slot_weight(kh, h, e)] * inv)));
+            for (int e = 0; e < 8; e++) o[e] = (_Float16)q[rein_xh_slot_weight(kh, h, e)];
             *reinterpret_cast<rein_v8h*>(rec + (sb & 1u) * 2048u + kh * 1024u + (32u * h + j) * 16u) = o;
         }
     if (!with_xsum) return;                          // the image of a format without minimums has no xsum part

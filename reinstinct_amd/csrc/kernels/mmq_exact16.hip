@@ -2,9 +2,10 @@
 #include "mmq_exact16.h"
 
 extern "C" __global__ __launch_bounds__(256) void rein_xh_quantize(const float* __restrict__ x, unsigned char* __restrict__ img,
-                                                                   unsigned int in_dim, unsigned int p_rows, unsigned int with_xsum)
+                                                                   BlockQ8* __restrict__ xq, unsigned int in_dim, unsigned int p_rows,
+                                                                   unsigned int with_xsum)
 {
-    rein_xh_quantize_body(x, img, in_dim, p_rows, with_xsum);
+    rein_xh_quantize_body(x, img, xq, in_dim, p_rows, with_xsum);
 }
 
 extern "C" __global__ __launch_bounds__(256) void rein_xh_sum(const float* __restrict__ parts, float* __restrict__ y, unsigned int out_dim,

@@ -65,6 +65,27 @@ def test_against_the_oracle(fmt, rows, in_dim, out_dim, split):
     assert_close_f32(got / scale, want / scale, what=f"fmt {fmt}")
 
 
+@pytest.mark.parametrize("fmt", [rein.Q4_K, rein.Q6_K])
+@pytest.mark.parametrize("rows, in_dim, skip", [(33, 256, 0), (129, 1280, 0), (77, 768, 1)])          # skip: x not 16-byte aligned
+def test_the_scratch_holds_the_quantized_rows(fmt, rows, in_dim, skip):
+    """the first part of the scratch is what rein_quantize_q8 writes, here as on every other launch of rein_matmul_ws: a caller that
+    quantizes with one projection may run the next one on it"""
+    out_dim = 96
+    x = np.random.default_rng(rows).standard_normal((rows, in_dim)).astype(np.float32)
+    x[rows // 2] = 0.0
+    set_option("REIN_MMQXH", "2")
+    size = runtime.matmul_scratch_bytes(fmt, in_dim, rows)
+    dw, dx = hip.DeviceBuf.from_host(weights(fmt, in_dim, out_dim, 1)), hip.DeviceBuf.from_host(np.concatenate([np.zeros(skip, np.float32), x.reshape(-1)]))
+    scratch, dy = hip.DeviceBuf.from_host(np.full(size, 0xA5, np.uint8)), hip.DeviceBuf(rows * out_dim * 4)
+    runtime.matmul_ws(fmt, dw, dx.ptr + 4 * skip, dy, in_dim, out_dim, rows, scratch, size)
+    hip.synchronize()
+    want = orc.quantize_q8(x)
+    got = scratch.to_host(np.uint8)
+    assert np.array_equal(got[:want.size], want)
+    behind = (want.size + 255) // 256 * 256               # up to the image nothing is touched
+    assert (got[want.size:behind] == 0xA5).all()
+
+
 @pytest.mark.parametrize("fmt", [rein.Q4_K, rein.Q5_K, rein.Q6_K])
 def test_no_further_from_64_bits_than_the_int8_tile(fmt):
     rows, in_dim, out_dim = 160, 4352, 256
