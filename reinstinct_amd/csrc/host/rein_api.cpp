@@ -1840,10 +1840,10 @@ namespace {
 // ---- Q4_K / Q5_K / Q6_K prefill with exact block dots on the fp16 instruction (kernels/mmq_exact16.h), out of rein_matmul_ws
 struct XhPlan {
     unsigned n_grp, n_unit, n_whole, split;
-    size_t image;                                    // bytes of the activation image, partial tiles behind it
+    size_t image, parts;                             // bytes of the activation image and of the partial tiles behind it
 };
 constexpr size_t kXhPart = (size_t)4 * 16 * 256 * 4;
-constexpr size_t kXhParts = (size_t)64 << 20;        // room for partial tiles: 1024
+constexpr unsigned kXhMostParts = 1024;              // partial tiles of one launch: 64 MiB
 bool xh_format(int fmt) { return fmt == REIN_TYPE_Q4_K || fmt == REIN_TYPE_Q5_K || fmt == REIN_TYPE_Q6_K; }
 bool xh_has_min(int fmt) { return fmt != REIN_TYPE_Q6_K; }
 size_t xh_image_bytes(int fmt, unsigned in_dim, unsigned p_rows)
@@ -1881,27 +1881,43 @@ bool xh_take(int fmt, unsigned in_dim, unsigned out_dim, unsigned p_rows)
 // and a half for its start; a last round of at most one workgroup per CU takes 0.6 of one with two; a partial tile is
 // written and read once.  Q6_K, us at 1 / 2 / 3 / 4 / 6 ranges: 17408 -> 5120, 777 rows (280 units) 475 / 409 / 382 / 382 /
 // 382, 512 rows (160 units) 349 / 290 / 228 / 249 / 240; 5120 -> 17408, 512 rows (a round and 32) 274 / 228 / 214 / 208 / 208.
+unsigned xh_split(unsigned tail, unsigned chunks)
+{
+    if (tail == 0) return 1;
+    const unsigned most = std::max(1u, std::min(std::min(16u, chunks), kXhMostParts / tail));
+    const unsigned forced = opt_u(O_MMQXH_SPLIT, 0);
+    if (forced) return std::min(forced, most);
+    unsigned split = 1;
+    double best = 0.0;
+    for (unsigned k = 1; k <= most; k++) {
+        const unsigned wg = tail * k, rem = wg % 512;
+        const double rounds = wg / 512 + (rem == 0 ? 0.0 : rem <= kCUs ? 0.6 : 1.0);
+        const double cost = rounds * (chunks / (double)k + 1.5) + (k > 1 ? 0.4 + wg * 0.0012 : 0.0);
+        if (k == 1 || cost < best) { best = cost; split = k; }
+    }
+    return split;
+}
+size_t xh_parts_bytes(unsigned tail, unsigned split) { return split > 1 ? (size_t)tail * split * kXhPart : 0; }
 XhPlan xh_plan(int fmt, unsigned in_dim, unsigned out_dim, unsigned p_rows)
 {
     XhPlan p{};
     p.n_grp = (p_rows + 127) / 128;
     p.n_unit = (out_dim + 127) / 128 * p.n_grp;
     p.n_whole = p.n_unit / 512 * 512;
-    p.split = 1;
+    p.split = xh_split(p.n_unit - p.n_whole, in_dim / 256);
     p.image = (xh_image_bytes(fmt, in_dim, p_rows) + 255) & ~(size_t)255;
-    const unsigned tail = p.n_unit - p.n_whole, chunks = in_dim / 256;
-    if (tail == 0) return p;
-    const unsigned most = std::min<unsigned>(std::min(16u, chunks), (unsigned)(kXhParts / kXhPart / tail));
-    double best = 0.0;
-    for (unsigned k = 1; k <= std::max(1u, most); k++) {
-        const unsigned wg = tail * k, rem = wg % 512;
-        const double rounds = wg / 512 + (rem == 0 ? 0.0 : rem <= kCUs ? 0.6 : 1.0);
-        const double cost = rounds * (chunks / (double)k + 1.5) + (k > 1 ? 0.4 + wg * 0.0012 : 0.0);
-        if (k == 1 || cost < best) { best = cost; p.split = k; }
-    }
-    const unsigned forced = opt_u(O_MMQXH_SPLIT, 0);
-    if (forced) p.split = std::max(1u, std::min(forced, most));
+    p.parts = xh_parts_bytes(p.n_unit - p.n_whole, p.split);
     return p;
+}
+// The most bytes of partial tiles that any number of weight rows leaves behind whole rounds of `n_grp` token groups (the size query
+// does not know the matrix): none for contractions of one or two superblocks, which are never split, 16 MiB up to five, 64 from ten.
+size_t xh_most_parts_bytes(unsigned in_dim, unsigned p_rows)
+{
+    unsigned step = (p_rows + 127) / 128 % 512;
+    step = step == 0 ? 512 : step & (0u - step);     // the remainders of its multiples by 512 are those of this power of two
+    size_t most = 0;
+    for (unsigned tail = step; tail < 512; tail += step) most = std::max(most, xh_parts_bytes(tail, xh_split(tail, in_dim / 256)));
+    return most;
 }
 }  // namespace
 
@@ -1911,7 +1927,7 @@ size_t rein_matmul_scratch_bytes(int fmt, unsigned in_dim, unsigned n_rows)
     const size_t xq = ((size_t)n_rows * (in_dim / 32) * 40 + 255) & ~(size_t)255;
     size_t behind = rein_matmul_path(fmt, n_rows) == 2 ? rein_mmq_workspace_bytes(fmt, in_dim, n_rows) : 0;
     if (rein_matmul_path(fmt, n_rows) == 2 && xh_shape(fmt, in_dim, n_rows))
-        behind = std::max(behind, ((xh_image_bytes(fmt, in_dim, n_rows) + 255) & ~(size_t)255) + kXhParts);
+        behind = std::max(behind, ((xh_image_bytes(fmt, in_dim, n_rows) + 255) & ~(size_t)255) + xh_most_parts_bytes(in_dim, n_rows));
     return xq + behind;
 }
 
@@ -1924,21 +1940,16 @@ int rein_matmul_ws(int fmt, const void* w, const float* x, float* y, unsigned in
     const size_t xq = ((size_t)n_rows * (in_dim / 32) * 40 + 255) & ~(size_t)255;
     if (scratch_bytes < (size_t)n_rows * (in_dim / 32) * 40)
         return fail(REIN_E_BAD_SHAPE, "rein_matmul_ws: scratch smaller than the quantized activations");
-    // nothing behind the activations that a workspace launch could use: the plain dispatch
-    const size_t least = rein_mmq_workspace_min_bytes(fmt, in_dim, n_rows);
-    if (rein_matmul_path(fmt, n_rows) != 2 || rein_mmq_workspace_bytes(fmt, in_dim, n_rows) == 0 ||
-        scratch_bytes < xq + std::max<size_t>(least, 16))
-        return rein_matmul(fmt, w, x, y, in_dim, out_dim, n_rows, scratch, s);
-    if (n_rows <= 65535 && xh_take(fmt, in_dim, out_dim, n_rows) && scratch_bytes >= rein_matmul_scratch_bytes(fmt, in_dim, n_rows)) {
-        if (int rc = check_ptr("rein_matmul_ws", x, 4, "x")) return rc;
-        if (int rc = check_ptr("rein_matmul_ws", w, 16, "w")) return rc;
-        if (int rc = check_ptr("rein_matmul_ws", y, 4, "y")) return rc;
+    if (n_rows <= 65535 && xh_take(fmt, in_dim, out_dim, n_rows)) {
         const XhPlan p = xh_plan(fmt, in_dim, out_dim, n_rows);
         char* const img = static_cast<char*>(scratch) + xq;
         char* const parts = img + p.image;
         const unsigned tail = p.n_unit - p.n_whole, with_xsum = xh_has_min(fmt);
         const unsigned long long grid = p.n_whole + 8ull * (((unsigned long long)tail * p.split + 7) / 8);
-        if (grid <= 0x7FFFFFFFull && in_dim / 256 <= 65535) {
+        if (scratch_bytes >= xq + p.image + p.parts && grid <= 0x7FFFFFFFull && in_dim / 256 <= 65535) {
+            if (int rc = check_ptr("rein_matmul_ws", x, 4, "x")) return rc;
+            if (int rc = check_ptr("rein_matmul_ws", w, 16, "w")) return rc;
+            if (int rc = check_ptr("rein_matmul_ws", y, 4, "y")) return rc;
             void* pa[] = {(void*)&x, (void*)&img, (void*)&scratch, (void*)&in_dim, (void*)&n_rows, (void*)&with_xsum};
             if (int rc = launch("rein_xh_quantize", (n_rows + 31) / 32, in_dim / 256, 1, 256, 0, s, pa)) return rc;
             void* a[] = {(void*)&w, (void*)&img, (void*)&y, (void*)&parts, (void*)&in_dim, (void*)&out_dim, (void*)&n_rows, (void*)&p.n_whole, (void*)&p.split};
@@ -1948,6 +1959,11 @@ int rein_matmul_ws(int fmt, const void* w, const float* x, float* y, unsigned in
             return launch("rein_xh_sum", tail, 16, 1, 256, 0, s, b);
         }
     }
+    // nothing behind the activations that a workspace launch could use: the plain dispatch
+    const size_t least = rein_mmq_workspace_min_bytes(fmt, in_dim, n_rows);
+    if (rein_matmul_path(fmt, n_rows) != 2 || rein_mmq_workspace_bytes(fmt, in_dim, n_rows) == 0 ||
+        scratch_bytes < xq + std::max<size_t>(least, 16))
+        return rein_matmul(fmt, w, x, y, in_dim, out_dim, n_rows, scratch, s);
     if (int rc = rein_quantize_q8(x, scratch, in_dim, n_rows, s)) return rc;
     return rein_mmq_xq8_ws(fmt, w, scratch, y, in_dim, out_dim, n_rows, static_cast<char*>(scratch) + xq, scratch_bytes - xq, s);
 }

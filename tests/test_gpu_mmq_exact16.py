@@ -142,9 +142,14 @@ def test_smaller_scratch_and_capture():
     call(size)
     hip.synchronize()
     eager = dy.to_host(np.uint32)
-    call(size - 1)
+    small = (rows * in_dim // 32 * 40 + 255) // 256 * 256 + 4096             # less than the activation image
+    call(small)
     hip.synchronize()
-    assert np.array_equal(dy.to_host(np.uint32).reshape(rows, out_dim), matmul(fmt, packed, x, out_dim, 0).view(np.uint32))
+    without = dy.to_host(np.uint32)
+    set_option("REIN_MMQXH", "0")
+    call(small)
+    hip.synchronize()
+    assert np.array_equal(without, dy.to_host(np.uint32)) and not np.array_equal(without, eager)
     set_option("REIN_MMQXH", None)
     stream = hip.Stream()
     stream.begin_capture()

@@ -60,3 +60,44 @@ def test_every_few_row_kernel_of_the_code_object_can_be_launched(tmp_path):
     reached = {r[0] for d in record(calls, tmp_path) for r in d["launches"]}
     assert len(there) > 100
     assert there - reached == set()
+
+
+def xh(done):
+    return [r[0] for r in done["launches"] if r[0].startswith("rein_xh_")]
+
+
+def test_exact_dot_gemm_needs_no_more_scratch_than_its_plan(tmp_path):
+    """rein_matmul_ws: a scratch of the size the query gives runs the exact-dot GEMM for every number of weight rows; one that holds
+    the shape's own image and partial tiles does too; one that does not runs the other launches"""
+    rng = random.Random(9)
+    shapes = [(fmt, k, rows) for fmt in (rein.Q4_K, rein.Q5_K, rein.Q6_K) for k, rows in
+              [(256, 33), (512, 4097), (768, 200), (4096, 128), (17408, 777), (5120, 65535), *((256 * rng.randint(1, 72), rng.randint(33, 3000)) for _ in range(6))]]
+    sizes = record([("option", ["REIN_MMQXH", 2])] + [("matmul_scratch_bytes", list(s)) for s in shapes], tmp_path)[1:]
+    calls = [("option", ["REIN_MMQXH", 2])]
+    for (fmt, k, rows), size in zip(shapes, sizes):
+        for n in [1, 640, 5120, 17408, *(rng.randint(1, 40000) for _ in range(20))]:
+            calls.append(("matmul_ws", [fmt, P, P, P, k, n, rows, P, size["value"]]))
+    for call, done in zip(calls[1:], record(calls, tmp_path)[1:]):
+        assert xh(done)[:1] == ["rein_xh_quantize"], call
+    # 200 rows against 4096 -> 640: ten units of sixteen superblocks in sixteen ranges at most
+    fmt, k, n, rows = rein.Q6_K, 4096, 640, 200
+    front = (rows * k // 32 * 40 + 255) // 256 * 256
+    image = k // 64 * 7 * 4352
+    call = [fmt, P, P, P, k, n, rows, P]
+    calls = [("option", ["REIN_MMQXH_SPLIT", 1]), ("matmul_ws", call + [front + image]), ("option", ["REIN_MMQXH_SPLIT", None]),
+             ("matmul_ws", call + [front + image + 160 * 65536]), ("matmul_ws", call + [front + image - 1]), ("matmul_ws", call + [front + image])]
+    _, unsplit, _, split, none, least = record(calls, tmp_path)
+    assert xh(unsplit) == ["rein_xh_quantize", "rein_xh_q6k"]
+    assert xh(split) == ["rein_xh_quantize", "rein_xh_q6k", "rein_xh_sum"]
+    assert xh(none) == [] and xh(least) == [] and none["launches"]
+    # the int8 tile's split-tail launch switched off does not switch this one off
+    off = record([("option", ["REIN_MMQ_SK", 0]), *(("matmul_ws", [f] + call[1:] + [front + image + (64 << 20)]) for f in (rein.Q5_K, rein.Q6_K)),
+                  ("option", ["REIN_MMQXH", 2]), ("matmul_ws", [rein.Q5_K] + call[1:] + [front + image + (64 << 20)])], tmp_path)
+    assert [bool(xh(d)) for d in off[1:3] + off[4:]] == [False, True, True]          # (Q5_K below 384 rows only where it is asked for)
+
+
+def test_exact_dot_gemm_and_the_scratch_query_without_partial_tiles(tmp_path):
+    """a contraction of one superblock is never split: the query asks for no more than the other launches want"""
+    from reinstinct_amd import runtime
+    for fmt in (rein.Q5_K, rein.Q6_K):
+        assert runtime.matmul_scratch_bytes(fmt, 256, 64) <= (64 * 8 * 40 + 255) // 256 * 256 + (16 << 20)
