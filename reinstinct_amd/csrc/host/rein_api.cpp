@@ -1158,13 +1158,19 @@ int rein_matvec_ondisk_xq8(int fmt, const void* w_blocks, const void* xq, float*
     if (int rc = check_ptr(who, xq, 8, "xq")) return rc;
     if (int rc = check_ptr(who, y, 4, "y")) return rc;
     void* a[] = {(void*)&w_blocks, (void*)&xq, (void*)&y, (void*)&in_dim, (void*)&out_dim};
-    // rein_mvd_<fmt> pairs sub-blocks and keeps the activations in LDS: every shape but a Q8_0 row of an odd number of blocks
-    // (which starts at 2-byte alignment) and a contraction whose activations do not fit, about 100 000 values.  Grids: the comment at
+    // rein_mvd_<fmt> pairs sub-blocks and keeps the activations in LDS: not for a Q8_0 row of an odd number of blocks (which
+    // starts at 2-byte alignment) and a contraction whose activations do not fit, about 100 000 values.  Grids: the comment at
     // the kernel.
+    // Up to 2048 rows the other kernel has a workgroup of eight rows per CU at most, and its rows go over 64 lanes, 2048 weights a
+    // trip, where sixteen lanes take 1024: Q8_0 is 1.01-1.28 x faster there (2048 -> 1024, us, mvd / other: 3.61 / 3.24; 8192 -> 512
+    // 7.67 / 6.40), and so is Q6_K unless its last trip of 2048 would be half idle (1.06-1.17: 2048 -> 1024 3.91 / 3.39, 6144 -> 2048
+    // 7.08 / 6.72; the other way round at 1024 -> 1024 2.87 / 3.35, 5120 -> 1024 6.15 / 6.53).  Q4_K and Q5_K are faster on mvd from 32
+    // rows (1.00-1.45), every format from 2049 (1.00-1.53 at 2304-2560 rows, up to 2.6 at 32768; 13 contractions 1024-16384).
     const unsigned n_sub = in_dim / 32, n_pad = (n_sub + 7) & ~7u;
     const unsigned pad = fmt == REIN_TYPE_Q6_K ? 32 : 16, words = fmt == REIN_TYPE_Q6_K ? 3 : fmt == REIN_TYPE_Q8_0 ? 1 : 2;
     const size_t lds = (size_t)n_pad / 8 * (256 + pad) + (size_t)n_pad * 4 * words;
-    if (n_sub % 2 == 0 && lds <= kLdsPerCu) {
+    const bool narrow = out_dim <= 8 * kCUs && (fmt == REIN_TYPE_Q8_0 || (fmt == REIN_TYPE_Q6_K && (in_dim + 1023) / 1024 % 2 == 0));
+    if (n_sub % 2 == 0 && lds <= kLdsPerCu && !narrow) {
         const unsigned most = fmt == REIN_TYPE_Q6_K || fmt == REIN_TYPE_Q8_0 ? 2 * kCUs : 4 * kCUs;
         return launch(KName("rein_mvd_", fmt_tag(fmt)), std::min((out_dim + 15) / 16, most), 1, 1, 256, (unsigned)lds, s, a);
     }

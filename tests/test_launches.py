@@ -101,3 +101,14 @@ def test_exact_dot_gemm_and_the_scratch_query_without_partial_tiles(tmp_path):
     from reinstinct_amd import runtime
     for fmt in (rein.Q5_K, rein.Q6_K):
         assert runtime.matmul_scratch_bytes(fmt, 256, 64) <= (64 * 8 * 40 + 255) // 256 * 256 + (16 << 20)
+
+
+def test_narrow_on_disk_matrices_keep_the_kernel_of_64_lanes(tmp_path):
+    """Q8_0, and Q6_K where the last 2048 weights of a row fill it, up to a workgroup of eight rows per CU"""
+    shapes = [(rein.Q6_K, 2048, 1024, 0), (rein.Q6_K, 2048, 2048, 0), (rein.Q6_K, 2048, 2049, 1), (rein.Q6_K, 1024, 256, 1), (rein.Q6_K, 3072, 2048, 1),
+              (rein.Q6_K, 1280, 64, 0), (rein.Q8_0, 1024, 2048, 0), (rein.Q8_0, 5120, 512, 0), (rein.Q8_0, 5120, 2049, 1), (rein.Q4_K, 2048, 32, 1),
+              (rein.Q5_K, 4096, 1024, 1), (rein.Q8_0, 5152, 4096, 0), (rein.Q4_K, 131072, 4096, 0), (rein.Q6_K, 2048, 151936, 1)]
+    done = record([("matvec_ondisk_xq8", [f, P, P, P, k, n]) for f, k, n, _ in shapes], tmp_path)
+    for (f, k, n, lds), d in zip(shapes, done):
+        (kernel, *_), = d["launches"]
+        assert kernel.startswith("rein_mvd_" if lds else "matvec_q"), (f, k, n, kernel)
