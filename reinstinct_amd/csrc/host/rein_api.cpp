@@ -2369,21 +2369,27 @@ bool moe_few_fits(const rein_moe_shape& sh)
     return sh.hidden % 64 == 0 && sh.expert_ff % 64 == 0 && sh.n_tok <= 1024 && (unsigned long long)sh.n_tok * sh.n_used <= 65535ull &&
            moe_few_lds(REIN_TYPE_Q6_K, std::max(sh.hidden, sh.expert_ff), 16) <= 128u * 1024u;
 }
-// Where they pay, from eight expert shapes x 4 .. 192 tokens against the decode launches and the pipeline.  Below: the decode launches read
-// an expert again for every entry, which costs nothing while the entries meet different experts, and are one launch fewer -- from
-// 0.8 entries per expert (Q8_0, whose decode launch runs at 5.6 TB/s, 0.95), or once 160 MB are read twice (us, decode / these: 128
-// experts top-8, 2048 x 768, 12 / 16 / 24 tokens 68 / 71, 87 / 77, 122 / 88; 256 top-6, 1280 x 1280, 16 / 64 tokens 107 / 88, 393 / 160).
-// Above: every further entry costs its dots, while a 32-token tile costs the same until it is full -- up to 5.5 entries per expert
-// (48 / 64 / 96 / 128 tokens of the first shape: pipeline 149-154, these 106 / 121 / 150 / 180), 4 where the experts are small and the tiles
-// few (64 top-6, 1792 x 512, 32 / 48 tokens 60 / 51, 61 / 64).
+// Up to here the decode launches are the other choice, beyond the grouped-GEMM pipeline: 1.6 entries per expert (28 tokens of 128
+// experts top-8: 141 us against 143, 32 tokens 160 against 145).
+bool moe_decode_range(const rein_moe_shape& sh) { return 5ull * sh.n_tok * sh.n_used <= 8ull * sh.n_expert; }
+// Where they pay.
+// Against the decode launches, which are two launches fewer, stream at a higher rate and read an expert again for every entry:
+// once what is read again outweighs 30 MB and 0.3 of what both read (0.45 for Q8_0, whose decode launch runs at 5.6 TB/s); an
+// entry counts as 0.2 MB more, the workgroups it costs there.  From 319 cells -- nine expert shapes of 1 to 20 MB, 2-256 experts, top
+// 1-8, 1-48 tokens, the weights of several layers in turn -- of which 301 are within 3 % of the better side (us, decode / these:
+// 128 experts top-8, 2048 x 768, 12 / 16 / 24 tokens 71 / 75, 89 / 82, 124 / 91; 256 experts of 1280 x 1280, 16 / 32 tokens 96 / 107,
+// 178 / 143; few experts hardly gain, 8 top-2 at 4 tokens 15 / 24, 4 top-4 at one 12 / 21, 16 top-8 of 4096 x 1536 at 2 and 3 62 / 60,
+// 83 / 66; furthest off 16 top-2 of that size at 8 tokens, 49 / 59, and 32 top-2 of 2048 x 768 at 20, 34 / 39, both on these).
+// Against the pipeline, from eight expert shapes x 4 .. 192 tokens: every further entry costs its dots, while a 32-token tile costs the
+// same until it is full -- up to 5.5 entries per expert (48 / 64 / 96 / 128 tokens of the first shape: pipeline 149-154, these 106 / 121 /
+// 150 / 180), 4 where the experts are small and the tiles few (64 top-6, 1792 x 512, 32 / 48 tokens 60 / 51, 61 / 64).
 bool moe_few_pays(const rein_moe_shape& sh)
 {
     const double entries = (double)sh.n_tok * sh.n_used, per_expert = entries / sh.n_expert;
     const double bytes = 2.0 * rein_repacked_len(sh.gate_up_fmt, sh.hidden, sh.expert_ff) + (double)rein_repacked_len(sh.down_fmt, sh.expert_ff, sh.hidden);
-    if (per_expert > (bytes * sh.n_expert < 134e6 ? 4.0 : 5.5)) return false;
-    if (per_expert >= (sh.gate_up_fmt == REIN_TYPE_Q8_0 ? 0.95 : 0.8)) return true;
+    if (!moe_decode_range(sh)) return per_expert <= (bytes * sh.n_expert < 134e6 ? 4.0 : 5.5);
     const double touched = sh.n_expert * (1.0 - std::pow(1.0 - (double)sh.n_used / sh.n_expert, (double)sh.n_tok));
-    return (entries - touched) * bytes >= 160e6;
+    return (entries - touched) * bytes + entries * 0.2e6 >= 30e6 + (sh.gate_up_fmt == REIN_TYPE_Q8_0 ? 0.45 : 0.3) * touched * bytes;
 }
 }  // namespace
 
@@ -2434,9 +2440,9 @@ int rein_moe_ffn(const rein_moe_shape* shp, const float* x, const float* logits,
     // Few tokens: with about one routing entry per expert nearly every entry meets an expert of its own, a
     // 32-token tile of the grouped GEMM holds one or two tokens, and the sort is pure overhead.  The decode kernels
     // (qwen35.rs:3071-3167, here in their two fused launches) read an expert per entry -- streaming, where a
-    // mostly empty tile pays its full matrix work -- and are ahead up to 1.6 entries per expert: 128 experts top-8
-    // at 1 / 4 / 16 / 24 tokens 16 / 33 / 89 / 125 us against 48 / 61 / 126 / 141 for the pipeline below, at 28
-    // tokens 141 against 143, at 32 tokens 160 against 145.  Same integer dots, fp32 sums in the decode kernels' order.
+    // mostly empty tile pays its full matrix work: 128 experts top-8 at 1 / 4 / 16 / 24 tokens 16 / 33 / 89 / 125 us against
+    // 48 / 61 / 126 / 141 for the pipeline below.  Same integer dots, fp32 sums in the decode kernels' order.  Where experts
+    // are read several times over, moe_few_pays.
     const bool wave = sh.n_expert <= 256 && sh.n_used <= 64 && sh.n_used <= sh.n_expert && opt_u(O_TOPK_WAVE, 1) != 0;
     const auto route_quantize = [&]() -> int {       // router and quantizer as one small launch
         int n_e = (int)sh.n_expert, n_u = (int)sh.n_used, n_t = (int)sh.n_tok;
@@ -2468,7 +2474,7 @@ int rein_moe_ffn(const rein_moe_shape* shp, const float* x, const float* logits,
                      (void*)&sh.n_expert};
         return launch("rein_moe_combine_rows4_f32", (sh.hidden / 4 + 127) / 128, sh.n_tok, 1, 128, 0, s, c);
     }
-    const bool chain = 5ull * ne <= 8ull * sh.n_expert && sh.expert_ff % 32 == 0 && opt_u(O_MOE_CHAIN, 1) != 0;
+    const bool chain = moe_decode_range(sh) && sh.expert_ff % 32 == 0 && opt_u(O_MOE_CHAIN, 1) != 0;
     if (chain) {
         const unsigned ns_h = sh.hidden / 32, ns_f = sh.expert_ff / 32;
         // Where the one-wavefront router applies it shares a launch: for one or two tokens the gate / up launch

@@ -112,3 +112,19 @@ def test_narrow_on_disk_matrices_keep_the_kernel_of_64_lanes(tmp_path):
     for (f, k, n, lds), d in zip(shapes, done):
         (kernel, *_), = d["launches"]
         assert kernel.startswith("rein_mvd_" if lds else "matvec_q"), (f, k, n, kernel)
+
+
+def test_form_of_the_expert_ffn(tmp_path):
+    """rein_moe_ffn: the decode launches while little is read twice, then every touched expert once, then the pipeline"""
+    q4, q6, q8 = rein.Q4_K, rein.Q6_K, rein.Q8_0
+    few, decode, tiles = "rein_moe_few_gate_up", "gate_up_swiglu_q8", "rein_mmq_"
+    # tokens, hidden, experts, used, width, formats
+    cases = [((1, 2048, 4, 4, 768, q4, q6), decode), ((1, 2048, 8, 8, 768, q4, q6), decode), ((2, 2048, 4, 2, 768, q4, q6), decode),
+             ((4, 2048, 8, 2, 768, q4, q6), decode), ((8, 2048, 8, 2, 768, q4, q6), few), ((1, 4096, 8, 8, 1536, q4, q6), decode),
+             ((3, 4096, 32, 8, 1536, q4, q6), decode), ((4, 4096, 32, 8, 1536, q4, q6), few), ((10, 2048, 128, 8, 768, q4, q6), decode),
+             ((16, 2048, 128, 8, 768, q4, q6), few), ((12, 2048, 128, 8, 768, q8, q8), decode), ((20, 2048, 128, 8, 768, q8, q8), few),
+             ((48, 2048, 128, 8, 768, q4, q6), few), ((96, 2048, 128, 8, 768, q4, q6), tiles)]
+    for (shape, form), d in zip(cases, record([("moe_ffn", list(s)) for s, _ in cases], tmp_path)):
+        kernels = [r[0] for r in d["launches"]]
+        assert any(form in k for k in kernels), (shape, kernels)
+        assert form == few or not any(few in k for k in kernels), (shape, kernels)
