@@ -1,18 +1,26 @@
 """Launch sites of the path, as thin wrappers over the C ABI.  Arguments are
 device pointers (ints or DeviceBuf) exactly as the C functions take them.
 
-The calls that launch are compiled (csrc/python/native.cpp); what follows here asks, sizes or places something."""
+The calls that launch are compiled (csrc/python/native.cpp), or ctypes' where that extension is not built for this interpreter
+(_calls.py); what follows here asks, sizes or places something.  Importing needs nothing built; a call without librein.so raises."""
 import ctypes as C
 
-from ._lib import MoeShape, check, lib, need_built
+from ._lib import MoeShape, check, lib
 
-need_built("_native.so")
-from ._native import (  # noqa: E402, F401
-    quantize_q8, rmsnorm_q8, add_rmsnorm_q8, swiglu_q8, sigmoid_mul_q8, rmsnorm_gated_q8, moe_geglu_q8, matvec_xq8,
-    matvec_batched_xq8, matvec_multi_xq8, matvec_ondisk_xq8, matvec_q8_0_splitk, mmq_xq8, mmq_xq8_ws,
-    mmq_xq8_noalloc, matmul, matmul_ws, moe_topk, moe_sort, moe_gather_xq, moe_quantize_scatter, moe_scatter_rows,
-    moe_grouped_gemm, moe_grouped_swiglu_q8, moe_expert_matvec, moe_down, moe_gate_up_swiglu, moe_gate_up_swiglu_q8,
-    moe_down_combine, swiglu_mul, moe_combine, moe_ffn)
+try:
+    from ._native import (  # noqa: F401
+        quantize_q8, rmsnorm_q8, add_rmsnorm_q8, swiglu_q8, sigmoid_mul_q8, rmsnorm_gated_q8, moe_geglu_q8, matvec_xq8,
+        matvec_batched_xq8, matvec_multi_xq8, matvec_ondisk_xq8, matvec_q8_0_splitk, mmq_xq8, mmq_xq8_ws,
+        mmq_xq8_noalloc, matmul, matmul_ws, moe_topk, moe_sort, moe_gather_xq, moe_quantize_scatter, moe_scatter_rows,
+        moe_grouped_gemm, moe_grouped_swiglu_q8, moe_expert_matvec, moe_down, moe_gate_up_swiglu, moe_gate_up_swiglu_q8,
+        moe_down_combine, swiglu_mul, moe_combine, moe_ffn)
+except ImportError:
+    from ._calls import (  # noqa: F401
+        quantize_q8, rmsnorm_q8, add_rmsnorm_q8, swiglu_q8, sigmoid_mul_q8, rmsnorm_gated_q8, moe_geglu_q8, matvec_xq8,
+        matvec_batched_xq8, matvec_multi_xq8, matvec_ondisk_xq8, matvec_q8_0_splitk, mmq_xq8, mmq_xq8_ws,
+        mmq_xq8_noalloc, matmul, matmul_ws, moe_topk, moe_sort, moe_gather_xq, moe_quantize_scatter, moe_scatter_rows,
+        moe_grouped_gemm, moe_grouped_swiglu_q8, moe_expert_matvec, moe_down, moe_gate_up_swiglu, moe_gate_up_swiglu_q8,
+        moe_down_combine, swiglu_mul, moe_combine, moe_ffn)
 
 
 def matvec_kernel_name(fmt, in_dim, out_dim, n_rows):

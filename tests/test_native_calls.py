@@ -2,11 +2,18 @@
 refused by the library's or the wrapper's own checks)."""
 import ctypes as C
 import inspect
+import json
+import os
+import shutil
+import subprocess
+import sys
 
 import pytest
 
 import reinstinct_amd as rein
 from reinstinct_amd import runtime
+
+PKG = os.path.dirname(os.path.abspath(rein.__file__))
 
 
 class Buf:
@@ -46,3 +53,61 @@ def test_multi_tables():
 def test_signatures_are_visible():
     assert str(inspect.signature(runtime.rmsnorm_q8)) == "(x, w, xq, n, n_vec=1, eps=1e-06, stream=None)"
     assert "quantize_q8" in runtime.quantize_q8.__doc__
+
+
+def child(code, root):
+    return subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120, cwd=root,
+                          env=dict(os.environ, PYTHONPATH=str(root)))
+
+
+def package(root, *built):
+    """a copy of the package's Python files, with these of the built ones"""
+    there = root / "reinstinct_amd"
+    there.mkdir()
+    for f in os.listdir(PKG):
+        if f.endswith(".py") or f in built:
+            os.symlink(os.path.join(PKG, f), there / f)
+    return root
+
+
+def test_import_and_calls_without_anything_built(tmp_path):
+    run = child("from reinstinct_amd import runtime, hip, quant, gguf, ReinError\n"
+                "try: runtime.quantize_q8(64, 64, 32)\n"
+                "except ReinError as e: print(e.code, e)\n", package(tmp_path))
+    assert run.returncode == 0, run.stderr
+    assert run.stdout.startswith("-1 ") and "librein.so is not built" in run.stdout
+
+
+def test_the_extension_is_the_one_in_use():
+    assert inspect.isbuiltin(runtime.quantize_q8) and inspect.isbuiltin(runtime.moe_ffn)
+
+
+def test_calls_by_ctypes_are_the_same(tmp_path):
+    """without the compiled extension: every launch call is there, with its parameters and defaults, and reaches the library"""
+    names = [n for n in dir(runtime) if inspect.isbuiltin(getattr(runtime, n))]
+    assert len(names) == 32
+    run = child("import inspect, json\n"
+                "from reinstinct_amd import runtime, ReinError\n"
+                f"names = {names!r}\n"
+                "assert not any(inspect.isbuiltin(getattr(runtime, n)) for n in names)\n"
+                "codes = []\n"
+                "for call in (lambda: runtime.quantize_q8(64, 64, 31), lambda: runtime.matvec_multi_xq8([12] * 5, [64] * 5, [64] * 5, [32] * 5, 64, 256),\n"
+                "             lambda: runtime.moe_ffn(runtime.moe_shape(0, 256, 8, 2, 256, 12, 12), 64, 64, 64, 64, 64, 64, 256, 64),\n"
+                "             lambda: runtime.matmul_ws(12, 64, 64, 64, 256, 32, 40, 64, n_scratch)):\n"
+                "    n_scratch = 8\n"
+                "    try: call()\n"
+                "    except ReinError as e: codes.append(e.code)\n"
+                "print(json.dumps([codes, [str(inspect.signature(getattr(runtime, n))) for n in names]]))\n", package(tmp_path, "librein.so"))
+    assert run.returncode == 0, run.stderr
+    codes, signatures = json.loads(run.stdout)
+    assert codes == [-3, -3, -3, -3]
+    assert signatures == [str(inspect.signature(getattr(runtime, n))) for n in names]
+
+
+@pytest.mark.skipif(shutil.which("make") is None, reason="no make")
+def test_the_library_builds_without_pythons_headers(tmp_path):
+    csrc = os.path.join(PKG, "csrc")
+    for setting in (f"PY_INC={tmp_path}", "PYTHON=/nonexistent/python"):
+        plan = subprocess.run(["make", "-n", "-B", "-C", csrc, setting], capture_output=True, text=True)
+        assert plan.returncode == 0, plan.stderr
+        assert "rein_api.cpp" in plan.stdout and "rein_kernels.hip" in plan.stdout and "native.cpp" not in plan.stdout
