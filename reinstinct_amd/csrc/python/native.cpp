@@ -15,11 +15,41 @@
 namespace {
 
 PyObject* g_check;        // reinstinct_amd._lib.check: raises ReinError with rein_last_error()
+PyObject* g_shape;        // reinstinct_amd._lib.MoeShape
 PyObject* g_as_parameter;
 PyObject* g_value;
+PyObject *g_cast, *g_void_p, *g_int, *g_uint, *g_size, *g_float;        // of ctypes
 
-// ---- one argument.  A pointer is an int, None, an object with ctypes' `_as_parameter_` (DeviceBuf, Stream) or a ctypes
-// pointer value; whole numbers are cut to their C type as ctypes does.
+// ---- one argument.  What ctypes takes for a parameter of its C type is taken, and nothing else: the quick ways are a test of the
+// type, the others go through ctypes' own types.  Whole numbers are cut to their C type as ctypes does.
+bool to_c(PyObject* o, void** out);
+bool to_c(PyObject* o, unsigned* out);
+bool to_c(PyObject* o, int* out);
+bool to_c(PyObject* o, size_t* out);
+bool to_c(PyObject* o, float* out);
+
+// the attribute of o called name, converted; -1: there is none
+template <class T> int from_attribute(PyObject* o, PyObject* name, T* out)
+{
+    PyObject* v = PyObject_GetAttr(o, name);
+    if (!v) {
+        PyErr_Clear();
+        return -1;
+    }
+    bool ok = false;
+    if (Py_EnterRecursiveCall(" in an argument") == 0) {
+        ok = to_c(v, out);
+        Py_LeaveRecursiveCall();
+    }
+    Py_DECREF(v);
+    return ok;
+}
+bool wrong(const char* want, PyObject* o)
+{
+    PyErr_Format(PyExc_TypeError, "%s is wanted, not %.80s", want, Py_TYPE(o)->tp_name);
+    return false;
+}
+// a pointer: an int, None, an object that stands for one (DeviceBuf), or what ctypes turns into a void pointer
 bool to_c(PyObject* o, void** out)
 {
     if (PyLong_Check(o)) {
@@ -30,54 +60,43 @@ bool to_c(PyObject* o, void** out)
         *out = nullptr;
         return true;
     }
-    PyObject* v = PyObject_GetAttr(o, g_as_parameter);
-    if (!v) {
+    const int got = from_attribute(o, g_as_parameter, out);
+    if (got >= 0) return got;
+    PyObject* p = PyObject_CallFunctionObjArgs(g_cast, o, g_void_p, nullptr);
+    if (!p) {
         PyErr_Clear();
-        v = PyObject_GetAttr(o, g_value);
+        return wrong("a device pointer (an int, None or a DeviceBuf)", o);
     }
-    if (!v) {
-        PyErr_Clear();
-        PyErr_Format(PyExc_TypeError, "a device pointer is an int, None, a DeviceBuf or a Stream, not %.80s", Py_TYPE(o)->tp_name);
-        return false;
-    }
-    bool ok = false;
-    if (Py_EnterRecursiveCall(" in a pointer argument") == 0) {
-        ok = to_c(v, out);
-        Py_LeaveRecursiveCall();
-    }
-    Py_DECREF(v);
-    return ok;
+    const int ok = from_attribute(p, g_value, out);          // the memory it points to is o's, which the caller holds
+    Py_DECREF(p);
+    return ok > 0;
 }
 template <class T> bool to_c(PyObject* o, T** out) { return to_c(o, reinterpret_cast<void**>(const_cast<std::remove_const_t<T>**>(out))); }
-bool whole(PyObject* o, unsigned long long* out)
+template <class T> bool whole(PyObject* o, PyObject* ctype, T* out)
 {
-    if (!PyLong_Check(o)) {
-        PyErr_Format(PyExc_TypeError, "a whole number is wanted, not %.80s", Py_TYPE(o)->tp_name);
-        return false;
+    if (PyLong_Check(o) || PyIndex_Check(o)) {
+        const unsigned long long v = PyLong_AsUnsignedLongLongMask(o);
+        *out = (T)v;
+        return v != (unsigned long long)-1 || !PyErr_Occurred();
     }
-    *out = PyLong_AsUnsignedLongLongMask(o);
-    return !PyErr_Occurred();
+    const int is = PyObject_IsInstance(o, ctype);
+    if (is < 0) return false;
+    const int got = from_attribute(o, is ? g_value : g_as_parameter, out);
+    return got < 0 ? wrong("a whole number", o) : got;
 }
-bool to_c(PyObject* o, unsigned* out)
-{
-    unsigned long long v;
-    return whole(o, &v) && (*out = (unsigned)v, true);
-}
-bool to_c(PyObject* o, int* out)
-{
-    unsigned long long v;
-    return whole(o, &v) && (*out = (int)(unsigned)v, true);
-}
-bool to_c(PyObject* o, size_t* out)
-{
-    unsigned long long v;
-    return whole(o, &v) && (*out = (size_t)v, true);
-}
+bool to_c(PyObject* o, unsigned* out) { return whole(o, g_uint, out); }
+bool to_c(PyObject* o, int* out) { return whole(o, g_int, out); }
+bool to_c(PyObject* o, size_t* out) { return whole(o, g_size, out); }
 bool to_c(PyObject* o, float* out)
 {
     const double v = PyFloat_AsDouble(o);
     *out = (float)v;
-    return v != -1.0 || !PyErr_Occurred();
+    if (v != -1.0 || !PyErr_Occurred()) return true;
+    PyErr_Clear();
+    const int is = PyObject_IsInstance(o, g_float);
+    if (is < 0) return false;
+    const int got = from_attribute(o, is ? g_value : g_as_parameter, out);
+    return got < 0 ? wrong("a number", o) : got;
 }
 
 // ---- the arguments of a call in the order of the parameters, keywords and defaults filled in.  `names` ends with NULL;
@@ -232,16 +251,16 @@ PyObject* py_moe_ffn(PyObject*, PyObject* const* a, Py_ssize_t nargs, PyObject* 
                                         "stream", nullptr};
     std::array<PyObject*, 10> got;
     if (!gather("moe_ffn", names, g_none, 1, a, nargs, kw, got)) return nullptr;
+    const int is = PyObject_IsInstance(got[0], g_shape);
+    if (is <= 0) {
+        if (is == 0) PyErr_SetString(PyExc_TypeError, "moe_ffn: shape is what moe_shape() returns");
+        return nullptr;
+    }
     Py_buffer b;
     if (PyObject_GetBuffer(got[0], &b, PyBUF_SIMPLE) != 0) return nullptr;
     rein_moe_shape shape;
-    const bool fits = b.len == (Py_ssize_t)sizeof shape;
-    if (fits) std::memcpy(&shape, b.buf, sizeof shape);
+    std::memcpy(&shape, b.buf, sizeof shape);
     PyBuffer_Release(&b);
-    if (!fits) {
-        PyErr_SetString(PyExc_TypeError, "moe_ffn: shape is what moe_shape() returns");
-        return nullptr;
-    }
     void *p[8], *stream;
     for (int i = 0; i < 8; i++)
         if (!to_c(got[1 + i], &p[i])) return nullptr;
@@ -319,14 +338,19 @@ PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_native", "The launch calls of r
 
 PyMODINIT_FUNC PyInit__native(void)
 {
-    PyObject* lib = PyImport_ImportModule("reinstinct_amd._lib");
-    if (!lib) return nullptr;
-    g_check = PyObject_GetAttrString(lib, "check");
+    PyObject *lib = PyImport_ImportModule("reinstinct_amd._lib"), *ctypes = PyImport_ImportModule("ctypes");
+    if (!lib || !ctypes) return nullptr;
+    const auto take = [](PyObject* m, const char* name, PyObject** to) { return (*to = PyObject_GetAttrString(m, name)) != nullptr; };
+    const bool ok = take(lib, "check", &g_check) && take(lib, "MoeShape", &g_shape) && take(ctypes, "cast", &g_cast) &&
+                    take(ctypes, "c_void_p", &g_void_p) && take(ctypes, "c_int", &g_int) && take(ctypes, "c_uint", &g_uint) &&
+                    take(ctypes, "c_size_t", &g_size) && take(ctypes, "c_float", &g_float);
     Py_DECREF(lib);
+    Py_DECREF(ctypes);
+    if (!ok) return nullptr;
     g_as_parameter = PyUnicode_InternFromString("_as_parameter_");
     g_value = PyUnicode_InternFromString("value");
     PyObject *one = PyLong_FromLong(1), *eps = PyFloat_FromDouble(1e-6);
-    if (!g_check || !g_as_parameter || !g_value || !one || !eps) return nullptr;
+    if (!g_as_parameter || !g_value || !one || !eps) return nullptr;
     g_none[0] = g_one_none[1] = g_one_eps_none[2] = g_eps_none[1] = Py_None;
     g_one_none[0] = g_one_eps_none[0] = one;
     g_one_eps_none[1] = g_eps_none[0] = eps;

@@ -8,6 +8,7 @@ import shutil
 import subprocess
 import sys
 
+import numpy as np
 import pytest
 
 import reinstinct_amd as rein
@@ -37,6 +38,47 @@ def test_wrong_arguments():
                  lambda: runtime.moe_ffn(b"short", 64, 64, 64, 64, 64, 64, 64, 64)):
         with pytest.raises(TypeError):
             call()
+
+
+class Four:
+    def __index__(self):
+        return 4
+
+
+COUNTS = (32, True, np.int64(32), np.uint8(32), Four(), C.c_uint(32))
+POINTERS = (64, None, Buf(), C.c_void_p(64), C.c_void_p(None), C.create_string_buffer(64), C.pointer(C.c_int(1)), C.byref(C.c_int(1)), b"host", C.c_char_p(b"host"))
+NUMBERS = (1e-6, 1, np.float32(1e-6), np.int32(1), C.c_float(1e-6))
+NEITHER = (1.5, "32", C.c_int(32), C.c_long(32), C.c_float(1.0), [32], object(), np.float32(4.0), np.zeros(4))
+
+
+@pytest.mark.parametrize("o", [*COUNTS, *POINTERS, *NUMBERS, *NEITHER], ids=repr)
+def test_arguments_are_those_of_ctypes(o):
+    """what ctypes takes for an unsigned, a pointer and a float parameter is taken, what it refuses is refused"""
+    def taken(ctype):
+        try:
+            ctype.from_param(o)
+            return True
+        except (TypeError, C.ArgumentError):
+            return False
+
+    def called(call):
+        try:
+            call()
+        except rein.ReinError:                                # the library's own refusal: every argument was converted
+            return True
+        except TypeError:
+            return False
+
+    assert called(lambda: runtime.quantize_q8(64, 64, 31, o)) == taken(C.c_uint)
+    assert called(lambda: runtime.quantize_q8(o, 64, 31)) == taken(C.c_void_p)
+    assert called(lambda: runtime.rmsnorm_q8(64, 64, 64, 31, 1, o)) == taken(C.c_float)
+    assert called(lambda: runtime.matmul_ws(12, 64, 64, 64, 31, 32, 40, 64, o)) == taken(C.c_size_t)
+    assert called(lambda: runtime.matvec_xq8(o, 64, 64, 64, 0, 32)) == taken(C.c_int)
+
+
+def test_the_shape_of_moe_ffn():
+    with pytest.raises(TypeError):
+        runtime.moe_ffn(bytes(C.sizeof(runtime.MoeShape)), 64, 64, 64, 64, 64, 64, 64, 64)
 
 
 def test_multi_tables():
