@@ -18,6 +18,7 @@ PyObject* g_check;        // reinstinct_amd._lib.check: raises ReinError with re
 PyObject* g_shape;        // reinstinct_amd._lib.MoeShape
 PyObject* g_as_parameter;
 PyObject* g_value;
+PyObject* g_raw;
 PyObject *g_cast, *g_void_p, *g_int, *g_uint, *g_size, *g_float;        // of ctypes
 
 // ---- one argument.  What ctypes takes for a parameter of its C type is taken, and nothing else: the quick ways are a test of the
@@ -70,6 +71,16 @@ bool to_c(PyObject* o, void** out)
     const int ok = from_attribute(p, g_value, out);          // the memory it points to is o's, which the caller holds
     Py_DECREF(p);
     return ok > 0;
+}
+// a stream: None or a hip.Stream, an object whose `raw` is the handle.  Nothing else: a number here is a count or a pointer that
+// slipped by one parameter
+struct Stream { void* raw; operator void*() const { return raw; } };
+bool to_c(PyObject* o, Stream* out)
+{
+    out->raw = nullptr;
+    if (o == Py_None) return true;
+    const int got = from_attribute(o, g_raw, &out->raw);
+    return got < 0 ? wrong("a stream (a hip.Stream or None)", o) : got;
 }
 template <class T> bool to_c(PyObject* o, T** out) { return to_c(o, reinterpret_cast<void**>(const_cast<std::remove_const_t<T>**>(out))); }
 template <class T> bool whole(PyObject* o, PyObject* ctype, T* out)
@@ -142,7 +153,8 @@ PyObject* result(int rc)
 template <class... A, size_t... I>
 PyObject* call(int (*fn)(A...), const std::array<PyObject*, sizeof...(A)>& got, std::index_sequence<I...>)
 {
-    std::tuple<A...> c;
+    // (the last parameter of every one of them is the stream)
+    std::tuple<std::conditional_t<I + 1 == sizeof...(A), Stream, A>...> c;
     if (!(to_c(got[I], &std::get<I>(c)) && ...)) return nullptr;
     int rc;
     Py_BEGIN_ALLOW_THREADS
@@ -233,7 +245,7 @@ PyObject* py_matvec_multi_xq8(PyObject*, PyObject* const* a, Py_ssize_t nargs, P
     float* ys[4] = {};
     unsigned dims[4] = {}, in_dim, n_rows;
     const void* xq;
-    void* stream;
+    Stream stream;
     if (!table(got[0], "fmts", n, fmts) || !table(got[1], "ws", n, ws) || !table(got[2], "ys", n, ys) || !table(got[3], "out_dims", n, dims) ||
         !to_c(got[4], &xq) || !to_c(got[5], &in_dim) || !to_c(got[6], &n_rows) || !to_c(got[7], &stream))
         return nullptr;
@@ -261,7 +273,8 @@ PyObject* py_moe_ffn(PyObject*, PyObject* const* a, Py_ssize_t nargs, PyObject* 
     rein_moe_shape shape;
     std::memcpy(&shape, b.buf, sizeof shape);
     PyBuffer_Release(&b);
-    void *p[8], *stream;
+    void* p[8];
+    Stream stream;
     for (int i = 0; i < 8; i++)
         if (!to_c(got[1 + i], &p[i])) return nullptr;
     if (!to_c(got[9], &stream)) return nullptr;
@@ -349,8 +362,9 @@ PyMODINIT_FUNC PyInit__native(void)
     if (!ok) return nullptr;
     g_as_parameter = PyUnicode_InternFromString("_as_parameter_");
     g_value = PyUnicode_InternFromString("value");
+    g_raw = PyUnicode_InternFromString("raw");
     PyObject *one = PyLong_FromLong(1), *eps = PyFloat_FromDouble(1e-6);
-    if (!g_as_parameter || !g_value || !one || !eps) return nullptr;
+    if (!g_as_parameter || !g_value || !g_raw || !one || !eps) return nullptr;
     g_none[0] = g_one_none[1] = g_one_eps_none[2] = g_eps_none[1] = Py_None;
     g_one_none[0] = g_one_eps_none[0] = one;
     g_one_eps_none[1] = g_eps_none[0] = eps;

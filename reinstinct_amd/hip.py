@@ -86,7 +86,7 @@ class Stream:
     def __init__(self):
         p = C.c_void_p(0)
         check(lib.rein_stream_create(C.byref(p)))
-        self.raw = self._as_parameter_ = p.value
+        self.raw = p.value
 
     def synchronize(self):
         check(lib.rein_stream_synchronize(self.raw))

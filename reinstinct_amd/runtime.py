@@ -60,7 +60,7 @@ def mmq_tile_plan_ws(fmt, out_dim, p_rows):
 
 def mmq_block_dots_ws(fmt, w, xq, out, in_dim, out_dim, n_rows, workspace, workspace_bytes, stream=None):
     check(lib.rein_mmq_block_dots_ws(fmt, w, xq, out, in_dim, out_dim, n_rows, workspace, workspace_bytes,
-                                     stream))
+                                     stream.raw if stream is not None else None))
 
 
 def matmul_scratch_bytes(fmt, in_dim, n_rows):
@@ -83,7 +83,8 @@ def mmq_tile_plan(fmt, in_dim, out_dim, p_rows):
 
 
 def block_dots(fmt, w, xq, out, in_dim, out_dim, n_rows, via_mfma=False, stream=None):
-    check(lib.rein_block_dots(fmt, w, xq, out, in_dim, out_dim, n_rows, int(via_mfma), stream))
+    check(lib.rein_block_dots(fmt, w, xq, out, in_dim, out_dim, n_rows, int(via_mfma),
+                              stream.raw if stream is not None else None))
 
 
 def moe_gemm_bn():

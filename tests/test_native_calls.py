@@ -12,7 +12,7 @@ import numpy as np
 import pytest
 
 import reinstinct_amd as rein
-from reinstinct_amd import runtime
+from reinstinct_amd import hip, runtime
 
 PKG = os.path.dirname(os.path.abspath(rein.__file__))
 
@@ -27,8 +27,31 @@ def test_pointer_arguments(x):
         runtime.quantize_q8(x, 64, 31)
     assert e.value.code == -3
     with pytest.raises(rein.ReinError) as e:
-        runtime.quantize_q8(x, xq=64, in_dim=31, n_vec=2, stream=x)
+        runtime.quantize_q8(x, xq=64, in_dim=31, n_vec=2, stream=None)
     assert e.value.code == -3
+
+
+class OnStream:
+    raw = 64
+
+
+@pytest.mark.parametrize("call", [lambda s: runtime.quantize_q8(64, 64, 31, 1, s), lambda s: runtime.quantize_q8(64, 64, 31, stream=s),
+                                  lambda s: runtime.matvec_multi_xq8([12], [64], [64], [32], 64, 255, 1, s),
+                                  lambda s: runtime.moe_ffn(runtime.moe_shape(0, 256, 8, 2, 256, 12, 12), 64, 64, 64, 64, 64, 64, 64, 64, s)])
+def test_a_stream_is_a_stream(call):
+    """None or an object whose `raw` is the handle; a number, a pointer or a buffer in its place is a mistake"""
+    for stream in (None, OnStream()):
+        with pytest.raises(rein.ReinError) as e:
+            call(stream)
+        assert e.value.code == -3
+    for stream in (64, True, Buf(), C.c_void_p(64), "s"):
+        with pytest.raises(TypeError):
+            call(stream)
+
+
+def test_a_stream_is_no_pointer():
+    with pytest.raises(TypeError):
+        runtime.quantize_q8(hip.Stream.__new__(hip.Stream), 64, 31)
 
 
 def test_wrong_arguments():
