@@ -90,7 +90,9 @@ int rein_is_loaded(void);
  * overrides them is set, and setting it back to NULL / "" hands the choice back.  Entries are
  * single atomic words; changing one while another thread launches is safe.
  * Names (rein_option_name enumerates them): REIN_MV_ROWS, REIN_MV_WPB (decode matvec rows per
- * wavefront 1/2/4, wavefronts per workgroup 1/2/4; 1..16 for the LDS-staged kernel), REIN_MV_LDS
+ * wavefront 1/2/4, wavefronts per workgroup 1/2/4; 1..16 for the LDS-staged kernel), REIN_MV_LOADS
+ * (how a decode matvec loads its weights: 0 plain, 1 the wide planes nontemporal, 2 all of them where
+ * that is built, up to four rows; the same bits), REIN_MV_LDS
  * (batched decode of 2..4 rows on the kernel that stages the activation rows in LDS: 0 never,
  * 1 whenever the rows fit), REIN_QUAD_LDS (the same for the 4x4x4 kernel, 3..8 rows),
  * REIN_QUAD_SLICES, REIN_QUAD_DEPTH (wavefronts that share a row group of that kernel, 1..8;

@@ -1,5 +1,5 @@
 """The few-row kernels in the builds that differ in how they load the weights, on both sides of the sizes where one follows the
-other, with a remainder of rows; one matrix and several in one launch."""
+other, with a remainder of rows; one matrix and several in one launch; every build against the others, bit for bit."""
 import numpy as np
 import pytest
 
@@ -51,3 +51,50 @@ def test_loads_of_several_matrices(outs, rows):
     hip.synchronize()
     for f, n, w, y in zip(fmts, outs, ws, ys):
         assert_close_f32(y.to_host(np.float32).reshape(rows, n), orc.matvec_q8(f, w, in_dim, n, xq, rows).reshape(rows, n), what=f"fmt {f} -> {n}")
+
+
+FAMILIES = {                                        # options that keep every row count on one family
+    "rein_mv_": {"REIN_MV_LDS": 0, "REIN_QUAD_LDS": 0, "REIN_SKINNY_FROM": 99, "REIN_QUAD_FROM": 99},
+    "rein_mvl_": {"REIN_MV_LDS": 1},
+    "rein_mvql_": {"REIN_QUAD_LDS": 1},
+}
+
+
+@pytest.mark.parametrize("family, rows", [("rein_mv_", (1, 2, 4)), ("rein_mvl_", (2, 4)), ("rein_mvql_", (4, 8, 16))])
+@pytest.mark.parametrize("fmt", [rein.Q4_0, rein.Q4_K, rein.Q5_K, rein.Q6_K, rein.Q8_0, rein.IQ4_XS, rein.IQ3_S])
+def test_every_build_gives_the_same_bits(family, rows, fmt, options):
+    in_dim, out_dim = 1536, 1031
+    w = orc.repack_for_matvec(fmt, random_raw_weights(fmt, in_dim, out_dim, seed=fmt), in_dim, out_dim)
+    dw, dx = dev(w), dev(orc.quantize_q8(np.random.default_rng(fmt).standard_normal((16, in_dim)).astype(np.float32)))
+    for name, value in FAMILIES[family].items():
+        options.set(name, value)
+    for n in rows:
+        seen = {}
+        for build in (0, 1, 2):
+            options.set("REIN_MV_LOADS", build)
+            kernel = runtime.matvec_kernel_name(fmt, in_dim, out_dim, n)
+            assert kernel.startswith(family)
+            dy = dev(np.full(n * out_dim, np.nan, np.float32))
+            runtime.mmq_xq8(fmt, dw, dx, dy, in_dim, out_dim, n)
+            hip.synchronize()
+            seen[kernel] = dy.to_host(np.uint32)
+        assert len(seen) == (3 if n <= 4 else 2)
+        first = next(iter(seen.values()))
+        assert not np.isnan(first.view(np.float32)).any()
+        assert all(np.array_equal(v, first) for v in seen.values())
+
+
+@pytest.mark.parametrize("rows", [1, 2, 4])
+def test_every_build_of_the_multi_matrix_launch_gives_the_same_bits(rows, options):
+    in_dim, outs, fmts = 1536, (517, 130, 65), (rein.Q5_K, rein.Q6_K, rein.Q8_0)
+    dx = dev(orc.quantize_q8(np.random.default_rng(3).standard_normal((rows, in_dim)).astype(np.float32)))
+    dws = [dev(orc.repack_for_matvec(f, random_raw_weights(f, in_dim, n, seed=n), in_dim, n)) for f, n in zip(fmts, outs)]
+    got = []
+    for build in (0, 1, 2):
+        options.set("REIN_MV_LOADS", build)
+        ys = [dev(np.full(rows * n, np.nan, np.float32)) for n in outs]
+        runtime.matvec_multi_xq8(list(fmts), dws, ys, list(outs), dx, in_dim, rows)
+        hip.synchronize()
+        got.append(np.concatenate([y.to_host(np.uint32) for y in ys]))
+    assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
+    assert not np.isnan(got[0].view(np.float32)).any()

@@ -161,3 +161,34 @@ def test_smaller_scratch_and_capture():
         graph.launch(stream)
         stream.synchronize()
         assert np.array_equal(dy.to_host(np.uint32), eager)
+
+
+D_AT = {rein.Q4_K: (144, 0), rein.Q5_K: (176, 0), rein.Q6_K: (210, 208)}        # bytes of a block, where d lies
+
+
+@pytest.mark.parametrize("fmt", list(D_AT))
+@pytest.mark.parametrize("split", [1, 2])
+def test_infinities_and_nan_stay_where_they_are(fmt, split):
+    """rows of x with an infinity or a NaN and weight rows with such a scale: non-finite where the int8 tile is, every other result
+    the bits of a product without them"""
+    rows, in_dim, out_dim = 97, 1024, 200
+    rng = np.random.default_rng(fmt)
+    x = rng.standard_normal((rows, in_dim)).astype(np.float32)
+    blocks = quant.quantize_weights(fmt, rng.standard_normal((out_dim, in_dim)).astype(np.float32) * 0.02).reshape(out_dim, -1, D_AT[fmt][0])
+    at = D_AT[fmt][1]
+    bad_x, bad_w = x.copy(), blocks.copy()
+    for r, v in {3: np.inf, 40: np.nan, 64: -np.inf, 96: np.inf}.items():
+        bad_x[r, (11 * r) % in_dim] = v
+    for r, v in {0: np.nan, 77: np.inf, 130: -np.inf, 199: np.nan}.items():
+        bad_w[r, r % 4, at:at + 2] = np.array([v], np.float16).view(np.uint8)
+
+    def product(w, x, mode):
+        return matmul(fmt, quant.repack_for_matvec(fmt, np.ascontiguousarray(w).reshape(-1), in_dim, out_dim), x, out_dim, mode, split)
+
+    clean, got, tile = product(blocks, x, 2), product(bad_w, bad_x, 2), product(bad_w, bad_x, 0)
+    assert np.array_equal(np.isfinite(got), np.isfinite(tile))
+    assert not np.isfinite(got[[3, 64, 96]]).any() and not np.isfinite(got[:, [0, 77, 130, 199]]).any()
+    rest = np.ix_(np.setdiff1d(np.arange(rows), [3, 40, 64, 96]), np.setdiff1d(np.arange(out_dim), [0, 77, 130, 199]))
+    assert np.array_equal(got[rest].view(np.uint32), clean[rest].view(np.uint32))
+    nan_row = got[40][np.isfinite(got[40])]
+    assert_close_f32(nan_row, tile[40][np.isfinite(got[40])], what="row with a NaN")

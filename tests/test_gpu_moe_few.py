@@ -61,3 +61,44 @@ def test_few_tokens_per_expert(gu, dn, n_tok, n_expert, n_used, hidden, ff, skew
     # the intermediate is re-quantized after SwiGLU: fp32 noise in gate / up can move a quant by one step
     assert rel_l2(got, want) < 2e-3
     assert_close_f32(got, want, rel=2e-2, abs_=2e-3, what="moe_ffn, touched experts once")
+
+
+@pytest.mark.parametrize("gu,dn", [(rein.Q4_K, rein.Q6_K), (rein.Q6_K, rein.Q5_K), (rein.Q8_0, rein.Q8_0)])
+@pytest.mark.parametrize("hidden, ff", [(1024, 256), (1280, 512)])          # without and with lanes past the contraction
+def test_infinities_and_nan_stay_where_they_are(gu, dn, hidden, ff, options):
+    """tokens with an infinity or a NaN, and an expert with such a scale in one row of its down projection: non-finite where the
+    pipeline is, every other result the bits of a call without them"""
+    n_tok, n_expert, n_used = 30, 6, 2
+    rng = np.random.default_rng(hidden)
+    x = rng.standard_normal((n_tok, hidden)).astype(np.float32)
+    logits = rng.standard_normal((n_tok, n_expert)).astype(np.float32)
+    gate, up = slab(gu, hidden, ff, n_expert, 1), slab(gu, hidden, ff, n_expert, 2)
+    blocks = quant.quantize_weights(dn, (rng.standard_normal((n_expert, hidden, ff)) * 0.02).astype(np.float32)).reshape(n_expert, hidden, -1)
+    size, at = {rein.Q5_K: (176, 0), rein.Q6_K: (210, 208), rein.Q8_0: (34, 0)}[dn]
+    bad_x, bad = x.copy(), blocks.copy()
+    for t, v in {2: np.inf, 17: np.nan, 29: -np.inf}.items():
+        bad_x[t, 9 * t] = v
+    row, expert = 77, 4
+    bad[expert, row, at:at + 2] = np.array([np.inf], np.float16).view(np.uint8)
+    scale = np.ones(n_expert, np.float32)
+    sh = runtime.moe_shape(n_tok, hidden, n_expert, n_used, ff, gu, dn)
+    ws = hip.DeviceBuf(runtime.moe_workspace_bytes(sh))
+
+    def ffn(x, down, few):
+        options.set("REIN_MOE_FEW", few)
+        down = np.concatenate([quant.repack_for_matvec(dn, down[e].reshape(-1), ff, hidden) for e in range(n_expert)])
+        d_out = dev(np.full(n_tok * hidden, 12345.0, np.float32))
+        runtime.moe_ffn(sh, dev(x), dev(logits), dev(gate), dev(up), dev(down), dev(scale), ws, d_out)
+        hip.synchronize()
+        return d_out.to_host(np.float32).reshape(n_tok, hidden)
+
+    clean, got, other = ffn(x, blocks, 1), ffn(bad_x, bad, 1), ffn(bad_x, bad, 0)
+    assert np.array_equal(np.isfinite(got), np.isfinite(other))
+    # gate and up of these tokens are NaN, whose blocks of the intermediate have quants of 0 and a NaN for their sum: only formats with
+    # minimums read the sum (the pipeline the same)
+    assert np.isfinite(got[[2, 29]]).any() != (dn == rein.Q5_K)
+    ids, _ = orc.moe_topk(logits, n_used)
+    there = (ids.reshape(n_tok, n_used) == expert).any(axis=1)
+    assert there.any() and not np.isfinite(got[there, row]).any()
+    rest = np.ix_(np.setdiff1d(np.arange(n_tok), [2, 17, 29]), np.setdiff1d(np.arange(hidden), [row]))
+    assert np.array_equal(got[rest].view(np.uint32), clean[rest].view(np.uint32))
