@@ -1861,35 +1861,38 @@ size_t xh_image_bytes(int fmt, unsigned in_dim, unsigned p_rows)
     return (in_dim / 64) * n_tt * 4352 + (xh_has_min(fmt) ? (in_dim / 256) * n_tt * 2048 : 0);
 }
 unsigned xh_lds_bytes(int fmt) { return 2 * 17408 + 4 * 4096 + 4 * 3584 + (xh_has_min(fmt) ? 8192 : 0); }     // rein_xh_lds_bytes
-// Where it is taken, from a sweep of 11 model shapes (hidden 1024-18432 against 1024-18944) x 20 row counts 33-2048 through
-// rein_matmul_ws, every cell beside the launches of rein_mmq_xq8_ws (their time / this one's):
-//   Q6_K  0.99-2.1 in all 154 cells (17408 -> 5120, 45 rows 58.8 / 46.3 us, 512 rows 444 / 216; 5120 -> 17408 512 rows 307 / 208):
-//         everywhere from two token tiles; below 2.5e8 operations nothing was measured.
-//   Q4_K  contractions of 3584 and more, 33-64 rows 1.02-1.24 (17408 -> 5120, 45 rows 38.0 / 31.8 us), 80 rows 0.89-1.26 (three tiles
-//         of a group of four at the cost of a whole group's unpack against the int8 split tail's 32-token units), from
-//         100 rows 0.96-1.25, median 1.06; 2048 and less 0.59-1.16: a range of few superblocks does not pay back its start
-//         and the image.  The line is between them.
-//   Q5_K  the same contractions from 384 rows 0.97-1.46, median 1.11 (5120 -> 17408, 512 rows 190 / 167); below, groups of two
-//         and three tiles share the unpack of its fifth bits too little (33-320 rows 0.75-1.8, median 0.98).
+// Where it is taken, from sweeps through rein_matmul_ws, every cell beside the launches of rein_mmq_xq8_ws (their time / this one's),
+// the weights of two to four matrices in turn, 33-2048 rows:
+//   Q6_K  0.98-2.0 in all 104 cells of 13 shapes (17408 -> 5120, 45 rows 62.5 / 51.0 us, 512 rows 451 / 222; 5120 -> 17408 512 rows
+//         311 / 200): everywhere from two token tiles; below 2.5e8 operations nothing was measured.
+//   Q4_K  contractions of 3072 and more at 33-64 rows 0.97-1.20, median 1.1 (17408 -> 5120, 45 rows 40.5 / 34.9 us; 2304-2560
+//         0.97-1.14, median 1.0); 80 rows 0.89-1.26 (three tiles of a group of four at the cost of a whole group's unpack against the int8 split
+//         tail's 32-token units); from 96 rows contractions of 4096 and more, 0.91-1.78, median 1.06 (3072-3584: 0.75-1.17, in the
+//         mean 0.97: ranges of few superblocks do not pay back their starts and the image).
+//   Q5_K  from 384 rows, contractions of 4096 and more 0.90-1.53, median 1.13 (5120 -> 17408, 512 rows 194 / 172), of 3072-3584 against
+//         16384 rows and more (18944: 1.05-1.18 in 22 cells; 2560-12288 rows 0.78-1.35, in the mean 0.99); below 384 rows groups of two and
+//         three tiles share the unpack of its fifth bits too little (33-320 rows 0.75-1.8, median 0.98).
 // From two token tiles on a group has at least two (rein_xh_group), which is what the kernel is built for.
-bool xh_shape(int fmt, unsigned in_dim, unsigned p_rows)
+bool xh_shape(int fmt, unsigned in_dim, unsigned p_rows)          // for any number of weight rows
 {
     const unsigned mode = opt_u(O_MMQXH, 1);
     if (mode == 0 || !xh_format(fmt) || in_dim == 0 || in_dim % 256 != 0 || p_rows <= 32) return false;
     if (mode == 2 || fmt == REIN_TYPE_Q6_K) return true;
-    if (in_dim < 3072) return false;
-    return fmt == REIN_TYPE_Q4_K ? p_rows <= 64 || p_rows >= 96 : p_rows >= 384;
+    if (fmt == REIN_TYPE_Q4_K && p_rows > 64) return in_dim >= 4096 && p_rows >= 96;
+    return in_dim >= 3072 && (fmt == REIN_TYPE_Q4_K || p_rows >= 384);
 }
 bool xh_take(int fmt, unsigned in_dim, unsigned out_dim, unsigned p_rows)
 {
     if (!xh_shape(fmt, in_dim, p_rows)) return false;
-    return fmt != REIN_TYPE_Q6_K || opt_u(O_MMQXH, 1) == 2 || 2.0 * p_rows * (double)out_dim * in_dim >= 2.5e8;
+    if (opt_u(O_MMQXH, 1) == 2) return true;
+    if (fmt == REIN_TYPE_Q5_K) return in_dim >= 4096 || out_dim >= 16384;
+    return fmt != REIN_TYPE_Q6_K || 2.0 * p_rows * (double)out_dim * in_dim >= 2.5e8;
 }
 // Units of 128 rows x 64..128 tokens, 512 resident workgroups.  Whole rounds run unsplit; what is left over is cut into the
 // cheapest number of ranges, counted in superblocks of a workgroup that shares its CU: a range costs its superblocks and one
 // and a half for its start; a last round of at most one workgroup per CU takes 0.6 of one with two; a partial tile is
-// written and read once.  Q6_K, us at 1 / 2 / 3 / 4 / 6 ranges: 17408 -> 5120, 777 rows (280 units) 475 / 409 / 382 / 382 /
-// 382, 512 rows (160 units) 349 / 290 / 228 / 249 / 240; 5120 -> 17408, 512 rows (a round and 32) 274 / 228 / 214 / 208 / 208.
+// written and read once.  Q6_K, us at 1 / 2 / 3 / 4 / 6 ranges: 17408 -> 5120, 777 rows (280 units) 467 / 409 / 371 / 370 /
+// 369, 512 rows (160 units) 357 / 278 / 223 / 252 / 232; 5120 -> 17408, 512 rows (a round and 32) 272 / 224 / 211 / 201 / 200.
 unsigned xh_split(unsigned tail, unsigned chunks)
 {
     if (tail == 0) return 1;

@@ -128,3 +128,15 @@ def test_form_of_the_expert_ffn(tmp_path):
         kernels = [r[0] for r in d["launches"]]
         assert any(form in k for k in kernels), (shape, kernels)
         assert form == few or not any(few in k for k in kernels), (shape, kernels)
+
+
+def test_where_the_exact_dot_gemm_is_taken(tmp_path):
+    cases = [(rein.Q6_K, 256, 20000, 33, 1), (rein.Q6_K, 256, 4096, 33, 0), (rein.Q6_K, 1024, 4096, 64, 1), (rein.Q6_K, 5120, 17408, 32, 0),
+             (rein.Q4_K, 2816, 8192, 64, 0), (rein.Q4_K, 3072, 8192, 64, 1), (rein.Q4_K, 3584, 18944, 65, 0), (rein.Q4_K, 3584, 18944, 512, 0),
+             (rein.Q4_K, 4096, 4096, 95, 0), (rein.Q4_K, 4096, 4096, 96, 1), (rein.Q4_K, 3840, 4096, 2048, 0),
+             (rein.Q5_K, 4096, 4096, 383, 0), (rein.Q5_K, 4096, 4096, 384, 1), (rein.Q5_K, 3584, 3584, 512, 0), (rein.Q5_K, 3584, 18944, 512, 1),
+             (rein.Q5_K, 2816, 18944, 512, 0), (rein.Q8_0, 5120, 17408, 512, 0)]
+    sizes = record([("matmul_scratch_bytes", [f, k, rows]) for f, k, _, rows, _ in cases], tmp_path)
+    done = record([("matmul_ws", [f, P, P, P, k, n, rows, P, size["value"]]) for (f, k, n, rows, _), size in zip(cases, sizes)], tmp_path)
+    for case, d in zip(cases, done):
+        assert bool(xh(d)) == bool(case[-1]), case
