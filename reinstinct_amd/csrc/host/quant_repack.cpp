@@ -4,6 +4,7 @@
 // a plane per step.  Rows are split over threads.
 #include <algorithm>
 #include <cstring>
+#include <exception>
 #include <thread>
 #include <vector>
 
@@ -297,9 +298,15 @@ void rein::repack_parallel(int fmt, size_t in_dim, size_t out_dim, uint8_t* dst,
     n_threads = std::max<size_t>(1, std::min({n_threads, in_dim * out_dim >> 20, out_dim}));
     std::vector<std::thread> pool;
     const size_t step = (out_dim + n_threads - 1) / n_threads;
-    for (size_t a = step; a < out_dim; a += step)
-        pool.emplace_back(repack_range, fmt, std::cref(l), row_bytes, dst, source, ctx, staged, a, std::min(out_dim, a + step));
+    size_t next = step;
+    try {
+        pool.reserve(n_threads);
+        for (; next < out_dim; next += step)
+            pool.emplace_back(repack_range, fmt, std::cref(l), row_bytes, dst, source, ctx, staged, next, std::min(out_dim, next + step));
+    } catch (const std::exception&) {                // no more threads to be had: the calling one does the rows that are left
+    }
     repack_range(fmt, l, row_bytes, dst, source, ctx, staged, 0, std::min(out_dim, step));
+    if (next < out_dim) repack_range(fmt, l, row_bytes, dst, source, ctx, staged, next, out_dim);
     for (auto& th : pool) th.join();
 }
 

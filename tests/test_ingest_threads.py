@@ -1,6 +1,9 @@
 """Load-time repack with its rows split over threads (CPU): shapes on either side of the split, rows that do not divide over
 the threads, padded and unpadded contractions, into memory that holds other bytes before -- against the oracle."""
 import ctypes as C
+import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -10,6 +13,7 @@ from reinstinct_amd import quant
 from reinstinct_amd._lib import check, lib
 from oracle import orc
 
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 PTR = C.c_void_p
 SHAPES = [(1024, 1), (1024, 2049), (1280, 1639), (256, 8193)]          # one thread; two, padded; two, not padded; two, one superblock a row
 
@@ -44,3 +48,23 @@ def test_bf16_rows_with_half_steps_and_extremes(in_dim, out_dim):
     slab, _ = quant.ingest_for_matvec(quant.GGML_BF16, bf.view(np.uint8), in_dim, out_dim)
     want = orc.repack_for_matvec(rein.Q8_0, orc.q8_0_quantize_from_f32(orc.bf16_to_f32(bf)), in_dim, out_dim)
     assert np.array_equal(slab, want)
+
+
+def test_no_thread_to_be_had():
+    """a process at its limits gets the same bytes from the calling thread alone (a child whose address space has no room for a
+    thread's stack)"""
+    code = ("import resource, numpy as np\n"
+            "from reinstinct_amd import quant\n"
+            "from reinstinct_amd._lib import lib\n"
+            "raw = np.random.default_rng(1).integers(0, 256, 2048 * 2304 // 32 * 18, dtype=np.uint8)\n"
+            "got = np.full(quant.repacked_len(2, 2048, 2304), 0xA5, np.uint8)\n"
+            "args = (2, raw.ctypes.data, 2048, 2304, got.ctypes.data)\n"
+            "size = int(open('/proc/self/statm').read().split()[0]) * resource.getpagesize()\n"
+            "before = resource.getrlimit(resource.RLIMIT_AS)\n"
+            "resource.setrlimit(resource.RLIMIT_AS, (size + (1 << 20), before[1]))\n"
+            "rc = lib.rein_repack_for_matvec(*args)\n"
+            "resource.setrlimit(resource.RLIMIT_AS, before)\n"
+            "assert rc == 0 and np.array_equal(got, quant.repack_for_matvec(2, raw, 2048, 2304))\n"
+            "print('same')\n")
+    run = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120, cwd=ROOT)
+    assert run.stdout.strip() == "same", (run.returncode, run.stderr[-500:])
