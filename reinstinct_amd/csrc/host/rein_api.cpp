@@ -2379,7 +2379,7 @@ bool moe_few_fits(const rein_moe_shape& sh)
 // experts top-8: 141 us against 143, 32 tokens 160 against 145).
 bool moe_decode_range(const rein_moe_shape& sh) { return 5ull * sh.n_tok * sh.n_used <= 8ull * sh.n_expert; }
 // Where they pay.
-// Against the decode launches, which are two launches fewer, stream at a higher rate and read an expert again for every entry:
+// Against the decode launches, which are one or two launches fewer, stream at a higher rate and read an expert again for every entry:
 // once what is read again outweighs 30 MB and 0.3 of what both read (0.45 for Q8_0, whose decode launch runs at 5.6 TB/s); an
 // entry counts as 0.2 MB more, the workgroups it costs there.  From 319 cells -- nine expert shapes of 1 to 20 MB, 2-256 experts, top
 // 1-8, 1-48 tokens, the weights of several layers in turn -- of which 301 are within 3 % of the better side (us, decode / these:

@@ -236,7 +236,8 @@ template <> struct DiskPart<REIN_Q8_0> {        // two 34-byte blocks; rows are 
 // workgroups at once are 5-20 % slower.  us before -> now (TB/s of weights), three matrices in turn:
 //   2048 -> 151936   Q6_K 80.2 -> 45.5 (5.6)   Q4_K 48.0 -> 30.5 (5.7)   Q5_K 60.0 -> 37.3 (5.7)   Q8_0 81.7 -> 54.4 (6.1)
 //   5120 -> 151936   Q6_K 235 -> 107 (6.0)     Q4_K 124 -> 72.2 (6.1)    Q5_K 158 -> 89.7 (6.0)    Q8_0 202 -> 139 (5.9)
-// which is the rate at which this part reads: what bounds it now is HBM.
+// which is the rate at which this part reads: what bounds it now is HBM.  Up to 2048 rows, where the kernels of matvec_ondisk.hip have a
+// workgroup per CU, rein_matvec_ondisk_xq8 keeps those for Q8_0 and for most contractions of Q6_K.
 template <int FMT>
 __device__ __forceinline__ void rein_matvec_disk(const uint8_t* __restrict__ w, const BlockQ8* __restrict__ xq, float* __restrict__ y,
                                                  unsigned in_dim, unsigned out_dim)

@@ -19,10 +19,10 @@
 // four 128 rows x 32 NT tokens; two workgroups per CU.
 //
 // Bound: matrix unit (2 / 4 fp16 instructions of 32 cycles per tile and sub-block, Q4_K and Q5_K / Q6_K) plus the 16
-// multiply-adds and the share of the unpack, which issue between them.  Measured per tile and sub-block and SIMD at 2048 x 5120 x
-// 17408: 104 / 122 / 150 ns, the launches before it (fp6, int8, int8) 108 / 139 / 211.  Whole calls of rein_matmul_ws, us before
-// and now: Q6_K 777 x 17408 -> 5120 523 / 379, 512 x 5120 -> 17408 307 / 208; Q5_K the same 190 / 167; Q4_K 147 / 145, 512 x
-// 17408 -> 5120 166 / 152.
+// multiply-adds and the share of the unpack, which issue between them.  Whole calls of rein_matmul_ws against the launches of
+// rein_mmq_xq8_ws (fp6 for Q4_K, else int8), weights of several matrices in turn, us: 2048 x 5120 -> 17408 Q4_K / Q5_K / Q6_K 580 /
+// 723 / 1130 -> 555 / 652 / 753 (102 / 120 / 138 ns per tile and sub-block and SIMD); 512 x 5120 -> 17408 152 / 194 / 311 -> 142 /
+// 172 / 200; 512 x 17408 -> 5120 172 / 250 / 451 -> 160 / 193 / 222; Q6_K 777 x 17408 -> 5120 526 -> 369.
 //
 // Replaces, from 33 rows, kernels/mmq_gemm_{q4k,q5k,q6k}_repacked.cpp of the reference behind rein_matmul_ws.
 #pragma once
