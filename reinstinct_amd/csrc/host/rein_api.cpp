@@ -192,8 +192,8 @@ int check_ptr(const char* who, const void* p, size_t align, const char* what)
 // rein_set_option changes an entry, so the launch an entry point chooses depends on its arguments
 // and on this table alone.  Entries are single atomic words: setting one while another thread
 // launches is safe, the launch sees the old or the new value.
-enum Opt : int { O_MV_ROWS, O_MV_WPB, O_MV_LOADS, O_MV_LDS, O_QUAD_LDS, O_QUAD_SLICES, O_QUAD_DEPTH, O_QUAD_WIDE32, O_SKINNY_KS, O_SKINNY_FROM, O_QUAD_FROM, O_GROUPED_STRIDED, O_MMQ_TM, O_MMQ_N64, O_MMQ6, O_MMQ6_N4, O_MMQ6_N2, O_MMQ6_SK_GRID, O_MMQ6_SK_SPLIT, O_MMQ6_SK, O_MMQ6_FROM, O_MMQ_SK, O_MMQ_SK_GRID, O_MMQ_SK_SPLIT, O_MMQ_SK_TM, O_MMQ16, O_MMQXH, O_MMQXH_SPLIT, O_TOPK_WAVE, O_MOE_SORT_SPLIT, O_MOE_GU_ROWS, O_MOE_DC_ROWS, O_MOE_CHAIN, O_MOE_FUSED, O_MOE_FEW, O_COUNT };
-const char* const kOptNames[O_COUNT] = {"REIN_MV_ROWS", "REIN_MV_WPB", "REIN_MV_LOADS", "REIN_MV_LDS", "REIN_QUAD_LDS", "REIN_QUAD_SLICES", "REIN_QUAD_DEPTH", "REIN_QUAD_WIDE32", "REIN_SKINNY_KS", "REIN_SKINNY_FROM", "REIN_QUAD_FROM", "REIN_GROUPED_STRIDED", "REIN_MMQ_TM", "REIN_MMQ_N64", "REIN_MMQ6", "REIN_MMQ6_N4", "REIN_MMQ6_N2", "REIN_MMQ6_SK_GRID", "REIN_MMQ6_SK_SPLIT", "REIN_MMQ6_SK", "REIN_MMQ6_FROM", "REIN_MMQ_SK", "REIN_MMQ_SK_GRID", "REIN_MMQ_SK_SPLIT", "REIN_MMQ_SK_TM", "REIN_MMQ16", "REIN_MMQXH", "REIN_MMQXH_SPLIT", "REIN_TOPK_WAVE", "REIN_MOE_SORT_SPLIT", "REIN_MOE_GU_ROWS", "REIN_MOE_DC_ROWS", "REIN_MOE_CHAIN", "REIN_MOE_FUSED", "REIN_MOE_FEW"};
+enum Opt : int { O_MV_ROWS, O_MV_WPB, O_MV_LOADS, O_MV_LDS, O_QUAD_LDS, O_QUAD_SLICES, O_QUAD_DEPTH, O_QUAD_WIDE32, O_SKINNY_KS, O_SKINNY_FROM, O_QUAD_FROM, O_GROUPED_STRIDED, O_MMQ_TM, O_MMQ_N64, O_MMQ6, O_MMQ6_N4, O_MMQ6_N2, O_MMQ6_SK_GRID, O_MMQ6_SK_SPLIT, O_MMQ6_SK, O_MMQ6_FROM, O_MMQ_SK, O_MMQ_SK_GRID, O_MMQ_SK_SPLIT, O_MMQ_SK_TM, O_MMQ16, O_MMQXH, O_MMQXH_SPLIT, O_MMQXH_GROUPS, O_TOPK_WAVE, O_MOE_SORT_SPLIT, O_MOE_GU_ROWS, O_MOE_DC_ROWS, O_MOE_CHAIN, O_MOE_FUSED, O_MOE_FEW, O_COUNT };
+const char* const kOptNames[O_COUNT] = {"REIN_MV_ROWS", "REIN_MV_WPB", "REIN_MV_LOADS", "REIN_MV_LDS", "REIN_QUAD_LDS", "REIN_QUAD_SLICES", "REIN_QUAD_DEPTH", "REIN_QUAD_WIDE32", "REIN_SKINNY_KS", "REIN_SKINNY_FROM", "REIN_QUAD_FROM", "REIN_GROUPED_STRIDED", "REIN_MMQ_TM", "REIN_MMQ_N64", "REIN_MMQ6", "REIN_MMQ6_N4", "REIN_MMQ6_N2", "REIN_MMQ6_SK_GRID", "REIN_MMQ6_SK_SPLIT", "REIN_MMQ6_SK", "REIN_MMQ6_FROM", "REIN_MMQ_SK", "REIN_MMQ_SK_GRID", "REIN_MMQ_SK_SPLIT", "REIN_MMQ_SK_TM", "REIN_MMQ16", "REIN_MMQXH", "REIN_MMQXH_SPLIT", "REIN_MMQXH_GROUPS", "REIN_TOPK_WAVE", "REIN_MOE_SORT_SPLIT", "REIN_MOE_GU_ROWS", "REIN_MOE_DC_ROWS", "REIN_MOE_CHAIN", "REIN_MOE_FUSED", "REIN_MOE_FEW"};
 constexpr uint64_t kOptSet = 1ull << 63;
 std::atomic<uint64_t> g_opts[O_COUNT];          // zero = unset
 std::once_flag g_opts_env_once;
@@ -1846,23 +1846,36 @@ int rein_matmul(int fmt, const void* w, const float* x, float* y, unsigned in_di
 }
 
 namespace {
-// ---- Q4_K / Q5_K / Q6_K prefill with exact block dots on the fp16 instruction (kernels/mmq_exact16.h), out of rein_matmul_ws
+// ---- prefill out of rein_matmul_ws: 32 rows x up to 128 tokens per wavefront, activations as an image in operand order.  Q4_K / Q5_K /
+// Q6_K with exact block dots on the fp16 instruction (kernels/mmq_exact16.h), Q8_0 / Q4_0 / IQ4_XS / IQ3_S on the int8 one (mmq_x8.h)
 struct XhPlan {
     unsigned n_grp, n_unit, n_whole, split;
     size_t image, parts;                             // bytes of the activation image and of the partial tiles behind it
 };
-constexpr size_t kXhPart = (size_t)4 * 16 * 256 * 4;
-constexpr unsigned kXhMostParts = 1024;              // partial tiles of one launch: 64 MiB
+constexpr size_t kXhPart = (size_t)16 * 256 * 4;     // 128 rows x a token tile, fp32
+constexpr unsigned kXhMostParts = 1024;              // ranges of one launch: at most 64 MiB of partial tiles
 bool xh_format(int fmt) { return fmt == REIN_TYPE_Q4_K || fmt == REIN_TYPE_Q5_K || fmt == REIN_TYPE_Q6_K; }
-bool xh_has_min(int fmt) { return fmt != REIN_TYPE_Q6_K; }
+bool xh_has_min(int fmt) { return fmt == REIN_TYPE_Q4_K || fmt == REIN_TYPE_Q5_K; }
 size_t xh_image_bytes(int fmt, unsigned in_dim, unsigned p_rows)
 {
     const size_t n_tt = ((size_t)p_rows + 31) / 32;
+    if (!xh_format(fmt)) return (in_dim / 64) * n_tt * 2304;                                                 // REIN_X8_REC
     return (in_dim / 64) * n_tt * 4352 + (xh_has_min(fmt) ? (in_dim / 256) * n_tt * 2048 : 0);
 }
-unsigned xh_lds_bytes(int fmt) { return 2 * 17408 + 4 * 4096 + 4 * 3584 + (xh_has_min(fmt) ? 8192 : 0); }     // rein_xh_lds_bytes
+unsigned xh_lds_bytes(int fmt)
+{
+    if (!xh_format(fmt)) return 2 * 18432 + 4 * (fmt == REIN_TYPE_Q8_0 ? 8192 : 4096) + 4 * 2048;            // X8Lds
+    return 2 * 17408 + 4 * 4096 + 4 * 3584 + (xh_has_min(fmt) ? 8192 : 0);                                   // rein_xh_lds_bytes
+}
 // Where it is taken, from sweeps through rein_matmul_ws, every cell beside the launches of rein_mmq_xq8_ws (their time / this one's),
-// the weights of two to four matrices in turn, 33-2048 rows:
+// the weights of two to six matrices in turn, 9-2048 rows:
+//   Q8_0, Q4_0, IQ4_XS  12 shapes (1024 -> 4096 ... 17408 -> 5120, 1536 -> 32000) x 17 row counts: from 24 rows 0.95-2.0 in 612 cells, 7 of
+//         them below 0.98, 1.14-1.27 in the geometric mean of every row count (Q8_0 5120 -> 17408, 2048 rows 648 / 507 us; 17408 ->
+//         5120, 200 rows 135 / 77, 45 rows 44 / 35; 5632 -> 2048, 32 rows 16.7 / 13.0).  All four from 17 rows on 13 shapes 1.03-1.44
+//         at 17-28 rows.  Not contractions below 2048 against 4096 rows and more at 65-400 rows (1024 -> 4096 and 1536 -> 32000
+//         0.96-1.03: three launches for little work).  9-16 rows: contractions of three times the rows of weights (1.04-1.33 in 60
+//         cells; 5632 -> 2048 0.92-0.96, 5120 -> 5120 0.86-1.0), and the 4-bit formats from 48M weights (5120 -> 17408, 4096 ->
+//         14336, 8192 -> 8192 1.01-1.15; Q8_0 there 0.82-1.01).
 //   Q6_K  0.98-2.0 in all 104 cells of 13 shapes (17408 -> 5120, 45 rows 62.5 / 51.0 us, 512 rows 451 / 222; 5120 -> 17408 512 rows
 //         311 / 200): everywhere from two token tiles; below 2.5e8 operations nothing was measured.
 //   Q4_K  contractions of 3072 and more at 33-64 rows 0.97-1.20, median 1.1 (17408 -> 5120, 45 rows 40.5 / 34.9 us; 2304-2560
@@ -1872,12 +1885,13 @@ unsigned xh_lds_bytes(int fmt) { return 2 * 17408 + 4 * 4096 + 4 * 3584 + (xh_ha
 //   Q5_K  from 384 rows, contractions of 4096 and more 0.90-1.53, median 1.13 (5120 -> 17408, 512 rows 194 / 172), of 3072-3584 against
 //         16384 rows and more (18944: 1.05-1.18 in 22 cells; 2560-12288 rows 0.78-1.35, in the mean 0.99); below 384 rows groups of two and
 //         three tiles share the unpack of its fifth bits too little (33-320 rows 0.75-1.8, median 0.98).
-// From two token tiles on a group has at least two (rein_xh_group), which is what the kernel is built for.
+// The K-quants' kernel is built for groups of at least two tiles.
 bool xh_shape(int fmt, unsigned in_dim, unsigned p_rows)          // for any number of weight rows
 {
     const unsigned mode = opt_u(O_MMQXH, 1);
-    if (mode == 0 || !xh_format(fmt) || in_dim == 0 || in_dim % 256 != 0 || p_rows <= 32) return false;
-    if (mode == 2 || fmt == REIN_TYPE_Q6_K) return true;
+    const bool k_quant = xh_format(fmt);
+    if (mode == 0 || in_dim == 0 || in_dim % 256 != 0 || p_rows <= (k_quant ? 32u : 8u)) return false;
+    if (mode == 2 || fmt == REIN_TYPE_Q6_K || !k_quant) return true;
     if (fmt == REIN_TYPE_Q4_K && p_rows > 64) return in_dim >= 4096 && p_rows >= 96;
     return in_dim >= 3072 && (fmt == REIN_TYPE_Q4_K || p_rows >= 384);
 }
@@ -1885,14 +1899,62 @@ bool xh_take(int fmt, unsigned in_dim, unsigned out_dim, unsigned p_rows)
 {
     if (!xh_shape(fmt, in_dim, p_rows)) return false;
     if (opt_u(O_MMQXH, 1) == 2) return true;
+    if (!xh_format(fmt)) {
+        if (p_rows <= 16) return in_dim >= 3ull * out_dim || (fmt != REIN_TYPE_Q8_0 && (unsigned long long)in_dim * out_dim >= 48ull << 20);
+        return in_dim >= 2048 || p_rows <= 64 || p_rows > 400 || out_dim < 4096;
+    }
     if (fmt == REIN_TYPE_Q5_K) return in_dim >= 4096 || out_dim >= 16384;
     return fmt != REIN_TYPE_Q6_K || 2.0 * p_rows * (double)out_dim * in_dim >= 2.5e8;
 }
-// Units of 128 rows x 64..128 tokens, 512 resident workgroups.  Whole rounds run unsplit; what is left over is cut into the
-// cheapest number of ranges, counted in superblocks of a workgroup that shares its CU: a range costs its superblocks and one
-// and a half for its start; a last round of at most one workgroup per CU takes 0.6 of one with two; a partial tile is
-// written and read once.  Q6_K, us at 1 / 2 / 3 / 4 / 6 ranges: 17408 -> 5120, 777 rows (280 units) 467 / 409 / 371 / 370 /
-// 369, 512 rows (160 units) 357 / 278 / 223 / 252 / 232; 5120 -> 17408, 512 rows (a round and 32) 272 / 224 / 211 / 201 / 200.
+// Units of 128 rows x a group of token tiles, 512 resident workgroups.  Whole rounds run unsplit; what is left over is cut into
+// ranges of superblocks.  How many tiles a group has and how many ranges there are is the cheapest by this price, in microseconds:
+// a superblock of a workgroup with t tiles a2 + b2 t beside another workgroup on its CU, a1 + b1 t alone (a last round of at most
+// one workgroup per CU), 2.4 for the launch that adds partial tiles, 6.1 ns for each tile of 16 KB that is written and read again.
+// Fitted to 600 cells (Q8_0, Q4_0, IQ4_XS; groups of 1-4 tiles x 1-16 ranges each): the pick is within 1 % of the best of its cell
+// in the mean, 16 % at most.  (Q8_0 5120 -> 1024, 160 rows, groups x ranges: 5 x 5 15.5 us, 2 x 12 20.3; 17408 -> 5120, 45 rows 1 x 12
+// 35.0, 2 x 6 36.5, 1 x 4 44; 2048 -> 5632, 300 rows 10 x 1 24.7, 5 x 1 26.2, 3 x 6 32.7.)
+struct XhGroups { unsigned n_grp, split; };
+constexpr double kX8Pair = 1.0, kX8PairTile = 1.68, kX8Alone = 0.47, kX8AloneTile = 1.2, kXhSum = 2.4, kXhTilePart = 0.0061;
+double x8_price(unsigned units, unsigned n_tt, unsigned n_grp, unsigned chunks, unsigned split)
+{
+    const double tiles = n_tt / (double)n_grp, most_tiles = (n_tt + n_grp - 1) / n_grp, pair = kX8Pair + kX8PairTile * tiles;
+    const unsigned wg = units % 512 * split, rem = wg % 512;
+    const double range = 0.5 * (chunks / (double)split + (chunks + split - 1) / split);
+    double t = (units / 512) * (chunks * pair) + (wg / 512) * (range * pair);
+    if (rem) t += range * (rem <= kCUs ? kX8Alone + kX8AloneTile * most_tiles : kX8Pair + kX8PairTile * most_tiles);
+    return split > 1 ? t + kXhSum + wg * tiles * kXhTilePart : t;
+}
+// the cheapest number of ranges for `units` units of n_grp groups, and its price
+unsigned x8_split(unsigned units, unsigned n_tt, unsigned n_grp, unsigned chunks, double* price)
+{
+    const unsigned tail = units % 512, most = tail == 0 ? 1 : std::max(1u, std::min(std::min(16u, chunks), kXhMostParts / tail));
+    const unsigned forced = opt_u(O_MMQXH_SPLIT, 0);
+    unsigned split = std::min(std::max(1u, forced), most);
+    *price = x8_price(units, n_tt, n_grp, chunks, split);
+    for (unsigned k = 2; k <= most && !forced; k++) {
+        const double t = x8_price(units, n_tt, n_grp, chunks, k);
+        if (t < *price) { *price = t; split = k; }
+    }
+    return split;
+}
+XhGroups x8_groups(unsigned in_dim, unsigned out_dim, unsigned p_rows)
+{
+    const unsigned n_tt = (p_rows + 31) / 32, n_rb = (out_dim + 127) / 128, least = (n_tt + 3) / 4, forced = opt_u(O_MMQXH_GROUPS, 0);
+    XhGroups best{0, 1};
+    double best_price = 0.0;
+    for (unsigned size = 4; size >= 1; size--) {
+        const unsigned n_grp = forced ? std::min(n_tt, std::max(forced, least)) : (n_tt + size - 1) / size;
+        double price;
+        const unsigned split = x8_split(n_rb * n_grp, n_tt, n_grp, in_dim / 256, &price);
+        if (best.n_grp == 0 || price < best_price) { best = XhGroups{n_grp, split}; best_price = price; }
+    }
+    return best;
+}
+// The K-quants: groups of up to four tiles; the cheapest number of ranges, counted in superblocks of a workgroup that shares its
+// CU: a range costs its superblocks and one and a half for its start; a last round of at most one workgroup per CU takes 0.6 of
+// one with two; a partial tile is written and read once.  Q6_K, us at 1 / 2 / 3 / 4 / 6 ranges: 17408 -> 5120, 777 rows (280 units)
+// 467 / 409 / 371 / 370 / 369, 512 rows (160 units) 357 / 278 / 223 / 252 / 232; 5120 -> 17408, 512 rows (a round and 32) 272 / 224 /
+// 211 / 201 / 200.
 unsigned xh_split(unsigned tail, unsigned chunks)
 {
     if (tail == 0) return 1;
@@ -1909,26 +1971,43 @@ unsigned xh_split(unsigned tail, unsigned chunks)
     }
     return split;
 }
-size_t xh_parts_bytes(unsigned tail, unsigned split) { return split > 1 ? (size_t)tail * split * kXhPart : 0; }
+size_t xh_parts_bytes(unsigned tail, unsigned split, unsigned n_tt, unsigned n_grp)
+{
+    return split > 1 ? (size_t)tail * split * ((n_tt + n_grp - 1) / n_grp) * kXhPart : 0;
+}
 XhPlan xh_plan(int fmt, unsigned in_dim, unsigned out_dim, unsigned p_rows)
 {
     XhPlan p{};
-    p.n_grp = (p_rows + 127) / 128;
-    p.n_unit = (out_dim + 127) / 128 * p.n_grp;
+    const unsigned n_tt = (p_rows + 31) / 32, n_rb = (out_dim + 127) / 128;
+    if (xh_format(fmt)) {
+        p.n_grp = std::min(std::max(1u, n_tt / 2), std::max((n_tt + 3) / 4, opt_u(O_MMQXH_GROUPS, 0)));
+        p.split = xh_split(n_rb * p.n_grp % 512, in_dim / 256);
+    } else {
+        const XhGroups g = x8_groups(in_dim, out_dim, p_rows);
+        p.n_grp = g.n_grp;
+        p.split = g.split;
+    }
+    p.n_unit = n_rb * p.n_grp;
     p.n_whole = p.n_unit / 512 * 512;
-    p.split = xh_split(p.n_unit - p.n_whole, in_dim / 256);
     p.image = (xh_image_bytes(fmt, in_dim, p_rows) + 255) & ~(size_t)255;
-    p.parts = xh_parts_bytes(p.n_unit - p.n_whole, p.split);
+    p.parts = xh_parts_bytes(p.n_unit - p.n_whole, p.split, n_tt, p.n_grp);
     return p;
 }
-// The most bytes of partial tiles that any number of weight rows leaves behind whole rounds of `n_grp` token groups (the size query
-// does not know the matrix): none for contractions of one or two superblocks, which are never split, 16 MiB up to five, 64 from ten.
-size_t xh_most_parts_bytes(unsigned in_dim, unsigned p_rows)
+// The most bytes of partial tiles that any number of weight rows leaves behind whole rounds of n_grp token groups (the size query does
+// not know the matrix): the remainders of the units by 512 are the multiples of the power of two in n_grp.  At most 64 MiB.
+size_t xh_most_parts_bytes(int fmt, unsigned in_dim, unsigned p_rows)
 {
-    unsigned step = (p_rows + 127) / 128 % 512;
-    step = step == 0 ? 512 : step & (0u - step);     // the remainders of its multiples by 512 are those of this power of two
+    const unsigned n_tt = (p_rows + 31) / 32, least = (n_tt + 3) / 4, most_grp = xh_format(fmt) ? std::max(1u, n_tt / 2) : n_tt;
+    const unsigned forced = opt_u(O_MMQXH_GROUPS, 0);
     size_t most = 0;
-    for (unsigned tail = step; tail < 512; tail += step) most = std::max(most, xh_parts_bytes(tail, xh_split(tail, in_dim / 256)));
+    for (unsigned size = 4; size >= 1; size--) {
+        const unsigned n_grp = forced ? std::min(most_grp, std::max(forced, least)) : (n_tt + size - 1) / size;
+        const unsigned step = std::min(512u, n_grp & (0u - n_grp));
+        double price;
+        for (unsigned tail = step; tail < 512; tail += step)
+            most = std::max(most, xh_parts_bytes(tail, xh_format(fmt) ? xh_split(tail, in_dim / 256) : x8_split(tail, n_tt, n_grp, in_dim / 256, &price), n_tt, n_grp));
+        if (xh_format(fmt)) break;
+    }
     return most;
 }
 }  // namespace
@@ -1939,7 +2018,7 @@ size_t rein_matmul_scratch_bytes(int fmt, unsigned in_dim, unsigned n_rows)
     const size_t xq = ((size_t)n_rows * (in_dim / 32) * 40 + 255) & ~(size_t)255;
     size_t behind = rein_matmul_path(fmt, n_rows) == 2 ? rein_mmq_workspace_bytes(fmt, in_dim, n_rows) : 0;
     if (rein_matmul_path(fmt, n_rows) == 2 && xh_shape(fmt, in_dim, n_rows))
-        behind = std::max(behind, ((xh_image_bytes(fmt, in_dim, n_rows) + 255) & ~(size_t)255) + xh_most_parts_bytes(in_dim, n_rows));
+        behind = std::max(behind, ((xh_image_bytes(fmt, in_dim, n_rows) + 255) & ~(size_t)255) + xh_most_parts_bytes(fmt, in_dim, n_rows));
     return xq + behind;
 }
 
@@ -1962,13 +2041,14 @@ int rein_matmul_ws(int fmt, const void* w, const float* x, float* y, unsigned in
             if (int rc = check_ptr("rein_matmul_ws", x, 4, "x")) return rc;
             if (int rc = check_ptr("rein_matmul_ws", w, 16, "w")) return rc;
             if (int rc = check_ptr("rein_matmul_ws", y, 4, "y")) return rc;
-            void* pa[] = {(void*)&x, (void*)&img, (void*)&scratch, (void*)&in_dim, (void*)&n_rows, (void*)&with_xsum};
-            if (int rc = launch("rein_xh_quantize", (n_rows + 31) / 32, in_dim / 256, 1, 256, 0, s, pa)) return rc;
-            void* a[] = {(void*)&w, (void*)&img, (void*)&y, (void*)&parts, (void*)&in_dim, (void*)&out_dim, (void*)&n_rows, (void*)&p.n_whole, (void*)&p.split};
-            if (int rc = launch(KName("rein_xh_", fmt_tag(fmt), ""), (unsigned)grid, 1, 1, 256, xh_lds_bytes(fmt), s, a)) return rc;
+            const bool k_quant = xh_format(fmt);
+            void* pa[] = {(void*)&x, (void*)&img, (void*)&scratch, (void*)&in_dim, (void*)&n_rows, (void*)&with_xsum};          // rein_x8_quantize: the first five
+            if (int rc = launch(k_quant ? "rein_xh_quantize" : "rein_x8_quantize", (n_rows + 31) / 32, in_dim / 256, 1, 256, 0, s, pa)) return rc;
+            void* a[] = {(void*)&w, (void*)&img, (void*)&y, (void*)&parts, (void*)&in_dim, (void*)&out_dim, (void*)&n_rows, (void*)&p.n_grp, (void*)&p.n_whole, (void*)&p.split};
+            if (int rc = launch(KName(k_quant ? "rein_xh_" : "rein_x8_", fmt_tag(fmt), ""), (unsigned)grid, 1, 1, 256, xh_lds_bytes(fmt), s, a)) return rc;
             if (p.split == 1) return 0;
-            void* b[] = {(void*)&parts, (void*)&y, (void*)&out_dim, (void*)&n_rows, (void*)&p.n_whole, (void*)&p.split};
-            return launch("rein_xh_sum", tail, 16, 1, 256, 0, s, b);
+            void* b[] = {(void*)&parts, (void*)&y, (void*)&out_dim, (void*)&n_rows, (void*)&p.n_grp, (void*)&p.n_whole, (void*)&p.split};
+            return launch(k_quant ? "rein_xh_sum" : "rein_x8_sum", tail, 16, 1, 256, 0, s, b);
         }
     }
     // nothing behind the activations that a workspace launch could use: the plain dispatch

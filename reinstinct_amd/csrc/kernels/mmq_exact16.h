@@ -61,21 +61,16 @@ __host__ __device__ constexpr int rein_xh_slot_weight(int kh, int h, int e)
 #define REIN_XH_REC 4352u
 #define REIN_XH_XS  2048u
 
-// x [p_rows][in_dim] fp32 -> image, and the blocks themselves to xq [p_rows][in_dim / 32] (the caller of rein_matmul_ws may read
-// them there), with the numbers that quantize_q8_f32 gives: the same sum tree (halves of 16, 8, 4, 2, 1), divisions and rounding,
-// by one thread for a block of 32.  blockIdx.x = token tile, blockIdx.y = superblock, 256 threads: thread 8 j + s handles token j,
-// sub-block s: eight threads read a kilobyte of a row and write runs of 128 bytes to the image and 320 to xq.
-// Bound by memory: 4 bytes in, 3.4 out per value (777 x 17408: 54 + 46 MB).
-__device__ __forceinline__ void rein_xh_quantize_body(const float* __restrict__ x, uint8_t* __restrict__ img, BlockQ8* __restrict__ xq, unsigned in_dim,
-                                                      unsigned p_rows, unsigned with_xsum)
+// One block of 32 values of row `tok` (zeros past p_rows, with d = 0) with the numbers that quantize_q8_f32 gives: the same sum tree
+// (halves of 16, 8, 4, 2, 1), divisions and rounding, by one thread.  The block itself goes to xq.
+struct XhBlock { float d, sum; int q[32]; };
+__device__ __forceinline__ void rein_xh_quantize_block(XhBlock& b, const float* __restrict__ x, BlockQ8* __restrict__ xq, unsigned in_dim, unsigned p_rows,
+                                                       unsigned tok, unsigned sb)
 {
 #pragma clang fp contract(off)
-    __shared__ float xsum[8][33];
-    const unsigned n_tt = (p_rows + 31u) / 32u, n_sub = in_dim >> 5, tt = blockIdx.x, c = blockIdx.y;
-    const unsigned j = threadIdx.x >> 3, s = threadIdx.x & 7u, tok = tt * 32u + j, sb = c * 8u + s;
-
     float v[32];
-    float d = 0.0f, inv = 0.0f, sum = 0.0f;
+    float inv = 0.0f;
+    b.d = b.sum = 0.0f;
     if (tok < p_rows) {
         const float* p = x + (size_t)tok * in_dim + sb * 32u;
         if (((size_t)x & 15u) == 0u) {
@@ -97,37 +92,50 @@ __device__ __forceinline__ void rein_xh_quantize_body(const float* __restrict__ 
         for (int m = 8; m >= 1; m >>= 1)
 #pragma unroll
             for (int i = 0; i < m; i++) t[i] = t[i] + t[i + m];
-        sum = t[0];
-        d   = amax > 0.0f ? amax / 127.0f : 1.0f;
-        inv = amax > 0.0f ? 127.0f / amax : 0.0f;
+        b.sum = t[0];
+        b.d   = amax > 0.0f ? amax / 127.0f : 1.0f;
+        inv   = amax > 0.0f ? 127.0f / amax : 0.0f;
     } else {
 #pragma unroll
         for (int i = 0; i < 32; i++) v[i] = 0.0f;
     }
-    int q[32];
 #pragma unroll
-    for (int i = 0; i < 32; i++) q[i] = max(-127, min(127, (int)rintf(v[i] * inv)));
+    for (int i = 0; i < 32; i++) b.q[i] = max(-127, min(127, (int)rintf(v[i] * inv)));
     if (tok < p_rows) {
-        BlockQ8 b;
-        b.d = d;
-        b.xsum = sum;
+        BlockQ8 o;
+        o.d = b.d;
+        o.xsum = b.sum;
 #pragma unroll
-        for (int i = 0; i < 8; i++) b.qs[i] = (q[4 * i] & 0xFF) | (q[4 * i + 1] & 0xFF) << 8 | (q[4 * i + 2] & 0xFF) << 16 | q[4 * i + 3] << 24;
-        xq[(size_t)tok * n_sub + sb] = b;
+        for (int i = 0; i < 8; i++) o.qs[i] = (b.q[4 * i] & 0xFF) | (b.q[4 * i + 1] & 0xFF) << 8 | (b.q[4 * i + 2] & 0xFF) << 16 | b.q[4 * i + 3] << 24;
+        xq[(size_t)tok * (in_dim >> 5) + sb] = o;
     }
+}
+
+// x [p_rows][in_dim] fp32 -> image, and the blocks themselves to xq [p_rows][in_dim / 32] (the caller of rein_matmul_ws may read
+// them there).  blockIdx.x = token tile, blockIdx.y = superblock, 256 threads: thread 8 j + s handles token j,
+// sub-block s: eight threads read a kilobyte of a row and write runs of 128 bytes to the image and 320 to xq.
+// Bound by memory: 4 bytes in, 3.4 out per value (777 x 17408: 54 + 46 MB).
+__device__ __forceinline__ void rein_xh_quantize_body(const float* __restrict__ x, uint8_t* __restrict__ img, BlockQ8* __restrict__ xq, unsigned in_dim,
+                                                      unsigned p_rows, unsigned with_xsum)
+{
+    __shared__ float xsum[8][33];
+    const unsigned n_tt = (p_rows + 31u) / 32u, n_sub = in_dim >> 5, tt = blockIdx.x, c = blockIdx.y;
+    const unsigned j = threadIdx.x >> 3, s = threadIdx.x & 7u, sb = c * 8u + s;
+    XhBlock b;
+    rein_xh_quantize_block(b, x, xq, in_dim, p_rows, tt * 32u + j, sb);
     uint8_t* rec = img + ((size_t)(sb >> 1) * n_tt + tt) * REIN_XH_REC;
-    reinterpret_cast<float*>(rec + REIN_XH_X)[(sb & 1u) * 32u + j] = d;
+    reinterpret_cast<float*>(rec + REIN_XH_X)[(sb & 1u) * 32u + j] = b.d;
 #pragma unroll
     for (int kh = 0; kh < 2; kh++)
 #pragma unroll
         for (int h = 0; h < 2; h++) {
             rein_v8h o;
 #pragma unroll
-            for (int e = 0; e < 8; e++) o[e] = (_Float16)q[rein_xh_slot_weight(kh, h, e)];
+            for (int e = 0; e < 8; e++) o[e] = (_Float16)b.q[rein_xh_slot_weight(kh, h, e)];
             *reinterpret_cast<rein_v8h*>(rec + (sb & 1u) * 2048u + kh * 1024u + (32u * h + j) * 16u) = o;
         }
     if (!with_xsum) return;                          // the image of a format without minimums has no xsum part
-    xsum[s][j] = sum;
+    xsum[s][j] = b.sum;
     __syncthreads();
     if (threadIdx.x < 128u) {                        // op = threadIdx.x / 64, lane = threadIdx.x % 64
         const unsigned op = threadIdx.x >> 6, h = (threadIdx.x >> 5) & 1u;
@@ -137,8 +145,8 @@ __device__ __forceinline__ void rein_xh_quantize_body(const float* __restrict__ 
             for (int k = 0; k < 8; k++) {
                 uint16_t p3[3];
                 rein_mmq_split_xsum(xsum[k][threadIdx.x & 31u], p3);
-                const uint32_t b = op ? p3[2] : (h ? p3[1] : p3[0]);
-                o[k >> 1] |= b << (16 * (k & 1));
+                const uint32_t x3 = op ? p3[2] : (h ? p3[1] : p3[0]);
+                o[k >> 1] |= x3 << (16 * (k & 1));
             }
         }
         uint8_t* dst = img + (size_t)(n_sub >> 1) * n_tt * REIN_XH_REC + ((size_t)c * n_tt + tt) * REIN_XH_XS;
@@ -146,14 +154,17 @@ __device__ __forceinline__ void rein_xh_quantize_body(const float* __restrict__ 
     }
 }
 
-// Token tiles are dealt evenly over ceil(tiles / 4) groups: 25 tiles are four groups of 4 and three of 3, not six of 4 and
-// one of 1.  From two tiles on every group has at least two.
+// Token tiles are dealt evenly over the n_grp groups of the launch (at least ceil(tiles / 4), at most one per tile): 25 tiles in
+// seven groups are four of 4 and three of 3, not six of 4 and one of 1.
 struct XhGroup { unsigned tile, n; };
-__device__ __forceinline__ XhGroup rein_xh_group(unsigned p_rows, unsigned g)
+__device__ __forceinline__ XhGroup rein_xh_group(unsigned p_rows, unsigned n_grp, unsigned g)
 {
-    const unsigned n_tt = (p_rows + 31u) >> 5, n_grp = (n_tt + 3u) >> 2, base = n_tt / n_grp, more = n_tt - base * n_grp;
+    const unsigned n_tt = (p_rows + 31u) >> 5, base = n_tt / n_grp, more = n_tt - base * n_grp;
     return XhGroup{g * base + min(g, more), base + (g < more ? 1u : 0u)};
 }
+
+// floats of the partial tiles of one range: of the largest group of the launch
+__device__ __forceinline__ unsigned rein_xh_part(unsigned p_rows, unsigned n_grp) { return (((p_rows + 31u) >> 5) + n_grp - 1u) / n_grp * 4096u; }
 
 // ---- weight operands ------------------------------------------------------------------
 // A nibble or-ed into the mantissa of 1024 (low nibble) or 64 (high nibble, which sits four bits up) is 1024 + n or 64 + n;
@@ -460,15 +471,25 @@ __device__ __forceinline__ void rein_xh_acc(const uint8_t* __restrict__ w, const
     REIN_WAIT_VMCNT(0);
 }
 
+template <int FMT> struct XhTile {
+    static constexpr bool kOne = false;              // groups of one tile: the stages of a tile on its own are not built
+    template <int NT>
+    static __device__ __forceinline__ void run(const uint8_t* __restrict__ w, const uint8_t* __restrict__ img, unsigned in_dim, unsigned out_dim, unsigned n_tt,
+                                               unsigned rb, unsigned tile, unsigned c0, unsigned c1, unsigned char* const raw, float (&acc)[NT][16])
+    {
+        rein_xh_acc<FMT, NT>(w, img, in_dim, out_dim, n_tt, rb, tile, c0, c1, raw, acc);
+    }
+};
+
 // One piece of the launch: superblocks [c0, c1) of unit (rb, grp), to y or (part not null) to a partial tile
 // [t][v / 4][thread] of float4.
-template <int FMT, int NT>
+template <class Tile, int NT>
 __device__ __forceinline__ void rein_xh_piece(const uint8_t* __restrict__ w, const uint8_t* __restrict__ img, float* __restrict__ y, float* __restrict__ part,
                                               unsigned in_dim, unsigned out_dim, unsigned p_rows, unsigned rb, unsigned tile, unsigned c0, unsigned c1,
                                               unsigned char* raw)
 {
     float acc[NT][16];
-    rein_xh_acc<FMT, NT>(w, img, in_dim, out_dim, (p_rows + 31u) / 32u, rb, tile, c0, c1, raw, acc);
+    Tile::template run<NT>(w, img, in_dim, out_dim, (p_rows + 31u) / 32u, rb, tile, c0, c1, raw, acc);
     const unsigned lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, j = lane & 31u, h = lane >> 5;
     if (part) {
 #pragma unroll
@@ -507,12 +528,12 @@ __device__ __forceinline__ unsigned rein_xh_deal(unsigned i, unsigned n)
     const unsigned per = (n + 7u) >> 3, k = i >> 3;
     return k < per ? (i & 7u) * per + k : 0xFFFFFFFFu;
 }
-template <int FMT>
+template <class Tile>
 __device__ __forceinline__ void rein_xh_dense(const uint8_t* __restrict__ w, const uint8_t* __restrict__ img, float* __restrict__ y, float* __restrict__ parts,
-                                              unsigned in_dim, unsigned out_dim, unsigned p_rows, unsigned n_whole, unsigned split)
+                                              unsigned in_dim, unsigned out_dim, unsigned p_rows, unsigned n_grp, unsigned n_whole, unsigned split)
 {
     extern __shared__ __attribute__((aligned(16))) unsigned char rein_xh_lds[];
-    const unsigned n_grp = (p_rows + 127u) / 128u, n_unit = ((out_dim + 127u) / 128u) * n_grp, n_chunk = in_dim >> 8;
+    const unsigned n_unit = ((out_dim + 127u) / 128u) * n_grp, n_chunk = in_dim >> 8;
     unsigned u, c0 = 0u, c1 = n_chunk;
     float* part = nullptr;
     if (blockIdx.x < n_whole) {
@@ -523,29 +544,30 @@ __device__ __forceinline__ void rein_xh_dense(const uint8_t* __restrict__ w, con
         const unsigned tu = seg / split, k = seg - tu * split;
         u = n_whole + tu;
         c0 = n_chunk * k / split; c1 = n_chunk * (k + 1u) / split;       // split <= n_chunk: no range is empty
-        if (split > 1u) part = parts + (size_t)seg * (4u * 16u * 256u);
+        if (split > 1u) part = parts + (size_t)seg * rein_xh_part(p_rows, n_grp);
     }
     if (u >= n_unit) return;
     const unsigned rb = u / n_grp;
-    const XhGroup g = rein_xh_group(p_rows, u - rb * n_grp);
-    if (g.n == 4u) rein_xh_piece<FMT, 4>(w, img, y, part, in_dim, out_dim, p_rows, rb, g.tile, c0, c1, rein_xh_lds);
-    else if (g.n == 3u) rein_xh_piece<FMT, 3>(w, img, y, part, in_dim, out_dim, p_rows, rb, g.tile, c0, c1, rein_xh_lds);
-    else if (g.n == 2u) rein_xh_piece<FMT, 2>(w, img, y, part, in_dim, out_dim, p_rows, rb, g.tile, c0, c1, rein_xh_lds);
+    const XhGroup g = rein_xh_group(p_rows, n_grp, u - rb * n_grp);
+    if (g.n == 4u) rein_xh_piece<Tile, 4>(w, img, y, part, in_dim, out_dim, p_rows, rb, g.tile, c0, c1, rein_xh_lds);
+    else if (g.n == 3u) rein_xh_piece<Tile, 3>(w, img, y, part, in_dim, out_dim, p_rows, rb, g.tile, c0, c1, rein_xh_lds);
+    else if (g.n == 2u) rein_xh_piece<Tile, 2>(w, img, y, part, in_dim, out_dim, p_rows, rb, g.tile, c0, c1, rein_xh_lds);
+    else if constexpr (Tile::kOne) { if (g.n == 1u) rein_xh_piece<Tile, 1>(w, img, y, part, in_dim, out_dim, p_rows, rb, g.tile, c0, c1, rein_xh_lds); }
 }
 
 // y of the split units.  Grid (units - n_whole, 16): blockIdx.y = 4 t + v / 4, 256 threads as in the GEMM.
-__device__ __forceinline__ void rein_xh_sum_body(const float* __restrict__ parts, float* __restrict__ y, unsigned out_dim, unsigned p_rows, unsigned n_whole, unsigned split)
+__device__ __forceinline__ void rein_xh_sum_body(const float* __restrict__ parts, float* __restrict__ y, unsigned out_dim, unsigned p_rows, unsigned n_grp, unsigned n_whole, unsigned split)
 {
-    const unsigned n_grp = (p_rows + 127u) / 128u, u = n_whole + blockIdx.x, rb = u / n_grp;
-    const XhGroup grp = rein_xh_group(p_rows, u - rb * n_grp);
+    const unsigned u = n_whole + blockIdx.x, rb = u / n_grp;
+    const XhGroup grp = rein_xh_group(p_rows, n_grp, u - rb * n_grp);
     const unsigned lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, j = lane & 31u, h = lane >> 5, t = blockIdx.y >> 2, g = blockIdx.y & 3u;
     const unsigned tok = (grp.tile + t) * 32u + j, row = rb * 128u + wave * 32u + 8u * g + 4u * h;
     if (t >= grp.n || tok >= p_rows) return;
     float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    const float4* src = reinterpret_cast<const float4*>(parts + (size_t)blockIdx.x * split * (4u * 16u * 256u)) + blockIdx.y * 256u + threadIdx.x;
+    const float4* src = reinterpret_cast<const float4*>(parts + (size_t)blockIdx.x * split * rein_xh_part(p_rows, n_grp)) + blockIdx.y * 256u + threadIdx.x;
 #pragma unroll 4
     for (unsigned k = 0; k < split; k++) {
-        const float4 p = src[(size_t)k * (4u * 4u * 256u)];
+        const float4 p = src[(size_t)k * (rein_xh_part(p_rows, n_grp) / 4u)];
         s[0] += p.x; s[1] += p.y; s[2] += p.z; s[3] += p.w;
     }
     float* o = y + (size_t)tok * out_dim + row;
