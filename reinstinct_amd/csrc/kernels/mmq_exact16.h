@@ -191,8 +191,8 @@ template <> struct XhWeights<REIN_Q4_K> {
     static constexpr int kOps = 1;                   // operands per instruction position
     static constexpr bool kHasMin = true;
     static constexpr float kUnit = 1.0f;             // what the operands were divided by
-    // plane of extra bits: bytes per sub-block (0: none) and the lane half's word in them; plane of the superblocks' scales
-    static constexpr unsigned kHiBytes = 0, kHiHalf = 0, kDBytes = 4;
+    // plane of extra bits: bytes per sub-block (0: none); plane of the superblocks' scales
+    static constexpr unsigned kHiBytes = 0, kDBytes = 4;
     static __device__ __forceinline__ const char* hi(const Fmt<REIN_Q4_K>&) { return nullptr; }
     static __device__ __forceinline__ const char* d(const Fmt<REIN_Q4_K>& f) { return reinterpret_cast<const char*>(f.ddp); }
     static __device__ __forceinline__ float scale(uint32_t dd) { return rein_h2f((uint16_t)(dd & 0xFFFFu)); }
@@ -215,7 +215,7 @@ template <> struct XhWeights<REIN_Q5_K> {
     static constexpr int kOps = 1;
     static constexpr bool kHasMin = true;
     static constexpr float kUnit = 1.0f;
-    static constexpr unsigned kHiBytes = 4, kHiHalf = 0, kDBytes = 4;
+    static constexpr unsigned kHiBytes = 4, kDBytes = 4;
     static __device__ __forceinline__ const char* hi(const Fmt<REIN_Q5_K>& f) { return reinterpret_cast<const char*>(f.qhp); }
     static __device__ __forceinline__ const char* d(const Fmt<REIN_Q5_K>& f) { return reinterpret_cast<const char*>(f.ddp); }
     static __device__ __forceinline__ float scale(uint32_t dd) { return rein_h2f((uint16_t)(dd & 0xFFFFu)); }
@@ -244,7 +244,7 @@ template <> struct XhWeights<REIN_Q6_K> {
     static constexpr int kOps = 2;
     static constexpr bool kHasMin = false;
     static constexpr float kUnit = 4.0f;
-    static constexpr unsigned kHiBytes = 8, kHiHalf = 4, kDBytes = 2;
+    static constexpr unsigned kHiBytes = 8, kDBytes = 2;
     static __device__ __forceinline__ const char* hi(const Fmt<REIN_Q6_K>& f) { return reinterpret_cast<const char*>(f.h2p); }
     static __device__ __forceinline__ const char* d(const Fmt<REIN_Q6_K>& f) { return reinterpret_cast<const char*>(f.dp); }
     static __device__ __forceinline__ float scale(uint32_t dd) { return rein_h2f((uint16_t)dd) * kUnit; }
@@ -284,8 +284,9 @@ __device__ __forceinline__ void rein_xh_pin(float (&s)[16])
 // LDS of one workgroup:
 //   acts  2 x 4 x 4352     records of two consecutive sub-block pairs
 //   ring  4 x 2 x 2048     per wavefront: two slots of 4 sub-blocks x 32 rows x 16 B
-//   small 4 x 3584         per wavefront: extra bits of a superblock [sub-block][lane], (sc, m) or both group scales
-//                          [row][sub-block], each in a dword, and the scale words of two superblocks [row]
+//   small 4 x 3584         per wavefront: extra bits of a superblock [row][sub-block] in granules of 16 bytes, rotated; (sc, m) or
+//                          both group scales [row][sub-block], in two bytes each or (padded rows) four; the scale words of two
+//                          superblocks [row]
 //   xs    4 x 2048             xsum operands of a superblock (formats with minimums)
 template <int FMT> constexpr unsigned rein_xh_lds_bytes()
 {
@@ -308,13 +309,31 @@ __device__ __forceinline__ void rein_xh_acc(const uint8_t* __restrict__ w, const
     const unsigned row_base = rb * 128u + wave * 32u, first = min(row_base, out_dim - 1u);
     // rows past the matrix read its last one; offsets from the wavefront's first row
     const unsigned row = min(row_base + j, out_dim - 1u) - first;
-    const unsigned hi_off = row * fmt.nsp * W::kHiBytes + h * W::kHiHalf, d_off = row * fmt.n_super * W::kDBytes;
-    unsigned sm_off[4];
+    const unsigned d_off = row * fmt.n_super * W::kDBytes;
+    // Extra bits and scales come sixteen bytes a lane, one to three transfers a superblock (by dword and 16-bit word they were
+    // thirteen, each as long as a kilobyte's: 2048 x 5120 -> 17408 Q6_K 749 -> 699 us, Q5_K 633 -> 569, Q5_K 45 x 17408 -> 5120 43 -> 38).
+    // A row's superblock of extra bits is four granules (Q6_K) or two (Q5_K), rotated so that the reads of one granule of every row
+    // meet every bank; its scales are one, unless the slab's rows are padded (a power of two of sub-blocks), which leaves them at
+    // two-byte alignment: then they come by 16-bit words.
+    const bool padded = (fmt.nsp & 1u) != 0u;
+    auto row_at = [&](unsigned n) { return min(row_base + n, out_dim - 1u) - first; };
+    unsigned hi_off[2] = {0u, 0u}, sm_off[4];
+    if constexpr (W::kHiBytes == 8) {
 #pragma unroll
-    for (unsigned k = 0; k < 4; k++) sm_off[k] = ((min(row_base + 8u * k + (lane >> 3), out_dim - 1u) - first) * fmt.nsp + (lane & 7u)) * 2u;
+        for (unsigned k = 0; k < 2; k++) {
+            const unsigned n = 16u * k + (lane >> 2);
+            hi_off[k] = row_at(n) * fmt.nsp * 8u + (((lane & 3u) - (n >> 1)) & 3u) * 16u;
+        }
+    } else if constexpr (W::kHiBytes == 4) {
+        hi_off[0] = row_at(lane >> 1) * fmt.nsp * 4u + ((lane ^ (lane >> 3)) & 1u) * 16u;
+    }
+#pragma unroll
+    for (unsigned k = 0; k < 4; k++)                 // (unpadded: the upper lanes fetch the rows again)
+        sm_off[k] = padded ? (row_at(8u * k + (lane >> 3)) * fmt.nsp + (lane & 7u)) * 2u : row * fmt.nsp * 2u;
+    const unsigned sm_step = padded ? 4u : 2u;
 
     const uint4* const ring = reinterpret_cast<const uint4*>(raw + kRing + wave * 4096u);
-    const uint32_t* const small = reinterpret_cast<const uint32_t*>(raw + kSmall + wave * 3584u);
+    const unsigned char* const small = raw + kSmall + wave * 3584u;
     const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(lptr_t)raw);
     MmqWSrc<FMT> wsrc;
     wsrc.init(*reinterpret_cast<const MmqWLds<FMT>*>(ring), fmt, row_base, out_dim, lane);
@@ -344,12 +363,16 @@ __device__ __forceinline__ void rein_xh_acc(const uint8_t* __restrict__ w, const
         const unsigned dst = lds0 + kSmall + wave * 3584u;
         if constexpr (W::kHiBytes != 0) {
             const char* hp = W::hi(fmt) + ((size_t)first * fmt.nsp + c * 8u) * W::kHiBytes;
-#pragma unroll
-            for (unsigned k = 0; k < 8; k++) rein_xh_dma_u32(hi_off, hp + k * W::kHiBytes, dst + k * 256u);
+            rein_lds_dma16_s(hi_off[0], hp, dst);
+            if constexpr (W::kHiBytes == 8) rein_lds_dma16_s(hi_off[1], hp, dst + 1024u);
         }
         const char* sp = reinterpret_cast<const char*>(fmt.smp) + ((size_t)first * fmt.nsp + c * 8u) * 2u;
+        if (padded) {
 #pragma unroll
-        for (unsigned k = 0; k < 4; k++) rein_xh_dma_u16(sm_off[k], sp, dst + 2048u + k * 256u);
+            for (unsigned k = 0; k < 4; k++) rein_xh_dma_u16(sm_off[k], sp, dst + 2048u + k * 256u);
+        } else {
+            rein_lds_dma16_s(sm_off[0], sp, dst + 2048u);
+        }
         const char* dp = W::d(fmt) + ((size_t)first * fmt.n_super + c) * W::kDBytes;
         if constexpr (W::kDBytes == 4) rein_xh_dma_u32(d_off, dp, dst + 3072u + (c & 1u) * 256u);
         else rein_xh_dma_u16(d_off, dp, dst + 3072u + (c & 1u) * 256u);
@@ -380,8 +403,16 @@ __device__ __forceinline__ void rein_xh_acc(const uint8_t* __restrict__ w, const
             const bool last = c + 1u == c1;
             REIN_WAIT_VMCNT(0);
             __syncthreads();
-            const uint2 sm2 = *reinterpret_cast<const uint2*>(small + 512u + j * 8u + 2u * u);
-            const uint32_t hi2[2] = {small[2u * u * 64u + lane], small[(2u * u + 1u) * 64u + lane]};
+            const unsigned char* const sms = small + 2048u + (8u * j + 2u * u) * sm_step;
+            const uint32_t sm2[2] = {*reinterpret_cast<const uint16_t*>(sms), *reinterpret_cast<const uint16_t*>(sms + sm_step)};
+            uint32_t hi2[2] = {0u, 0u};
+            if constexpr (W::kHiBytes == 8) {
+                const uint4 g = *reinterpret_cast<const uint4*>(small + j * 64u + ((u + rot) & 3u) * 16u);
+                hi2[0] = h ? g.y : g.x; hi2[1] = h ? g.w : g.z;
+            } else if constexpr (W::kHiBytes == 4) {
+                const uint2 g = *reinterpret_cast<const uint2*>(small + j * 32u + (((u >> 1) ^ (j >> 2)) & 1u) * 16u + (u & 1u) * 8u);
+                hi2[0] = g.x; hi2[1] = g.y;
+            }
             if (u < 3u || !last) issue_acts(pair + 1u);
             if (u == 0u) rein_mmq_wload<FMT>(wsrc, 1u, fmt, c * 8u + 4u, n_sub);
             if (u == 1u) issue_xs(c);                // read at the superblock's end; the barrier of u = 0 freed it
@@ -396,7 +427,7 @@ __device__ __forceinline__ void rein_xh_acc(const uint8_t* __restrict__ w, const
                 const unsigned sb = 2u * u + q, s4 = sb & 3u;
                 const uint2 w2 = reinterpret_cast<const uint2*>(ring + (u >> 1) * 128u + 4u * j + ((s4 + rot) & 3u))[h];
                 rein_v8h a[2][W::kOps];
-                const uint32_t sm = q ? sm2.y : sm2.x;
+                const uint32_t sm = sm2[q];
                 W::unpack(a, w2, hi2[q], sm, h, mk);
                 if constexpr (W::kHasMin) {
                     const uint32_t m = rein_bf16_of_u8(sm >> 8);
@@ -450,7 +481,7 @@ __device__ __forceinline__ void rein_xh_acc(const uint8_t* __restrict__ w, const
         float dv[16], nv[16];
 #pragma unroll
         for (int g = 0; g < 4; g++) {
-            const uint4 d4 = *reinterpret_cast<const uint4*>(small + 768u + (c & 1u) * 64u + 8 * g + 4u * h);
+            const uint4 d4 = *reinterpret_cast<const uint4*>(small + 3072u + (c & 1u) * 256u + (8 * g + 4u * h) * 4u);
             const uint32_t dw[4] = {d4.x, d4.y, d4.z, d4.w};
 #pragma unroll
             for (int v = 0; v < 4; v++) { dv[4 * g + v] = W::scale(dw[v]); nv[4 * g + v] = W::min_scale(dw[v]); }

@@ -52,7 +52,7 @@ __device__ __forceinline__ void rein_x8_quantize_body(const float* __restrict__ 
 // LDS of one workgroup:
 //   acts  2 x 8 x 2304               records of two consecutive steps (a step: two sub-block pairs), [pair of the step][tile]
 //   ring  4 x 2 x planes x 2048      per wavefront: two slots of 4 sub-blocks x 32 rows x 16 B (Q8_0: of both planes)
-//   scale 4 x 2 x 1024               per wavefront: fp16 scales of two superblocks: [row][8], or a dword each (PAD)
+//   scale 4 x 2 x 1024               per wavefront: fp16 scales of two superblocks: [row][8], or (padded rows) a dword each
 template <int FMT> struct X8Lds {
     static constexpr unsigned kAct = 8u * REIN_X8_REC, kPlanes = FMT == REIN_Q8_0 ? 2u : 1u, kRing = 2u * kAct, kRingWave = 2u * kPlanes * 2048u;
     static constexpr unsigned kScale = kRing + 4u * kRingWave, kBytes = kScale + 4u * 2048u;
@@ -75,9 +75,9 @@ __device__ __forceinline__ void rein_x8_step(float (&acc)[16], const rein_v16i& 
 
 // Superblocks [c0, c1) of rows 128 rb .. and the NT token tiles from `tile` on, into acc.  One barrier per step of four
 // sub-blocks: at its top everything that the step reads has landed (issued a whole step earlier: 4 NT matrix instructions of dots and
-// NT of scales per wavefront), behind it the next step's transfers go out.  PAD: the slab's rows are padded (a power of two of
-// sub-blocks), which leaves a row's scales at 2-byte alignment: they come by 16-bit transfers.
-template <int FMT, int NT, bool PAD>
+// NT of scales per wavefront), behind it the next step's transfers go out.  Padded rows of the slab (a power of two of sub-blocks)
+// leave a row's scales at two-byte alignment: then they come by 16-bit words.
+template <int FMT, int NT>
 __device__ __forceinline__ void rein_x8_acc(const uint8_t* __restrict__ w, const uint8_t* __restrict__ img, unsigned in_dim, unsigned out_dim,
                                             unsigned n_tt, unsigned rb, unsigned tile, unsigned c0, unsigned c1, unsigned char* const raw, float (&acc)[NT][16])
 {
@@ -90,18 +90,17 @@ __device__ __forceinline__ void rein_x8_acc(const uint8_t* __restrict__ w, const
     // rows past the matrix read its last one; offsets from the wavefront's first row
     const unsigned row_base = rb * 128u + wave * 32u, first = min(row_base, out_dim - 1u);
     auto row_at = [&](unsigned n) { return min(row_base + n, out_dim - 1u) - first; };
-    unsigned w_off[2], sc_off[PAD ? 4 : 1];
+    const bool padded = (fmt.nsp & 1u) != 0u;
+    unsigned w_off[2], sc_off[4];
 #pragma unroll
     for (unsigned k = 0; k < 2; k++) {               // slot entry of (row n, sub-block s): 4 n + ((s + n / 2) & 3), as in MmqWLds
         const unsigned n = 16u * k + (lane >> 2);
         w_off[k] = (row_at(n) * fmt.nsp + (((lane & 3u) - (n >> 1)) & 3u)) * 16u;
     }
-    if constexpr (PAD) {
 #pragma unroll
-        for (unsigned k = 0; k < 4; k++) sc_off[k] = (row_at(8u * k + (lane >> 3)) * fmt.nsp + (lane & 7u)) * 2u;
-    } else {
-        sc_off[0] = row_at(j) * fmt.nsp * 2u;        // 16 bytes a row; the upper lanes fetch the rows again
-    }
+    for (unsigned k = 0; k < 4; k++)                 // (unpadded: sixteen bytes a row; the upper lanes fetch the rows again)
+        sc_off[k] = padded ? (row_at(8u * k + (lane >> 3)) * fmt.nsp + (lane & 7u)) * 2u : row_at(j) * fmt.nsp * 2u;
+    const unsigned sc_step = padded ? 4u : 2u;
     const unsigned ring_at = L::kRing + wave * L::kRingWave, sc_at = L::kScale + wave * 2048u;
     const uint4* const ring = reinterpret_cast<const uint4*>(raw + ring_at);
     const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(lptr_t)raw);
@@ -132,7 +131,7 @@ __device__ __forceinline__ void rein_x8_acc(const uint8_t* __restrict__ w, const
     auto issue_scales = [&](unsigned c) {
         const unsigned dst = lds0 + sc_at + (c & 1u) * 1024u;
         const char* p = reinterpret_cast<const char*>(fmt.dp) + ((size_t)first * fmt.nsp + c * 8u) * 2u;
-        if constexpr (PAD) {
+        if (padded) {
 #pragma unroll
             for (unsigned k = 0; k < 4; k++) rein_xh_dma_u16(sc_off[k], p, dst + k * 256u);
         } else {
@@ -163,7 +162,7 @@ __device__ __forceinline__ void rein_x8_acc(const uint8_t* __restrict__ w, const
     const unsigned rot = j >> 1;
 
     for (unsigned c = c0; c < c1; c++) {
-        const unsigned char* const sc_base = raw + sc_at + (c & 1u) * 1024u + (PAD ? j * 32u : j * 16u);
+        const unsigned char* const sc_base = raw + sc_at + (c & 1u) * 1024u + (8u * j + h) * sc_step;
 #pragma unroll
         for (unsigned u = 0; u < 2; u++) {
             const unsigned step = c * 2u + u;
@@ -182,7 +181,7 @@ __device__ __forceinline__ void rein_x8_acc(const uint8_t* __restrict__ w, const
 #pragma unroll
                 for (unsigned q = 0; q < 2; q++)
                     b[q] = C::operand_at(ring + (u * L::kPlanes + (L::kPlanes == 2u ? h : 0u)) * 128u + 4u * j + ((2u * pr + q + rot) & 3u), none, 0, h);
-                const float sc = rein_h2f(*reinterpret_cast<const uint16_t*>(sc_base + (4u * u + 2u * pr + h) * (PAD ? 4u : 2u)));
+                const float sc = rein_h2f(*reinterpret_cast<const uint16_t*>(sc_base + (4u * u + 2u * pr) * sc_step));
                 rein_v4i xa[2][2];
                 float dx[2];
                 auto read = [&](int t) {
@@ -224,7 +223,6 @@ template <int FMT> struct X8Tile {
     static __device__ __forceinline__ void run(const uint8_t* __restrict__ w, const uint8_t* __restrict__ img, unsigned in_dim, unsigned out_dim, unsigned n_tt,
                                                unsigned rb, unsigned tile, unsigned c0, unsigned c1, unsigned char* const raw, float (&acc)[NT][16])
     {
-        if (rein_nsp(in_dim >> 5) & 1u) rein_x8_acc<FMT, NT, true>(w, img, in_dim, out_dim, n_tt, rb, tile, c0, c1, raw, acc);
-        else rein_x8_acc<FMT, NT, false>(w, img, in_dim, out_dim, n_tt, rb, tile, c0, c1, raw, acc);
+        rein_x8_acc<FMT, NT>(w, img, in_dim, out_dim, n_tt, rb, tile, c0, c1, raw, acc);
     }
 };
