@@ -107,8 +107,8 @@ int rein_is_loaded(void);
  * width), REIN_MMQ6, REIN_MMQ6_FROM, REIN_MMQ6_N4, REIN_MMQ6_N2, REIN_MMQ6_SK,
  * REIN_MMQ6_SK_GRID, REIN_MMQ6_SK_SPLIT (Q4_K fp6 launch: 0 off, first row count, token groups
  * of four / two tiles per row block, split-tail 0 off / 2 forced, its grid and ranges),
- * REIN_MMQ16 (1: the fp16 formulation where the code object holds it), REIN_MMQXH (0 / 2: the GEMMs of
- * rein_matmul_ws on 32 x 128 wavefront tiles, exact-dot fp16 and int8, off / wherever they can run), REIN_MMQXH_SPLIT,
+ * REIN_MMQ16 (1: the fp16 formulation where the code object holds it), REIN_MMQXH (0 / 2 / 3: the GEMMs of
+ * rein_matmul_ws on 32 x 128 wavefront tiles, exact-dot fp16 and int8, off / wherever they can run / the K-quants' in groups of one and two token tiles), REIN_MMQXH_SPLIT,
  * REIN_MMQXH_GROUPS (their ranges per unit, their groups of token tiles), REIN_TOPK_WAVE,
  * REIN_MOE_SORT_SPLIT, REIN_MOE_CHAIN, REIN_MOE_FUSED, REIN_MOE_FEW, REIN_MOE_GU_ROWS, REIN_MOE_DC_ROWS
  * (MoE glue: 0 = the workgroup router, 1 = the four-launch sort, 0 = no decode chain for few

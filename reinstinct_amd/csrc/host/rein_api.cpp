@@ -1846,167 +1846,177 @@ int rein_matmul(int fmt, const void* w, const float* x, float* y, unsigned in_di
 }
 
 namespace {
-// ---- prefill out of rein_matmul_ws: 32 rows x up to 128 tokens per wavefront, activations as an image in operand order.  Q4_K / Q5_K /
-// Q6_K with exact block dots on the fp16 instruction (kernels/mmq_exact16.h), Q8_0 / Q4_0 / IQ4_XS / IQ3_S on the int8 one (mmq_x8.h)
-struct XhPlan {
+// ---- prefill out of rein_matmul_ws: 32 rows x a group of token tiles per wavefront, activations as an image in operand order.
+//   exact  Q4_K, Q5_K, Q6_K   exact block dots on the fp16 instruction (kernels/mmq_exact16.h), groups of two to four tiles
+//   few    the same           groups of one and two tiles, three workgroups per CU
+//   int8   Q8_0, Q4_0, IQ4_XS, IQ3_S   the int8 instruction (mmq_x8.h), groups of one to four tiles
+// Units of 128 rows x a group; whole rounds of the resident workgroups run unsplit, what is left over is cut into ranges of
+// superblocks.  How many tiles a group has and how many ranges there are is the cheapest by a price in microseconds: a superblock of
+// a workgroup with t tiles costs alone[n] + tile[n] t with n + 1 workgroups on its CU (the last round may leave fewer than fit),
+// `sum` the launch that adds partial tiles, `part` each tile of 16 KB that is written and read again.  Fitted per kind to every group
+// size x 1-16 ranges on 12-13 shapes x 17 row counts: the pick is within 1 % of the best of its cell in the mean, at most 8-16 % (Q8_0 5120 ->
+// 1024, 160 rows, groups x ranges: 5 x 5 15.5 us, 2 x 12 20.3; 17408 -> 5120, 45 rows 1 x 12 35.0, 2 x 6 36.5, 1 x 4 44; 2048 -> 5632,
+// 300 rows 10 x 1 24.7, 5 x 1 26.2, 3 x 6 32.7).
+struct WideKind {
+    const char* tag;                                 // of the kernels' names: rein_<tag>_quantize, _<fmt>, _sum
+    unsigned most, least, slots;                     // tiles of a group, resident workgroups
+    double alone[3], tile[3], sum, part;
+};
+const WideKind kWideQ4 = {"xh", 4, 2, 512, {0.9, 3.0}, {1.44, 1.27}, 1.2, 0.0087}, kWideQ5 = {"xh", 4, 2, 512, {0.3, 2.3}, {1.41, 1.25}, 1.5, 0.0077},
+               kWideQ6 = {"xh", 4, 2, 512, {0.4, 3.85}, {1.47, 0.82}, 0.42, 0.0075}, kWideInt8 = {"x8", 4, 1, 512, {0.47, 1.0}, {1.2, 1.68}, 2.4, 0.0061},
+               kWideFew = {"xf", 2, 1, 768, {1.0, 2.1, 2.7}, {0.81, 0.67, 0.90}, 1.14, 0.0071};
+struct WidePlan {
     unsigned n_grp, n_unit, n_whole, split;
     size_t image, parts;                             // bytes of the activation image and of the partial tiles behind it
 };
-constexpr size_t kXhPart = (size_t)16 * 256 * 4;     // 128 rows x a token tile, fp32
-constexpr unsigned kXhMostParts = 1024;              // ranges of one launch: at most 64 MiB of partial tiles
-bool xh_format(int fmt) { return fmt == REIN_TYPE_Q4_K || fmt == REIN_TYPE_Q5_K || fmt == REIN_TYPE_Q6_K; }
-bool xh_has_min(int fmt) { return fmt == REIN_TYPE_Q4_K || fmt == REIN_TYPE_Q5_K; }
-size_t xh_image_bytes(int fmt, unsigned in_dim, unsigned p_rows)
+constexpr size_t kWidePart = (size_t)16 * 256 * 4;   // 128 rows x a token tile, fp32
+constexpr unsigned kWideMostParts = 1024;            // ranges of one launch: at most 64 MiB of partial tiles
+bool wide_k_quant(int fmt) { return fmt == REIN_TYPE_Q4_K || fmt == REIN_TYPE_Q5_K || fmt == REIN_TYPE_Q6_K; }
+bool wide_has_min(int fmt) { return fmt == REIN_TYPE_Q4_K || fmt == REIN_TYPE_Q5_K; }
+const WideKind& wide_exact(int fmt) { return fmt == REIN_TYPE_Q4_K ? kWideQ4 : fmt == REIN_TYPE_Q5_K ? kWideQ5 : kWideQ6; }
+size_t wide_image_bytes(int fmt, unsigned in_dim, unsigned p_rows)
 {
     const size_t n_tt = ((size_t)p_rows + 31) / 32;
-    if (!xh_format(fmt)) return (in_dim / 64) * n_tt * 2304;                                                 // REIN_X8_REC
-    return (in_dim / 64) * n_tt * 4352 + (xh_has_min(fmt) ? (in_dim / 256) * n_tt * 2048 : 0);
+    if (!wide_k_quant(fmt)) return (in_dim / 64) * n_tt * 2304;                                              // REIN_X8_REC
+    return (in_dim / 64) * n_tt * 4352 + (wide_has_min(fmt) ? (in_dim / 256) * n_tt * 2048 : 0);
 }
-unsigned xh_lds_bytes(int fmt)
+unsigned wide_lds_bytes(const WideKind& kind, int fmt)
 {
-    if (!xh_format(fmt)) return 2 * 18432 + 4 * (fmt == REIN_TYPE_Q8_0 ? 8192 : 4096) + 4 * 2048;            // X8Lds
-    return 2 * 17408 + 4 * 4096 + 4 * 3584 + (xh_has_min(fmt) ? 8192 : 0);                                   // rein_xh_lds_bytes
+    if (!wide_k_quant(fmt)) return 2 * 18432 + 4 * (fmt == REIN_TYPE_Q8_0 ? 8192 : 4096) + 4 * 2048;         // X8Lds
+    return 2 * kind.most * 4352 + 4 * 4096 + 4 * 3584 + (wide_has_min(fmt) ? kind.most * 2048 : 0);          // rein_xh_lds_bytes
 }
-// Where it is taken, from sweeps through rein_matmul_ws, every cell beside the launches of rein_mmq_xq8_ws (their time / this one's),
-// the weights of two to six matrices in turn, 9-2048 rows:
-//   Q8_0, Q4_0, IQ4_XS  12 shapes (1024 -> 4096 ... 17408 -> 5120, 1536 -> 32000) x 17 row counts: from 24 rows 0.95-2.0 in 612 cells, 7 of
-//         them below 0.98, 1.14-1.27 in the geometric mean of every row count (Q8_0 5120 -> 17408, 2048 rows 648 / 507 us; 17408 ->
-//         5120, 200 rows 135 / 77, 45 rows 44 / 35; 5632 -> 2048, 32 rows 16.7 / 13.0).  All four from 17 rows on 13 shapes 1.03-1.44
-//         at 17-28 rows.  Not contractions below 2048 against 4096 rows and more at 65-400 rows (1024 -> 4096 and 1536 -> 32000
-//         0.96-1.03: three launches for little work).  9-16 rows: contractions of three times the rows of weights (1.04-1.33 in 60
-//         cells; 5632 -> 2048 0.92-0.96, 5120 -> 5120 0.86-1.0), and the 4-bit formats from 48M weights (5120 -> 17408, 4096 ->
-//         14336, 8192 -> 8192 1.01-1.15; Q8_0 there 0.82-1.01).
-//   Q6_K  0.98-2.0 in all 104 cells of 13 shapes (17408 -> 5120, 45 rows 62.5 / 51.0 us, 512 rows 451 / 222; 5120 -> 17408 512 rows
-//         311 / 200): everywhere from two token tiles; below 2.5e8 operations nothing was measured.
-//   Q4_K  contractions of 3072 and more at 33-64 rows 0.97-1.20, median 1.1 (17408 -> 5120, 45 rows 40.5 / 34.9 us; 2304-2560
-//         0.97-1.14, median 1.0); 80 rows 0.89-1.26 (three tiles of a group of four at the cost of a whole group's unpack against the int8 split
-//         tail's 32-token units); from 96 rows contractions of 4096 and more, 0.91-1.78, median 1.06 (3072-3584: 0.75-1.17, in the
-//         mean 0.97: ranges of few superblocks do not pay back their starts and the image).
-//   Q5_K  from 384 rows, contractions of 4096 and more 0.90-1.53, median 1.13 (5120 -> 17408, 512 rows 194 / 172), of 3072-3584 against
-//         16384 rows and more (18944: 1.05-1.18 in 22 cells; 2560-12288 rows 0.78-1.35, in the mean 0.99); below 384 rows groups of two and
-//         three tiles share the unpack of its fifth bits too little (33-320 rows 0.75-1.8, median 0.98).
-// The K-quants' kernel is built for groups of at least two tiles.
-bool xh_shape(int fmt, unsigned in_dim, unsigned p_rows)          // for any number of weight rows
+// Where they are taken, from sweeps through rein_matmul_ws, every cell beside the launches of rein_mmq_xq8_ws (their time / this one's),
+// the weights of two to six matrices in turn:
+//   int8  12 shapes (1024 -> 4096 ... 17408 -> 5120, 1536 -> 32000) x 17 row counts: from 24 rows 0.95-2.0 in 612 cells, 7 of them below
+//         0.98, 1.14-1.27 in the geometric mean of every row count (Q8_0 5120 -> 17408, 2048 rows 648 / 507 us; 17408 -> 5120, 200 rows
+//         135 / 77, 45 rows 44 / 35; 5632 -> 2048, 32 rows 16.7 / 13.0).  All four from 17 rows on 13 shapes 1.03-1.44 at 17-28 rows.  Not
+//         contractions below 2048 against 4096 rows and more at 65-400 rows (1024 -> 4096 and 1536 -> 32000 0.96-1.03: three launches for
+//         little work).  9-16 rows: contractions of three times the rows of weights (1.04-1.33 in 60 cells; 5632 -> 2048 0.92-0.96, 5120 ->
+//         5120 0.86-1.0), and the 4-bit formats from 48M weights (5120 -> 17408, 4096 -> 14336, 8192 -> 8192 1.01-1.15; Q8_0 there 0.82-1.01).
+//   exact, 13 shapes (those and 3584 -> 18944) x 17 row counts from 33:
+//     Q6_K  1.07-3.0 in all 221 cells (17408 -> 5120, 200 rows 220 / 72 us; 5120 -> 17408, 512 rows 311 / 182); below 2.5e8 operations
+//           nothing was measured.
+//     Q4_K  33-64 rows contractions of 3072 and more 0.98-1.27 in 27 cells (2048 1.05-1.14, but 1536 -> 32000 0.85); 65-95 rows those of 4096
+//           and more against matrices of 48M weights (1.09-1.36; 5120 -> 5120 0.90: three tiles at the cost of a whole group's unpack);
+//           from 96 rows contractions of 4096 and more, 0.86-1.85, median 1.10 (below, 0.70-1.22: ranges of few superblocks do not
+//           pay back their starts and the image).
+//     Q5_K  65-383 rows contractions of 3072 and more against 48M weights (0.90-1.97, median 1.2), from 101 rows 24M (5120 -> 5120
+//           1.10-1.46; 80 rows 0.96), and narrow ones of 5M (5632 -> 2048, 5120 -> 1024 1.0-1.13); 3072 -> 3072 0.88-0.95 at 80-200 rows.  From 384 rows
+//           contractions of 4096 and more (1.07-1.52), of 3072 against 16384 rows and more (1.18-1.31), from 1024 rows of 1536 (1.04-1.29).
+//   few, the same shapes, 12-64 rows:
+//     Q6_K  17-32 rows 1.14-1.41 in all 26 cells (17408 -> 5120 43 / 34 us)
+//     Q4_K, Q5_K  17-32 rows up to 16384 rows of weights 1.01-1.23 (beyond 0.91-1.02); Q5_K at 33-64 rows 1.05-1.26 in all 26 (17408 -> 5120,
+//           45 rows 42 / 37).
+//     9-16 rows matrices of 60M weights (Q5_K 85M): 1.03-1.32; smaller ones 0.82-1.05.  Matrices below 4M weights were not measured.
+bool wide_exact_shape(int fmt, unsigned in_dim, unsigned p_rows)          // for any number of weight rows
 {
     const unsigned mode = opt_u(O_MMQXH, 1);
-    const bool k_quant = xh_format(fmt);
-    if (mode == 0 || in_dim == 0 || in_dim % 256 != 0 || p_rows <= (k_quant ? 32u : 8u)) return false;
-    if (mode == 2 || fmt == REIN_TYPE_Q6_K || !k_quant) return true;
-    if (fmt == REIN_TYPE_Q4_K && p_rows > 64) return in_dim >= 4096 && p_rows >= 96;
-    return in_dim >= 3072 && (fmt == REIN_TYPE_Q4_K || p_rows >= 384);
+    if (mode == 0 || mode == 3 || p_rows <= 32) return false;             // the kernel is built for groups of at least two tiles
+    if (mode == 2 || fmt == REIN_TYPE_Q6_K) return true;
+    if (fmt == REIN_TYPE_Q4_K) return in_dim >= (p_rows <= 64 ? 3072u : 4096u);
+    return p_rows > 64 && in_dim >= (p_rows >= 1024 ? 1536u : 3072u);
 }
-bool xh_take(int fmt, unsigned in_dim, unsigned out_dim, unsigned p_rows)
+bool wide_exact_take(int fmt, unsigned in_dim, unsigned out_dim, unsigned p_rows)
 {
-    if (!xh_shape(fmt, in_dim, p_rows)) return false;
+    if (!wide_exact_shape(fmt, in_dim, p_rows)) return false;
     if (opt_u(O_MMQXH, 1) == 2) return true;
-    if (!xh_format(fmt)) {
-        if (p_rows <= 16) return in_dim >= 3ull * out_dim || (fmt != REIN_TYPE_Q8_0 && (unsigned long long)in_dim * out_dim >= 48ull << 20);
-        return in_dim >= 2048 || p_rows <= 64 || p_rows > 400 || out_dim < 4096;
-    }
-    if (fmt == REIN_TYPE_Q5_K) return in_dim >= 4096 || out_dim >= 16384;
-    return fmt != REIN_TYPE_Q6_K || 2.0 * p_rows * (double)out_dim * in_dim >= 2.5e8;
+    const unsigned long long weights = (unsigned long long)in_dim * out_dim;
+    if (fmt == REIN_TYPE_Q6_K) return 2.0 * p_rows * (double)weights >= 2.5e8;
+    if (fmt == REIN_TYPE_Q4_K) return p_rows <= 64 || p_rows >= 96 || weights >= 48ull << 20;
+    if (p_rows >= 384) return in_dim >= 4096 || out_dim >= 16384 || p_rows >= 1024;
+    return weights >= (p_rows > 100 ? 24ull << 20 : 48ull << 20) || (2ull * in_dim >= 5ull * out_dim && weights >= 5ull << 20);
 }
-// Units of 128 rows x a group of token tiles, 512 resident workgroups.  Whole rounds run unsplit; what is left over is cut into
-// ranges of superblocks.  How many tiles a group has and how many ranges there are is the cheapest by this price, in microseconds:
-// a superblock of a workgroup with t tiles a2 + b2 t beside another workgroup on its CU, a1 + b1 t alone (a last round of at most
-// one workgroup per CU), 2.4 for the launch that adds partial tiles, 6.1 ns for each tile of 16 KB that is written and read again.
-// Fitted to 600 cells (Q8_0, Q4_0, IQ4_XS; groups of 1-4 tiles x 1-16 ranges each): the pick is within 1 % of the best of its cell
-// in the mean, 16 % at most.  (Q8_0 5120 -> 1024, 160 rows, groups x ranges: 5 x 5 15.5 us, 2 x 12 20.3; 17408 -> 5120, 45 rows 1 x 12
-// 35.0, 2 x 6 36.5, 1 x 4 44; 2048 -> 5632, 300 rows 10 x 1 24.7, 5 x 1 26.2, 3 x 6 32.7.)
-struct XhGroups { unsigned n_grp, split; };
-constexpr double kX8Pair = 1.0, kX8PairTile = 1.68, kX8Alone = 0.47, kX8AloneTile = 1.2, kXhSum = 2.4, kXhTilePart = 0.0061;
-double x8_price(unsigned units, unsigned n_tt, unsigned n_grp, unsigned chunks, unsigned split)
+bool wide_few_shape(int fmt, unsigned, unsigned p_rows)
 {
-    const double tiles = n_tt / (double)n_grp, most_tiles = (n_tt + n_grp - 1) / n_grp, pair = kX8Pair + kX8PairTile * tiles;
-    const unsigned wg = units % 512 * split, rem = wg % 512;
-    const double range = 0.5 * (chunks / (double)split + (chunks + split - 1) / split);
-    double t = (units / 512) * (chunks * pair) + (wg / 512) * (range * pair);
-    if (rem) t += range * (rem <= kCUs ? kX8Alone + kX8AloneTile * most_tiles : kX8Pair + kX8PairTile * most_tiles);
-    return split > 1 ? t + kXhSum + wg * tiles * kXhTilePart : t;
+    const unsigned mode = opt_u(O_MMQXH, 1);
+    if (mode == 3) return p_rows > 8;
+    return mode == 1 && p_rows > 8 && p_rows <= (fmt == REIN_TYPE_Q5_K ? 64u : 32u);
+}
+bool wide_few_take(int fmt, unsigned in_dim, unsigned out_dim, unsigned p_rows)
+{
+    if (!wide_few_shape(fmt, in_dim, p_rows)) return false;
+    if (opt_u(O_MMQXH, 1) == 3) return true;
+    const unsigned long long weights = (unsigned long long)in_dim * out_dim;
+    if (p_rows <= 16) return weights >= (fmt == REIN_TYPE_Q5_K ? 85ull << 20 : 60ull << 20);
+    return weights >= 4ull << 20 && (fmt == REIN_TYPE_Q6_K || p_rows > 32 || out_dim <= 16384);
+}
+bool wide_int8_take(int fmt, unsigned in_dim, unsigned out_dim, unsigned p_rows)
+{
+    if (opt_u(O_MMQXH, 1) >= 2) return true;
+    if (p_rows <= 16) return in_dim >= 3ull * out_dim || (fmt != REIN_TYPE_Q8_0 && (unsigned long long)in_dim * out_dim >= 48ull << 20);
+    return in_dim >= 2048 || p_rows <= 64 || p_rows > 400 || out_dim < 4096;
+}
+// the launch of a shape, or null: those of rein_mmq_xq8_ws
+const WideKind* wide_kind(int fmt, unsigned in_dim, unsigned out_dim, unsigned p_rows)
+{
+    if (opt_u(O_MMQXH, 1) == 0 || in_dim % 256 != 0 || p_rows <= 8) return nullptr;
+    if (!wide_k_quant(fmt)) return wide_int8_take(fmt, in_dim, out_dim, p_rows) ? &kWideInt8 : nullptr;
+    if (wide_exact_take(fmt, in_dim, out_dim, p_rows)) return &wide_exact(fmt);
+    return wide_few_take(fmt, in_dim, out_dim, p_rows) ? &kWideFew : nullptr;
+}
+double wide_price(const WideKind& kind, unsigned units, unsigned n_tt, unsigned n_grp, unsigned chunks, unsigned split)
+{
+    const double tiles = n_tt / (double)n_grp, most_tiles = (n_tt + n_grp - 1) / n_grp;
+    const unsigned full = kind.slots / kCUs - 1, wg = units % kind.slots * split, rem = wg % kind.slots;
+    const double range = 0.5 * (chunks / (double)split + (chunks + split - 1) / split), round = kind.alone[full] + kind.tile[full] * tiles;
+    double t = ((units / kind.slots) * (double)chunks + (wg / kind.slots) * range) * round;
+    if (rem) t += range * (kind.alone[(rem - 1) / kCUs] + kind.tile[(rem - 1) / kCUs] * most_tiles);
+    return split > 1 ? t + kind.sum + wg * tiles * kind.part : t;
 }
 // the cheapest number of ranges for `units` units of n_grp groups, and its price
-unsigned x8_split(unsigned units, unsigned n_tt, unsigned n_grp, unsigned chunks, double* price)
+unsigned wide_split(const WideKind& kind, unsigned units, unsigned n_tt, unsigned n_grp, unsigned chunks, double* price)
 {
-    const unsigned tail = units % 512, most = tail == 0 ? 1 : std::max(1u, std::min(std::min(16u, chunks), kXhMostParts / tail));
+    const unsigned tail = units % kind.slots, most = tail == 0 ? 1 : std::max(1u, std::min(std::min(16u, chunks), kWideMostParts / tail));
     const unsigned forced = opt_u(O_MMQXH_SPLIT, 0);
     unsigned split = std::min(std::max(1u, forced), most);
-    *price = x8_price(units, n_tt, n_grp, chunks, split);
+    *price = wide_price(kind, units, n_tt, n_grp, chunks, split);
     for (unsigned k = 2; k <= most && !forced; k++) {
-        const double t = x8_price(units, n_tt, n_grp, chunks, k);
+        const double t = wide_price(kind, units, n_tt, n_grp, chunks, k);
         if (t < *price) { *price = t; split = k; }
     }
     return split;
 }
-XhGroups x8_groups(unsigned in_dim, unsigned out_dim, unsigned p_rows)
+// groups of at most `size` tiles (or as many groups as are asked for), none smaller than the kernel is built for
+unsigned wide_groups(const WideKind& kind, unsigned n_tt, unsigned size)
 {
-    const unsigned n_tt = (p_rows + 31) / 32, n_rb = (out_dim + 127) / 128, least = (n_tt + 3) / 4, forced = opt_u(O_MMQXH_GROUPS, 0);
-    XhGroups best{0, 1};
-    double best_price = 0.0;
-    for (unsigned size = 4; size >= 1; size--) {
-        const unsigned n_grp = forced ? std::min(n_tt, std::max(forced, least)) : (n_tt + size - 1) / size;
-        double price;
-        const unsigned split = x8_split(n_rb * n_grp, n_tt, n_grp, in_dim / 256, &price);
-        if (best.n_grp == 0 || price < best_price) { best = XhGroups{n_grp, split}; best_price = price; }
-    }
-    return best;
+    const unsigned least = (n_tt + kind.most - 1) / kind.most, most = std::max(1u, n_tt / kind.least), forced = opt_u(O_MMQXH_GROUPS, 0);
+    return std::max(least, std::min(most, forced ? forced : (n_tt + size - 1) / size));
 }
-// The K-quants: groups of up to four tiles; the cheapest number of ranges, counted in superblocks of a workgroup that shares its
-// CU: a range costs its superblocks and one and a half for its start; a last round of at most one workgroup per CU takes 0.6 of
-// one with two; a partial tile is written and read once.  Q6_K, us at 1 / 2 / 3 / 4 / 6 ranges: 17408 -> 5120, 777 rows (280 units)
-// 467 / 409 / 371 / 370 / 369, 512 rows (160 units) 357 / 278 / 223 / 252 / 232; 5120 -> 17408, 512 rows (a round and 32) 272 / 224 /
-// 211 / 201 / 200.
-unsigned xh_split(unsigned tail, unsigned chunks)
+// partial tiles of the units behind n_whole (rein_xh_part, rein_xh_group)
+size_t wide_parts_bytes(unsigned n_rb, unsigned n_whole, unsigned split, unsigned n_tt, unsigned n_grp)
 {
-    if (tail == 0) return 1;
-    const unsigned most = std::max(1u, std::min(std::min(16u, chunks), kXhMostParts / tail));
-    const unsigned forced = opt_u(O_MMQXH_SPLIT, 0);
-    if (forced) return std::min(forced, most);
-    unsigned split = 1;
-    double best = 0.0;
-    for (unsigned k = 1; k <= most; k++) {
-        const unsigned wg = tail * k, rem = wg % 512;
-        const double rounds = wg / 512 + (rem == 0 ? 0.0 : rem <= kCUs ? 0.6 : 1.0);
-        const double cost = rounds * (chunks / (double)k + 1.5) + (k > 1 ? 0.4 + wg * 0.0012 : 0.0);
-        if (k == 1 || cost < best) { best = cost; split = k; }
-    }
-    return split;
+    const unsigned g0 = n_whole % n_grp, tile0 = g0 * (n_tt / n_grp) + std::min(g0, n_tt % n_grp);
+    return split > 1 ? ((size_t)(n_rb - n_whole / n_grp) * n_tt - tile0) * split * kWidePart : 0;
 }
-size_t xh_parts_bytes(unsigned tail, unsigned split, unsigned n_tt, unsigned n_grp)
+WidePlan wide_plan(const WideKind& kind, int fmt, unsigned in_dim, unsigned out_dim, unsigned p_rows)
 {
-    return split > 1 ? (size_t)tail * split * ((n_tt + n_grp - 1) / n_grp) * kXhPart : 0;
-}
-XhPlan xh_plan(int fmt, unsigned in_dim, unsigned out_dim, unsigned p_rows)
-{
-    XhPlan p{};
     const unsigned n_tt = (p_rows + 31) / 32, n_rb = (out_dim + 127) / 128;
-    if (xh_format(fmt)) {
-        p.n_grp = std::min(std::max(1u, n_tt / 2), std::max((n_tt + 3) / 4, opt_u(O_MMQXH_GROUPS, 0)));
-        p.split = xh_split(n_rb * p.n_grp % 512, in_dim / 256);
-    } else {
-        const XhGroups g = x8_groups(in_dim, out_dim, p_rows);
-        p.n_grp = g.n_grp;
-        p.split = g.split;
+    WidePlan p{};
+    double best = 0.0;
+    for (unsigned size = kind.most; size >= 1; size--) {
+        const unsigned n_grp = wide_groups(kind, n_tt, size);
+        double price;
+        const unsigned split = wide_split(kind, n_rb * n_grp, n_tt, n_grp, in_dim / 256, &price);
+        if (p.n_grp == 0 || price < best) { p.n_grp = n_grp; p.split = split; best = price; }
     }
     p.n_unit = n_rb * p.n_grp;
-    p.n_whole = p.n_unit / 512 * 512;
-    p.image = (xh_image_bytes(fmt, in_dim, p_rows) + 255) & ~(size_t)255;
-    p.parts = xh_parts_bytes(p.n_unit - p.n_whole, p.split, n_tt, p.n_grp);
+    p.n_whole = p.n_unit / kind.slots * kind.slots;
+    p.image = (wide_image_bytes(fmt, in_dim, p_rows) + 255) & ~(size_t)255;
+    p.parts = wide_parts_bytes(n_rb, p.n_whole, p.split, n_tt, p.n_grp);
     return p;
 }
-// The most bytes of partial tiles that any number of weight rows leaves behind whole rounds of n_grp token groups (the size query does
-// not know the matrix): the remainders of the units by 512 are the multiples of the power of two in n_grp.  At most 64 MiB.
-size_t xh_most_parts_bytes(int fmt, unsigned in_dim, unsigned p_rows)
+// The most bytes of partial tiles that any number of weight rows leaves behind whole rounds (the size query does not know the matrix)
+size_t wide_most_parts_bytes(const WideKind& kind, unsigned in_dim, unsigned p_rows)
 {
-    const unsigned n_tt = (p_rows + 31) / 32, least = (n_tt + 3) / 4, most_grp = xh_format(fmt) ? std::max(1u, n_tt / 2) : n_tt;
-    const unsigned forced = opt_u(O_MMQXH_GROUPS, 0);
+    const unsigned n_tt = (p_rows + 31) / 32;
     size_t most = 0;
-    for (unsigned size = 4; size >= 1; size--) {
-        const unsigned n_grp = forced ? std::min(most_grp, std::max(forced, least)) : (n_tt + size - 1) / size;
-        const unsigned step = std::min(512u, n_grp & (0u - n_grp));
-        double price;
-        for (unsigned tail = step; tail < 512; tail += step)
-            most = std::max(most, xh_parts_bytes(tail, xh_format(fmt) ? xh_split(tail, in_dim / 256) : x8_split(tail, n_tt, n_grp, in_dim / 256, &price), n_tt, n_grp));
-        if (xh_format(fmt)) break;
+    for (unsigned size = kind.most; size >= 1; size--) {
+        const unsigned n_grp = wide_groups(kind, n_tt, size);
+        for (unsigned n_rb = 1; n_rb <= kind.slots; n_rb++) {            // the remainders repeat
+            const unsigned units = n_rb * n_grp;
+            double price;
+            most = std::max(most, wide_parts_bytes(n_rb, units / kind.slots * kind.slots, wide_split(kind, units, n_tt, n_grp, in_dim / 256, &price), n_tt, n_grp));
+        }
     }
     return most;
 }
@@ -2017,8 +2027,14 @@ size_t rein_matmul_scratch_bytes(int fmt, unsigned in_dim, unsigned n_rows)
     if (!rein_block_size(fmt) || in_dim == 0 || in_dim % 32 != 0 || n_rows == 0) return 0;
     const size_t xq = ((size_t)n_rows * (in_dim / 32) * 40 + 255) & ~(size_t)255;
     size_t behind = rein_matmul_path(fmt, n_rows) == 2 ? rein_mmq_workspace_bytes(fmt, in_dim, n_rows) : 0;
-    if (rein_matmul_path(fmt, n_rows) == 2 && xh_shape(fmt, in_dim, n_rows))
-        behind = std::max(behind, ((xh_image_bytes(fmt, in_dim, n_rows) + 255) & ~(size_t)255) + xh_most_parts_bytes(fmt, in_dim, n_rows));
+    if (rein_matmul_path(fmt, n_rows) == 2 && opt_u(O_MMQXH, 1) != 0 && in_dim % 256 == 0) {
+        const size_t image = (wide_image_bytes(fmt, in_dim, n_rows) + 255) & ~(size_t)255;
+        if (!wide_k_quant(fmt)) behind = std::max(behind, image + wide_most_parts_bytes(kWideInt8, in_dim, n_rows));
+        else {
+            if (wide_exact_shape(fmt, in_dim, n_rows)) behind = std::max(behind, image + wide_most_parts_bytes(wide_exact(fmt), in_dim, n_rows));
+            if (wide_few_shape(fmt, in_dim, n_rows)) behind = std::max(behind, image + wide_most_parts_bytes(kWideFew, in_dim, n_rows));
+        }
+    }
     return xq + behind;
 }
 
@@ -2031,24 +2047,23 @@ int rein_matmul_ws(int fmt, const void* w, const float* x, float* y, unsigned in
     const size_t xq = ((size_t)n_rows * (in_dim / 32) * 40 + 255) & ~(size_t)255;
     if (scratch_bytes < (size_t)n_rows * (in_dim / 32) * 40)
         return fail(REIN_E_BAD_SHAPE, "rein_matmul_ws: scratch smaller than the quantized activations");
-    if (n_rows <= 65535 && xh_take(fmt, in_dim, out_dim, n_rows)) {
-        const XhPlan p = xh_plan(fmt, in_dim, out_dim, n_rows);
+    if (const WideKind* const kind = n_rows <= 65535 ? wide_kind(fmt, in_dim, out_dim, n_rows) : nullptr) {
+        const WidePlan p = wide_plan(*kind, fmt, in_dim, out_dim, n_rows);
         char* const img = static_cast<char*>(scratch) + xq;
         char* const parts = img + p.image;
-        const unsigned tail = p.n_unit - p.n_whole, with_xsum = xh_has_min(fmt);
+        const unsigned tail = p.n_unit - p.n_whole, with_xsum = wide_has_min(fmt);
         const unsigned long long grid = p.n_whole + 8ull * (((unsigned long long)tail * p.split + 7) / 8);
         if (scratch_bytes >= xq + p.image + p.parts && grid <= 0x7FFFFFFFull && in_dim / 256 <= 65535) {
             if (int rc = check_ptr("rein_matmul_ws", x, 4, "x")) return rc;
             if (int rc = check_ptr("rein_matmul_ws", w, 16, "w")) return rc;
             if (int rc = check_ptr("rein_matmul_ws", y, 4, "y")) return rc;
-            const bool k_quant = xh_format(fmt);
             void* pa[] = {(void*)&x, (void*)&img, (void*)&scratch, (void*)&in_dim, (void*)&n_rows, (void*)&with_xsum};          // rein_x8_quantize: the first five
-            if (int rc = launch(k_quant ? "rein_xh_quantize" : "rein_x8_quantize", (n_rows + 31) / 32, in_dim / 256, 1, 256, 0, s, pa)) return rc;
+            if (int rc = launch(KName("rein_", kind->tag, "_quantize"), (n_rows + 31) / 32, in_dim / 256, 1, 256, 0, s, pa)) return rc;
             void* a[] = {(void*)&w, (void*)&img, (void*)&y, (void*)&parts, (void*)&in_dim, (void*)&out_dim, (void*)&n_rows, (void*)&p.n_grp, (void*)&p.n_whole, (void*)&p.split};
-            if (int rc = launch(KName(k_quant ? "rein_xh_" : "rein_x8_", fmt_tag(fmt), ""), (unsigned)grid, 1, 1, 256, xh_lds_bytes(fmt), s, a)) return rc;
+            if (int rc = launch(KName("rein_", kind->tag, "_", fmt_tag(fmt)), (unsigned)grid, 1, 1, 256, wide_lds_bytes(*kind, fmt), s, a)) return rc;
             if (p.split == 1) return 0;
             void* b[] = {(void*)&parts, (void*)&y, (void*)&out_dim, (void*)&n_rows, (void*)&p.n_grp, (void*)&p.n_whole, (void*)&p.split};
-            return launch(k_quant ? "rein_xh_sum" : "rein_x8_sum", tail, 16, 1, 256, 0, s, b);
+            return launch(KName("rein_", kind->tag, "_sum"), tail, 16, 1, 256, 0, s, b);
         }
     }
     // nothing behind the activations that a workspace launch could use: the plain dispatch

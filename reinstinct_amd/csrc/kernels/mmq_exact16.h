@@ -15,14 +15,17 @@
 // sums that the int8 tile makes in fp32, fewer of them.  The minimum term of Q4_K and Q5_K is the int8 tile's: bf16 instructions on
 // the three-way bf16 split of xsum (24 bits) against the integer minimums, scaled by -dmin.
 //
-// A wavefront owns 32 weight rows x 32 NT tokens, NT up to 4 (the unpack of a weight is shared by NT tiles), a workgroup of
-// four 128 rows x 32 NT tokens; two workgroups per CU.
+// A wavefront owns 32 weight rows x 32 NT tokens (the unpack of a weight is shared by NT tiles), a workgroup of four 128 rows x
+// 32 NT tokens: NT two to four, two workgroups per CU (rein_xh_*), or one and two, three per CU (rein_xf_*: one tile leaves
+// registers and LDS for the third, which fills the waits of the others' short steps; Q4_K 64 x 5120 -> 17408 45 -> 40 us).
 //
-// Bound: matrix unit (2 / 4 fp16 instructions of 32 cycles per tile and sub-block, Q4_K and Q5_K / Q6_K) plus the 16
-// multiply-adds and the share of the unpack, which issue between them.  Whole calls of rein_matmul_ws against the launches of
-// rein_mmq_xq8_ws (fp6 for Q4_K, else int8), weights of several matrices in turn, us: 2048 x 5120 -> 17408 Q4_K / Q5_K / Q6_K 580 /
-// 723 / 1130 -> 555 / 652 / 753 (102 / 120 / 138 ns per tile and sub-block and SIMD); 512 x 5120 -> 17408 152 / 194 / 311 -> 142 /
-// 172 / 200; 512 x 17408 -> 5120 172 / 250 / 451 -> 160 / 193 / 222; Q6_K 777 x 17408 -> 5120 526 -> 369.
+// Bound: the same instructions alone, on every CU, take 65 ns (Q4_K) and 90 (Q6_K) per tile and sub-block and SIMD -- two / four matrix
+// instructions, the 16 multiply-adds and a quarter of the unpack, the two units overlapping but for issue, the clock at 1.8-2.0 of
+// 2.4 GHz under this load; the kernel without its transfers 75 and 108, with them 97 and 129.  Whole calls of rein_matmul_ws against
+// the launches of rein_mmq_xq8_ws (fp6 for Q4_K, else int8), weights of several matrices in turn, us, Q4_K / Q5_K / Q6_K: 2048 x 5120 ->
+// 17408 633 / 809 / 1268 -> 588 / 645 / 786; 512 x 5120 -> 17408 169 / 203 / 347 -> 149 / 160 / 198; 512 x 17408 -> 5120 195 / 271 /
+// 494 -> 163 / 176 / 214; Q6_K 777 x
+// 17408 -> 5120 569 -> 363; 45 x 17408 -> 5120 (one group of two tiles) Q5_K 42.1 -> 36.3.
 //
 // Replaces, from 33 rows, kernels/mmq_gemm_{q4k,q5k,q6k}_repacked.cpp of the reference behind rein_matmul_ws.
 #pragma once
@@ -163,8 +166,13 @@ __device__ __forceinline__ XhGroup rein_xh_group(unsigned p_rows, unsigned n_grp
     return XhGroup{g * base + min(g, more), base + (g < more ? 1u : 0u)};
 }
 
-// floats of the partial tiles of one range: of the largest group of the launch
-__device__ __forceinline__ unsigned rein_xh_part(unsigned p_rows, unsigned n_grp) { return (((p_rows + 31u) >> 5) + n_grp - 1u) / n_grp * 4096u; }
+// Partial tiles of unit (rb, group g) of the ones that are cut: ranges one after the other, the tiles of a range together, units in
+// order from the first that is cut.
+__device__ __forceinline__ size_t rein_xh_part(unsigned p_rows, unsigned n_grp, unsigned n_whole, unsigned rb, const XhGroup& g, unsigned split)
+{
+    const unsigned n_tt = (p_rows + 31u) >> 5, rb0 = n_whole / n_grp, tile0 = rein_xh_group(p_rows, n_grp, n_whole - rb0 * n_grp).tile;
+    return ((size_t)(rb - rb0) * n_tt + g.tile - tile0) * split * 4096u;
+}
 
 // ---- weight operands ------------------------------------------------------------------
 // A nibble or-ed into the mantissa of 1024 (low nibble) or 64 (high nibble, which sits four bits up) is 1024 + n or 64 + n;
@@ -282,27 +290,28 @@ __device__ __forceinline__ void rein_xh_pin(float (&s)[16])
 
 // ---- the tile -------------------------------------------------------------------------
 // LDS of one workgroup:
-//   acts  2 x 4 x 4352     records of two consecutive sub-block pairs
+//   acts  2 x MOST x 4352  records of two consecutive sub-block pairs
 //   ring  4 x 2 x 2048     per wavefront: two slots of 4 sub-blocks x 32 rows x 16 B
 //   small 4 x 3584         per wavefront: extra bits of a superblock [row][sub-block] in granules of 16 bytes, rotated; (sc, m) or
 //                          both group scales [row][sub-block], in two bytes each or (padded rows) four; the scale words of two
 //                          superblocks [row]
-//   xs    4 x 2048             xsum operands of a superblock (formats with minimums)
-template <int FMT> constexpr unsigned rein_xh_lds_bytes()
+//   xs    MOST x 2048          xsum operands of a superblock (formats with minimums)
+// MOST: tiles of the launch's largest group, 4 or (rein_xf_*) 2.
+template <int FMT, unsigned MOST> constexpr unsigned rein_xh_lds_bytes()
 {
-    return 8u * REIN_XH_REC + 4u * 2u * 2048u + 4u * 3584u + (XhWeights<FMT>::kHasMin ? 4u * REIN_XH_XS : 0u);
+    return 2u * MOST * REIN_XH_REC + 4u * 2u * 2048u + 4u * 3584u + (XhWeights<FMT>::kHasMin ? MOST * REIN_XH_XS : 0u);
 }
 
 // Superblocks [c0, c1) of rows 128 rb .. and the NT token tiles from `tile` on, into acc.  One barrier per sub-block
 // pair: at its top everything in flight has landed (it was issued a whole pair earlier: 8 NT or 16 NT matrix instructions per
 // wavefront), behind it the next pair's transfers go out.
-template <int FMT, int NT>
+template <int FMT, int NT, unsigned MOST>
 __device__ __forceinline__ void rein_xh_acc(const uint8_t* __restrict__ w, const uint8_t* __restrict__ img, unsigned in_dim, unsigned out_dim,
                                             unsigned n_tt, unsigned rb, unsigned tile, unsigned c0, unsigned c1, unsigned char* const raw, float (&acc)[NT][16])
 {
     using W = XhWeights<FMT>;
     typedef __attribute__((address_space(3))) const void* lptr_t;
-    constexpr unsigned kRing = 8u * REIN_XH_REC, kSmall = kRing + 4u * 4096u, kXs = kSmall + 4u * 3584u;
+    constexpr unsigned kRing = 2u * MOST * REIN_XH_REC, kSmall = kRing + 4u * 4096u, kXs = kSmall + 4u * 3584u;
     const unsigned lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), j = lane & 31u, h = lane >> 5;
     const unsigned n_sub = in_dim >> 5;
     const Fmt<FMT> fmt(w, n_sub, out_dim);
@@ -341,7 +350,7 @@ __device__ __forceinline__ void rein_xh_acc(const uint8_t* __restrict__ w, const
 
     auto issue_acts = [&](unsigned pair) {
         const uint8_t* src = img + ((size_t)pair * n_tt + tile) * REIN_XH_REC;
-        const unsigned buf = lds0 + (pair & 1u) * (4u * REIN_XH_REC);
+        const unsigned buf = lds0 + (pair & 1u) * (MOST * REIN_XH_REC);
 #pragma unroll
         for (unsigned t = 0; t < (unsigned)NT; t++) {
             const unsigned off = t * REIN_XH_REC + wave * 1024u;
@@ -421,7 +430,7 @@ __device__ __forceinline__ void rein_xh_acc(const uint8_t* __restrict__ w, const
                 __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the reads above have left the buffer
                 issue_small(c + 1u);
             }
-            const unsigned char* const act = raw + (pair & 1u) * (4u * REIN_XH_REC);
+            const unsigned char* const act = raw + (pair & 1u) * (MOST * REIN_XH_REC);
 #pragma unroll
             for (unsigned q = 0; q < 2; q++) {
                 const unsigned sb = 2u * u + q, s4 = sb & 3u;
@@ -502,13 +511,14 @@ __device__ __forceinline__ void rein_xh_acc(const uint8_t* __restrict__ w, const
     REIN_WAIT_VMCNT(0);
 }
 
-template <int FMT> struct XhTile {
-    static constexpr bool kOne = false;              // groups of one tile: the stages of a tile on its own are not built
+// kMost / kLeast: tiles of the largest and of the smallest group that the launch may have; kSlots: resident workgroups
+template <int FMT, unsigned MOST> struct XhTile {
+    static constexpr unsigned kMost = MOST, kLeast = MOST == 2u ? 1u : 2u, kSlots = MOST == 2u ? 768u : 512u;
     template <int NT>
     static __device__ __forceinline__ void run(const uint8_t* __restrict__ w, const uint8_t* __restrict__ img, unsigned in_dim, unsigned out_dim, unsigned n_tt,
                                                unsigned rb, unsigned tile, unsigned c0, unsigned c1, unsigned char* const raw, float (&acc)[NT][16])
     {
-        rein_xh_acc<FMT, NT>(w, img, in_dim, out_dim, n_tt, rb, tile, c0, c1, raw, acc);
+        rein_xh_acc<FMT, NT, MOST>(w, img, in_dim, out_dim, n_tt, rb, tile, c0, c1, raw, acc);
     }
 };
 
@@ -550,8 +560,8 @@ __device__ __forceinline__ void rein_xh_piece(const uint8_t* __restrict__ w, con
     }
 }
 
-// Units u = (128-row block u / n_grp, token group u % n_grp).  The first n_whole (whole rounds of 512 workgroups, two per
-// CU) are one workgroup each; the others are cut into `split` ranges of superblocks, a workgroup each, whose partial tiles
+// Units u = (128-row block u / n_grp, token group u % n_grp).  The first n_whole (whole rounds of resident
+// workgroups) are one workgroup each; the others are cut into `split` ranges of superblocks, a workgroup each, whose partial tiles
 // rein_xh_sum_body adds in range order.  Workgroup i runs on XCD i % 8: neighbouring units and ranges go to one XCD, so the
 // token groups of a row block meet its weights in one L2.  Grid: n_whole + 8 ceil((units - n_whole) split / 8).
 __device__ __forceinline__ unsigned rein_xh_deal(unsigned i, unsigned n)
@@ -565,25 +575,29 @@ __device__ __forceinline__ void rein_xh_dense(const uint8_t* __restrict__ w, con
 {
     extern __shared__ __attribute__((aligned(16))) unsigned char rein_xh_lds[];
     const unsigned n_unit = ((out_dim + 127u) / 128u) * n_grp, n_chunk = in_dim >> 8;
-    unsigned u, c0 = 0u, c1 = n_chunk;
-    float* part = nullptr;
+    unsigned u, c0 = 0u, c1 = n_chunk, k = 0u;
     if (blockIdx.x < n_whole) {
-        u = (blockIdx.x & ~511u) + rein_xh_deal(blockIdx.x & 511u, 512u);
+        u = blockIdx.x / Tile::kSlots * Tile::kSlots + rein_xh_deal(blockIdx.x % Tile::kSlots, Tile::kSlots);
     } else {
         const unsigned n_seg = (n_unit - n_whole) * split, seg = rein_xh_deal(blockIdx.x - n_whole, n_seg);
         if (seg >= n_seg) return;
-        const unsigned tu = seg / split, k = seg - tu * split;
+        const unsigned tu = seg / split;
+        k = seg - tu * split;
         u = n_whole + tu;
         c0 = n_chunk * k / split; c1 = n_chunk * (k + 1u) / split;       // split <= n_chunk: no range is empty
-        if (split > 1u) part = parts + (size_t)seg * rein_xh_part(p_rows, n_grp);
     }
     if (u >= n_unit) return;
     const unsigned rb = u / n_grp;
     const XhGroup g = rein_xh_group(p_rows, n_grp, u - rb * n_grp);
-    if (g.n == 4u) rein_xh_piece<Tile, 4>(w, img, y, part, in_dim, out_dim, p_rows, rb, g.tile, c0, c1, rein_xh_lds);
-    else if (g.n == 3u) rein_xh_piece<Tile, 3>(w, img, y, part, in_dim, out_dim, p_rows, rb, g.tile, c0, c1, rein_xh_lds);
-    else if (g.n == 2u) rein_xh_piece<Tile, 2>(w, img, y, part, in_dim, out_dim, p_rows, rb, g.tile, c0, c1, rein_xh_lds);
-    else if constexpr (Tile::kOne) { if (g.n == 1u) rein_xh_piece<Tile, 1>(w, img, y, part, in_dim, out_dim, p_rows, rb, g.tile, c0, c1, rein_xh_lds); }
+    float* const part = u >= n_whole && split > 1u ? parts + rein_xh_part(p_rows, n_grp, n_whole, rb, g, split) + (size_t)k * g.n * 4096u : nullptr;
+    if (g.n == 2u) { rein_xh_piece<Tile, 2>(w, img, y, part, in_dim, out_dim, p_rows, rb, g.tile, c0, c1, rein_xh_lds); return; }
+    if constexpr (Tile::kMost == 4u) {
+        if (g.n == 4u) rein_xh_piece<Tile, 4>(w, img, y, part, in_dim, out_dim, p_rows, rb, g.tile, c0, c1, rein_xh_lds);
+        else if (g.n == 3u) rein_xh_piece<Tile, 3>(w, img, y, part, in_dim, out_dim, p_rows, rb, g.tile, c0, c1, rein_xh_lds);
+    }
+    if constexpr (Tile::kLeast == 1u) {
+        if (g.n == 1u) rein_xh_piece<Tile, 1>(w, img, y, part, in_dim, out_dim, p_rows, rb, g.tile, c0, c1, rein_xh_lds);
+    }
 }
 
 // y of the split units.  Grid (units - n_whole, 16): blockIdx.y = 4 t + v / 4, 256 threads as in the GEMM.
@@ -595,10 +609,10 @@ __device__ __forceinline__ void rein_xh_sum_body(const float* __restrict__ parts
     const unsigned tok = (grp.tile + t) * 32u + j, row = rb * 128u + wave * 32u + 8u * g + 4u * h;
     if (t >= grp.n || tok >= p_rows) return;
     float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    const float4* src = reinterpret_cast<const float4*>(parts + (size_t)blockIdx.x * split * rein_xh_part(p_rows, n_grp)) + blockIdx.y * 256u + threadIdx.x;
+    const float4* src = reinterpret_cast<const float4*>(parts + rein_xh_part(p_rows, n_grp, n_whole, rb, grp, split)) + blockIdx.y * 256u + threadIdx.x;
 #pragma unroll 4
     for (unsigned k = 0; k < split; k++) {
-        const float4 p = src[(size_t)k * (rein_xh_part(p_rows, n_grp) / 4u)];
+        const float4 p = src[(size_t)k * (grp.n * 1024u)];
         s[0] += p.x; s[1] += p.y; s[2] += p.z; s[3] += p.w;
     }
     float* o = y + (size_t)tok * out_dim + row;

@@ -218,7 +218,7 @@ __device__ __forceinline__ void rein_x8_acc(const uint8_t* __restrict__ w, const
 }
 
 template <int FMT> struct X8Tile {
-    static constexpr bool kOne = true;
+    static constexpr unsigned kMost = 4, kLeast = 1, kSlots = 512;
     template <int NT>
     static __device__ __forceinline__ void run(const uint8_t* __restrict__ w, const uint8_t* __restrict__ img, unsigned in_dim, unsigned out_dim, unsigned n_tt,
                                                unsigned rb, unsigned tile, unsigned c0, unsigned c1, unsigned char* const raw, float (&acc)[NT][16])
