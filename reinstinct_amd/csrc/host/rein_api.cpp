@@ -552,10 +552,16 @@ bool mvql_wide32(int fmt)
 {
     return opt_u(O_QUAD_WIDE32, fmt == REIN_TYPE_Q6_K ? 0u : 1u) != 0;
 }
+size_t quad_lds_bytes(unsigned t, unsigned n_stage, unsigned wpb, unsigned parts)
+{
+    const unsigned stride = n_stage + ((20u - (n_stage & 15u)) & 15u);
+    return (size_t)t * stride * 40 + (size_t)wpb * parts * 76 * 16;
+}
+unsigned quad_raw_parts(int fmt) { return fmt == REIN_TYPE_Q8_0 ? 3 : 2; }            // 16-byte parts of Fmt<FMT>::Raw
 QuadLdsGeometry mvql_geometry(int fmt, unsigned in_dim, unsigned out_dim, unsigned n_rows)
 {
     const unsigned n_sub = in_dim / 32, t = n_rows <= 4 ? 4 : n_rows <= 8 ? 8 : n_rows <= 16 ? 16 : 32;
-    const unsigned parts = fmt == REIN_TYPE_Q8_0 ? 3 : 2;               // 16-byte parts of Fmt<FMT>::Raw
+    const unsigned parts = quad_raw_parts(fmt);
     const unsigned groups = (out_dim + 3) / 4;
     QuadLdsGeometry g;
     g.slices = 1;
@@ -586,10 +592,7 @@ QuadLdsGeometry mvql_geometry(int fmt, unsigned in_dim, unsigned out_dim, unsign
         g.wpb = gpb * g.slices;
         g.grid = (groups + gpb - 1) / gpb;
     }
-    const auto bytes = [&](unsigned n_stage) {
-        const unsigned stride = n_stage + ((20u - (n_stage & 15u)) & 15u);
-        return (size_t)t * stride * 40 + (size_t)g.wpb * parts * 76 * 16;
-    };
+    const auto bytes = [&](unsigned n_stage) { return quad_lds_bytes(t, n_stage, g.wpb, parts); };
     g.phase_sub = n_sub;
     g.lds = bytes(n_sub);
     if (g.lds > kLdsPerCu) {
@@ -685,25 +688,28 @@ KName mvql_name(int fmt, unsigned in_dim, unsigned out_dim, unsigned n_rows)
     return KName("rein_mvql_", fmt_tag(fmt), n_rows <= 4 ? "_t4" : n_rows <= 8 ? "_t8" : "_t16",
                  load_tag(fmt, in_dim, rein_repacked_len(fmt, in_dim, out_dim), n_rows));
 }
-int launch_quad_lds(int fmt, const void* w, const void* xq, float* y, unsigned in_dim, unsigned out_dim,
-                    unsigned n_rows, rein_stream_t s)
+// Trips of weights in flight per wavefront where wavefronts stride over row groups or own a whole one (no slices,
+// no phases): two for the formats with little arithmetic per sub-block at 3-4 rows -- two register sets taking
+// turns -- (us, 5120 -> 34816 / 5120 -> 17408 / 3584 -> 18944 at 4 rows, one -> two: Q4_K 28.3 -> 26.0, 18.8 -> 17.3,
+// 14.2 -> 13.0; Q4_0 27.4 -> 23.7, 18.9 -> 16.1, 14.4 -> 12.2; IQ3_S 27.8 -> 24.2, 18.7 -> 16.2; Q8_0 40.1 -> 37.5,
+// 25.8 -> 23.0; Q5_K 33.0 -> 32.3, 21.2 -> 20.3) and for Q8_0 / Q4_0 / IQ3_S at 5-8 rows against 16384 rows and more
+// (1.05-1.07 x); Q6_K and IQ4_XS lose 3-10 % to the registers it costs, Q4_K and Q5_K at 8 rows 1-4 %.
+unsigned quad_lds_depth(int fmt, unsigned out_dim, unsigned n_rows, bool strided)
 {
-    const QuadLdsGeometry g = mvql_geometry(fmt, in_dim, out_dim, n_rows);
-    // Trips of weights in flight per wavefront where wavefronts stride over row groups or own a whole one (no slices,
-    // no phases): two for the formats with little arithmetic per sub-block at 3-4 rows -- two register sets taking
-    // turns -- (us, 5120 -> 34816 / 5120 -> 17408 / 3584 -> 18944 at 4 rows, one -> two: Q4_K 28.3 -> 26.0, 18.8 -> 17.3,
-    // 14.2 -> 13.0; Q4_0 27.4 -> 23.7, 18.9 -> 16.1, 14.4 -> 12.2; IQ3_S 27.8 -> 24.2, 18.7 -> 16.2; Q8_0 40.1 -> 37.5,
-    // 25.8 -> 23.0; Q5_K 33.0 -> 32.3, 21.2 -> 20.3) and for Q8_0 / Q4_0 / IQ3_S at 5-8 rows against 16384 rows and more
-    // (1.05-1.07 x); Q6_K and IQ4_XS lose 3-10 % to the registers it costs, Q4_K and Q5_K at 8 rows 1-4 %.
     const bool light = fmt == REIN_TYPE_Q4_K || fmt == REIN_TYPE_Q4_0 || fmt == REIN_TYPE_Q8_0 || fmt == REIN_TYPE_IQ3_S || fmt == REIN_TYPE_Q5_K;
     // With slices or phases (narrow matrices) the second register set gains only where a wavefront has the CU nearly to
     // itself: 5120 -> 1024 1.05-1.20 x for every format at 4 and 8 rows, 0.86-1.05 from 4096 rows on.
-    const bool strided = g.slices == 1 && g.phase_sub >= in_dim / 32;
     unsigned depth = 1;
     if (!strided) depth = out_dim <= 1536 ? 2 : 1;
     else if (n_rows <= 4 && light) depth = 2;
     else if (n_rows <= 8 && out_dim >= 16384 && (fmt == REIN_TYPE_Q8_0 || fmt == REIN_TYPE_Q4_0 || fmt == REIN_TYPE_IQ3_S)) depth = 2;
-    depth = opt_u(O_QUAD_DEPTH, depth);
+    return opt_u(O_QUAD_DEPTH, depth);
+}
+int launch_quad_lds(int fmt, const void* w, const void* xq, float* y, unsigned in_dim, unsigned out_dim,
+                    unsigned n_rows, rein_stream_t s)
+{
+    const QuadLdsGeometry g = mvql_geometry(fmt, in_dim, out_dim, n_rows);
+    const unsigned depth = quad_lds_depth(fmt, out_dim, n_rows, g.slices == 1 && g.phase_sub >= in_dim / 32);
     void* args[] = {(void*)&w, (void*)&xq, (void*)&y, (void*)&in_dim, (void*)&out_dim, (void*)&n_rows, (void*)&g.phase_sub, (void*)&g.slices,
                     (void*)&depth};
     return launch(mvql_name(fmt, in_dim, out_dim, n_rows), g.grid, 1, 1, g.wpb * 64, (unsigned)g.lds, s, args);
@@ -753,6 +759,110 @@ KName matvec_kernel_name(int fmt, unsigned in_dim, unsigned out_dim, unsigned n_
     }
     default: return mv_name(fmt, in_dim, out_dim, n_rows);
     }
+}
+
+// Launches of several matrices whose workgroups stage the activation rows in LDS (kernels/matvec_multi.hip): wpb wavefronts, rows[i] of
+// matrix i to a workgroup.  wpb == 0: none.
+struct MultiLds { unsigned wpb, rows[4], rows_per_wave; size_t bytes; };
+unsigned multi_blocks(unsigned n_mat, const unsigned* out_dims, unsigned rows)
+{
+    unsigned n = 0;
+    for (unsigned i = 0; i < n_mat; i++) n += (out_dims[i] + rows - 1) / rows;
+    return n;
+}
+
+// Two to four activation rows on the LDS-staged dot4 kernel, whose bits are those of rein_mv_multi_*.  Geometry as mvl_geometry's, over
+// the rows of all matrices.  Where it is taken, from 26 shapes in two to six formats (us, rein_mv_multi_* / this):
+//   3-4 rows  matrices of at most twice the contraction together (Q, K, V), every format: 1.00-1.52 x (4 rows: 2048 -> 2048 + 2 x 512
+//             IQ3_S 6.0 / 4.2, 4096 -> 4096 + 2 x 1024 Q5_K with Q6_K 11.8 / 9.1, Q8_0 9.5 / 8.0, 5120 -> 5120 + 2 x 1024 Q4_K with Q6_K
+//             13.1 / 11.6, Q8_0 13.8 / 9.9; least 4096 -> 4096 + 2 x 1024 Q4_K with Q6_K, level).  Beyond that two matrices (gate, up) from
+//             eight million weights in Q5_K, Q6_K and Q8_0 (2048 -> 2 x 8192 10.6 / 9.7, 14.3 / 11.4, 11.3 / 10.5; least 0.99) and in Q4_K,
+//             Q4_0, IQ3_S from a contraction of 3072 (3072 -> 2 x 8192 Q4_K 14.3 / 11.8, 1536 -> 2 x 5120 6.4 / 6.5), not in IQ4_XS
+//             (2560 -> 2 x 8960 14.5 / 16.6), nor three (4096 -> 3 x 4096 Q4_K with Q6_K 14.3 / 14.8).
+//   2 rows    at most 8192 rows in all and at most one and a half times the contraction (5120 -> 5120 + 2 x 1024 9.7 / 9.2, 2560 -> 2560 +
+//             2 x 640 Q5_K with Q6_K 6.1 / 5.4; Q8_0 and Q4_0 not from 4097 to 5120 rows of 3584 and more: 4096 -> 4096 + 2 x 512 6.9 /
+//             7.2); contractions of 8192 and more (8192 -> 2 x 24576 Q4_K 50.8 / 42.2, Q8_0 83.1 / 71.8); Q4_K and Q8_0 from 6144 against
+//             four times that (6144 -> 2 x 18432 26.4 / 24.3, 41.8 / 39.1, but Q6_K 37.6 / 39.3).  Between, level or behind (2048 -> 2 x
+//             8192 Q4_K 6.7 / 7.8, 4096 -> 2 x 14336 Q6_K 22.0 / 24.5).
+MultiLds multi_dot4_lds(unsigned n_mat, unsigned in_dim, const unsigned* out_dims, unsigned n_rows, int lead)
+{
+    MultiLds p{};
+    const unsigned forced = opt_u(O_MV_ROWS, 0);
+    if (n_mat < 2 || n_rows < 2 || mvl_lds_bytes(in_dim, n_rows) > kLdsPerCu || opt_is_set(O_MV_WPB)) return p;
+    const unsigned long long total = multi_blocks(n_mat, out_dims, 1);
+    if (opt_is_set(O_MV_LDS)) {
+        if (!opt_u(O_MV_LDS, 0) || forced > 2) return p;
+    } else {
+        if (opt_is_set(O_SKINNY_FROM) || opt_is_set(O_QUAD_FROM) || opt_is_set(O_MV_ROWS)) return p;
+        const bool heavy = lead == REIN_TYPE_Q5_K || lead == REIN_TYPE_Q6_K || lead == REIN_TYPE_Q8_0;
+        if (n_rows >= 3) {
+            if (total > 2ull * in_dim && !(n_mat == 2 && (heavy ? total * in_dim >= (8ull << 20) : in_dim >= 3072 && lead != REIN_TYPE_IQ4_XS))) return p;
+        } else {
+            const bool light = lead == REIN_TYPE_Q8_0 || lead == REIN_TYPE_Q4_0;
+            const bool narrow = total <= 8192 && 2 * total <= 3ull * in_dim && !(light && in_dim >= 3584 && total > 4096 && total <= 5120);
+            const bool tall = in_dim >= 6144 && total >= 4ull * in_dim && (lead == REIN_TYPE_Q4_K || lead == REIN_TYPE_Q8_0);
+            if (!narrow && !tall && in_dim < 8192) return p;
+        }
+    }
+    const unsigned copies = (unsigned)std::min<size_t>(4, kLdsPerCu / mvl_lds_bytes(in_dim, n_rows));
+    unsigned rr = forced ? forced : 1, per = 0;
+    for (; rr <= 2 && !p.wpb; rr *= 2) {
+        const unsigned c = (multi_blocks(n_mat, out_dims, rr) + kCUs * 16 - 1) / (kCUs * 16);
+        if (c > std::min(2u, copies) && !(forced && rr == forced)) continue;
+        p.rows_per_wave = rr;
+        for (p.wpb = 1; p.wpb < 16 && multi_blocks(n_mat, out_dims, rr * p.wpb) > kCUs * c; p.wpb++) {}
+        per = rr * p.wpb;
+    }
+    if (!p.wpb) {                                         // persistent
+        p.rows_per_wave = 2;
+        p.wpb = n_rows <= 2 ? 4 : 8;
+        while (copies * p.wpb < 16) p.wpb *= 2;
+        const unsigned wave = 2 * p.wpb;
+        for (per = (unsigned)(total / (kCUs * copies) / wave) * wave + wave; multi_blocks(n_mat, out_dims, per) > kCUs * copies; per += wave) {}
+    }
+    for (unsigned& r : p.rows) r = per;
+    p.bytes = mvl_lds_bytes(in_dim, n_rows);
+    return p;
+}
+
+// Two matrices of an FFN's size on the 4x4x4 kernel with the rows in LDS, each in as many slices as its launch alone (the order of a
+// row's sums): the activations are staged once, a wavefront's weights come in without a break, and 28 to 63 row groups to a CU deal
+// better than half as many (us at 4 rows, two launches / this: 4096 -> 2 x 14336 Q4_K 20.1 / 17.4, Q5_K 23.8 / 20.6, Q6_K 30.2 / 26.3,
+// Q8_0 29.6 / 26.6; 5120 -> 2 x 17408 30.2 / 22.6, 33.8 / 26.9, 42.8 / 33.9, 41.2 / 31.3; 7168 -> 2 x 24576 42.3 / 37.5, 47.9 / 44.7, 59.0 / 58.2,
+// 60.7 / 57.5; Q4_K with Q6_K 5120 -> 2 x 17408 36.5 / 33.4, but three matrices 51.3 / 53.6).  One workgroup per CU, sixteen wavefronts
+// at most; two of ten for Q8_0 from a contraction of 8192 (8192 -> 2 x 24576 85.5 on two launches, 87.7 / 85.5 with one / two).
+MultiLds multi_quad_lds(unsigned n_mat, const int* fmts, unsigned in_dim, const unsigned* out_dims, unsigned n_rows)
+{
+    MultiLds p{};
+    if (n_mat != 2) return p;
+    unsigned parts = 0;
+    QuadLdsGeometry g[2];
+    for (unsigned i = 0; i < 2; i++) {
+        if (matvec_family(fmts[i], in_dim, out_dims[i], n_rows) != MvFamily::QuadLds) return p;
+        if (std::strcmp(load_tag(fmts[i], in_dim, 1ull << 30, n_rows), "_m") != 0) return p;
+        g[i] = mvql_geometry(fmts[i], in_dim, out_dims[i], n_rows);
+        if (g[i].phase_sub < in_dim / 32) return p;
+        parts = std::max(parts, quad_raw_parts(fmts[i]));
+    }
+    p.rows_per_wave = 4;
+    if (g[0].slices > 1 || g[1].slices > 1) {
+        // sliced: workgroups as they would be alone, both matrices' alike (5120 -> 8192 and 12288, two slices and one: 21.9 / 23.6)
+        const bool alike = g[0].slices == g[1].slices && g[0].wpb == g[1].wpb;
+        if (!alike && !opt_is_set(O_QUAD_LDS)) return p;
+        p.wpb = alike ? g[0].wpb : 16;
+        for (unsigned i = 0; i < 2; i++)
+            p.rows[i] = 4 * (g[i].slices > 1 ? p.wpb / g[i].slices : p.wpb * (((out_dims[i] + 3) / 4 + kCUs * p.wpb - 1) / (kCUs * p.wpb)));
+    } else {
+        const unsigned c = parts == 3 && in_dim >= 8192 ? 2 : 1, most = c == 2 ? 10 : 16;
+        unsigned rounds = (multi_blocks(2, out_dims, 4) + kCUs * c * most - 1) / (kCUs * c * most);
+        while (multi_blocks(2, out_dims, 4 * most * rounds) > kCUs * c) rounds++;
+        for (p.wpb = 1; multi_blocks(2, out_dims, 4 * p.wpb * rounds) > kCUs * c; p.wpb++) {}
+        p.rows[0] = p.rows[1] = 4 * p.wpb * rounds;
+    }
+    p.rows[2] = p.rows[3] = p.rows[1];
+    p.bytes = quad_lds_bytes(4, in_dim / 32, p.wpb, parts);
+    if (p.bytes > kLdsPerCu) p.wpb = 0;
+    return p;
 }
 
 int launch_matvec(const char* who, int fmt, const void* w, const void* xq, float* y, unsigned in_dim,
@@ -1101,11 +1211,35 @@ int rein_matvec_multi_xq8(unsigned n_mat, const int* fmts, const void* const* ws
         if (out_dims[i] > out_dims[widest]) widest = i;
     }
     if (total > 0x3FFFFFFFull) return fail(REIN_E_TOO_LARGE, std::string(who) + ": too many rows for one launch");
-    // One matrix, or three to four rows against matrices of the size of an FFN's: the launches of the matrices one by
-    // one, whose few-row kernels (activations staged in LDS, matrix instructions) are further ahead of dot4 there than
-    // a launch costs (gate + up 5120 -> 17408 at 4 rows: 34.0 us as two launches, 38.6 as one; Q + K + V 5120 -> 5120 /
+    // One matrix, or three to four rows against matrices of the size of an FFN's: the kernels that the matrices take one by
+    // one, two of them in one launch where multi_quad_lds has one, whose few-row kernels (activations staged in LDS, matrix instructions) are further ahead of dot4 there than
+    // a launch costs (gate + up 5120 -> 17408 at 4 rows: 34.0 us as two launches, 38.6 as one of dot4; Q + K + V 5120 -> 5120 /
     // 1024 / 1024: 20.7 against 14.1, stays one launch; at 2 rows 26.9 against 25.7 and 15.4 against 10.1).
     const bool one_by_one = n_mat == 1 || (n_rows >= 3 && total * in_dim >= (64ull << 20) && !opt_is_set(O_MV_ROWS));
+    struct Mat { const void* w; float* y; unsigned out_dim; int fmt; unsigned end, slices; };
+    struct Args { Mat m[kMax]; } a{};
+    const auto table = [&](const unsigned* rows) {          // the matrices, each dealt out `rows` at a time
+        unsigned end = 0;
+        for (unsigned i = 0; i < kMax; i++) {
+            const unsigned j = std::min(i, n_mat - 1);
+            if (i < n_mat) end += (out_dims[i] + rows[i] - 1) / rows[i];
+            a.m[i] = Mat{ws[j], ys[j], out_dims[j], fmts[j], end, 0};
+        }
+        return end;
+    };
+    void* args[] = {(void*)&a, (void*)&xq, (void*)&in_dim, (void*)&n_mat, (void*)&n_rows};
+    const MultiLds lds = one_by_one ? multi_quad_lds(n_mat, fmts, in_dim, out_dims, n_rows)
+                                    : multi_dot4_lds(n_mat, in_dim, out_dims, n_rows, fmts[widest]);
+    if (lds.wpb) {
+        const unsigned grid = table(lds.rows);
+        for (unsigned i = 0; i < kMax && one_by_one; i++) {
+            const unsigned slices = mvql_geometry(a.m[i].fmt, in_dim, a.m[i].out_dim, n_rows).slices;
+            a.m[i].slices = slices | quad_lds_depth(a.m[i].fmt, a.m[i].out_dim, n_rows, slices == 1) << 16;
+        }
+        return launch(one_by_one ? KName("rein_mvql_multi_t4_m")
+                                 : KName("rein_mvl_multi_r", lds.rows_per_wave, "_b", n_rows <= 2 ? 2u : 4u, load_tag(fmts[widest], in_dim, bytes, n_rows)),
+                      grid, 1, 1, lds.wpb * 64, (unsigned)lds.bytes, s, args);
+    }
     if (one_by_one) {
         for (unsigned i = 0; i < n_mat; i++)
             if (int rc = launch_matvec(who, fmts[i], ws[i], xq, ys[i], in_dim, out_dims[i], n_rows, s)) return rc;
@@ -1124,16 +1258,8 @@ int rein_matvec_multi_xq8(unsigned n_mat, const int* fmts, const void* const* ws
         if (ri == 4 && total < 16384 && !opt_is_set(O_MV_ROWS)) ri = 2;
         r = std::min(r, ri);
     }
-    struct Mat { const void* w; float* y; unsigned out_dim; int fmt; unsigned group_end; unsigned pad; };
-    struct Args { Mat m[kMax]; } a{};
-    unsigned groups = 0;
-    for (unsigned i = 0; i < n_mat; i++) {
-        groups += (out_dims[i] + r - 1) / r;
-        a.m[i] = Mat{ws[i], ys[i], out_dims[i], fmts[i], groups, 0u};
-    }
-    for (unsigned i = n_mat; i < kMax; i++) a.m[i] = a.m[n_mat - 1];
+    const unsigned each[kMax] = {r, r, r, r}, groups = table(each);
     const unsigned wpb = pick_wpb(lead, groups, b);
-    void* args[] = {(void*)&a, (void*)&xq, (void*)&in_dim, (void*)&n_mat, (void*)&n_rows};
     return launch(KName("rein_mv_multi_r", r, "_b", b, load_tag(lead, in_dim, bytes, n_rows)), (groups + wpb - 1) / wpb, 1, 1, wpb * 64, 0, s, args);
 }
 

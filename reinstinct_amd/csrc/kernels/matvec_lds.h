@@ -30,7 +30,7 @@
 template <int FMT, int R, int B, int POL>
 __device__ __forceinline__ void rein_matvec_lds_body(const uint8_t* __restrict__ w, const BlockQ8* __restrict__ xq,
                                                      float* __restrict__ y, unsigned in_dim, unsigned out_dim,
-                                                     unsigned n_rows)
+                                                     unsigned n_rows, unsigned block, unsigned n_block)
 {
     using F = Fmt<FMT>;
     extern __shared__ uint4 rein_mvl_lds[];
@@ -40,13 +40,13 @@ __device__ __forceinline__ void rein_matvec_lds_body(const uint8_t* __restrict__
     const F fmt(w, n_sub, out_dim);
     const unsigned n_groups = (out_dim + R - 1) / R;
     const unsigned rmax = out_dim - 1, bmax = n_rows - 1;
-    const unsigned stride = gridDim.x * wpb;
+    const unsigned stride = n_block * wpb;
     uint4* qlo = rein_mvl_lds;
     uint4* qhi = rein_mvl_lds + (size_t)B * n_sub;
     float* dxs = reinterpret_cast<float*>(rein_mvl_lds + 2u * B * n_sub);
     float* xss = dxs + (size_t)B * n_sub;
 
-    unsigned g = blockIdx.x * wpb + (threadIdx.x >> 6);
+    unsigned g = block * wpb + (threadIdx.x >> 6);
     // A wavefront's trips in order: position (row group, first sub-block); the one after the last trip of a row
     // group is the first of the wavefront's next row group.  Lanes past the end of a row re-read its last
     // sub-block (loads stay unconditional) and are zeroed through dx / xsum; a position past the last row group
@@ -141,7 +141,7 @@ __device__ __forceinline__ void rein_matvec_lds_body(const uint8_t* __restrict__
 #define REIN_DEFINE_MATVEC_LDS_LD(name, FMT, R, B, POL)                                           \
     extern "C" __global__ __launch_bounds__(1024) void name(REIN_MATVEC_ARGS, unsigned int n_rows) \
     {                                                                                             \
-        rein_matvec_lds_body<FMT, R, B, POL>(w, xq, y, in_dim, out_dim, n_rows);                  \
+        rein_matvec_lds_body<FMT, R, B, POL>(w, xq, y, in_dim, out_dim, n_rows, blockIdx.x, gridDim.x); \
     }
 #define REIN_DEFINE_MATVEC_LDS(name, FMT, R, B)                                                   \
     REIN_DEFINE_MATVEC_LDS_LD(name, FMT, R, B, REIN_LD_STREAM)                                    \

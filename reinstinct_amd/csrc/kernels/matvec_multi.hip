@@ -10,6 +10,16 @@
 // single-matrix kernel rein_mv_<fmt>_r<R>_b<B> does (the same function, the same sums in the same
 // order: the outputs are the bits of those kernels).  The matrices may differ in format and in their
 // number of rows; they share in_dim and the activation rows.
+//
+// At two to four activation rows those kernels are bound by the activations: every wavefront reads them from memory again, 40-byte
+// records at a 40-byte stride, and with few wavefronts per CU the chain of its trips is what is left.  rein_mvl_multi_r<R>_b<B> (two
+// to four rows) and rein_mvql_multi_t4_m (three and four, two matrices of an FFN's size) deal whole workgroups instead, each staging the
+// activation rows in LDS and running its matrix as rein_mvl_<fmt> and rein_mvql_<fmt>_t4 would on its workgroups alone: the same
+// functions again, so the same bits.  One launch in place of two or three also means that the activations are staged once per CU and
+// that the tail of one matrix is covered by the next (us at 4 rows, before / after: Q, K, V 4096 -> 4096 + 2 x 1024 in Q5_K with Q6_K
+// 11.6 / 8.9, 1.7 TB/s; gate, up 4096 -> 2 x 14336 in Q5_K 24.0 / 20.6, 4.0 TB/s, 5120 -> 2 x 17408 in Q8_0 41.9 / 31.4, 6.0 TB/s).
+#include "matvec_lds.h"
+#include "matvec_quad.h"
 #include "matvec_repacked.h"
 
 #define REIN_MULTI_MAX 4
@@ -19,8 +29,8 @@ struct ReinMultiMat {
     float*         y;
     unsigned       out_dim;
     int            fmt;          // REIN_* format id of rein_formats.h
-    unsigned       group_end;    // row groups of this matrix and of those before it
-    unsigned       pad;
+    unsigned       end;          // row groups (workgroups) of this matrix and of those before it
+    unsigned       slices;       // rein_mvql_multi_t4_m: of the contraction, and << 16 the trips of weights in flight
 };
 struct ReinMultiArgs {
     ReinMultiMat m[REIN_MULTI_MAX];
@@ -32,14 +42,14 @@ __device__ __forceinline__ void rein_matvec_multi_body(const ReinMultiArgs& a, c
 {
     const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const unsigned wid = blockIdx.x * (blockDim.x >> 6) + wave;
-    unsigned base = 0, end = a.m[0].group_end, out_dim = a.m[0].out_dim;
+    unsigned base = 0, end = a.m[0].end, out_dim = a.m[0].out_dim;
     const uint8_t* w = a.m[0].w;
     float* y = a.m[0].y;
     int fmt = a.m[0].fmt;
 #pragma unroll
     for (int i = 1; i < REIN_MULTI_MAX; i++)
-        if ((unsigned)i < n_mat && wid >= a.m[i - 1].group_end) {
-            base = a.m[i - 1].group_end; end = a.m[i].group_end; out_dim = a.m[i].out_dim;
+        if ((unsigned)i < n_mat && wid >= a.m[i - 1].end) {
+            base = a.m[i - 1].end; end = a.m[i].end; out_dim = a.m[i].out_dim;
             w = a.m[i].w; y = a.m[i].y; fmt = a.m[i].fmt;
         }
     if (wid >= end) return;
@@ -81,3 +91,56 @@ REIN_DEFINE_MATVEC_MULTI(rein_mv_multi_r4_b2, 4, 2)
 REIN_DEFINE_MATVEC_MULTI(rein_mv_multi_r1_b4, 1, 4)
 REIN_DEFINE_MATVEC_MULTI(rein_mv_multi_r2_b4, 2, 4)
 REIN_DEFINE_MATVEC_MULTI(rein_mv_multi_r4_b4, 4, 4)
+
+// run(format as a constant, matrix, workgroup, workgroups of the matrix)
+template <int V> struct ReinFmtId { static constexpr int value = V; };
+template <class Run>
+__device__ __forceinline__ void rein_multi_blocks(const ReinMultiArgs& a, unsigned n_mat, const Run& run)
+{
+    unsigned base = 0;
+    ReinMultiMat m = a.m[0];
+#pragma unroll
+    for (int i = 1; i < REIN_MULTI_MAX; i++)
+        if ((unsigned)i < n_mat && blockIdx.x >= a.m[i - 1].end) {
+            base = a.m[i - 1].end;
+            m = a.m[i];
+        }
+    const unsigned block = blockIdx.x - base, n_block = m.end - base;
+    switch (m.fmt) {
+    case REIN_Q4_K:   run(ReinFmtId<REIN_Q4_K>(), m, block, n_block); break;
+    case REIN_Q6_K:   run(ReinFmtId<REIN_Q6_K>(), m, block, n_block); break;
+    case REIN_Q5_K:   run(ReinFmtId<REIN_Q5_K>(), m, block, n_block); break;
+    case REIN_Q8_0:   run(ReinFmtId<REIN_Q8_0>(), m, block, n_block); break;
+    case REIN_Q4_0:   run(ReinFmtId<REIN_Q4_0>(), m, block, n_block); break;
+    case REIN_IQ4_XS: run(ReinFmtId<REIN_IQ4_XS>(), m, block, n_block); break;
+    case REIN_IQ3_S:  run(ReinFmtId<REIN_IQ3_S>(), m, block, n_block); break;
+    default: break;
+    }
+}
+#define REIN_DEFINE_MATVEC_LDS_MULTI(name, R, B)                                                                                  \
+    REIN_DEFINE_MATVEC_LDS_MULTI_LD(name, R, B, REIN_LD_STREAM)                                                                   \
+    REIN_DEFINE_MATVEC_LDS_MULTI_LD(name##_m, R, B, REIN_LD_MIX)                                                                  \
+    REIN_DEFINE_MATVEC_LDS_MULTI_LD(name##_p, R, B, REIN_LD_PLAIN)
+#define REIN_DEFINE_MATVEC_LDS_MULTI_LD(name, R, B, POL)                                                                          \
+    extern "C" __global__ __launch_bounds__(1024) void name(ReinMultiArgs a, const BlockQ8* __restrict__ xq, unsigned int in_dim, \
+                                                            unsigned int n_mat, unsigned int n_rows)                              \
+    {                                                                                                                             \
+        rein_multi_blocks(a, n_mat, [&](auto fmt, const ReinMultiMat& m, unsigned block, unsigned n_block) {                      \
+            rein_matvec_lds_body<decltype(fmt)::value, R, B, POL>(m.w, xq, m.y, in_dim, m.out_dim, n_rows, block, n_block);       \
+        });                                                                                                                       \
+    }
+#define REIN_DEFINE_MATVEC_QUAD_LDS_MULTI_LD(name, POL)                                                                           \
+    extern "C" __global__ __launch_bounds__(1024) void name(ReinMultiArgs a, const BlockQ8* __restrict__ xq, unsigned int in_dim, \
+                                                            unsigned int n_mat, unsigned int n_rows)                              \
+    {                                                                                                                             \
+        rein_multi_blocks(a, n_mat, [&](auto fmt, const ReinMultiMat& m, unsigned block, unsigned n_block) {                      \
+            rein_matvec_quad_lds_body<decltype(fmt)::value, 1, POL>(m.w, xq, m.y, in_dim, m.out_dim, n_rows, in_dim >> 5,         \
+                                                                    m.slices & 0xFFFFu, m.slices >> 16, block, n_block);          \
+        });                                                                                                                       \
+    }
+
+REIN_DEFINE_MATVEC_LDS_MULTI(rein_mvl_multi_r1_b2, 1, 2)
+REIN_DEFINE_MATVEC_LDS_MULTI(rein_mvl_multi_r2_b2, 2, 2)
+REIN_DEFINE_MATVEC_LDS_MULTI(rein_mvl_multi_r1_b4, 1, 4)
+REIN_DEFINE_MATVEC_LDS_MULTI(rein_mvl_multi_r2_b4, 2, 4)
+REIN_DEFINE_MATVEC_QUAD_LDS_MULTI_LD(rein_mvql_multi_t4_m, REIN_LD_MIX)

@@ -262,7 +262,8 @@ __device__ __forceinline__ void rein_matvec_quad_body(const uint8_t* __restrict_
 template <int FMT, int NT, int POL>
 __device__ __forceinline__ void rein_matvec_quad_lds_body(const uint8_t* __restrict__ w, const BlockQ8* __restrict__ xq,
                                                           float* __restrict__ y, unsigned in_dim, unsigned out_dim,
-                                                          unsigned n_rows, unsigned phase_sub, unsigned slices, unsigned depth)
+                                                          unsigned n_rows, unsigned phase_sub, unsigned slices, unsigned depth,
+                                                          unsigned block, unsigned n_block)
 {
     using F = Fmt<FMT>;
     using Raw = typename F::Raw;
@@ -288,7 +289,7 @@ __device__ __forceinline__ void rein_matvec_quad_lds_body(const uint8_t* __restr
     uint4* stage = reinterpret_cast<uint4*>(xhd + T * stride) + wave * (kParts * 76u);
     const F fmt(w, n_sub, out_dim);
     const unsigned n_groups = (out_dim + 3u) / 4u;
-    const unsigned step = gridDim.x * wpb;
+    const unsigned step = n_block * wpb;
     const XSums no_xs = {0, 0};
 
     // sub-blocks [first, first + count) of every activation row -> planes
@@ -389,7 +390,7 @@ __device__ __forceinline__ void rein_matvec_quad_lds_body(const uint8_t* __restr
 #pragma unroll
         for (int r = 0; r < 4; r++) acc[t][r] = 0.0f;
     if (phase_sub >= n_sub && slices <= 1u) {
-        unsigned g = blockIdx.x * wpb + wave;
+        unsigned g = block * wpb + wave;
         {   // the first trip's weights are on their way while the activations are staged
             const unsigned row = min(min(g, n_groups - 1u) * 4u + lr, out_dim - 1u);
             rq = fmt.template load<POL>(row, min(ls, n_sub - 1u));
@@ -441,7 +442,7 @@ __device__ __forceinline__ void rein_matvec_quad_lds_body(const uint8_t* __restr
         // slices-th trip of it, from trip w % slices on
         const unsigned gpb = wpb / slices;                       // row groups per workgroup
         const unsigned slice = wave % slices;
-        const unsigned g = blockIdx.x * gpb + wave / slices;
+        const unsigned g = block * gpb + wave / slices;
         const bool has = wave < gpb * slices && g < n_groups;    // wave-uniform
         const unsigned ahead = 16u * slices;
         const bool two = kTwoSets && depth >= 2u;                // two register sets of weights taking turns
@@ -519,5 +520,5 @@ __device__ __forceinline__ void rein_matvec_quad_lds_body(const uint8_t* __restr
         unsigned int slices, unsigned int depth)                                                  \
     {                                                                                             \
         rein_matvec_quad_lds_body<FMT, NT, POL>(w, xq, y, in_dim, out_dim, n_rows, phase_sub,     \
-                                                slices, depth);                                   \
+                                                slices, depth, blockIdx.x, gridDim.x);            \
     }

@@ -140,3 +140,24 @@ def test_where_the_exact_dot_gemm_is_taken(tmp_path):
     done = record([("matmul_ws", [f, P, P, P, k, n, rows, P, size["value"]]) for (f, k, n, rows, _), size in zip(cases, sizes)], tmp_path)
     for case, d in zip(cases, done):
         assert bool(xh(d)) == bool(case[-1]), case
+
+
+def test_which_products_of_several_matrices_stage_their_activations_in_lds(tmp_path):
+    q4, q5, q6, q8, i4 = rein.Q4_K, rein.Q5_K, rein.Q6_K, rein.Q8_0, rein.IQ4_XS
+    dot4, matrix, plain = "rein_mvl_multi_", "rein_mvql_multi_t4_m", "rein_mv_multi_"
+    cases = [(([q5, q5, q6], 4096, [4096, 1024, 1024], 4), dot4), (([q4, q4, q6], 4096, [4096, 4096, 4096], 4), plain),
+             (([q8, q8], 2048, [8192, 8192], 3), dot4), (([q4, q4], 2048, [8192, 8192], 3), plain), (([q4, q4], 3072, [8192, 8192], 3), dot4),
+             (([i4, i4], 3072, [8192, 8192], 3), plain), (([q4, q4, q6], 5120, [5120, 1024, 1024], 2), dot4), (([q6, q6], 5120, [17408, 17408], 2), plain),
+             (([q6, q6], 8192, [24576, 24576], 2), dot4), (([q4, q4], 5120, [17408, 17408], 1), plain), (([q5, q5], 4096, [14336, 14336], 4), matrix),
+             (([q4, q6], 8192, [8192, 8192], 3), matrix), (([q4, q4, q4], 5120, [17408, 17408, 17408], 4), "rein_mvql_q4k_t4_m"),
+             (([q4, q6], 5120, [8192, 12288], 3), "rein_mvql_q4k_t4_m"), (([i4, i4], 5120, [17408, 17408], 4), "rein_mvq_iq4xs_t4")]
+    calls = [("matvec_multi_xq8", [f, [P] * len(f), [P] * len(f), outs, P, k, rows]) for (f, k, outs, rows), _ in cases]
+    for (case, kernel), d in zip(cases, record(calls, tmp_path)):
+        names = [r[0] for r in d["launches"]]
+        assert names[0].startswith(kernel), (case, names)
+        assert len(names) == (1 if "multi" in kernel else len(case[0])), (case, names)
+    # a pinned choice of the other forms keeps them
+    pins = [("REIN_MV_LDS", 0, 0), ("REIN_MV_ROWS", 2, 0), ("REIN_MV_WPB", 4, 0), ("REIN_QUAD_LDS", 0, 10), ("REIN_MV_LOADS", 0, 10)]
+    for name, value, at in pins:
+        _, d, _ = record([("option", [name, value]), calls[at], ("option", [name, None])], tmp_path)
+        assert not d["launches"][0][0].startswith(cases[at][1]), (name, d["launches"])
