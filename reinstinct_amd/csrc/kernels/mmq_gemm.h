@@ -359,13 +359,15 @@ template <> struct MmqChunk<REIN_Q6_K> : MmqChunkBase<REIN_Q6_K, MmqChunk<REIN_Q
     static __device__ __forceinline__ rein_v4i operand(const uint4& q, const Small& r, int s, unsigned h)
     {
         const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+        uint32_t lo[4], hi[4];
+        rein_spread2(r.h2.v[s].x >> (8 * h), lo);
+        rein_spread2(r.h2.v[s].y >> (8 * h), hi);
         rein_v4i o;
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             // hi2 byte 2j+h holds the 2-bit fields of this half's word j
-            const uint32_t hw = j < 2 ? r.h2.v[s].x : r.h2.v[s].y;
-            const uint32_t q6 = ((w[j] >> (4 * h)) & 0x0F0F0F0Fu) | rein_spread2(hw, 16 * (j & 1) + 8 * h);
-            o[j] = rein_sub_bytes(q6, 0x20202020u);
+            const uint32_t f = (j < 2 ? lo : hi)[2 * (j & 1)];
+            o[j] = rein_sub_bytes(((w[j] >> (4 * h)) & 0x0F0F0F0Fu) | (f & 0x30303030u), 0x20202020u);
         }
         return o;
     }
@@ -386,12 +388,13 @@ template <> struct MmqChunk<REIN_Q6_K> : MmqChunkBase<REIN_Q6_K, MmqChunk<REIN_Q
     static __device__ __forceinline__ rein_v4i operand_at(const uint4* e, const Small& r, int s, unsigned h)
     {
         const uint2 q = reinterpret_cast<const uint2*>(e)[h];
-        const uint32_t hw = h ? r.h2.v[s].y : r.h2.v[s].x;
+        uint32_t f[4];
+        rein_spread2(h ? r.h2.v[s].y : r.h2.v[s].x, f);
         rein_v4i o;
-        o[0] = rein_sub_bytes((q.x & 0x0F0F0F0Fu) | rein_spread2(hw, 0), 0x20202020u);
-        o[1] = rein_sub_bytes((q.y & 0x0F0F0F0Fu) | rein_spread2(hw, 16), 0x20202020u);
-        o[2] = rein_sub_bytes(((q.x >> 4) & 0x0F0F0F0Fu) | rein_spread2(hw, 8), 0x20202020u);
-        o[3] = rein_sub_bytes(((q.y >> 4) & 0x0F0F0F0Fu) | rein_spread2(hw, 24), 0x20202020u);
+        o[0] = rein_sub_bytes((q.x & 0x0F0F0F0Fu) | (f[0] & 0x30303030u), 0x20202020u);
+        o[1] = rein_sub_bytes((q.y & 0x0F0F0F0Fu) | (f[2] & 0x30303030u), 0x20202020u);
+        o[2] = rein_sub_bytes(((q.x >> 4) & 0x0F0F0F0Fu) | (f[1] & 0x30303030u), 0x20202020u);
+        o[3] = rein_sub_bytes(((q.y >> 4) & 0x0F0F0F0Fu) | (f[3] & 0x30303030u), 0x20202020u);
         return o;
     }
     // the int8 scales of sub-block s (0 or 1 after rotation) for the two groups
