@@ -48,6 +48,11 @@ template <int R> __device__ __forceinline__ float rein_quad_bcast(float v)
 {
     return rein_dpp_f32<R * 0x55>(0.0f, v);
 }
+// the same without the move that prepares an old value for lanes that have no source (here every lane has one)
+template <int R> __device__ __forceinline__ float rein_quad_bcast_all(float v)
+{
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), R * 0x55, 0xF, 0xF, true));
+}
 
 // One trip of a wavefront through LDS.  Memory wants lane l to read row l / 16, sub-block
 // l % 16 (16 lanes x 16 B contiguous per row and load); the matrix instruction wants lane
@@ -331,19 +336,34 @@ __device__ __forceinline__ void rein_matvec_quad_lds_body(const uint8_t* __restr
         int a[8];
 #pragma unroll
         for (int k = 0; k < 8; k++) a[k] = rein_fold_offset<FMT>(sw.w[k]);
+        // One scale for a sub-block: no preparing moves, and what lies past the contraction is zeroed by a mask, where a choice becomes a
+        // branch round the read (us, before / after: 4096 -> 14336 at 4 rows Q4_K 10.4 / 10.1, Q5_K 12.1 / 11.8, 17408 -> 5120 at 16
+        // 26.7 / 25.7, 28.6 / 28.0, Q8_0 27.1 / 25.8).  Q6_K, with two, keeps both: its loop is the slower without them (4096 -> 14336 at 4
+        // rows 14.7 / 15.3).
         float s0[4], s1[4];
-        s0[0] = rein_quad_bcast<0>(sw.s0); s0[1] = rein_quad_bcast<1>(sw.s0);
-        s0[2] = rein_quad_bcast<2>(sw.s0); s0[3] = rein_quad_bcast<3>(sw.s0);
-        s1[0] = rein_quad_bcast<0>(sw.s1); s1[1] = rein_quad_bcast<1>(sw.s1);
-        s1[2] = rein_quad_bcast<2>(sw.s1); s1[3] = rein_quad_bcast<3>(sw.s1);
+        if constexpr (kTwo) {
+            s0[0] = rein_quad_bcast<0>(sw.s0); s0[1] = rein_quad_bcast<1>(sw.s0);
+            s0[2] = rein_quad_bcast<2>(sw.s0); s0[3] = rein_quad_bcast<3>(sw.s0);
+            s1[0] = rein_quad_bcast<0>(sw.s1); s1[1] = rein_quad_bcast<1>(sw.s1);
+            s1[2] = rein_quad_bcast<2>(sw.s1); s1[3] = rein_quad_bcast<3>(sw.s1);
+        } else {
+            s0[0] = rein_quad_bcast_all<0>(sw.s0); s0[1] = rein_quad_bcast_all<1>(sw.s0);
+            s0[2] = rein_quad_bcast_all<2>(sw.s0); s0[3] = rein_quad_bcast_all<3>(sw.s0);
+            s1[0] = rein_quad_bcast_all<0>(sw.s1); s1[1] = rein_quad_bcast_all<1>(sw.s1);
+            s1[2] = rein_quad_bcast_all<2>(sw.s1); s1[3] = rein_quad_bcast_all<3>(sw.s1);
+        }
+        const unsigned mask = live ? ~0u : 0u;
 #pragma unroll
         for (int t = 0; t < NT; t++) {
             const unsigned at = (4u * t + j) * stride + sbx;
             const uint4 lo = xlo[at], hi = xhi[at];
             const uint2 hd = xhd[at];
-            const bool on = live && 4u * t + j < n_rows;
-            const float dx = on ? __builtin_bit_cast(float, hd.x) : 0.0f;
-            const float xsum = on ? __builtin_bit_cast(float, hd.y) : 0.0f;
+            float dx = __builtin_bit_cast(float, hd.x & mask), xsum = __builtin_bit_cast(float, hd.y & mask);
+            if constexpr (kTwo) {
+                const bool on = live && 4u * t + j < n_rows;
+                dx = on ? __builtin_bit_cast(float, hd.x) : 0.0f;
+                xsum = on ? __builtin_bit_cast(float, hd.y) : 0.0f;
+            }
             const int q[8] = {(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
             rein_quad_v4i d0 = {0, 0, 0, 0}, d1 = {0, 0, 0, 0};
 #pragma unroll
