@@ -2573,7 +2573,7 @@ MoeWs moe_ws(const rein_moe_shape& sh)
 namespace {
 // Lanes to a row of rein_moe_few_* (kernels/moe_few.hip): 16, 8 or 4, the least of trips x lanes (idle lanes count) times what
 // the narrower groups lose to their shorter runs of bytes.  gate + up of 2048 -> 768 (no idle lanes at any width), 48
-// tokens: 52.5 / 56.5 / 70.7 us; down 768 -> 2048 (a quarter of 16 or 8 lanes idle): 54.1 / 52.3 / 43.4.
+// tokens, with every entry on dot4: 52.5 / 56.5 / 70.7 us; down 768 -> 2048 (a quarter of 16 or 8 lanes idle): 54.1 / 52.3 / 43.4.
 unsigned moe_few_lanes(unsigned in_dim, bool two_slabs)
 {
     const unsigned n_unit = in_dim / 64;
@@ -2587,7 +2587,8 @@ unsigned moe_few_lanes(unsigned in_dim, bool two_slabs)
 }
 unsigned moe_few_lds(int fmt, unsigned in_dim, unsigned lanes)
 {
-    return 8 * (fmt == REIN_TYPE_Q6_K ? 96 : 80) * ((in_dim / 64 + lanes - 1) / lanes * lanes);
+    const unsigned words = (fmt == REIN_TYPE_Q6_K ? 6 : 5) * ((in_dim / 64 + lanes - 1) / lanes * lanes);
+    return 8 * 16 * (((words + 5) & ~7u) + 2);               // entry_stride
 }
 // their shapes: contractions of whole pairs of sub-blocks, eight entries of each in LDS beside the kernel's own arrays, at most
 // one entry of an expert per token and 1024 of those
@@ -2607,14 +2608,19 @@ bool moe_decode_range(const rein_moe_shape& sh) { return 5ull * sh.n_tok * sh.n_
 // 128 experts top-8, 2048 x 768, 12 / 16 / 24 tokens 71 / 75, 89 / 82, 124 / 91; 256 experts of 1280 x 1280, 16 / 32 tokens 96 / 107,
 // 178 / 143; few experts hardly gain, 8 top-2 at 4 tokens 15 / 24, 4 top-4 at one 12 / 21, 16 top-8 of 4096 x 1536 at 2 and 3 62 / 60,
 // 83 / 66; furthest off 16 top-2 of that size at 8 tokens, 49 / 59, and 32 top-2 of 2048 x 768 at 20, 34 / 39, both on these).
-// Against the pipeline, from eight expert shapes x 4 .. 192 tokens: every further entry costs its dots, while a 32-token tile costs the
-// same until it is full -- up to 5.5 entries per expert (48 / 64 / 96 / 128 tokens of the first shape: pipeline 149-154, these 106 / 121 /
-// 150 / 180), 4 where the experts are small and the tiles few (64 top-6, 1792 x 512, 32 / 48 tokens 60 / 51, 61 / 64).
+// Against the pipeline, from twelve expert shapes: every further entry costs its dots, while a 32-token tile costs the same until it is
+// full -- up to 5.9 entries per expert (pipeline / these: 48 / 64 / 80 tokens of the first shape 149-152 / 97 / 108 / 117, 47 of 32 top-4, 2048 x
+// 1536, 85.4 / 82.0), 7.2 from 450 MB of experts (6.5 and 7.9 entries: 256 top-8, 2048 x 512, 205 / 178, 209 / 205; 64 top-4, 4096 x 1024, 222 / 169,
+// 222 / 195; 128 top-8, 3072 x 768 in Q5_K 207 / 192, 208 / 216), 4.9 where the experts are small and the tiles few (4.5 and 5.1-5.2 entries: 64
+// top-8, 1024 x 512, 45.0 / 42.2, 44.6 / 45.4; 64 top-6, 1792 x 512, 56.5 / 51.9, 57.0 / 55.2).
 bool moe_few_pays(const rein_moe_shape& sh)
 {
     const double entries = (double)sh.n_tok * sh.n_used, per_expert = entries / sh.n_expert;
     const double bytes = 2.0 * rein_repacked_len(sh.gate_up_fmt, sh.hidden, sh.expert_ff) + (double)rein_repacked_len(sh.down_fmt, sh.expert_ff, sh.hidden);
-    if (!moe_decode_range(sh)) return per_expert <= (bytes * sh.n_expert < 134e6 ? 4.0 : 5.5);
+    if (!moe_decode_range(sh)) {
+        const double all = bytes * sh.n_expert;
+        return per_expert <= (all < 134e6 ? 4.9 : all < 450e6 ? 5.9 : 7.2);
+    }
     const double touched = sh.n_expert * (1.0 - std::pow(1.0 - (double)sh.n_used / sh.n_expert, (double)sh.n_tok));
     return (entries - touched) * bytes + entries * 0.2e6 >= 30e6 + (sh.gate_up_fmt == REIN_TYPE_Q8_0 ? 0.45 : 0.3) * touched * bytes;
 }

@@ -7,21 +7,26 @@
 // waited on was their own instructions.  Here a workgroup of four wavefronts owns an expert and a run of its rows.  It finds
 // the expert's entries by scanning the router's ids (a few KB: no sort, no gather), stages their activations in LDS, up to
 // eight at a time, and streams its rows past them: a lane owns 64 weights (FmtPair) of each of two rows -- gate and up of one column, or two
-// rows of down -- so that a fetch from LDS serves both, dot4 against every entry, one unpack for all of them.  The first
-// weights are requested before the scan: they depend on the expert alone.  G lanes share a row (16, or 4 for contractions
+// rows of down -- so that a fetch from LDS serves both, one unpack for all entries.  One or two entries go on dot4; three to eight on
+// v_mfma_i32_4x4x4_16b_i8, four rows of a unit (two sub-blocks) to a quad of lanes against four entries, where the dots of four cost what
+// one and a half do on dot4 and an operand of the activations is read once for four rows: each wavefront turns its weights through an LDS
+// image of 76 words, from the order in which memory is read fastest into the instruction's.  The first weights are requested before the
+// scan: they depend on the expert alone.  G lanes share a row (16, or 4 for contractions
 // that are not a multiple of 1024 values: 768 is three trips of 4 lanes without an idle one).
 //
-// grid = (runs of rows, n_expert), block = 64 * kGuWaves / kDownWaves; dynamic LDS = 8 * kParts * 16 * n_pad bytes, n_pad = in_dim / 64 in
-// whole trips of G.  Contractions are a multiple of 64; ids [n_entries], at most 65535, as the router wrote them, entry e = token
+// grid = (runs of rows, n_expert), block = 64 * kGuWaves / kDownWaves; dynamic LDS = 8 entries of entry_stride(n_pad) 16-byte words, n_pad =
+// in_dim / 64 in whole trips of G.  Contractions are a multiple of 64; ids [n_entries], at most 65535, as the router wrote them, entry e = token
 // e / n_used; at most kMaxEntries of one expert (the router picks an expert at most once per token).  An expert without
 // entries ends at once.
 //
-// Measured (us, gate + up / down of 128 experts top-8, 2048 x 768, Q4_K / Q6_K, against the tiles' 74 / 57 at any of these counts):
-// 24 tokens 43 / 37, 48 tokens 53 / 44, 96 tokens 74 / 59; the whole FFN at 16 / 32 / 48 / 64 / 96 tokens 77 / 93 / 106 / 121 / 150 against
-// 87 / 142 / 149 / 150 / 152.  What bounds it: at one entry per expert the chain of requests of short-lived workgroups (3.5-4.5 TB/s),
-// from about four the dot4 and scale instructions, 13 per sub-block and entry.  Tried without gain: 8 or 16 wavefronts to a
-// workgroup (31.7 against 24.7 us for gate + up at 8 tokens), two trips in flight per wavefront instead of
-// one (38.3 against 32.7 then), runs of 32 or 128 columns.
+// What bounds it (48 tokens of 128 experts top-8, 2048 x 768, Q4_K / Q6_K): not memory -- with every load from the cache the dot4 form took
+// 45 / 39 us of 52 / 45 -- but the vector instructions of unpack, dots and scales and the returns of 32-byte pieces to registers.  Hence the
+// matrix instruction, three wavefronts to a SIMD for Q4_K (168 registers; Q5_K and Q6_K would spill: 106 -> 118 us on dot4).  Whole FFN at 16 / 32 /
+// 48 / 64 / 80 tokens, dot4 for every count / this: 75.5 / 74.3, 92.3 / 89.7, 103.9 / 96.7, 119.2 / 108.2, 131.2 / 117.1 us; 44 tokens of 32
+// experts top-4, 4096 x 1536, 134.3 / 120.0; Q5_K at 60 tokens 122.5 / 111.8; Q8_0 at 48 134.4 / 130.8; the tiles of the pipeline 149-152 at any
+// of the counts of the first shape.  Tried without gain: 8 or 16 wavefronts to a workgroup, two trips in flight per wavefront
+// instead of one, runs of 32 or 128 columns, one sub-block at a time for fewer registers, the ids before the weights (-0.8 us), weights
+// requested in the matrix instruction's order (quads of lanes on four rows: 78.8 / 101.1 at 16 / 48 tokens).
 #include "matvec_pair.h"
 #include "q8_block.h"
 
@@ -56,18 +61,95 @@ __device__ __forceinline__ void stage(uint4* x, unsigned n_pad, unsigned sb, con
     }
 }
 
+// 16-byte words between staged entries: 2 modulo 8, so that the four entries that a quad of lanes reads lie in different banks
+template <int FMT> __device__ __forceinline__ unsigned entry_stride(unsigned n_pad) { return ((kParts<FMT> * n_pad + 5u) & ~7u) + 2u; }
+
+// Over the units of a row, on lanes l = unit (dot4) or on quads of lanes 4 unit + c (the 4x4x4 form): both add the units that differ
+// in bit 3, then 2, 1, 0, so an entry's result does not depend on the form that its batch took.
 template <int G> __device__ __forceinline__ float group_sum(float v)
 {
-    if constexpr (G == 16) return rein_row16_sum(v);
-    v += rein_dpp_f32<0xB1>(0.0f, v);
+    if constexpr (G == 16) v += rein_dpp_f32<0x128>(0.0f, v);           // row_ror 8
+    if constexpr (G == 16) v += rein_dpp_f32<0x124>(0.0f, v);           // row_ror 4
+    if constexpr (G == 8) v += rein_row_xor4(v);
     v += rein_dpp_f32<0x4E>(0.0f, v);
-    if constexpr (G == 8) v += rein_dpp_f32<0x141>(0.0f, v);
+    v += rein_dpp_f32<0xB1>(0.0f, v);
     return v;
+}
+// a + the same register 32 (16) lanes away, in the lower half (even rows of 16 lanes); b's in the others
+__device__ __forceinline__ float sum_far32(float a, float b)
+{
+    const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
+    return __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
+}
+__device__ __forceinline__ float sum_far16(float a, float b)
+{
+    const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
+    return __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
+}
+__device__ __forceinline__ float sum_quads(float v)
+{
+    v += rein_dpp_f32<0x128>(0.0f, v);
+    v += rein_dpp_f32<0x124>(0.0f, v);
+    return v;
+}
+// four sums over the G quads of a lane group at once; held() says which of them a lane ends with, stores() the lane of each that is first
+template <int G> __device__ __forceinline__ float group_sum4(const float (&v)[4])
+{
+    const unsigned lane = threadIdx.x & 63u;
+    if constexpr (G == 16) {
+        return sum_quads(sum_far16(sum_far32(v[0], v[2]), sum_far32(v[1], v[3])));
+    } else if constexpr (G == 8) {
+        const float a = sum_quads(sum_far16(v[0], v[1])), b = sum_quads(sum_far16(v[2], v[3]));
+        return lane & 8u ? b : a;
+    } else {
+        const float a = sum_quads(v[0]), b = sum_quads(v[1]), c = sum_quads(v[2]), d = sum_quads(v[3]);
+        const float ab = lane & 4u ? b : a, cd = lane & 4u ? d : c;
+        return lane & 8u ? cd : ab;
+    }
+}
+template <int G> __device__ __forceinline__ unsigned held()
+{
+    const unsigned lane = threadIdx.x & 63u;
+    return G == 16 ? lane >> 4 : G == 8 ? ((lane >> 4) & 1u) + ((lane >> 2) & 2u) : (lane >> 2) & 3u;
+}
+template <int G> __device__ __forceinline__ bool stores() { return G == 16 ? !(threadIdx.x & 12u) : G == 8 ? !(threadIdx.x & 4u) : true; }
+
+template <int R> __device__ __forceinline__ float quad_lane(float v)
+{
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), R * 0x55, 0xF, 0xF, true));
+}
+template <int R> __device__ __forceinline__ int quad_lane(int v) { return __builtin_amdgcn_mov_dpp(v, R * 0x55, 0xF, 0xF, true); }
+
+typedef int v4i __attribute__((ext_vector_type(4)));
+
+// A pair of sub-blocks as 16-byte words, and a wavefront's image of 64 of them: written in the order of memory (lane = row, unit), read in
+// the order of the 4x4x4 instruction (lane = unit, row).  Entry e lies at e + 4 (e / 16): sixteen lanes touch every bank once both ways.
+template <int FMT> constexpr unsigned kWords = FMT == REIN_Q8_0 ? 5 : FMT == REIN_Q6_K ? 4 : 3;
+constexpr unsigned kImage = 76;
+template <int FMT> __device__ __forceinline__ void pack(const FmtPair<FMT>& v, uint4 (&o)[kWords<FMT>])
+{
+    o[0] = v.q0;
+    o[1] = v.q1;
+    if constexpr (FMT == REIN_Q8_0) { o[2] = v.h0; o[3] = v.h1; o[4] = make_uint4(v.sm, 0, 0, 0); }
+    else if constexpr (FMT == REIN_Q6_K) { o[2] = make_uint4(v.h0.x, v.h0.y, v.h1.x, v.h1.y); o[3] = make_uint4(v.sm, v.dd, 0, 0); }
+    else if constexpr (FMT == REIN_Q5_1) o[2] = make_uint4(v.qh.x, v.qh.y, v.dm.x, v.dm.y);
+    else if constexpr (FMT == REIN_Q5_K) o[2] = make_uint4(v.sm, v.dd, v.qh.x, v.qh.y);
+    else o[2] = make_uint4(v.sm, v.dd, 0, 0);
+}
+template <int FMT> __device__ __forceinline__ void unpack_words(FmtPair<FMT>& v, const uint4 (&o)[kWords<FMT>])
+{
+    v.q0 = o[0];
+    v.q1 = o[1];
+    if constexpr (FMT == REIN_Q8_0) { v.h0 = o[2]; v.h1 = o[3]; v.sm = o[4].x; }
+    else if constexpr (FMT == REIN_Q6_K) { v.h0.x = o[2].x; v.h0.y = o[2].y; v.h1.x = o[2].z; v.h1.y = o[2].w; v.sm = o[3].x; v.dd = o[3].y; }
+    else if constexpr (FMT == REIN_Q5_1) { v.qh.x = o[2].x; v.qh.y = o[2].y; v.dm.x = o[2].z; v.dm.y = o[2].w; }
+    else { v.sm = o[2].x; v.dd = o[2].y; if constexpr (FMT == REIN_Q5_K) { v.qh.x = o[2].z; v.qh.y = o[2].w; } }
 }
 
 // A wavefront's rows: `rows(pass, lr, ra, rb)` says which row of wa and of wb the lane group lr works on in a pass.
 // done(pass, lr, b, sum_a, sum_b) gets the sums of entry b, each on a lane of its own: lane b % G of the group.
 template <int FMT, int G> struct Stream {
+    static constexpr bool q6 = FMT == REIN_Q6_K, mins = !q6 && FMT != REIN_Q8_0;
     using Planes = PairPlanes<FMT>;
     using Pair = FmtPair<FMT>[2];
     Pair cur;
@@ -84,7 +166,6 @@ template <int FMT, int G> struct Stream {
     template <int B>
     static __device__ __forceinline__ void multiply(const Pair& v, const uint4* lds, unsigned at, unsigned n_pad, float (&acc)[2][B])
     {
-        constexpr bool q6 = FMT == REIN_Q6_K, mins = !q6 && FMT != REIN_Q8_0;
         int w[2][2][8], sc[2][2][2];
         float s0[2][2], s1[2][2];
 #pragma unroll
@@ -106,7 +187,7 @@ template <int FMT, int G> struct Stream {
             }
         const uint4* x = lds + at;
 #pragma unroll
-        for (int b = 0; b < B; b++, x += kParts<FMT> * n_pad) {
+        for (int b = 0; b < B; b++, x += entry_stride<FMT>(n_pad)) {
             const uint4 hd = x[4 * n_pad];
             float2 d2;
             if constexpr (q6) d2 = reinterpret_cast<const float2*>(&x[5 * n_pad - at])[at];
@@ -130,6 +211,81 @@ template <int FMT, int G> struct Stream {
                     if constexpr (q6) i0 = __mul24(i0, sc[r][o][0]) + __mul24(i1, sc[r][o][1]);
                     acc[r][b] = fmaf(s0[r][o] * dx, (float)i0, acc[r][b]);
                     if constexpr (mins) acc[r][b] = fmaf(-s1[r][o], __builtin_bit_cast(float, o ? hd.w : hd.z), acc[r][b]);
+                }
+            }
+        }
+    }
+    struct Sub { int w[8]; float s0, s1; int sc[2]; };
+    static __device__ __forceinline__ void unpack(const FmtPair<FMT>& v, int o, Sub& s)
+    {
+        SubW sw;
+        const auto raw = v.get(o);
+        Fmt<FMT>::unpack(raw, sw);
+#pragma unroll
+        for (int k = 0; k < 8; k++) s.w[k] = sw.w[k];
+        s.s0 = sw.s0;
+        s.s1 = sw.s1;
+        if constexpr (q6) {
+            s.sc[0] = (int)(int8_t)(raw.sm & 0xFFu);
+            s.sc[1] = (int)(int8_t)(raw.sm >> 8);
+            s.s0 = rein_h2f(raw.d);
+        }
+    }
+    // what a lane reads of an entry for sub-block o of its unit
+    struct X { int q[8]; float dx, xsum; int fold[2]; };
+    static __device__ __forceinline__ void read(const uint4* x, unsigned u, unsigned n_pad, int o, X& v)
+    {
+        const uint4 x0 = x[2 * o * n_pad + u], x1 = x[(2 * o + 1) * n_pad + u], hd = x[4 * n_pad + u];
+        v.q[0] = x0.x; v.q[1] = x0.y; v.q[2] = x0.z; v.q[3] = x0.w;
+        v.q[4] = x1.x; v.q[5] = x1.y; v.q[6] = x1.z; v.q[7] = x1.w;
+        if constexpr (q6) {
+            v.fold[0] = o ? hd.z : hd.x;
+            v.fold[1] = o ? hd.w : hd.y;
+            const float2 d = reinterpret_cast<const float2*>(&x[5 * n_pad])[u];
+            v.dx = o ? d.y : d.x;
+        } else {
+            v.dx = __builtin_bit_cast(float, o ? hd.y : hd.x);
+            v.xsum = __builtin_bit_cast(float, o ? hd.w : hd.z);
+        }
+    }
+    template <int R> static __device__ __forceinline__ void scale(const Sub& s, const X& e, const v4i& d0, const v4i& d1, float& acc)
+    {
+        int i = d0[R];
+        if constexpr (q6) i = __mul24(i, quad_lane<R>(s.sc[0])) + __mul24(d1[R], quad_lane<R>(s.sc[1]));
+        acc = fmaf(quad_lane<R>(s.s0) * e.dx, (float)i, acc);
+        if constexpr (mins) acc = fmaf(-quad_lane<R>(s.s1), e.xsum, acc);
+    }
+    // NQ groups of four entries: lane 4 (G h + g) + c has the unit g of row 4 h + c, and of each group entry c with those four rows
+    template <int NQ>
+    static __device__ __forceinline__ void fours(const Pair& v, const uint4* lds, unsigned stride, unsigned u, unsigned n_pad, float (&acc)[2][NQ][4])
+    {
+#pragma unroll
+        for (int o = 0; o < 2; o++) {
+            Sub s[2];
+            unpack(v[0], o, s[0]);
+            unpack(v[1], o, s[1]);
+#pragma unroll
+            for (int n = 0; n < NQ; n++) {
+                X e;
+                read(lds + (4 * n + (threadIdx.x & 3u)) * stride, u, n_pad, o, e);
+#pragma unroll
+                for (int r = 0; r < 2; r++) {
+                    v4i d0 = {0, 0, 0, 0}, d1 = {0, 0, 0, 0};
+                    if constexpr (q6) {
+                        d0 = v4i{e.fold[0], e.fold[0], e.fold[0], e.fold[0]};
+                        d1 = v4i{e.fold[1], e.fold[1], e.fold[1], e.fold[1]};
+                    }
+#pragma unroll
+                    for (int k = 0; k < 4; k++) d0 = __builtin_amdgcn_mfma_i32_4x4x4i8(s[r].w[k], e.q[k], d0, 0, 0, 0);
+#pragma unroll
+                    for (int k = 4; k < 8; k++) {
+                        if constexpr (q6) d1 = __builtin_amdgcn_mfma_i32_4x4x4i8(s[r].w[k], e.q[k], d1, 0, 0, 0);
+                        else d0 = __builtin_amdgcn_mfma_i32_4x4x4i8(s[r].w[k], e.q[k], d0, 0, 0, 0);
+                    }
+                    scale<0>(s[r], e, d0, d1, acc[r][n][0]);
+                    scale<1>(s[r], e, d0, d1, acc[r][n][1]);
+                    scale<2>(s[r], e, d0, d1, acc[r][n][2]);
+                    scale<3>(s[r], e, d0, d1, acc[r][n][3]);
                 }
             }
         }
@@ -177,15 +333,65 @@ template <int FMT, int G> struct Stream {
             if (pass == n_pass) break;
         }
     }
-    // the loops are compiled for 1, 2, 3, 4, 6 and 8 entries: what lies in LDS behind the nb-th is computed and dropped
-    template <class Rows, class Done>
-    __device__ __forceinline__ void run_some(unsigned nb, const Planes& wa, const Planes& wb, const uint4* lds, unsigned n_unit, unsigned n_pad,
-                                             unsigned n_pass, const Rows& rows, const Done& done)
+    // three to eight entries on the 4x4x4 instruction, whose 4 NQ columns cost the same whatever they hold
+    template <int NQ, class Rows, class Done>
+    __device__ __forceinline__ void run_fours(const Planes& wa, const Planes& wb, const uint4* lds, uint4* image, unsigned n_unit, unsigned n_pad,
+                                              unsigned n_pass, const Rows& rows, const Done& done)
     {
-        if (nb > 6) run<8>(wa, wb, lds, n_unit, n_pad, n_pass, rows, done);
-        else if (nb > 4) run<6>(wa, wb, lds, n_unit, n_pad, n_pass, rows, done);
-        else if (nb == 4) run<4>(wa, wb, lds, n_unit, n_pad, n_pass, rows, done);
-        else if (nb == 3) run<3>(wa, wb, lds, n_unit, n_pad, n_pass, rows, done);
+        const unsigned lane = threadIdx.x & 63u, c = lane & 3u, g = (lane >> 2) % G, h4 = (lane >> 2) / G * 4u;
+        const unsigned trips = n_pad / G, stride = entry_stride<FMT>(n_pad);
+        const unsigned e = (h4 + c) * G + g;
+        uint4* const put = image + lane + 4u * (lane >> 4);
+        const uint4* const get = image + e + 4u * (e >> 4);
+        float acc[2][NQ][4] = {};
+        unsigned pass = 0, t = 0;
+        const auto step = [&](Pair& now, Pair& next) {
+            const bool last = t + 1 == trips;
+            const unsigned pass2 = last ? pass + 1 : pass, t2 = last ? 0 : t + 1;
+            request(wa, wb, n_unit, min(pass2, n_pass - 1), t2, rows, next);
+            Pair mine;
+#pragma unroll
+            for (int r = 0; r < 2; r++) {
+                uint4 o[kWords<FMT>];
+                pack<FMT>(now[r], o);
+#pragma unroll
+                for (unsigned k = 0; k < kWords<FMT>; k++) {
+                    *put = o[k];
+                    __builtin_amdgcn_wave_barrier();
+                    o[k] = *get;
+                    __builtin_amdgcn_wave_barrier();
+                }
+                unpack_words<FMT>(mine[r], o);
+            }
+            fours<NQ>(mine, lds, stride, g + G * t, n_pad, acc);
+            if (last) {
+#pragma unroll
+                for (int n = 0; n < NQ; n++) {
+                    const float a = group_sum4<G>(acc[0][n]), b = group_sum4<G>(acc[1][n]);
+                    if (stores<G>()) done(pass, h4 + held<G>(), 4 * n + c, a, b);
+#pragma unroll
+                    for (int i = 0; i < 4; i++) acc[0][n][i] = acc[1][n][i] = 0.0f;
+                }
+            }
+            pass = pass2;
+            t = t2;
+        };
+        Pair nxt;
+        for (;;) {
+            step(cur, nxt);
+            if (pass == n_pass) break;
+            step(nxt, cur);
+            if (pass == n_pass) break;
+        }
+    }
+    // what lies in LDS behind the nb-th entry is computed and dropped
+    template <class Rows, class Done>
+    __device__ __forceinline__ void run_some(unsigned nb, const Planes& wa, const Planes& wb, const uint4* lds, uint4* images, unsigned n_unit,
+                                             unsigned n_pad, unsigned n_pass, const Rows& rows, const Done& done)
+    {
+        uint4* image = images + (threadIdx.x >> 6) * kImage;
+        if (nb > 4) run_fours<2>(wa, wb, lds, image, n_unit, n_pad, n_pass, rows, done);
+        else if (nb > 2) run_fours<1>(wa, wb, lds, image, n_unit, n_pad, n_pass, rows, done);
         else if (nb == 2) run<2>(wa, wb, lds, n_unit, n_pad, n_pass, rows, done);
         else run<1>(wa, wb, lds, n_unit, n_pad, n_pass, rows, done);
     }
@@ -214,6 +420,7 @@ __device__ __forceinline__ void gate_up(const uint8_t* __restrict__ gate_slab, c
     __shared__ uint16_t list[kMaxEntries];
     __shared__ unsigned count;
     __shared__ float vals[kBatch][kGuCols + 4];
+    __shared__ uint4 images[kGuWaves * kImage];
     const unsigned e = blockIdx.y, c0 = blockIdx.x * kGuCols;
     const unsigned n_sub = in_dim >> 5, n_unit = n_sub >> 1, n_pad = (n_unit + G - 1) / G * G, wave = threadIdx.x >> 6;
     constexpr unsigned kRows = 64 / G, kStep = kGuWaves * kRows;                   // columns of a wavefront, of the workgroup, per pass
@@ -229,14 +436,14 @@ __device__ __forceinline__ void gate_up(const uint8_t* __restrict__ gate_slab, c
         const unsigned nb = min(kBatch, m - at);
         if (at) s.request(wg, wu, n_unit, 0, 0, rows, s.cur);
         if (n_pad > n_unit && at == 0)
-            for (unsigned i = threadIdx.x; i < kBatch * kParts<FMT> * n_pad; i += blockDim.x) rein_few_lds[i] = make_uint4(0, 0, 0, 0);
+            for (unsigned i = threadIdx.x; i < kBatch * entry_stride<FMT>(n_pad); i += blockDim.x) rein_few_lds[i] = make_uint4(0, 0, 0, 0);
         if (n_pad > n_unit && at == 0) __syncthreads();
         for (unsigned i = threadIdx.x; i < nb * n_sub; i += blockDim.x) {
             const unsigned b = i / n_sub, sb = i - b * n_sub;
-            stage<FMT>(rein_few_lds + b * kParts<FMT> * n_pad, n_pad, sb, xq[(size_t)(list[at + b] / n_used) * n_sub + sb]);
+            stage<FMT>(rein_few_lds + b * entry_stride<FMT>(n_pad), n_pad, sb, xq[(size_t)(list[at + b] / n_used) * n_sub + sb]);
         }
         __syncthreads();
-        s.run_some(nb, wg, wu, rein_few_lds, n_unit, n_pad, n_pass, rows, [&](unsigned pass, unsigned lr, unsigned b, float g, float u) {
+        s.run_some(nb, wg, wu, rein_few_lds, images, n_unit, n_pad, n_pass, rows, [&](unsigned pass, unsigned lr, unsigned b, float g, float u) {
             vals[b][pass * kStep + wave * kRows + lr] = rein_silu_det(g) * u;
         });
         __syncthreads();
@@ -255,6 +462,7 @@ __device__ __forceinline__ void down(const uint8_t* __restrict__ slab, unsigned 
 {
     extern __shared__ uint4 rein_few_lds[];
     __shared__ uint16_t list[kMaxEntries];
+    __shared__ uint4 images[kDownWaves * kImage];
     __shared__ unsigned count;
     const unsigned e = blockIdx.y, r0 = blockIdx.x * kDownRows;
     const unsigned n_sub = in_dim >> 5, n_unit = n_sub >> 1, n_pad = (n_unit + G - 1) / G * G, wave = threadIdx.x >> 6;
@@ -276,14 +484,14 @@ __device__ __forceinline__ void down(const uint8_t* __restrict__ slab, unsigned 
             s.request(w, w, n_unit, 0, 0, rows, s.cur);
         }
         if (n_pad > n_unit && at == 0)
-            for (unsigned i = threadIdx.x; i < kBatch * kParts<FMT> * n_pad; i += blockDim.x) rein_few_lds[i] = make_uint4(0, 0, 0, 0);
+            for (unsigned i = threadIdx.x; i < kBatch * entry_stride<FMT>(n_pad); i += blockDim.x) rein_few_lds[i] = make_uint4(0, 0, 0, 0);
         if (n_pad > n_unit && at == 0) __syncthreads();
         for (unsigned i = threadIdx.x; i < nb * n_sub; i += blockDim.x) {
             const unsigned b = i / n_sub, sb = i - b * n_sub;
-            stage<FMT>(rein_few_lds + b * kParts<FMT> * n_pad, n_pad, sb, xq[(size_t)list[at + b] * n_sub + sb]);
+            stage<FMT>(rein_few_lds + b * entry_stride<FMT>(n_pad), n_pad, sb, xq[(size_t)list[at + b] * n_sub + sb]);
         }
         __syncthreads();
-        s.run_some(nb, w, w, rein_few_lds, n_unit, n_pad, n_pass, rows, [&](unsigned pass, unsigned lr, unsigned b, float va, float vb) {
+        s.run_some(nb, w, w, rein_few_lds, images, n_unit, n_pad, n_pass, rows, [&](unsigned pass, unsigned lr, unsigned b, float va, float vb) {
             if (b >= nb) return;
             float* o = y + (size_t)list[at + b] * out_dim;
             const unsigned ra = first(pass, lr), rb = ra + kRows;
@@ -296,14 +504,14 @@ __device__ __forceinline__ void down(const uint8_t* __restrict__ slab, unsigned 
 }  // namespace rein_few
 
 #define REIN_DEFINE_MOE_FEW(tag, FMT, G)                                                                                     \
-    extern "C" __global__ __launch_bounds__(64 * rein_few::kGuWaves, 2) void rein_moe_few_gate_up_##tag##_g##G(              \
+    extern "C" __global__ __launch_bounds__(64 * rein_few::kGuWaves, (FMT == REIN_Q4_K ? 3 : 2)) void rein_moe_few_gate_up_##tag##_g##G(              \
         const unsigned char* __restrict__ gate_slab, const unsigned char* __restrict__ up_slab, const int* __restrict__ ids, \
         const BlockQ8* __restrict__ xq, BlockQ8* __restrict__ xq_out, unsigned int bytes_per_expert, unsigned int in_dim,    \
         unsigned int out_dim, unsigned int n_used, unsigned int n_entries)                                                   \
     {                                                                                                                        \
         rein_few::gate_up<FMT, G>(gate_slab, up_slab, bytes_per_expert, ids, xq, xq_out, in_dim, out_dim, n_used, n_entries); \
     }                                                                                                                        \
-    extern "C" __global__ __launch_bounds__(64 * rein_few::kDownWaves, 2) void rein_moe_few_down_##tag##_g##G(               \
+    extern "C" __global__ __launch_bounds__(64 * rein_few::kDownWaves, (FMT == REIN_Q4_K ? 3 : 2)) void rein_moe_few_down_##tag##_g##G(               \
         const unsigned char* __restrict__ slab, const int* __restrict__ ids, const BlockQ8* __restrict__ xq,                 \
         float* __restrict__ y, unsigned int bytes_per_expert, unsigned int in_dim, unsigned int out_dim,                     \
         unsigned int n_entries)                                                                                              \
