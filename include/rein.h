@@ -311,9 +311,9 @@ int rein_matvec_batched_xq8(int fmt, const void *w, const void *xq, float *y, un
  * (the two to four rows of the speculative-decode verify step, prefill.rs:448-508).  The matrices
  * share in_dim and may differ in format and in out_dims[i]; with one row every output is bit for
  * bit what rein_matvec_xq8 gives for that matrix, with more rows what the dot4 kernels behind
- * rein_matvec_batched_xq8 give (three and four rows against matrices of an FFN's size go out as
- * the launches of rein_matvec_batched_xq8 one by one, which are faster there).  The four tables are
- * host arrays, read before the call returns. */
+ * rein_matvec_batched_xq8 give (three and four rows against matrices of an FFN's size: what
+ * rein_matvec_batched_xq8 gives, whose launches go out one by one or two matrices in one).  The
+ * four tables are host arrays, read before the call returns. */
 int rein_matvec_multi_xq8(unsigned n_mat, const int *fmts, const void *const *ws, float *const *ys,
                           const unsigned *out_dims, const void *xq, unsigned in_dim, unsigned n_rows,
                           rein_stream_t s);

@@ -597,8 +597,8 @@ __device__ __forceinline__ void rein_mmq_chunk_math(const MmqLds<TM>& lds, const
                     }
                 }
             }
-            // keep the pairs apart: interleaving them buys nothing (MFMA and VALU of
-            // a SIMD do not overlap) and costs a second set of 96 live registers
+            // keep the pairs apart: interleaving them was level and costs a second set
+            // of 96 live registers
             __builtin_amdgcn_sched_barrier(0);
         }
         if constexpr (C::kHasMin && DOTS == 0) {
