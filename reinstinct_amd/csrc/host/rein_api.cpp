@@ -626,8 +626,7 @@ QuadLdsGeometry mvql_geometry(int fmt, unsigned in_dim, unsigned out_dim, unsign
 //             Q4_K, Q8_0, Q4_0, IQ3_S (skinny MMQ otherwise): ahead up to 20480 rows -- 17408 -> 5120 1.21-1.37, 14336 ->
 //             4096 1.25-1.46, 18944 -> 3584 1.27-1.50, 5120 -> 5120 1.12-1.16, 4096 -> 4096 1.12-1.35, 5120 -> 1024
 //             1.20-1.51, 8192 -> 8192 1.00-1.23, 4096 -> 14336 1.21-1.36, 2048 -> 16384 1.20-1.35 -- except where the rows
-//             need phases against more than 6144 rows (28672 -> 8192 0.88-1.06); behind or level beyond 20480 rows
-//             (5120 -> 34816 0.95-1.08, 8192 -> 28672 0.92-1.20).
+//             need phases against more than 6144 rows (28672 -> 8192 0.88-1.06); beyond 20480 rows by shape (the rule below).
 //   3-4 rows  up to 8192 rows and from 20 * 2^20 weights ahead of the LDS-staged dot4 kernel for every format but Q8_0
 //             (0.95-1.02): Q4_K 5120 -> 5120 1.05-1.08, 17408 -> 5120 1.24-1.26, 14336 -> 4096 1.09, 28672 -> 8192
 //             1.15-1.18, 18944 -> 3584 1.17, 5120 -> 7168 1.18-1.20, 8192 -> 8192 0.96; Q4_0 1.08-1.33; Q6_K 1.07-1.22;
@@ -678,14 +677,17 @@ bool use_mvql(int fmt, unsigned in_dim, unsigned out_dim, unsigned n_rows)
                (in_dim % 4096 == 0 && out_dim <= 14336);
     }
     if (n_rows >= 5) {
-        // (from four million weights with a contraction of 4096, every format but Q5_K: 4096 -> 1024 at 8 rows Q6_K 8.6 -> 6.7 us,
-        // Q8_0 7.4 -> 6.4, IQ4_XS 8.0 -> 6.3, Q4_0 7.7 -> 6.3, IQ3_S 7.5 -> 6.2, Q4_K 6.5 -> 6.3; Q5_K 5.8 -> 6.5 and 2048 -> 2048
-        // Q4_K 5.6 -> 6.0, Q5_K 5.3 -> 6.1 stay on dot4)
-        const bool from_4m = fmt != REIN_TYPE_Q5_K && weights >= (4ull << 20) && in_dim >= 4096;
-        if (weights < (5ull << 20) && !from_4m) return false;
+        // from 3.5 * 2^20 weights, and with contractions of 1024 from 1536 rows, every format (dot4 -> this, 5 / 8 rows: 2304 -> 1664 Q4_K
+        // 1.39 / 1.32 x, Q5_K 1.26 / 1.15, Q6_K 1.52 / 1.53; 6144 -> 640 1.30 / 1.23, 1.13 / 1.10, 1.72 / 1.73; 1024 -> 1536 1.28 / 1.11, 1.14 / 1.07,
+        // 1.29 / 1.28; below that 2048 -> 1536 Q8_0 0.95 / 1.03, Q5_K 0.97 / 0.88, 1024 -> 1024 0.8-1.0, 2048 -> 512 0.7-0.9)
+        if (weights < (7ull << 19) && !(in_dim <= 1024 && out_dim >= 1536)) return false;
         if (fmt == REIN_TYPE_Q6_K || fmt == REIN_TYPE_Q5_K || fmt == REIN_TYPE_IQ4_XS) return true;
+        // the other formats beyond 20480 rows: from 28672 where two workgroups of eight rows fit the CU and no trip is part empty (5 / 8 rows: 4096 -> 28672 Q8_0 1.44 /
+        // 1.41 x, Q4_K 1.36 / 1.37, 2048 -> 32768 1.28 / 1.27, 1.23 / 1.24, 5120 -> 151936 1.15 / 1.16, 1.10 / 1.17; 2304 -> 30720 Q4_0 0.95, 6144 ->
+        // 22528 Q4_K 0.83 / 0.86, 7168 -> 24576 0.82 / 0.87), Q8_0 also from contractions of 8192 (8192 -> 28672 1.31 x; 7168 -> 24576 0.97 / 1.00)
         const bool phased = g.phase_sub < in_dim / 32;
-        return out_dim <= 20480 && !(phased && out_dim > 6144);
+        if (out_dim > 20480) return (in_dim <= 5120 && in_dim % 512 == 0 && out_dim >= 28672) || (fmt == REIN_TYPE_Q8_0 && in_dim >= 8192 && !phased);
+        return !(phased && out_dim > 6144);
     }
     return mvql_few_rows(fmt, in_dim, out_dim, n_rows);
 }

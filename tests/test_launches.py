@@ -163,12 +163,13 @@ def test_which_products_of_several_matrices_stage_their_activations_in_lds(tmp_p
         assert not d["launches"][0][0].startswith(cases[at][1]), (name, d["launches"])
 
 
-def test_which_products_of_three_and_four_rows_take_the_4x4x4_kernel_with_the_rows_in_lds(tmp_path):
+def test_which_products_of_three_to_eight_rows_take_the_4x4x4_kernel_with_the_rows_in_lds(tmp_path):
     q4, q5, q6, q8, i4, i3 = rein.Q4_K, rein.Q5_K, rein.Q6_K, rein.Q8_0, rein.IQ4_XS, rein.IQ3_S
     cases = [(q4, 1024, 4096, 3, 1), (q4, 1024, 4064, 3, 0), (q4, 2560, 6496, 4, 1), (q4, 2816, 5120, 4, 0), (q5, 2048, 4608, 3, 1), (q6, 1280, 5120, 3, 1),
              (q6, 1536, 5120, 3, 0), (q8, 2048, 4608, 4, 1), (q8, 2048, 4608, 3, 0), (i4, 1536, 4096, 4, 1), (i4, 1536, 4096, 3, 0), (q8, 7168, 7168, 3, 1),
              (q8, 8192, 8192, 4, 0), (q8, 8192, 10240, 4, 1), (q8, 5120, 5120, 4, 0), (i4, 5120, 16384, 3, 1), (i4, 5120, 16416, 3, 0), (i3, 2048, 8192, 4, 1),
-             (q4, 2048, 8192, 4, 0), (q4, 1024, 4096, 2, 0)]
+             (q4, 2048, 8192, 4, 0), (q4, 1024, 4096, 2, 0), (q5, 2304, 1664, 5, 1), (q5, 2048, 1536, 8, 0), (q8, 1024, 1536, 6, 1), (q4, 1024, 1504, 7, 0),
+             (q4, 4096, 28672, 5, 1), (q4, 4096, 28640, 5, 0), (q4, 2304, 30720, 8, 0), (q4, 6144, 30720, 8, 0), (q8, 8192, 20512, 8, 1), (q8, 7168, 24576, 5, 0)]
     calls = [("mmq_xq8", [f, P, P, P, k, n, rows]) for f, k, n, rows, _ in cases]
     for case, d in zip(cases, record(calls, tmp_path)):
         assert d["launches"][0][0].startswith("rein_mvql_") == bool(case[-1]), (case, d["launches"])
