@@ -682,11 +682,12 @@ bool use_mvql(int fmt, unsigned in_dim, unsigned out_dim, unsigned n_rows)
         // 1.29 / 1.28; below that 2048 -> 1536 Q8_0 0.95 / 1.03, Q5_K 0.97 / 0.88, 1024 -> 1024 0.8-1.0, 2048 -> 512 0.7-0.9)
         if (weights < (7ull << 19) && !(in_dim <= 1024 && out_dim >= 1536)) return false;
         if (fmt == REIN_TYPE_Q6_K || fmt == REIN_TYPE_Q5_K || fmt == REIN_TYPE_IQ4_XS) return true;
-        // the other formats beyond 20480 rows: from 28672 where two workgroups of eight rows fit the CU and no trip is part empty (5 / 8 rows: 4096 -> 28672 Q8_0 1.44 /
-        // 1.41 x, Q4_K 1.36 / 1.37, 2048 -> 32768 1.28 / 1.27, 1.23 / 1.24, 5120 -> 151936 1.15 / 1.16, 1.10 / 1.17; 2304 -> 30720 Q4_0 0.95, 6144 ->
-        // 22528 Q4_K 0.83 / 0.86, 7168 -> 24576 0.82 / 0.87), Q8_0 also from contractions of 8192 (8192 -> 28672 1.31 x; 7168 -> 24576 0.97 / 1.00)
+        // the other formats beyond 20480 rows: from 28672 up to contractions of 4608, where workgroups of eight rows leave the CU room for two,
+        // and no trip is part empty (5 or 8 rows: 4096 -> 28672 Q8_0 1.46 x, Q4_K 1.39, 4096 -> 65536 1.52, 1.39, 2048 -> 34816 1.31, 1.30; 5120 ->
+        // 34816 Q4_K 1.05-1.12 but Q4_0 5120 -> 49152 1.02; 2304 -> 30720 Q4_0 0.95, 6144 -> 22528 Q4_K 0.83-0.86, 7168 -> 24576 0.82-0.87), Q8_0 also
+        // from contractions of 8192 (8192 -> 28672 1.31 x, 8192 -> 36864 1.40; 7168 -> 24576 0.97-1.00)
         const bool phased = g.phase_sub < in_dim / 32;
-        if (out_dim > 20480) return (in_dim <= 5120 && in_dim % 512 == 0 && out_dim >= 28672) || (fmt == REIN_TYPE_Q8_0 && in_dim >= 8192 && !phased);
+        if (out_dim > 20480) return (in_dim <= 4608 && in_dim % 512 == 0 && out_dim >= 28672) || (fmt == REIN_TYPE_Q8_0 && in_dim >= 8192 && !phased);
         return !(phased && out_dim > 6144);
     }
     return mvql_few_rows(fmt, in_dim, out_dim, n_rows);
