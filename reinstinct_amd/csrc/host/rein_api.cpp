@@ -2074,13 +2074,28 @@ bool wide_few_take(int fmt, unsigned in_dim, unsigned out_dim, unsigned p_rows)
     if (!wide_few_shape(fmt, in_dim, p_rows)) return false;
     if (opt_u(O_MMQXH, 1) == 3) return true;
     const unsigned long long weights = (unsigned long long)in_dim * out_dim;
-    if (p_rows <= 16) return weights >= (fmt == REIN_TYPE_Q5_K ? 85ull << 20 : 60ull << 20);
-    return weights >= 4ull << 20 && (fmt == REIN_TYPE_Q6_K || p_rows > 32 || out_dim <= 16384);
+    // (9-16 rows, other launches / this: Q4_K 8192 -> 8192 24.8 / 21.7, 5120 -> 17408 26.5 / 24.5, but 5120 -> 13824 20.1 / 21.6, 3072 -> 24576 19.7 /
+    // 21.3; Q5_K 6144 -> 18432 37.6 / 34.9, 8192 -> 14336 41.0 / 42.7 at 9 rows, 8192 -> 24576 60.5 / 75.0; Q6_K 5120 -> 17408 40.0 / 32.4, 8192 ->
+    // 24576 70.1 / 76.6)
+    if (p_rows <= 16) {
+        if (out_dim > 18432) return false;
+        if (fmt == REIN_TYPE_Q6_K) return weights >= 60ull << 20;
+        if (fmt == REIN_TYPE_Q5_K) return weights >= 85ull << 20 && (in_dim < 8192 || out_dim <= 8192);
+        return weights >= (in_dim >= 8192 ? 60ull << 20 : 85ull << 20);
+    }
+    // (17-32 rows: Q4_K 8192 -> 8192 23.9 / 22.0, 8192 -> 14336 33.0 / 34.0, 5120 -> 13824 23.1 / 23.9, Q5_K 8192 -> 14336 39.8 / 42.9)
+    return weights >= 4ull << 20 && (fmt == REIN_TYPE_Q6_K || p_rows > 32 || out_dim <= 12288);
 }
 bool wide_int8_take(int fmt, unsigned in_dim, unsigned out_dim, unsigned p_rows)
 {
     if (opt_u(O_MMQXH, 1) >= 2) return true;
-    if (p_rows <= 16) return in_dim >= 3ull * out_dim || (fmt != REIN_TYPE_Q8_0 && (unsigned long long)in_dim * out_dim >= 48ull << 20);
+    // (9-16 rows, other launches / this: 14336 -> 5120 Q4_0 26.2 / 20.4, 8192 -> 14336 IQ4_XS 34.3 / 30.5, 4096 -> 16384 22.1 / 21.3; 4096 -> 12288 19.0 / 20.3, 3072 -> 24576
+    // IQ4_XS 21.8 / 26.9, Q4_0 19.4 / 24.2, 8192 -> 24576 at 9 rows 45.4 / 48.7)
+    if (p_rows <= 16)
+        return in_dim >= 3ull * out_dim ||
+               (fmt != REIN_TYPE_Q8_0 && in_dim >= 4096 && out_dim <= 18432 && (unsigned long long)in_dim * out_dim >= 56ull << 20);
+    // (17-32 rows: 3072 -> 24576 IQ4_XS 26.9 / 28.1 at 32, 1024 -> 20000 13.6 / 14.3; 4096 -> 18432 26.4 / 25.1, Q8_0 3072 -> 24576 29.7 / 27.6)
+    if (p_rows <= 32 && fmt != REIN_TYPE_Q8_0 && out_dim > 18432 && in_dim < 4096) return false;
     return in_dim >= 2048 || p_rows <= 64 || p_rows > 400 || out_dim < 4096;
 }
 // the launch of a shape, or null: those of rein_mmq_xq8_ws
