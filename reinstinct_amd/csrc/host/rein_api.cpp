@@ -2096,6 +2096,10 @@ bool wide_int8_take(int fmt, unsigned in_dim, unsigned out_dim, unsigned p_rows)
                (fmt != REIN_TYPE_Q8_0 && in_dim >= 4096 && out_dim <= 18432 && (unsigned long long)in_dim * out_dim >= 56ull << 20);
     // (17-32 rows: 3072 -> 24576 IQ4_XS 26.9 / 28.1 at 32, 1024 -> 20000 13.6 / 14.3; 4096 -> 18432 26.4 / 25.1, Q8_0 3072 -> 24576 29.7 / 27.6)
     if (p_rows <= 32 && fmt != REIN_TYPE_Q8_0 && out_dim > 18432 && in_dim < 4096) return false;
+    // (33-128 rows: 2048 -> 32768 at 96 IQ4_XS 34.3 / 37.6, Q8_0 38.2 / 39.6, 1024 -> 20000 at 64 16.4 / 17.6, 16.3 / 17.7; 3072 -> 24576 36.9 / 35.5)
+    if (p_rows > 32 && p_rows <= 128 && in_dim <= 2048 && out_dim > 18432) return false;
+    // (65-192 rows: 2048 -> 12288 at 128 / 160 Q8_0 24.3 / 26.5, 24.7 / 26.2, IQ4_XS 26.2 / 26.9; level at 256, 58.1 / 45.7 at 400)
+    if (p_rows > 64 && p_rows <= 192 && in_dim <= 2048 && out_dim >= 4096 && out_dim <= 18432) return false;
     return in_dim >= 2048 || p_rows <= 64 || p_rows > 400 || out_dim < 4096;
 }
 // the launch of a shape, or null: those of rein_mmq_xq8_ws
