@@ -2161,20 +2161,15 @@ WidePlan wide_plan(const WideKind& kind, int fmt, unsigned in_dim, unsigned out_
     p.parts = wide_parts_bytes(n_rb, p.n_whole, p.split, n_tt, p.n_grp);
     return p;
 }
-// The most bytes of partial tiles that any number of weight rows leaves behind whole rounds (the size query does not know the matrix)
+// No number of weight rows leaves more bytes of partial tiles behind whole rounds (the size query does not know the matrix): at most
+// kWideMostParts ranges, and of a tail's units at most one for each of sixteen superblocks, each of a group of the most tiles.  A bound
+// and not the largest plan: that is within a fifth of it from sixteen superblocks on and a half to a quarter below, but pricing a
+// round's plans takes the query from 1 to 70-270 us, and a program whose prompts differ in length asks before each.
 size_t wide_most_parts_bytes(const WideKind& kind, unsigned in_dim, unsigned p_rows)
 {
-    const unsigned n_tt = (p_rows + 31) / 32;
-    size_t most = 0;
-    for (unsigned size = kind.most; size >= 1; size--) {
-        const unsigned n_grp = wide_groups(kind, n_tt, size);
-        for (unsigned n_rb = 1; n_rb <= kind.slots; n_rb++) {            // the remainders repeat
-            const unsigned units = n_rb * n_grp;
-            double price;
-            most = std::max(most, wide_parts_bytes(n_rb, units / kind.slots * kind.slots, wide_split(kind, units, n_tt, n_grp, in_dim / 256, &price), n_tt, n_grp));
-        }
-    }
-    return most;
+    const unsigned n_tt = (p_rows + 31) / 32, most_split = std::min(16u, in_dim / 256);
+    if (most_split < 2) return 0;
+    return (size_t)std::min(kWideMostParts, (kind.slots - 1) * most_split) * std::min(kind.most, n_tt) * kWidePart;
 }
 }  // namespace
 
