@@ -2024,12 +2024,16 @@ unsigned wide_lds_bytes(const WideKind& kind, int fmt)
 }
 // Where they are taken, from sweeps through rein_matmul_ws, every cell beside the launches of rein_mmq_xq8_ws (their time / this one's),
 // the weights of two to six matrices in turn:
-//   int8  12 shapes (1024 -> 4096 ... 17408 -> 5120, 1536 -> 32000) x 17 row counts: from 24 rows 0.95-2.0 in 612 cells, 7 of them below
-//         0.98, 1.14-1.27 in the geometric mean of every row count (Q8_0 5120 -> 17408, 2048 rows 648 / 507 us; 17408 -> 5120, 200 rows
-//         135 / 77, 45 rows 44 / 35; 5632 -> 2048, 32 rows 16.7 / 13.0).  All four from 17 rows on 13 shapes 1.03-1.44 at 17-28 rows.  Not
-//         contractions below 2048 against 4096 rows and more at 65-400 rows (1024 -> 4096 and 1536 -> 32000 0.96-1.03: three launches for
-//         little work).  9-16 rows: contractions of three times the rows of weights (1.04-1.33 in 60 cells; 5632 -> 2048 0.92-0.96, 5120 ->
-//         5120 0.86-1.0), and the 4-bit formats from 48M weights (5120 -> 17408, 4096 -> 14336, 8192 -> 8192 1.01-1.15; Q8_0 there 0.82-1.01).
+//   int8, 17 contractions x 44 row counts of weights x 25 of activations, 17-2048 rows, in pieces of 128 rows x 32 tokens -- the workgroups of
+//         the plain launch, which are resident at once up to 768: contractions of 1536 and more 0.98-1.62 in the mean of every cell of (contraction,
+//         pieces), 1.20 over all (Q8_0 5120 -> 17408, 2048 rows 648 / 507 us; 17408 -> 5120, 200 rows 135 / 77).  Below, three launches and a start-up
+//         of four tiles against little work: 256 and 512 0.80-0.95 at any size; 768 to 1280 1.02-1.6 up to 64 pieces, 0.92-1.02 beyond, from 1024
+//         pieces 1.04-1.15 again (768: 0.98-1.10).  2048, whose padded rows bring their scales by 16-bit words: 0.90-0.98 between 256 and
+//         512 pieces (Q8_0 up to 1.10), 1.03-1.25 on both sides.
+//         9-16 rows: narrow matrices, where the few-row kernels have too few workgroups -- up to 1024 rows of weights from contractions of 3072
+//         (1.0-1.9; 2048 0.92-1.05, below 0.7-0.9), beyond from 8192, four times the rows of weights, or 11008 and three times (1.01-1.21; 5120 -> 1536
+//         0.84, 6144 -> 2048 0.91) -- and the 4-bit formats from 56M weights with a contraction of 6144 or against more than 16384 rows
+//         (5120 -> 18432 1.07, 6144 -> 12288 1.08, 11008 -> 12288 1.45; 4096 and 5120 -> 14336 0.87-0.97; Q8_0 there 0.75-1.0).
 //   exact, 13 shapes (those and 3584 -> 18944) x 17 row counts from 33:
 //     Q6_K  1.07-3.0 in all 221 cells (17408 -> 5120, 200 rows 220 / 72 us; 5120 -> 17408, 512 rows 311 / 182); below 2.5e8 operations
 //           nothing was measured.
@@ -2086,21 +2090,18 @@ bool wide_few_take(int fmt, unsigned in_dim, unsigned out_dim, unsigned p_rows)
     // (17-32 rows: Q4_K 8192 -> 8192 23.9 / 22.0, 8192 -> 14336 33.0 / 34.0, 5120 -> 13824 23.1 / 23.9, Q5_K 8192 -> 14336 39.8 / 42.9)
     return weights >= 4ull << 20 && (fmt == REIN_TYPE_Q6_K || p_rows > 32 || out_dim <= 12288);
 }
+bool wide_int8_shape(unsigned in_dim) { return in_dim >= 768 || opt_u(O_MMQXH, 1) >= 2; }          // for any number of weight rows
 bool wide_int8_take(int fmt, unsigned in_dim, unsigned out_dim, unsigned p_rows)
 {
     if (opt_u(O_MMQXH, 1) >= 2) return true;
-    // (9-16 rows, other launches / this: 14336 -> 5120 Q4_0 26.2 / 20.4, 8192 -> 14336 IQ4_XS 34.3 / 30.5, 4096 -> 16384 22.1 / 21.3; 4096 -> 12288 19.0 / 20.3, 3072 -> 24576
-    // IQ4_XS 21.8 / 26.9, Q4_0 19.4 / 24.2, 8192 -> 24576 at 9 rows 45.4 / 48.7)
-    if (p_rows <= 16)
-        return in_dim >= 3ull * out_dim ||
-               (fmt != REIN_TYPE_Q8_0 && in_dim >= 4096 && out_dim <= 18432 && (unsigned long long)in_dim * out_dim >= 56ull << 20);
-    // (17-32 rows: 3072 -> 24576 IQ4_XS 26.9 / 28.1 at 32, 1024 -> 20000 13.6 / 14.3; 4096 -> 18432 26.4 / 25.1, Q8_0 3072 -> 24576 29.7 / 27.6)
-    if (p_rows <= 32 && fmt != REIN_TYPE_Q8_0 && out_dim > 18432 && in_dim < 4096) return false;
-    // (33-128 rows: 2048 -> 32768 at 96 IQ4_XS 34.3 / 37.6, Q8_0 38.2 / 39.6, 1024 -> 20000 at 64 16.4 / 17.6, 16.3 / 17.7; 3072 -> 24576 36.9 / 35.5)
-    if (p_rows > 32 && p_rows <= 128 && in_dim <= 2048 && out_dim > 18432) return false;
-    // (65-192 rows: 2048 -> 12288 at 128 / 160 Q8_0 24.3 / 26.5, 24.7 / 26.2, IQ4_XS 26.2 / 26.9; level at 256, 58.1 / 45.7 at 400)
-    if (p_rows > 64 && p_rows <= 192 && in_dim <= 2048 && out_dim >= 4096 && out_dim <= 18432) return false;
-    return in_dim >= 2048 || p_rows <= 64 || p_rows > 400 || out_dim < 4096;
+    if (p_rows <= 16) {
+        if (out_dim <= 1024) return in_dim >= 3072;
+        if (in_dim >= 8192 && in_dim >= (in_dim >= 11008 ? 3ull : 4ull) * out_dim) return true;
+        return fmt != REIN_TYPE_Q8_0 && (in_dim >= 6144 || out_dim >= 16384) && out_dim <= 18432 && (unsigned long long)in_dim * out_dim >= 56ull << 20;
+    }
+    const unsigned long long pieces = ((unsigned long long)out_dim + 127) / 128 * ((p_rows + 31) / 32);
+    if (in_dim < 1536) return in_dim >= 768 && (pieces <= 64 || (pieces > 1024 && in_dim >= 1024));
+    return in_dim != 2048 || pieces <= 256 || pieces > 512;
 }
 // the launch of a shape, or null: those of rein_mmq_xq8_ws
 const WideKind* wide_kind(int fmt, unsigned in_dim, unsigned out_dim, unsigned p_rows)
@@ -2180,8 +2181,9 @@ size_t rein_matmul_scratch_bytes(int fmt, unsigned in_dim, unsigned n_rows)
     size_t behind = rein_matmul_path(fmt, n_rows) == 2 ? rein_mmq_workspace_bytes(fmt, in_dim, n_rows) : 0;
     if (rein_matmul_path(fmt, n_rows) == 2 && opt_u(O_MMQXH, 1) != 0 && in_dim % 256 == 0) {
         const size_t image = (wide_image_bytes(fmt, in_dim, n_rows) + 255) & ~(size_t)255;
-        if (!wide_k_quant(fmt)) behind = std::max(behind, image + wide_most_parts_bytes(kWideInt8, in_dim, n_rows));
-        else {
+        if (!wide_k_quant(fmt)) {
+            if (wide_int8_shape(in_dim)) behind = std::max(behind, image + wide_most_parts_bytes(kWideInt8, in_dim, n_rows));
+        } else {
             if (wide_exact_shape(fmt, in_dim, n_rows)) behind = std::max(behind, image + wide_most_parts_bytes(wide_exact(fmt), in_dim, n_rows));
             if (wide_few_shape(fmt, in_dim, n_rows)) behind = std::max(behind, image + wide_most_parts_bytes(kWideFew, in_dim, n_rows));
         }

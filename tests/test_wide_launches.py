@@ -40,3 +40,28 @@ def test_a_scratch_of_the_size_asked_for_holds_every_plan(mode, tags, tmp_path):
         names = [r[0] for r in done["launches"]]
         tag = tags[call[1][0]]
         assert names[:2] == [f"rein_{tag[:3]}quantize", "rein_" + tag] and names[2:] in ([], [f"rein_{tag[:3]}sum"]), call
+
+
+def wide(done):
+    return any(r[0].startswith(("rein_x8_", "rein_xf_", "rein_xh_")) for r in done["launches"])
+
+
+def taken(cases, tmp_path):
+    sizes = record([("matmul_scratch_bytes", [f, k, rows]) for f, k, _, rows, _ in cases], tmp_path)
+    done = record([("matmul_ws", [f, P, P, P, k, n, rows, P, size["value"]]) for (f, k, n, rows, _), size in zip(cases, sizes)], tmp_path)
+    for case, d in zip(cases, done):
+        kernels = [r[0] for r in d["launches"]]
+        assert wide(d) == bool(case[-1]), (case, kernels)
+        assert not wide(d) or f"rein_{case[-1]}" in kernels, (case, kernels)
+
+
+def test_where_the_int8_gemm_is_taken(tmp_path):
+    q8, q4, i4, i3 = rein.Q8_0, rein.Q4_0, rein.IQ4_XS, rein.IQ3_S
+    taken([(q8, 512, 4096, 64, 0), (q8, 512, 32, 33, 0), (i3, 256, 151936, 512, 0), (q4, 512, 65536, 2048, 0),          # short contractions
+           (q8, 768, 8192, 32, "x8_q8_0"), (q8, 768, 8320, 32, 0), (i4, 1024, 2048, 128, "x8_iq4xs"), (i4, 1024, 2048, 129, 0),          # 64 pieces and 65
+           (q4, 1280, 32768, 128, 0), (q4, 1280, 32768, 129, "x8_q4_0"), (q4, 768, 65536, 512, 0),          # 1024 pieces and 1280
+           (i3, 2048, 8192, 128, "x8_iq3s"), (i3, 2048, 8192, 129, 0), (q8, 2048, 8192, 256, 0), (q8, 2048, 8192, 257, "x8_q8_0"),
+           (q8, 1536, 32, 17, "x8_q8_0"), (i4, 2304, 8192, 256, "x8_iq4xs"), (q8, 5120, 17408, 2048, "x8_q8_0"),
+           (q8, 3072, 1024, 9, "x8_q8_0"), (q8, 2816, 256, 16, 0), (q4, 5120, 1536, 16, 0), (q8, 8192, 2048, 9, "x8_q8_0"), (q8, 8192, 2080, 9, 0),
+           (i4, 11008, 3584, 12, "x8_iq4xs"), (q4, 5120, 14336, 9, 0), (q4, 5120, 16384, 9, "x8_q4_0"), (i3, 6144, 12288, 16, "x8_iq3s"),
+           (q8, 6144, 12288, 16, 0), (q4, 5120, 18464, 16, 0)], tmp_path)
