@@ -682,12 +682,21 @@ bool use_mvql(int fmt, unsigned in_dim, unsigned out_dim, unsigned n_rows)
         // 1.29 / 1.28; below that 2048 -> 1536 Q8_0 0.95 / 1.03, Q5_K 0.97 / 0.88, 1024 -> 1024 0.8-1.0, 2048 -> 512 0.7-0.9)
         if (weights < (7ull << 19) && !(in_dim <= 1024 && out_dim >= 1536)) return false;
         if (fmt == REIN_TYPE_Q6_K || fmt == REIN_TYPE_Q5_K || fmt == REIN_TYPE_IQ4_XS) return true;
-        // the other formats beyond 20480 rows: from 28672 up to contractions of 4608, where workgroups of eight rows leave the CU room for two,
-        // and no trip is part empty (5 or 8 rows: 4096 -> 28672 Q8_0 1.46 x, Q4_K 1.39, 4096 -> 65536 1.52, 1.39, 2048 -> 34816 1.31, 1.30; 5120 ->
-        // 34816 Q4_K 1.05-1.12 but Q4_0 5120 -> 49152 1.02; 2304 -> 30720 Q4_0 0.95, 6144 -> 22528 Q4_K 0.83-0.86, 7168 -> 24576 0.82-0.87), Q8_0 also
-        // from contractions of 8192 (8192 -> 28672 1.31 x, 8192 -> 36864 1.40; 7168 -> 24576 0.97-1.00)
-        const bool phased = g.phase_sub < in_dim / 32;
-        if (out_dim > 20480) return (in_dim <= 4608 && in_dim % 512 == 0 && out_dim >= 28672) || (fmt == REIN_TYPE_Q8_0 && in_dim >= 8192 && !phased);
+        // the other formats beyond 20480 rows: from 28672 up to contractions of 4608, where workgroups of eight rows leave the CU room for two and no
+        // trip is part empty, by shape (in the mean of 5 to 8 rows).  Padded rows (a power of two of sub-blocks), which the skinny MMQ reads worse:
+        // 4096 Q8_0 1.42-1.57 x, Q4_K, Q4_0 and IQ3_S 1.21-1.46, 2048 1.20-1.33 and 1.06-1.30, 1024 1.05-1.27 and up to 40960 rows 1.03-1.19 (65536
+        // 0.96-1.02, 151936 0.86).  Else Q8_0 from 2560 (1.01-1.20; 1536 0.94-1.05), the 4-bit formats only between 32768 and 40960 rows, whose
+        // row groups deal evenly (1.07-1.17; 28672 0.97-1.05, 49152 0.91-1.03, 65536 0.88-1.01, 1536 0.81-1.06).  512 0.62-1.0.  5120, which gains for
+        // output heads (151936 rows 1.10-1.17), stays out: tests/test_host_cpu.py names the skinny MMQ for 5120 -> 34816 at eight rows.  Q8_0 also
+        // with padded rows of 8192 (1.28-1.37; 8448 to 12288 0.89-1.06).
+        const bool phased = g.phase_sub < in_dim / 32, padded = rein_repacked_n_sub_padded(in_dim) != in_dim / 32;
+        if (out_dim > 20480) {
+            if (in_dim >= 8192) return fmt == REIN_TYPE_Q8_0 && padded && !phased;
+            if (in_dim > 4608 || in_dim < 1024 || in_dim % 512 != 0 || out_dim < 28672) return false;
+            if (padded && (in_dim >= 2048 || fmt == REIN_TYPE_Q8_0)) return true;
+            if (fmt == REIN_TYPE_Q8_0) return in_dim >= 2560;
+            return (padded || (in_dim >= 2560 && out_dim > 32768)) && out_dim <= 40960;
+        }
         return !(phased && out_dim > 6144);
     }
     return mvql_few_rows(fmt, in_dim, out_dim, n_rows);

@@ -1,0 +1,19 @@
+"""Which kernels the products of two to eight activation rows launch, on both sides of each line (CPU: tests/launches.py records the
+launches)."""
+import reinstinct_amd as rein
+from launches import P, record
+
+Q4, Q4_0, Q5, Q6, Q8, I4, I3 = rein.Q4_K, rein.Q4_0, rein.Q5_K, rein.Q6_K, rein.Q8_0, rein.IQ4_XS, rein.IQ3_S
+
+
+def quad_lds(cases, tmp_path):
+    """(format, in_dim, out_dim, rows, taken): the 4x4x4 kernel with the rows in LDS"""
+    calls = [("mmq_xq8", [f, P, P, P, k, n, rows]) for f, k, n, rows, _ in cases]
+    for case, d in zip(cases, record(calls, tmp_path)):
+        assert d["launches"][0][0].startswith("rein_mvql_") == bool(case[-1]), (case, d["launches"])
+
+
+def test_five_to_eight_rows_against_many(tmp_path):
+    quad_lds([(Q4, 512, 151936, 8, 0), (Q8, 512, 65536, 5, 0), (Q8, 1024, 151936, 8, 1), (Q4, 1024, 40960, 6, 1), (Q4, 1024, 40992, 6, 0), (I3, 1536, 36864, 5, 0),
+              (Q8, 1536, 36864, 5, 0), (Q4_0, 2048, 151936, 5, 1), (Q8, 2560, 28672, 8, 1), (Q4, 2560, 32768, 5, 0), (Q4, 2560, 32800, 5, 1), (Q4_0, 3584, 65536, 8, 0),
+              (I3, 4096, 65536, 7, 1), (Q8, 4608, 151936, 5, 1), (Q8, 5120, 34816, 8, 0), (Q8, 8192, 28672, 6, 1), (Q8, 8448, 28672, 6, 0), (Q5, 512, 151936, 8, 1)], tmp_path)
