@@ -679,8 +679,11 @@ bool use_mvql(int fmt, unsigned in_dim, unsigned out_dim, unsigned n_rows)
     if (n_rows >= 5) {
         // from 3.5 * 2^20 weights, and with contractions of 1024 from 1536 rows, every format (dot4 -> this, 5 / 8 rows: 2304 -> 1664 Q4_K
         // 1.39 / 1.32 x, Q5_K 1.26 / 1.15, Q6_K 1.52 / 1.53; 6144 -> 640 1.30 / 1.23, 1.13 / 1.10, 1.72 / 1.73; 1024 -> 1536 1.28 / 1.11, 1.14 / 1.07,
-        // 1.29 / 1.28; below that 2048 -> 1536 Q8_0 0.95 / 1.03, Q5_K 0.97 / 0.88, 1024 -> 1024 0.8-1.0, 2048 -> 512 0.7-0.9)
+        // 1.29 / 1.28; below that 2048 -> 1536 Q8_0 0.95 / 1.03, Q5_K 0.97 / 0.88, 1024 -> 1024 0.8-1.0, 2048 -> 512 0.7-0.9), but for Q5_K, whose
+        // dot4 kernel fills the chip with one row to a wavefront from there, not between 832 and 1024 rows below five million (3584 -> 1024
+        // 0.83-0.86, 4096 -> 1024 0.88-0.91, 4096 -> 896 0.88; 4608 -> 832 1.01, 3584 -> 1088 1.21)
         if (weights < (7ull << 19) && !(in_dim <= 1024 && out_dim >= 1536)) return false;
+        if (fmt == REIN_TYPE_Q5_K && weights < (5ull << 20) && out_dim > 832 && out_dim <= 1024) return false;
         if (fmt == REIN_TYPE_Q6_K || fmt == REIN_TYPE_Q5_K || fmt == REIN_TYPE_IQ4_XS) return true;
         // the other formats beyond 20480 rows: from 28672 up to contractions of 4608, where workgroups of eight rows leave the CU room for two and no
         // trip is part empty, by shape (in the mean of 5 to 8 rows).  Padded rows (a power of two of sub-blocks), which the skinny MMQ reads worse:

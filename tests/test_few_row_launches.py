@@ -17,3 +17,8 @@ def test_five_to_eight_rows_against_many(tmp_path):
     quad_lds([(Q4, 512, 151936, 8, 0), (Q8, 512, 65536, 5, 0), (Q8, 1024, 151936, 8, 1), (Q4, 1024, 40960, 6, 1), (Q4, 1024, 40992, 6, 0), (I3, 1536, 36864, 5, 0),
               (Q8, 1536, 36864, 5, 0), (Q4_0, 2048, 151936, 5, 1), (Q8, 2560, 28672, 8, 1), (Q4, 2560, 32768, 5, 0), (Q4, 2560, 32800, 5, 1), (Q4_0, 3584, 65536, 8, 0),
               (I3, 4096, 65536, 7, 1), (Q8, 4608, 151936, 5, 1), (Q8, 5120, 34816, 8, 0), (Q8, 8192, 28672, 6, 1), (Q8, 8448, 28672, 6, 0), (Q5, 512, 151936, 8, 1)], tmp_path)
+
+
+def test_five_to_eight_rows_of_q5_k_against_a_thousand(tmp_path):
+    quad_lds([(Q5, 3584, 1024, 5, 0), (Q5, 4096, 864, 8, 0), (Q5, 4608, 832, 5, 1), (Q5, 3584, 1088, 6, 1), (Q5, 5120, 1024, 5, 1), (Q4, 4096, 1024, 5, 1),
+              (Q6, 3584, 1024, 5, 1)], tmp_path)
