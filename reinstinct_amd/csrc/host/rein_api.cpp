@@ -479,12 +479,13 @@ void mvl_geometry(int fmt, unsigned in_dim, unsigned out_dim, unsigned n_rows, u
 //   * between 8192 and 14336 rows, every format (us at 4 rows, 4x4x4 without LDS or dot4 with it -> this: 5120 -> 13824 Q4_K 14.0 -> 12.4, Q5_K
 //     17.7 -> 14.7; 8192 -> 10240 16.8 -> 15.6, 20.0 -> 19.1, Q6_K 24.5 -> 21.9; 4096 -> 11008 Q8_0 14.6 -> 11.7, IQ4_XS 10.0 -> 9.1; least Q8_0
 //     8192 -> 10240 1.04-1.06 x), with IQ3_S and IQ4_XS from 8192 (2048 -> 8192 1.08-1.13 x; Q4_K, Q5_K, Q6_K 0.9);
-//   * Q8_0 from 7168 rows where the contraction is shorter than 8192 (4096 -> 8192 11.2 -> 10.5, 6144 -> 8192 13.2 -> 11.8, 7168 -> 7168 12.5 ->
-//     12.0; 8192 -> 8192 14.6 -> 18.1, 5120 -> 5120 8.0 -> 8.6);
+//   * Q8_0 from 7168 rows at contractions from 3584 and shorter than 8192 (4096 -> 8192 11.2 -> 10.5, 6144 -> 8192 13.2 -> 11.8, 7168 -> 7168 12.5 ->
+//     12.0; 3072 -> 7168 7.5 -> 7.9, 2560 -> 7168 7.0 -> 7.4, 8192 -> 8192 14.6 -> 18.1, 5120 -> 5120 8.0 -> 8.6);
 //   * from 14336 rows: every format, IQ4_XS up to 16384 (4096 -> 14336 12.0 -> 10.7, 5120 -> 16384 1.05 x, 5120 -> 17408 16.0 -> 16.3; measured
 //     from steady clocks, 4x4x4 without LDS -> this at 4 rows: Q6_K 5120 -> 34816 40.7 -> 36.7, 6144 -> 16384 23.6 -> 21.7, 3584 -> 18944 18.2 -> 17.9);
 //   * below 2^24 weights, from 4096 rows and four million weights against contractions up to 2560 (dot4 -> this at 3 / 4 rows: 1024 -> 6144 Q4_K
-//     1.35 / 1.47 x, 2048 -> 4608 1.22 / 1.36, 2560 -> 6912 1.12 / 1.12, Q5_K 1.30 / 1.40, 1.07 / 1.14, 0.99 / 1.00, Q4_0 and IQ3_S as Q4_K; at four
+//     1.35 / 1.47 x, 2048 -> 4608 1.22 / 1.36, 2560 -> 6912 1.12 / 1.12, Q4_0 and IQ3_S as Q4_K; Q5_K, against the 4x4x4 kernel without LDS, up to ten
+//     million: 1024 -> 6144 1.06, 1536 -> 6144 1.07, 2048 -> 4096 1.14, but 1536 -> 7168 0.95, 2048 -> 7168 0.90, 2304 -> 5120 0.99; at four
 //     rows only Q8_0 1.36, 1.12, 0.98 (three: 1.08, 0.96, 0.96) and IQ4_XS 1.49, 1.33, 1.12 (1.05, 1.06, 0.97); Q6_K up to 1280 only: 1024 -> 6144
 //     1.12 / 1.17, 1536 -> 6144 0.93 / 0.95).
 bool mvql_few_rows(int fmt, unsigned in_dim, unsigned out_dim, unsigned n_rows)
@@ -497,11 +498,12 @@ bool mvql_few_rows(int fmt, unsigned in_dim, unsigned out_dim, unsigned n_rows)
     if (weights >= (6ull << 20) && weights < (1ull << 24) && out_dim >= 8192) return true;
     if (weights < (1ull << 24)) {
         const bool four = fmt == REIN_TYPE_Q8_0 || fmt == REIN_TYPE_IQ4_XS;
+        if (fmt == REIN_TYPE_Q5_K && weights >= (10ull << 20)) return false;
         return out_dim >= 4096 && weights >= (4ull << 20) && in_dim <= (fmt == REIN_TYPE_Q6_K ? 1280u : 2560u) && (n_rows == 4 || !four);
     }
-    if (fmt == REIN_TYPE_Q8_0) return out_dim > 8192 || (out_dim >= 7168 && in_dim < 8192);
+    if (fmt == REIN_TYPE_Q8_0) return out_dim > 8192 || (out_dim >= 7168 && in_dim >= 3584 && in_dim < 8192);
     if (fmt == REIN_TYPE_IQ4_XS) return out_dim >= 8192 && out_dim <= 16384;
-    return out_dim > 8192 || (fmt == REIN_TYPE_IQ3_S && out_dim == 8192);
+    return out_dim >= (fmt == REIN_TYPE_IQ3_S ? 8192u : 8193u);
 }
 
 bool use_mvl(int fmt, unsigned in_dim, unsigned out_dim, unsigned n_rows)
