@@ -2058,11 +2058,16 @@ unsigned wide_lds_bytes(const WideKind& kind, int fmt)
 //     Q5_K  65-383 rows contractions of 3072 and more against 48M weights (0.90-1.97, median 1.2), from 101 rows 24M (5120 -> 5120
 //           1.10-1.46; 80 rows 0.96), and narrow ones of 5M (5632 -> 2048, 5120 -> 1024 1.0-1.13); 3072 -> 3072 0.88-0.95 at 80-200 rows.  From 384 rows
 //           contractions of 4096 and more (1.07-1.52), of 3072 against 16384 rows and more (1.18-1.31), from 1024 rows of 1536 (1.04-1.29).
-//   few, the same shapes, 12-64 rows:
-//     Q6_K  17-32 rows 1.14-1.41 in all 26 cells (17408 -> 5120 43 / 34 us)
-//     Q4_K, Q5_K  17-32 rows up to 16384 rows of weights 1.01-1.23 (beyond 0.91-1.02); Q5_K at 33-64 rows 1.05-1.26 in all 26 (17408 -> 5120,
-//           45 rows 42 / 37).
-//     9-16 rows matrices of 60M weights (Q5_K 85M): 1.03-1.32; smaller ones 0.82-1.05.  Matrices below 4M weights were not measured.
+//   few, 18 contractions x 44 row counts of weights x 9 of activations, 9-64 rows (Q5_K 33-64), from 4M weights:
+//     17-32 rows Q6_K 1.03-1.69 in the mean of every cell of (contraction, weight rows) from contractions of 512 (256 0.97; 17408 -> 5120 43 / 34 us);
+//           Q4_K and Q5_K from 1024 up to 8192 rows of weights 1.02-1.36 (10240 0.91 and 0.97), from 1280 up to 12288 (0.96-1.23; beyond 0.85-1.04),
+//           from 10240 up to 5120 (1.03-1.13; 14336 -> 10240 0.94 and 0.91, 17408 -> 6144 0.94 and 0.95).  512 and 768 0.83-0.95.
+//     33-64 rows Q5_K 1.00-1.38 from contractions of 1024 (17408 -> 5120, 45 rows 42 / 37); 256 to 768 0.78-0.95, and below 3072 against 32769 to
+//           49152 rows, where every workgroup of the plain launch is resident at once, 0.87-0.94 (65536 1.07-1.19).
+//     9-16 rows large matrices against which the few-row kernels deal badly: Q6_K 60M weights up to 18432 rows (1.05-1.51), 72M where those
+//           deal evenly (8192 -> 8192 0.95, 4096 -> 16384 0.89, 14336 -> 8192 1.08); Q4_K
+//           contractions of 10752 and more up to 6144 rows and from 8193 to 18432 (60M: 1.01-1.33; 11008 -> 7168 and 8192 0.91-0.93), shorter ones
+//           and Q5_K's below 8192 against more than 16384 rows (85M: 1.06-1.21; 8192 -> 14336 0.93, 6144 -> 16384 0.96, Q5_K 11008 -> 8192 0.91).
 bool wide_exact_shape(int fmt, unsigned in_dim, unsigned p_rows)          // for any number of weight rows
 {
     const unsigned mode = opt_u(O_MMQXH, 1);
@@ -2081,28 +2086,26 @@ bool wide_exact_take(int fmt, unsigned in_dim, unsigned out_dim, unsigned p_rows
     if (p_rows >= 384) return in_dim >= 4096 || out_dim >= 16384 || p_rows >= 1024;
     return weights >= (p_rows > 100 ? 24ull << 20 : 48ull << 20) || (2ull * in_dim >= 5ull * out_dim && weights >= 5ull << 20);
 }
-bool wide_few_shape(int fmt, unsigned, unsigned p_rows)
+bool wide_few_shape(int fmt, unsigned in_dim, unsigned p_rows)
 {
     const unsigned mode = opt_u(O_MMQXH, 1);
     if (mode == 3) return p_rows > 8;
-    return mode == 1 && p_rows > 8 && p_rows <= (fmt == REIN_TYPE_Q5_K ? 64u : 32u);
+    return mode == 1 && p_rows > 8 && p_rows <= (fmt == REIN_TYPE_Q5_K ? 64u : 32u) && in_dim >= (fmt == REIN_TYPE_Q6_K ? 512u : 1024u);
 }
 bool wide_few_take(int fmt, unsigned in_dim, unsigned out_dim, unsigned p_rows)
 {
     if (!wide_few_shape(fmt, in_dim, p_rows)) return false;
     if (opt_u(O_MMQXH, 1) == 3) return true;
     const unsigned long long weights = (unsigned long long)in_dim * out_dim;
-    // (9-16 rows, other launches / this: Q4_K 8192 -> 8192 24.8 / 21.7, 5120 -> 17408 26.5 / 24.5, but 5120 -> 13824 20.1 / 21.6, 3072 -> 24576 19.7 /
-    // 21.3; Q5_K 6144 -> 18432 37.6 / 34.9, 8192 -> 14336 41.0 / 42.7 at 9 rows, 8192 -> 24576 60.5 / 75.0; Q6_K 5120 -> 17408 40.0 / 32.4, 8192 ->
-    // 24576 70.1 / 76.6)
     if (p_rows <= 16) {
         if (out_dim > 18432) return false;
-        if (fmt == REIN_TYPE_Q6_K) return weights >= 60ull << 20;
-        if (fmt == REIN_TYPE_Q5_K) return weights >= 85ull << 20 && (in_dim < 8192 || out_dim <= 8192);
-        return weights >= (in_dim >= 8192 ? 60ull << 20 : 85ull << 20);
+        if (fmt == REIN_TYPE_Q6_K) return weights >= (out_dim % 8192 ? 60ull : 72ull) << 20;
+        if (fmt == REIN_TYPE_Q4_K && in_dim >= 10752) return weights >= 60ull << 20 && (out_dim <= 6144 || out_dim > 8192);
+        return weights >= 85ull << 20 && out_dim > 16384 && (fmt == REIN_TYPE_Q4_K || in_dim < 8192);
     }
-    // (17-32 rows: Q4_K 8192 -> 8192 23.9 / 22.0, 8192 -> 14336 33.0 / 34.0, 5120 -> 13824 23.1 / 23.9, Q5_K 8192 -> 14336 39.8 / 42.9)
-    return weights >= 4ull << 20 && (fmt == REIN_TYPE_Q6_K || p_rows > 32 || out_dim <= 12288);
+    if (weights < 4ull << 20) return false;
+    if (p_rows > 32) return in_dim >= 3072 || out_dim <= 32768 || out_dim > 49152;          // 513 to 768 workgroups of the plain launch
+    return fmt == REIN_TYPE_Q6_K || out_dim <= (in_dim < 1280 ? 8192u : in_dim < 10240 ? 12288u : 5120u);
 }
 bool wide_int8_shape(unsigned in_dim) { return in_dim >= 768 || opt_u(O_MMQXH, 1) >= 2; }          // for any number of weight rows
 bool wide_int8_take(int fmt, unsigned in_dim, unsigned out_dim, unsigned p_rows)

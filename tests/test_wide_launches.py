@@ -65,3 +65,14 @@ def test_where_the_int8_gemm_is_taken(tmp_path):
            (q8, 3072, 1024, 9, "x8_q8_0"), (q8, 2816, 256, 16, 0), (q4, 5120, 1536, 16, 0), (q8, 8192, 2048, 9, "x8_q8_0"), (q8, 8192, 2080, 9, 0),
            (i4, 11008, 3584, 12, "x8_iq4xs"), (q4, 5120, 14336, 9, 0), (q4, 5120, 16384, 9, "x8_q4_0"), (i3, 6144, 12288, 16, "x8_iq3s"),
            (q8, 6144, 12288, 16, 0), (q4, 5120, 18464, 16, 0)], tmp_path)
+
+
+def test_where_the_small_groups_are_taken(tmp_path):
+    q4, q5, q6 = rein.Q4_K, rein.Q5_K, rein.Q6_K
+    taken([(q6, 256, 32768, 17, 0), (q6, 512, 16384, 32, "xf_q6k"), (q6, 8192, 8192, 9, 0), (q6, 11008, 8192, 9, "xf_q6k"), (q6, 6144, 10240, 16, "xf_q6k"), (q6, 8192, 18464, 16, 0), (q6, 2048, 1024, 32, 0),
+           (q4, 768, 8192, 32, 0), (q4, 1024, 8192, 32, "xf_q4k"), (q5, 1024, 8224, 17, 0), (q4, 1280, 12288, 24, "xf_q4k"), (q4, 4096, 12320, 24, 0),
+           (q5, 9984, 12288, 32, "xf_q5k"), (q5, 10240, 5152, 32, 0), (q5, 17408, 5120, 17, "xf_q5k"), (q4, 14336, 10240, 24, 0),
+           (q5, 768, 32768, 33, 0), (q5, 1024, 32768, 64, "xf_q5k"), (q5, 2816, 32800, 64, 0), (q5, 3072, 32800, 64, "xf_q5k"), (q5, 2816, 49184, 33, "xf_q5k"),
+           (q5, 256, 151936, 64, 0),
+           (q4, 11008, 8192, 9, 0), (q4, 11008, 6144, 9, "xf_q4k"), (q4, 10752, 8224, 16, "xf_q4k"), (q4, 8192, 14336, 12, 0), (q4, 6144, 16384, 9, 0),
+           (q4, 5120, 17408, 9, "xf_q4k"), (q5, 6144, 18432, 16, "xf_q5k"), (q5, 11008, 8192, 9, 0), (q5, 17408, 5120, 12, 0)], tmp_path)
