@@ -805,10 +805,14 @@ unsigned multi_blocks(unsigned n_mat, const unsigned* out_dims, unsigned rows)
 //             Q4_0, IQ3_S from a contraction of 3072 (3072 -> 2 x 8192 Q4_K 14.3 / 11.8, 1536 -> 2 x 5120 6.4 / 6.5), not in IQ4_XS
 //             (2560 -> 2 x 8960 14.5 / 16.6), nor three (4096 -> 3 x 4096 Q4_K with Q6_K 14.3 / 14.8).
 //   2 rows    at most 8192 rows in all and at most one and a half times the contraction (5120 -> 5120 + 2 x 1024 9.7 / 9.2, 2560 -> 2560 +
-//             2 x 640 Q5_K with Q6_K 6.1 / 5.4; Q8_0 and Q4_0 not from 4097 to 5120 rows of 3584 and more: 4096 -> 4096 + 2 x 512 6.9 /
-//             7.2); contractions of 8192 and more (8192 -> 2 x 24576 Q4_K 50.8 / 42.2, Q8_0 83.1 / 71.8); Q4_K and Q8_0 from 6144 against
+//             2 x 640 Q5_K with Q6_K 6.1 / 5.4), but Q8_0, Q4_0, IQ3_S and IQ4_XS not with 4097 to 5120 rows, where two workgroups
+//             of nine or ten wavefronts to a CU both stage the activations (Q4_0 0.89-0.93 x whatever the contraction, IQ3_S 0.89-0.99, Q8_0
+//             0.94-1.00, IQ4_XS 0.92-1.03; 5376 rows 0.99-1.20), and Q8_0 up to contractions of 4096 not up to 6144 (0.93-0.96);
+//             contractions of 8192 and more (8192 -> 2 x 24576 Q4_K 50.8 / 42.2, Q8_0 83.1 / 71.8; IQ4_XS up to
+//             three times that, 1.06-1.23, but 2 x 24576 51.2 / 54.4, 2 x 28672 60.5 / 68.1); Q4_K and Q8_0 from 6144 against
 //             four times that (6144 -> 2 x 18432 26.4 / 24.3, 41.8 / 39.1, but Q6_K 37.6 / 39.3).  Between, level or behind (2048 -> 2 x
 //             8192 Q4_K 6.7 / 7.8, 4096 -> 2 x 14336 Q6_K 22.0 / 24.5).
+//   none from contractions below 512 (256: 2.6 / 2.8 whatever the format and the rows; 512 0.97-1.18 x).
 MultiLds multi_dot4_lds(unsigned n_mat, unsigned in_dim, const unsigned* out_dims, unsigned n_rows, int lead)
 {
     MultiLds p{};
@@ -820,13 +824,15 @@ MultiLds multi_dot4_lds(unsigned n_mat, unsigned in_dim, const unsigned* out_dim
     } else {
         if (opt_is_set(O_SKINNY_FROM) || opt_is_set(O_QUAD_FROM) || opt_is_set(O_MV_ROWS)) return p;
         const bool heavy = lead == REIN_TYPE_Q5_K || lead == REIN_TYPE_Q6_K || lead == REIN_TYPE_Q8_0;
+        if (in_dim < 512) return p;
         if (n_rows >= 3) {
             if (total > 2ull * in_dim && !(n_mat == 2 && (heavy ? total * in_dim >= (8ull << 20) : in_dim >= 3072 && lead != REIN_TYPE_IQ4_XS))) return p;
         } else {
-            const bool light = lead == REIN_TYPE_Q8_0 || lead == REIN_TYPE_Q4_0;
-            const bool narrow = total <= 8192 && 2 * total <= 3ull * in_dim && !(light && in_dim >= 3584 && total > 4096 && total <= 5120);
+            const bool light = lead != REIN_TYPE_Q4_K && lead != REIN_TYPE_Q5_K && lead != REIN_TYPE_Q6_K;
+            const bool narrow = total <= 8192 && 2 * total <= 3ull * in_dim && !(light && total > 4096 && total <= (lead == REIN_TYPE_Q8_0 && in_dim <= 4096 ? 6144u : 5120u));
             const bool tall = in_dim >= 6144 && total >= 4ull * in_dim && (lead == REIN_TYPE_Q4_K || lead == REIN_TYPE_Q8_0);
-            if (!narrow && !tall && in_dim < 8192) return p;
+            const bool deep = in_dim >= 8192 && (lead != REIN_TYPE_IQ4_XS || total <= 3ull * in_dim);
+            if (!narrow && !tall && !deep) return p;
         }
     }
     const unsigned copies = (unsigned)std::min<size_t>(4, kLdsPerCu / mvl_lds_bytes(in_dim, n_rows));

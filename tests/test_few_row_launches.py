@@ -28,3 +28,15 @@ def test_three_and_four_rows_of_q5_k_and_q8_0(tmp_path):
     quad_lds([(Q5, 2048, 5088, 3, 1), (Q5, 2048, 5120, 3, 0), (Q5, 1536, 7168, 4, 0), (Q5, 1536, 6144, 4, 1), (Q5, 2560, 4608, 3, 0), (Q5, 1024, 8192, 3, 1),
               (Q4, 2048, 7168, 4, 1), (Q8, 3072, 7168, 3, 0), (Q8, 3328, 8192, 4, 0), (Q8, 3584, 7168, 3, 1), (Q8, 3072, 8224, 4, 1),
               (I3, 2304, 8192, 3, 1), (I3, 2304, 8224, 3, 1), (Q4, 2304, 8192, 3, 0)], tmp_path)
+
+
+def test_several_matrices_with_the_activations_in_lds(tmp_path):
+    cases = [([Q4, Q4, Q6], 256, [256, 128, 128], 3, 0), ([Q8, Q8], 256, [256, 256], 4, 0), ([Q4, Q4, Q6], 512, [512, 128, 128], 3, 1),
+             ([Q4_0] * 3, 3072, [3072, 768, 768], 2, 0), ([I3] * 3, 4096, [4096, 512, 512], 2, 0), ([I4, I4, Q5], 3584, [3584, 448, 448], 2, 0),
+             ([Q8] * 3, 4096, [4096, 1024, 1024], 2, 0), ([Q8] * 3, 5120, [4096, 1024, 1024], 2, 1), ([Q4_0] * 3, 5120, [4096, 512, 513], 2, 1), ([Q4, Q4, Q6], 4096, [4096, 1024, 1024], 2, 1),
+             ([Q8] * 3, 3072, [3072, 512, 512], 2, 1), ([I4, I4], 8192, [12288, 12288], 2, 1), ([I4, I4], 8192, [12288, 12320], 2, 0),
+             ([Q4_0, Q4_0], 8192, [24576, 24576], 2, 1)]
+    calls = [("matvec_multi_xq8", [f, [P] * len(f), [P] * len(f), outs, P, k, rows]) for f, k, outs, rows, _ in cases]
+    for case, d in zip(cases, record(calls, tmp_path)):
+        (kernel, *_), = d["launches"]
+        assert kernel.startswith("rein_mvl_multi_" if case[-1] else "rein_mv_multi_"), (case, kernel)
