@@ -2061,9 +2061,12 @@ unsigned wide_lds_bytes(const WideKind& kind, int fmt)
 //           and more against matrices of 48M weights (1.09-1.36; 5120 -> 5120 0.90: three tiles at the cost of a whole group's unpack);
 //           from 96 rows contractions of 4096 and more, 0.86-1.85, median 1.10 (below, 0.70-1.22: ranges of few superblocks do not
 //           pay back their starts and the image).
-//     Q5_K  65-383 rows contractions of 3072 and more against 48M weights (0.90-1.97, median 1.2), from 101 rows 24M (5120 -> 5120
-//           1.10-1.46; 80 rows 0.96), and narrow ones of 5M (5632 -> 2048, 5120 -> 1024 1.0-1.13); 3072 -> 3072 0.88-0.95 at 80-200 rows.  From 384 rows
-//           contractions of 4096 and more (1.07-1.52), of 3072 against 16384 rows and more (1.18-1.31), from 1024 rows of 1536 (1.04-1.29).
+//     Q5_K  65-383 rows contractions of 3072 and more against 48M weights (0.96-1.97, mean 1.27), from 101 rows 24M (5120 -> 5120
+//           1.10-1.46; 80 rows 0.96), and narrow ones of 5M (5632 -> 2048, 5120 -> 1024 1.0-1.13; up to 100 rows not against less than a
+//           twentieth of the contraction, 17408 -> 640 0.91-0.94); not 3072 against what the plain launch has on the chip at once with three
+//           workgroups to a CU (160 x 3072 -> 17408 0.92, 18432 0.91; 200 1.1).  From 384 rows contractions of 4096 and more (1.07-1.52), of
+//           3072 against 16384 rows and more (1.18-1.31), from 1024 rows 3072 (1.00-1.26) and, against 4096 rows and more, 1536
+//           (1.01-1.32 in the mean; 1536 -> 3072 0.85, 2304 -> 3072 0.89).
 //   few, 18 contractions x 44 row counts of weights x 9 of activations, 9-64 rows (Q5_K 33-64), from 4M weights:
 //     17-32 rows Q6_K 1.03-1.69 in the mean of every cell of (contraction, weight rows) from contractions of 512 (256 0.97; 17408 -> 5120 43 / 34 us);
 //           Q4_K and Q5_K from 1024 up to 8192 rows of weights 1.02-1.36 (10240 0.91 and 0.97), from 1280 up to 12288 (0.96-1.23; beyond 0.85-1.04),
@@ -2089,8 +2092,11 @@ bool wide_exact_take(int fmt, unsigned in_dim, unsigned out_dim, unsigned p_rows
     const unsigned long long weights = (unsigned long long)in_dim * out_dim;
     if (fmt == REIN_TYPE_Q6_K) return 2.0 * p_rows * (double)weights >= 2.5e8;
     if (fmt == REIN_TYPE_Q4_K) return p_rows <= 64 || p_rows >= 96 || weights >= 48ull << 20;
-    if (p_rows >= 384) return in_dim >= 4096 || out_dim >= 16384 || p_rows >= 1024;
-    return weights >= (p_rows > 100 ? 24ull << 20 : 48ull << 20) || (2ull * in_dim >= 5ull * out_dim && weights >= 5ull << 20);
+    if (p_rows >= 384) return in_dim >= 4096 || out_dim >= 16384 || (p_rows >= 1024 && (in_dim >= 3072 || out_dim >= 4096));
+    const unsigned long long pieces = ((unsigned long long)out_dim + 127) / 128 * ((p_rows + 31) / 32);
+    if (in_dim < 4096 && pieces > 640 && pieces <= 768) return false;                 // the plain launch's three workgroups on every CU
+    return weights >= (p_rows > 100 ? 24ull << 20 : 48ull << 20) ||
+           (2ull * in_dim >= 5ull * out_dim && weights >= 5ull << 20 && (p_rows > 100 || in_dim <= 20ull * out_dim));
 }
 bool wide_few_shape(int fmt, unsigned in_dim, unsigned p_rows)
 {

@@ -76,3 +76,10 @@ def test_where_the_small_groups_are_taken(tmp_path):
            (q5, 256, 151936, 64, 0),
            (q4, 11008, 8192, 9, 0), (q4, 11008, 6144, 9, "xf_q4k"), (q4, 10752, 8224, 16, "xf_q4k"), (q4, 8192, 14336, 12, 0), (q4, 6144, 16384, 9, 0),
            (q4, 5120, 17408, 9, "xf_q4k"), (q5, 6144, 18432, 16, "xf_q5k"), (q5, 11008, 8192, 9, 0), (q5, 17408, 5120, 12, 0)], tmp_path)
+
+
+def test_where_the_exact_dot_gemm_of_q5_k_is_taken(tmp_path):
+    q5, kernel = rein.Q5_K, "xh_q5k"
+    taken([(q5, 1536, 4064, 1024, 0), (q5, 1536, 4096, 1024, kernel), (q5, 2816, 3072, 1024, 0), (q5, 3072, 512, 1024, kernel), (q5, 2816, 18944, 1023, 0),
+           (q5, 3072, 17408, 160, 0), (q5, 3072, 17408, 161, kernel), (q5, 4096, 17408, 160, kernel), (q5, 17408, 832, 65, 0), (q5, 17408, 1024, 65, kernel),
+           (q5, 17408, 640, 101, kernel), (q5, 8192, 640, 100, kernel)], tmp_path)
