@@ -859,9 +859,11 @@ MultiLds multi_dot4_lds(unsigned n_mat, unsigned in_dim, const unsigned* out_dim
 // Two matrices of an FFN's size on the 4x4x4 kernel with the rows in LDS, each in as many slices as its launch alone (the order of a
 // row's sums): the activations are staged once, a wavefront's weights come in without a break, and 28 to 63 row groups to a CU deal
 // better than half as many (us at 4 rows, two launches / this: 4096 -> 2 x 14336 Q4_K 20.1 / 17.4, Q5_K 23.8 / 20.6, Q6_K 30.2 / 26.3,
-// Q8_0 29.6 / 26.6; 5120 -> 2 x 17408 30.2 / 22.6, 33.8 / 26.9, 42.8 / 33.9, 41.2 / 31.3; 7168 -> 2 x 24576 42.3 / 37.5, 47.9 / 44.7, 59.0 / 58.2,
-// 60.7 / 57.5; Q4_K with Q6_K 5120 -> 2 x 17408 36.5 / 33.4, but three matrices 51.3 / 53.6).  One workgroup per CU, sixteen wavefronts
-// at most; two of ten for Q8_0 from a contraction of 8192 (8192 -> 2 x 24576 85.5 on two launches, 87.7 / 85.5 with one / two).
+// 5120 -> 2 x 17408 30.2 / 22.6, 33.8 / 26.9, 42.8 / 33.9, Q8_0 41.2 / 31.3; 7168 -> 2 x 24576 42.3 / 37.5, 47.9 / 44.7, 59.0 / 58.2,
+// 60.7 / 57.5; Q4_K with Q6_K 5120 -> 2 x 17408 36.5 / 33.4, but three matrices 51.3 / 53.6).  Padded Q8_0 rows (4096, 8192) are read by the
+// plain build, which has no launch of two.  One workgroup per CU, sixteen wavefronts at most; two of ten for Q8_0 from a contraction of 8192
+// are level against many rows and behind against few (8448 -> 2 x 8200 one / two 26.5 / 28.6, 12288 -> 2 x 12288 50.7 / 56.9, 10240 -> 2 x 24576
+// 81.8 / 82.3; as two launches 37.3, 55.4, 86.7).
 MultiLds multi_quad_lds(unsigned n_mat, const int* fmts, unsigned in_dim, const unsigned* out_dims, unsigned n_rows)
 {
     MultiLds p{};
@@ -884,10 +886,11 @@ MultiLds multi_quad_lds(unsigned n_mat, const int* fmts, unsigned in_dim, const 
         for (unsigned i = 0; i < 2; i++)
             p.rows[i] = 4 * (g[i].slices > 1 ? p.wpb / g[i].slices : p.wpb * (((out_dims[i] + 3) / 4 + kCUs * p.wpb - 1) / (kCUs * p.wpb)));
     } else {
-        const unsigned c = parts == 3 && in_dim >= 8192 ? 2 : 1, most = c == 2 ? 10 : 16;
-        unsigned rounds = (multi_blocks(2, out_dims, 4) + kCUs * c * most - 1) / (kCUs * c * most);
-        while (multi_blocks(2, out_dims, 4 * most * rounds) > kCUs * c) rounds++;
-        for (p.wpb = 1; multi_blocks(2, out_dims, 4 * p.wpb * rounds) > kCUs * c; p.wpb++) {}
+        unsigned most = 16;
+        while (most > 1 && quad_lds_bytes(4, in_dim / 32, most, parts) > kLdsPerCu) most--;
+        unsigned rounds = (multi_blocks(2, out_dims, 4) + kCUs * most - 1) / (kCUs * most);
+        while (multi_blocks(2, out_dims, 4 * most * rounds) > kCUs) rounds++;
+        for (p.wpb = 1; multi_blocks(2, out_dims, 4 * p.wpb * rounds) > kCUs; p.wpb++) {}
         p.rows[0] = p.rows[1] = 4 * p.wpb * rounds;
     }
     p.rows[2] = p.rows[3] = p.rows[1];

@@ -40,3 +40,25 @@ def test_several_matrices_with_the_activations_in_lds(tmp_path):
     for case, d in zip(cases, record(calls, tmp_path)):
         (kernel, *_), = d["launches"]
         assert kernel.startswith("rein_mvl_multi_" if case[-1] else "rein_mv_multi_"), (case, kernel)
+
+
+def test_two_matrices_in_one_launch_of_the_4x4x4_kernel(tmp_path):
+    """(Q8_0 from a contraction of 8192: one workgroup to a CU, of as many wavefronts as its LDS holds)"""
+    cases = [([Q8, Q8], 8448, [8200, 8200], 1), ([Q8, Q8], 12288, [12288, 12288], 1), ([Q8, Q8], 22528, [8200, 8200], 1), ([Q8, Q8], 8192, [8200, 8200], 0),
+             ([Q4, Q4], 5120, [17408, 17408], 1)]
+    calls = [("matvec_multi_xq8", [f, [P] * 2, [P] * 2, outs, P, k, 4]) for f, k, outs, _ in cases]
+    for case, d in zip(cases, record(calls, tmp_path)):
+        assert len(d["launches"]) == (1 if case[-1] else 2), case
+        if case[-1]:
+            (kernel, grid, block, lds), = d["launches"]
+            assert kernel == "rein_mvql_multi_t4_m" and grid[0] <= 256 and lds <= 160 << 10, (case, d["launches"])
+
+
+def test_the_gpu_cases_of_several_matrices_launch_what_they_name(tmp_path):
+    from test_gpu_matvec_multi_lds import DOT4, MATRIX
+    for pin, cases, kernel in ((("REIN_MV_LDS", "1"), [c + (r, None) for c in DOT4 for r in (2, 3, 4)], "rein_mvl_multi_"), (None, MATRIX, "rein_mvql_multi_t4_m")):
+        for fmts, k, outs, rows, quad in cases:
+            pins = [("option", list(p)) for p in (pin, quad and ("REIN_QUAD_LDS", quad)) if p]
+            done = record(pins + [("matvec_multi_xq8", [fmts, [P] * len(fmts), [P] * len(fmts), outs, P, k, rows])], tmp_path)[-1]
+            (name, *_), = done["launches"]
+            assert name.startswith(kernel), (fmts, k, outs, rows, name)
