@@ -483,7 +483,8 @@ void mvl_geometry(int fmt, unsigned in_dim, unsigned out_dim, unsigned n_rows, u
 //     12.0; 3072 -> 7168 7.5 -> 7.9, 2560 -> 7168 7.0 -> 7.4, 8192 -> 8192 14.6 -> 18.1, 5120 -> 5120 8.0 -> 8.6);
 //   * from 14336 rows: every format, IQ4_XS up to 16384 (4096 -> 14336 12.0 -> 10.7, 5120 -> 16384 1.05 x, 5120 -> 17408 16.0 -> 16.3; measured
 //     from steady clocks, 4x4x4 without LDS -> this at 4 rows: Q6_K 5120 -> 34816 40.7 -> 36.7, 6144 -> 16384 23.6 -> 21.7, 3584 -> 18944 18.2 -> 17.9);
-//   * below 2^24 weights, from 4096 rows and four million weights against contractions up to 2560 (dot4 -> this at 3 / 4 rows: 1024 -> 6144 Q4_K
+//   * below 2^24 weights, from 4096 rows and four million weights against contractions of 512 to 2560 (Q8_0 256 -> 22464 at 4 rows, skinny MMQ ->
+//     this 3.9 -> 5.3 us; dot4 -> this at 3 / 4 rows: 1024 -> 6144 Q4_K
 //     1.35 / 1.47 x, 2048 -> 4608 1.22 / 1.36, 2560 -> 6912 1.12 / 1.12, Q4_0 and IQ3_S as Q4_K; Q5_K, against the 4x4x4 kernel without LDS, up to ten
 //     million: 1024 -> 6144 1.06, 1536 -> 6144 1.07, 2048 -> 4096 1.14, but 1536 -> 7168 0.95, 2048 -> 7168 0.90, 2304 -> 5120 0.99; at four
 //     rows only Q8_0 1.36, 1.12, 0.98 (three: 1.08, 0.96, 0.96) and IQ4_XS 1.49, 1.33, 1.12 (1.05, 1.06, 0.97); Q6_K up to 1280 only: 1024 -> 6144
@@ -498,7 +499,7 @@ bool mvql_few_rows(int fmt, unsigned in_dim, unsigned out_dim, unsigned n_rows)
     if (weights >= (6ull << 20) && weights < (1ull << 24) && out_dim >= 8192) return true;
     if (weights < (1ull << 24)) {
         const bool four = fmt == REIN_TYPE_Q8_0 || fmt == REIN_TYPE_IQ4_XS;
-        if (fmt == REIN_TYPE_Q5_K && weights >= (10ull << 20)) return false;
+        if (in_dim < 512 || (fmt == REIN_TYPE_Q5_K && weights >= (10ull << 20))) return false;
         return out_dim >= 4096 && weights >= (4ull << 20) && in_dim <= (fmt == REIN_TYPE_Q6_K ? 1280u : 2560u) && (n_rows == 4 || !four);
     }
     if (fmt == REIN_TYPE_Q8_0) return out_dim > 8192 || (out_dim >= 7168 && in_dim >= 3584 && in_dim < 8192);

@@ -26,7 +26,7 @@ def test_five_to_eight_rows_of_q5_k_against_a_thousand(tmp_path):
 
 def test_three_and_four_rows_of_q5_k_and_q8_0(tmp_path):
     quad_lds([(Q5, 2048, 5088, 3, 1), (Q5, 2048, 5120, 3, 0), (Q5, 1536, 7168, 4, 0), (Q5, 1536, 6144, 4, 1), (Q5, 2560, 4608, 3, 0), (Q5, 1024, 8192, 3, 1),
-              (Q4, 2048, 7168, 4, 1), (Q8, 3072, 7168, 3, 0), (Q8, 3328, 8192, 4, 0), (Q8, 3584, 7168, 3, 1), (Q8, 3072, 8224, 4, 1),
+              (Q4, 2048, 7168, 4, 1), (Q8, 3072, 7168, 3, 0), (Q8, 3328, 8192, 4, 0), (Q8, 3584, 7168, 3, 1), (Q8, 3072, 8224, 4, 1), (Q8, 256, 22464, 4, 0), (Q8, 512, 10240, 4, 1),
               (I3, 2304, 8192, 3, 1), (I3, 2304, 8224, 3, 1), (Q4, 2304, 8192, 3, 0)], tmp_path)
 
 
