@@ -2249,7 +2249,8 @@ int rein_matmul_ws(int fmt, const void* w, const float* x, float* y, unsigned in
             if (int rc = launch(KName("rein_", kind->tag, "_", fmt_tag(fmt)), (unsigned)grid, 1, 1, 256, wide_lds_bytes(*kind, fmt), s, a)) return rc;
             if (p.split == 1) return 0;
             void* b[] = {(void*)&parts, (void*)&y, (void*)&out_dim, (void*)&n_rows, (void*)&p.n_grp, (void*)&p.n_whole, (void*)&p.split};
-            return launch(KName("rein_", kind->tag, "_sum"), tail, 16, 1, 256, 0, s, b);
+            const unsigned most_tiles = ((n_rows + 31) / 32 + p.n_grp - 1) / p.n_grp;
+            return launch(KName("rein_", kind->tag, "_sum"), tail, 4 * most_tiles, 1, 256, 0, s, b);
         }
     }
     // nothing behind the activations that a workspace launch could use: the plain dispatch

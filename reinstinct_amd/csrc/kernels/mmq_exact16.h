@@ -27,7 +27,7 @@
 // 494 -> 163 / 176 / 214; Q6_K 777 x
 // 17408 -> 5120 569 -> 363; 45 x 17408 -> 5120 (one group of two tiles) Q5_K 42.1 -> 36.3.
 //
-// Replaces, from 33 rows, kernels/mmq_gemm_{q4k,q5k,q6k}_repacked.cpp of the reference behind rein_matmul_ws.
+// Replaces, from nine rows, kernels/mmq_gemm_{q4k,q5k,q6k}_repacked.cpp of the reference behind rein_matmul_ws.
 #pragma once
 
 #include "mmq_fp6.h"
@@ -600,7 +600,7 @@ __device__ __forceinline__ void rein_xh_dense(const uint8_t* __restrict__ w, con
     }
 }
 
-// y of the split units.  Grid (units - n_whole, 16): blockIdx.y = 4 t + v / 4, 256 threads as in the GEMM.
+// y of the split units.  Grid (units - n_whole, 4 x the tiles of the largest group): blockIdx.y = 4 t + v / 4, 256 threads as in the GEMM.
 __device__ __forceinline__ void rein_xh_sum_body(const float* __restrict__ parts, float* __restrict__ y, unsigned out_dim, unsigned p_rows, unsigned n_grp, unsigned n_whole, unsigned split)
 {
     const unsigned u = n_whole + blockIdx.x, rb = u / n_grp;

@@ -18,7 +18,7 @@
 // 17408 -> 5120 at 200 rows 195 -> 74.  Eight wavefronts per workgroup (256 rows share the activations) 519, one order left to the
 // scheduler 511, conversions instead of the biased dots 501-511 (2048 rows).
 //
-// Replaces, from 33 rows, kernels/mmq_gemm_{q8_0,q4_0,iq4xs}_repacked.cpp of the reference behind rein_matmul_ws.
+// Replaces, from nine rows, kernels/mmq_gemm_{q8_0,q4_0,iq4xs}_repacked.cpp of the reference behind rein_matmul_ws.
 #pragma once
 
 #include "mmq_exact16.h"

@@ -83,3 +83,10 @@ def test_where_the_exact_dot_gemm_of_q5_k_is_taken(tmp_path):
     taken([(q5, 1536, 4064, 1024, 0), (q5, 1536, 4096, 1024, kernel), (q5, 2816, 3072, 1024, 0), (q5, 3072, 512, 1024, kernel), (q5, 2816, 18944, 1023, 0),
            (q5, 3072, 17408, 160, 0), (q5, 3072, 17408, 161, kernel), (q5, 4096, 17408, 160, kernel), (q5, 17408, 832, 65, 0), (q5, 17408, 1024, 65, kernel),
            (q5, 17408, 640, 101, kernel), (q5, 8192, 640, 100, kernel)], tmp_path)
+
+
+def test_the_sum_has_workgroups_for_the_tiles_there_are(tmp_path):
+    for fmt, k, n, rows in [(rein.Q5_K, 17408, 5120, 45), (rein.Q8_0, 17408, 5120, 20), (rein.Q6_K, 17408, 5120, 777), (rein.Q8_0, 5120, 17408, 300)]:
+        size = runtime.matmul_scratch_bytes(fmt, k, rows)
+        (image, *_), (gemm, *_), (total, grid, *_) = record([("matmul_ws", [fmt, P, P, P, k, n, rows, P, size])], tmp_path)[0]["launches"]
+        assert total.endswith("_sum") and grid[1] % 4 == 0 and grid[1] // 4 <= min(4 if gemm[6] != "f" else 2, (rows + 31) // 32), (gemm, grid)
