@@ -416,10 +416,12 @@ int rein_matmul(int fmt, const void *w, const float *x, float *y, unsigned in_di
  * (16-byte aligned) that holds the quantized activations -- its first n_rows*in_dim/32*40 bytes, as
  * rein_quantize_q8 writes them, whichever launch is taken -- and, for the MMQ path, the workspace
  * of rein_mmq_xq8_ws.  A scratch that only holds the activations runs rein_matmul.
- * Q4_K, Q5_K and Q6_K from 33 rows: the fp16-instruction GEMM with exact block dots where it is the faster one
- * (activation image and up to 64 MiB of partial tiles in the scratch; three launches, no allocation) if the
- * scratch holds what the shape needs for it -- a scratch of the size asked for does, whatever out_dim is --
- * and what rein_mmq_xq8_ws takes for the scratch otherwise. */
+ * From nine rows, contractions that are a multiple of 256, every dense format: the GEMMs on 32 x 128 wavefront
+ * tiles where they are the faster ones (Q4_K, Q5_K, Q6_K with exact block dots on the fp16 instruction, the others
+ * on the int8 instruction; two or three launches, no allocation) if the scratch holds what the shape needs for it:
+ * behind the activations their image in operand order (2.25 to 4.5 bytes a value) and the partial tiles of what is cut
+ * over the contraction, 16 MiB for each 32 rows up to 64 MiB.  A scratch of the size asked for does, whatever
+ * out_dim is; a smaller one takes what rein_mmq_xq8_ws takes for it.  The query costs a microsecond. */
 size_t rein_matmul_scratch_bytes(int fmt, unsigned in_dim, unsigned n_rows);
 int rein_matmul_ws(int fmt, const void *w, const float *x, float *y, unsigned in_dim,
                    unsigned out_dim, unsigned n_rows, void *scratch, size_t scratch_bytes,
