@@ -2015,7 +2015,8 @@ namespace {
 // superblocks.  How many tiles a group has and how many ranges there are is the cheapest by a price in microseconds: a superblock of
 // a workgroup with t tiles costs alone[n] + tile[n] t with n + 1 workgroups on its CU (the last round may leave fewer than fit),
 // `sum` the launch that adds partial tiles, `part` each tile of 16 KB that is written and read again.  Fitted per kind to every group
-// size x 1-16 ranges on 12-13 shapes x 17 row counts: the pick is within 1 % of the best of its cell in the mean, at most 8-16 % (Q8_0 5120 ->
+// size x 1-16 ranges on 12-13 shapes x 17 row counts: the pick is within 1 % of the best of its cell in the mean, at most 8-16 %, and for the K-quants over 900 further cells
+// drawn at random within 1.1 %, at most 19 (Q6_K 278 x 4096 -> 160, groups x ranges: 3 x 16 17.6 us, 4 x 16 14.8; Q8_0 5120 ->
 // 1024, 160 rows, groups x ranges: 5 x 5 15.5 us, 2 x 12 20.3; 17408 -> 5120, 45 rows 1 x 12 35.0, 2 x 6 36.5, 1 x 4 44; 2048 -> 5632,
 // 300 rows 10 x 1 24.7, 5 x 1 26.2, 3 x 6 32.7).
 struct WideKind {
@@ -2196,9 +2197,9 @@ WidePlan wide_plan(const WideKind& kind, int fmt, unsigned in_dim, unsigned out_
     return p;
 }
 // No number of weight rows leaves more bytes of partial tiles behind whole rounds (the size query does not know the matrix): at most
-// kWideMostParts ranges, and of a tail's units at most one for each of sixteen superblocks, each of a group of the most tiles.  A bound
-// and not the largest plan: that is within a fifth of it from sixteen superblocks on and a half to a quarter below, but pricing a
-// round's plans takes the query from 1 to 70-270 us, and a program whose prompts differ in length asks before each.
+// kWideMostParts ranges, and of a tail's units at most one for each of sixteen superblocks, each of a group of the most tiles.  A bound,
+// not the largest plan, which needs four fifths of it and more from sixteen superblocks on and a quarter to three quarters below: to price
+// a round's plans takes 70-270 us where this takes one, and a program whose prompts differ in length asks before each.
 size_t wide_most_parts_bytes(const WideKind& kind, unsigned in_dim, unsigned p_rows)
 {
     const unsigned n_tt = (p_rows + 31) / 32, most_split = std::min(16u, in_dim / 256);
