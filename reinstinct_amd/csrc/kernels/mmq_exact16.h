@@ -187,7 +187,8 @@ struct XhMasks {
 };
 __device__ __forceinline__ uint32_t rein_xh_or(uint32_t v, uint32_t mask, uint32_t base) { return (v & mask) | base; }
 __device__ __forceinline__ rein_h2 rein_xh_fma(uint32_t v, rein_h2 sc, rein_h2 c) { return __builtin_elementwise_fma(__builtin_bit_cast(rein_h2, v), sc, c); }
-__device__ __forceinline__ rein_h2 rein_xh_splat(float v) { return rein_h2{(_Float16)v, (_Float16)v}; }
+// (as an operand of a packed instruction: its half of a register, no copy)
+__device__ __forceinline__ rein_h2 rein_xh_both(_Float16 v) { return rein_h2{v, v}; }
 __device__ __forceinline__ rein_v8h rein_xh_join(rein_h2 a, rein_h2 b, rein_h2 c, rein_h2 d)
 {
     return rein_v8h{a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
@@ -208,8 +209,8 @@ template <> struct XhWeights<REIN_Q4_K> {
     // words 2h, 2h + 1 of a sub-block's nibbles and its (sc, m)
     static __device__ __forceinline__ void unpack(rein_v8h (&o)[2][kOps], uint2 w2, uint32_t, uint32_t sm, unsigned, const XhMasks& mk)
     {
-        const float scf = (float)(sm & 0xFFu);
-        const rein_h2 sc = rein_xh_splat(scf), c1024 = rein_xh_splat(scf * -1024.0f), c64 = rein_xh_splat(scf * -64.0f);
+        const rein_h2 sc = rein_xh_both((_Float16)(uint16_t)(sm & 0xFFu)), c = sc * rein_h2{(_Float16)-1024.0f, (_Float16)-64.0f};
+        const rein_h2 c1024 = rein_xh_both(c[0]), c64 = rein_xh_both(c[1]);
 #pragma unroll
         for (int kh = 0; kh < 2; kh++) {
             const uint32_t w = kh ? w2.y : w2.x, w8 = w >> 8;
@@ -231,8 +232,8 @@ template <> struct XhWeights<REIN_Q5_K> {
     // words 2h, 2h + 1 of a sub-block's nibbles, its fifth bits and (sc, m)
     static __device__ __forceinline__ void unpack(rein_v8h (&o)[2][kOps], uint2 w2, uint32_t qh, uint32_t sm, unsigned h, const XhMasks& mk)
     {
-        const float scf = (float)(sm & 0xFFu);
-        const rein_h2 sc = rein_xh_splat(scf), c1024 = rein_xh_splat(scf * -1024.0f), c64 = rein_xh_splat(scf * -64.0f);
+        const rein_h2 sc = rein_xh_both((_Float16)(uint16_t)(sm & 0xFFu)), c = sc * rein_h2{(_Float16)-1024.0f, (_Float16)-64.0f};
+        const rein_h2 c1024 = rein_xh_both(c[0]), c64 = rein_xh_both(c[1]);
         const uint32_t q = qh >> (16u * h), q2 = q >> 2;      // bits f of byte kh: weights f of the low nibbles, bits 4 + f: of the high
 #pragma unroll
         for (int kh = 0; kh < 2; kh++) {
@@ -255,28 +256,31 @@ template <> struct XhWeights<REIN_Q6_K> {
     static constexpr unsigned kHiBytes = 8, kDBytes = 2;
     static __device__ __forceinline__ const char* hi(const Fmt<REIN_Q6_K>& f) { return reinterpret_cast<const char*>(f.h2p); }
     static __device__ __forceinline__ const char* d(const Fmt<REIN_Q6_K>& f) { return reinterpret_cast<const char*>(f.dp); }
-    static __device__ __forceinline__ float scale(uint32_t dd) { return rein_h2f((uint16_t)dd) * kUnit; }
+    static __device__ __forceinline__ float scale(uint32_t dd) { return rein_h2f((uint16_t)dd); }
     static __device__ __forceinline__ float min_scale(uint32_t) { return 0.0f; }
     // Words 2h, 2h + 1 of a sub-block's nibbles, the word of two-bit fields that goes with them, both group scales.  Low nibbles
-    // are weights 0..15 (first scale), high ones 16..31 (second).  A two-bit field at bits 8, 9 of 4.0 is 4 + c:
-    // (4 + c) 4 sc - 24 sc = 4 (c - 2) sc; 4 sc is at most 512, 24 sc has 9 bits: exact.  The nibble term is held as a quarter,
-    // so that 1024 * sc / 4 stays inside fp16.
+    // are weights 0..15 (first scale), high ones 16..31 (second).  Or-ed into the mantissas of 256 and 16 they are 256 + n / 4 and
+    // 16 + n / 4, a two-bit field at bits 8, 9 of 16 is 16 + 4 c: one packed fma with the scale itself and an offset of it makes
+    // n sc / 4 and 4 (c - 2) sc, and the offsets (256, 16, 24 times a scale of 8 bits) are exact.  The quarter is taken back at the
+    // end.  (With scales multiplied by 1/4 and 4 first it is eight conversions and twelve products a sub-block instead of two and two:
+    // 2048 x 5120 -> 17408 739 -> 719 us.)
     static __device__ __forceinline__ void unpack(rein_v8h (&o)[2][kOps], uint2 w2, uint32_t hw, uint32_t sm, unsigned, const XhMasks& mk)
     {
-        const float a = (float)(int)(int8_t)(sm & 0xFFu), b = (float)(int)(int8_t)((sm >> 8) & 0xFFu);
-        const rein_h2 na = rein_xh_splat(a * 0.25f), nb = rein_xh_splat(b * 0.25f), ca = rein_xh_splat(a * -256.0f), cb = rein_xh_splat(b * -16.0f);
-        const rein_h2 ha = rein_xh_splat(a * 4.0f), hb = rein_xh_splat(b * 4.0f), ga = rein_xh_splat(a * -24.0f), gb = rein_xh_splat(b * -24.0f);
+        const rein_h2 sc = {(_Float16)(short)(int8_t)(sm & 0xFFu), (_Float16)(short)(int8_t)((sm >> 8) & 0xFFu)};
+        const rein_h2 cn = sc * rein_h2{(_Float16)-256.0f, (_Float16)-16.0f}, cg = sc * rein_h2{(_Float16)-24.0f, (_Float16)-24.0f};
+        const rein_h2 a = rein_xh_both(sc[0]), b = rein_xh_both(sc[1]), ca = rein_xh_both(cn[0]), cb = rein_xh_both(cn[1]);
+        const rein_h2 ga = rein_xh_both(cg[0]), gb = rein_xh_both(cg[1]);
         const uint32_t hw4 = hw >> 4;
 #pragma unroll
         for (int kh = 0; kh < 2; kh++) {
             const uint32_t w = kh ? w2.y : w2.x, w8 = w >> 8;
-            o[kh][0] = rein_xh_join(rein_xh_fma(rein_xh_or(w, mk.lo, 0x64006400u), na, ca), rein_xh_fma(rein_xh_or(w, mk.hi, 0x54005400u), nb, cb),
-                                    rein_xh_fma(rein_xh_or(w8, mk.lo, 0x64006400u), na, ca), rein_xh_fma(rein_xh_or(w8, mk.hi, 0x54005400u), nb, cb));
+            o[kh][0] = rein_xh_join(rein_xh_fma(rein_xh_or(w, mk.lo, 0x5C005C00u), a, ca), rein_xh_fma(rein_xh_or(w, mk.hi, 0x4C004C00u), b, cb),
+                                    rein_xh_fma(rein_xh_or(w8, mk.lo, 0x5C005C00u), a, ca), rein_xh_fma(rein_xh_or(w8, mk.hi, 0x4C004C00u), b, cb));
             // byte 2 kh (weights of the low nibbles) / 2 kh + 1 (of the high ones): elements 0, 1 to bits 8..11, 2, 3 to bits 24..27
             const uint32_t pa = __builtin_amdgcn_perm(hw4, hw, kh ? 0x060C020Cu : 0x040C000Cu), pa2 = pa >> 2;
             const uint32_t pb = __builtin_amdgcn_perm(hw4, hw, kh ? 0x070C030Cu : 0x050C010Cu), pb2 = pb >> 2;
-            o[kh][1] = rein_xh_join(rein_xh_fma(rein_xh_or(pa, mk.two, 0x44004400u), ha, ga), rein_xh_fma(rein_xh_or(pb, mk.two, 0x44004400u), hb, gb),
-                                    rein_xh_fma(rein_xh_or(pa2, mk.two, 0x44004400u), ha, ga), rein_xh_fma(rein_xh_or(pb2, mk.two, 0x44004400u), hb, gb));
+            o[kh][1] = rein_xh_join(rein_xh_fma(rein_xh_or(pa, mk.two, 0x4C004C00u), a, ga), rein_xh_fma(rein_xh_or(pb, mk.two, 0x4C004C00u), b, gb),
+                                    rein_xh_fma(rein_xh_or(pa2, mk.two, 0x4C004C00u), a, ga), rein_xh_fma(rein_xh_or(pb2, mk.two, 0x4C004C00u), b, gb));
         }
     }
 };
@@ -386,16 +390,20 @@ __device__ __forceinline__ void rein_xh_acc(const uint8_t* __restrict__ w, const
         if constexpr (W::kDBytes == 4) rein_xh_dma_u32(d_off, dp, dst + 3072u + (c & 1u) * 256u);
         else rein_xh_dma_u16(d_off, dp, dst + 3072u + (c & 1u) * 256u);
     };
-    rein_v16f dot[2], z16;
+    // Dots are multiplied by their dx one stage after their instructions went out, two where a stage has two instructions and registers
+    // are left: nothing waits for the matrix unit then (Q4_K 2048 x 5120 -> 17408 540 -> 530 us).
+    constexpr int kLag = W::kOps == 1 && NT > 2 ? 2 : 1, kBuf = kLag + 1;
+    rein_v16f dot[kBuf], z16;
     float s1[NT][16];
-    float dx[2] = {0.0f, 0.0f};
+    float dx[kBuf];
 #pragma unroll
     for (int v = 0; v < 16; v++) z16[v] = 0.0f;
 #pragma unroll
     for (int t = 0; t < NT; t++)
 #pragma unroll
         for (int v = 0; v < 16; v++) acc[t][v] = s1[t][v] = 0.0f;
-    dot[0] = dot[1] = z16;
+#pragma unroll
+    for (int b = 0; b < kBuf; b++) { dot[b] = z16; dx[b] = 0.0f; }
 
     __syncthreads();                                 // the LDS may still be read by the caller's previous tile
     issue_acts(c0 * 4u);
@@ -456,7 +464,7 @@ __device__ __forceinline__ void rein_xh_acc(const uint8_t* __restrict__ w, const
                 // written: left alone, the scheduler starts all tiles at once and spills.
 #pragma unroll
                 for (int t = 0; t < NT; t++) {
-                    const int now = (int)(sb * NT + t) & 1;
+                    const int i = (int)(sb * NT) + t, now = i % kBuf;
                     if (t + 1 < NT) {
                         xa[(t + 1) & 1][0] = *reinterpret_cast<const rein_v8h*>(x + (t + 1) * REIN_XH_REC);
                         xa[(t + 1) & 1][1] = *reinterpret_cast<const rein_v8h*>(x + (t + 1) * REIN_XH_REC + 1024u);
@@ -468,23 +476,40 @@ __device__ __forceinline__ void rein_xh_acc(const uint8_t* __restrict__ w, const
                         dot[now] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[1][k], xa[t & 1][1], dot[now], 0, 0, 0);
                     }
                     dx[now] = dxp[t * (REIN_XH_REC / 4u)];
-                    if (sb * NT + t > 0u) {
-                        const int tp = (t + NT - 1) % NT;
-                        const bool first = sb * NT + t <= (unsigned)NT;              // the sums' first term of this superblock
+                    if (i >= kLag) {
+                        const int tp = (i - kLag) % NT, old = (i - kLag) % kBuf;
+                        const bool first = i - kLag < NT;                            // the sums' first term of this superblock
 #pragma unroll
-                        for (int v = 0; v < 16; v++) s1[tp][v] = first ? dx[now ^ 1] * dot[now ^ 1][v] : fmaf(dx[now ^ 1], dot[now ^ 1][v], s1[tp][v]);
+                        for (int v = 0; v < 16; v++) s1[tp][v] = first ? dx[old] * dot[old][v] : fmaf(dx[old], dot[old][v], s1[tp][v]);
                         rein_xh_pin(s1[tp]);
+                    }
+                    // the order in a stage: operand reads, then the matrix instructions with the multiply-adds behind them.  Left to
+                    // itself the scheduler puts multiply-adds behind the first one of Q6_K, where they wait for the stage before
+                    // (777 x 17408 -> 5120 335 -> 330 us).
+                    if constexpr (W::kOps == 1 && NT > 2) {
+                        __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x2, 8, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x2, 8, 0);
+                    }
+                    if constexpr (W::kOps == 2) {
+                        __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x8, 2, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x2, 8, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x2, 8, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
                     }
                     __builtin_amdgcn_sched_barrier(0);
                 }
                 __builtin_amdgcn_s_setprio(0);
             }
         }
-        {
-            constexpr int end = (8 * NT - 1) & 1;
 #pragma unroll
-            for (int v = 0; v < 16; v++) s1[NT - 1][v] = fmaf(dx[end], dot[end][v], s1[NT - 1][v]);
-        }
+        for (int i = 8 * NT - kLag; i < 8 * NT; i++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) s1[i % NT][v] = fmaf(dx[i % kBuf], dot[i % kBuf][v], s1[i % NT][v]);
         // acc += d s1 - dmin (m . xsum): register v is weight row 8 (v / 4) + 4 h + v % 4
         const unsigned char* const xb = raw + kXs + lane * 16u;
         float dv[16], nv[16];
@@ -507,6 +532,12 @@ __device__ __forceinline__ void rein_xh_acc(const uint8_t* __restrict__ w, const
                 for (int v = 0; v < 16; v++) acc[t][v] = fmaf(nv[v], s2[v], acc[t][v]);
             }
         }
+    }
+    if constexpr (W::kUnit != 1.0f) {
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) acc[t][v] *= W::kUnit;
     }
     REIN_WAIT_VMCNT(0);
 }
