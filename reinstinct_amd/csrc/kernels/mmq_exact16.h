@@ -352,15 +352,15 @@ __device__ __forceinline__ void rein_xh_acc(const uint8_t* __restrict__ w, const
     wsrc.init(*reinterpret_cast<const MmqWLds<FMT>*>(ring), fmt, row_base, out_dim, lane);
     const uint8_t* const xsimg = img + (size_t)(n_sub >> 1) * n_tt * REIN_XH_REC;
 
-    auto issue_acts = [&](unsigned pair) {
-        const uint8_t* src = img + ((size_t)pair * n_tt + tile) * REIN_XH_REC;
-        const unsigned buf = lds0 + (pair & 1u) * (MOST * REIN_XH_REC);
-#pragma unroll
-        for (unsigned t = 0; t < (unsigned)NT; t++) {
-            const unsigned off = t * REIN_XH_REC + wave * 1024u;
-            rein_lds_dma16_s(lane * 16u, src + off, buf + off);
-        }
-        if (wave < (unsigned)NT) rein_xh_dma_u32(lane * 4u, src + wave * REIN_XH_REC + REIN_XH_X, buf + wave * REIN_XH_REC + REIN_XH_X);
+    // src: a pair's record of the first tile.  It runs along with the pairs: addresses worked out of the pair's number for each transfer
+    // cost as much scalar issue as the transfers do (777 x 17408 -> 5120 Q6_K 328 -> 320 us).
+    auto issue_act = [&](const uint8_t* src, unsigned buf, unsigned t) {
+        const unsigned off = t * REIN_XH_REC + wave * 1024u;
+        rein_lds_dma16_s(lane * 16u, src + off, lds0 + buf * (MOST * REIN_XH_REC) + off);
+    };
+    auto issue_dx = [&](const uint8_t* src, unsigned buf) {              // (the wavefronts past the last tile fetch its scales again)
+        const unsigned off = min(wave, (unsigned)NT - 1u) * REIN_XH_REC + REIN_XH_X;
+        rein_xh_dma_u32(lane * 4u, src + off, lds0 + buf * (MOST * REIN_XH_REC) + off);
     };
     auto issue_xs = [&](unsigned c) {
         if constexpr (W::kHasMin) {
@@ -393,6 +393,9 @@ __device__ __forceinline__ void rein_xh_acc(const uint8_t* __restrict__ w, const
     // Dots are multiplied by their dx one stage after their instructions went out, two where a stage has two instructions and registers
     // are left: nothing waits for the matrix unit then (Q4_K 2048 x 5120 -> 17408 540 -> 530 us).
     constexpr int kLag = W::kOps == 1 && NT > 2 ? 2 : 1, kBuf = kLag + 1;
+    // Transfers of a step go out one by one between the matrix instructions of three and four tiles; with one or two tiles there are
+    // too few instructions for that, and they go out at the step's top (spread: Q4_K 60 x 5120 -> 5120 19.9 -> 20.9 us).
+    constexpr bool kSpread = NT > 2;
     rein_v16f dot[kBuf], z16;
     float s1[NT][16];
     float dx[kBuf];
@@ -405,8 +408,12 @@ __device__ __forceinline__ void rein_xh_acc(const uint8_t* __restrict__ w, const
 #pragma unroll
     for (int b = 0; b < kBuf; b++) { dot[b] = z16; dx[b] = 0.0f; }
 
+    const size_t src_step = (size_t)n_tt * REIN_XH_REC;
+    const uint8_t* src = img + (c0 * 4u) * src_step + tile * REIN_XH_REC;
     __syncthreads();                                 // the LDS may still be read by the caller's previous tile
-    issue_acts(c0 * 4u);
+#pragma unroll
+    for (unsigned t = 0; t < (unsigned)NT; t++) issue_act(src, 0u, t);
+    issue_dx(src, 0u);
     issue_small(c0);
     rein_mmq_wload<FMT>(wsrc, 0u, fmt, c0 * 8u, n_sub);
     const unsigned rot = j >> 1;
@@ -417,7 +424,8 @@ __device__ __forceinline__ void rein_xh_acc(const uint8_t* __restrict__ w, const
 #pragma unroll
         for (unsigned u = 0; u < 4; u++) {
             const unsigned pair = c * 4u + u;
-            const bool last = c + 1u == c1;
+            const bool more = c + 1u < c1;
+            if (u < 3u || more) src += src_step;     // (past the last pair: it again, read by nobody)
             REIN_WAIT_VMCNT(0);
             __syncthreads();
             const unsigned char* const sms = small + 2048u + (8u * j + 2u * u) * sm_step;
@@ -430,13 +438,23 @@ __device__ __forceinline__ void rein_xh_acc(const uint8_t* __restrict__ w, const
                 const uint2 g = *reinterpret_cast<const uint2*>(small + j * 32u + (((u >> 1) ^ (j >> 2)) & 1u) * 16u + (u & 1u) * 8u);
                 hi2[0] = g.x; hi2[1] = g.y;
             }
-            if (u < 3u || !last) issue_acts(pair + 1u);
-            if (u == 0u) rein_mmq_wload<FMT>(wsrc, 1u, fmt, c * 8u + 4u, n_sub);
-            if (u == 1u) issue_xs(c);                // read at the superblock's end; the barrier of u = 0 freed it
-            if (u == 2u && !last) rein_mmq_wload<FMT>(wsrc, 0u, fmt, c * 8u + 8u, n_sub);
-            if (u == 3u && !last) {
-                __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the reads above have left the buffer
-                issue_small(c + 1u);
+            const unsigned buf = (pair & 1u) ^ 1u;
+            auto issue_other = [&]() {
+                if (u == 0u) rein_mmq_wload<FMT>(wsrc, 1u, fmt, c * 8u + 4u, n_sub);
+                if (u == 1u) issue_xs(c);            // read at the superblock's end; the barrier of u = 0 freed it
+                if (u == 2u && more) rein_mmq_wload<FMT>(wsrc, 0u, fmt, c * 8u + 8u, n_sub);
+                if (u == 3u && more) {
+                    if constexpr (!kSpread) __builtin_amdgcn_s_waitcnt(0xC07F);          // lgkmcnt(0): the reads above have left the buffer
+                    issue_small(c + 1u);
+                }
+            };
+            if constexpr (!kSpread) {
+                if (u < 3u || more) {
+#pragma unroll
+                    for (unsigned t = 0; t < (unsigned)NT; t++) issue_act(src, buf, t);
+                    if (wave < (unsigned)NT) issue_dx(src, buf);
+                }
+                issue_other();
             }
             const unsigned char* const act = raw + (pair & 1u) * (MOST * REIN_XH_REC);
 #pragma unroll
@@ -468,6 +486,11 @@ __device__ __forceinline__ void rein_xh_acc(const uint8_t* __restrict__ w, const
                     if (t + 1 < NT) {
                         xa[(t + 1) & 1][0] = *reinterpret_cast<const rein_v8h*>(x + (t + 1) * REIN_XH_REC);
                         xa[(t + 1) & 1][1] = *reinterpret_cast<const rein_v8h*>(x + (t + 1) * REIN_XH_REC + 1024u);
+                    }
+                    if constexpr (kSpread) {
+                        if (q == 0u) issue_act(src, buf, (unsigned)t);
+                        if (q == 0u && t == NT - 1) issue_dx(src, buf);
+                        if (q == 1u && t == 0) issue_other();
                     }
                     dot[now] = z16;
 #pragma unroll
