@@ -21,11 +21,11 @@
 //
 // Bound: the same instructions alone, on every CU, take 65 ns (Q4_K) and 90 (Q6_K) per tile and sub-block and SIMD -- two / four matrix
 // instructions, the 16 multiply-adds and a quarter of the unpack, the two units overlapping but for issue, the clock at 1.8-2.0 of
-// 2.4 GHz under this load; the kernel without its transfers 75 and 108, with them 97 and 129.  Whole calls of rein_matmul_ws against
-// the launches of rein_mmq_xq8_ws (fp6 for Q4_K, else int8), weights of several matrices in turn, us, Q4_K / Q5_K / Q6_K: 2048 x 5120 ->
-// 17408 633 / 809 / 1268 -> 588 / 645 / 786; 512 x 5120 -> 17408 169 / 203 / 347 -> 149 / 160 / 198; 512 x 17408 -> 5120 195 / 271 /
-// 494 -> 163 / 176 / 214; Q6_K 777 x
-// 17408 -> 5120 569 -> 363; 45 x 17408 -> 5120 (one group of two tiles) Q5_K 42.1 -> 36.3.
+// 2.4 GHz under this load; the kernel takes 88 and 118.  Without its transfers it is 14 % faster (Q4_K 17 %), with the activations
+// always from one place in cache 3-7 %: what is left is the way from L2 to LDS and the scalar issue around it.  Waits, barriers and
+// the operand reads from LDS cost nothing measurable.  Whole calls of rein_matmul_ws against the launches of rein_mmq_xq8_ws (fp6 for
+// Q4_K, else int8), us, Q4_K / Q5_K / Q6_K: 2048 x 5120 -> 17408 633 / 809 / 1268 -> 512 / 557 / 670; 512 x 5120 -> 17408 169 / 203 /
+// 347 -> 138 / 149 / 184; 777 x 17408 -> 5120 Q6_K 569 -> 320; 45 x 17408 -> 5120 (one group of two tiles) Q5_K 42.1 -> 36.3.
 //
 // Replaces, from nine rows, kernels/mmq_gemm_{q4k,q5k,q6k}_repacked.cpp of the reference behind rein_matmul_ws.
 #pragma once
@@ -623,15 +623,30 @@ __device__ __forceinline__ unsigned rein_xh_deal(unsigned i, unsigned n)
     const unsigned per = (n + 7u) >> 3, k = i >> 3;
     return k < per ? (i & 7u) * per + k : 0xFFFFFFFFu;
 }
+// Unit `v` of n_rb x n_grp in the order of the launch: bands of up to four token groups, in a band row block by row block.  An XCD's
+// 64 resident workgroups are then 16 row blocks x 4 groups instead of 4 x 16: they share the activations sixteen ways in their L2, and what
+// it fetches is halved (a group's activations are 272 bytes a value of the contraction, a row block's weights 72 to 136).  2048 x 5120
+// -> 17408 Q4_K 548 -> 522 us, Q8_0 523 -> 500, Q8_0 1000 x 4096 -> 4096 75 -> 68; bands of eight 532 and 503.  Band b has the groups b,
+// b + n_band, ..., so that the longer groups, which come first, are in all of them.  Units that are cut keep their order, the ranges of
+// one side by side: banded, or range by range, 777 x 17408 -> 5120 takes 345 to 360 us instead of 333.
+__device__ __forceinline__ unsigned rein_xh_banded(unsigned v, unsigned n_rb, unsigned n_grp)
+{
+    const unsigned n_band = (n_grp + 3u) / 4u, base = n_grp / n_band, more = n_grp - base * n_band, wide = more * (base + 1u) * n_rb;
+    unsigned w = base + 1u, b0 = 0u;
+    if (v >= wide) { v -= wide; w = base; b0 = more; }
+    const unsigned b = v / (w * n_rb), r = (v - b * w * n_rb) / w;
+    return r * n_grp + b0 + b + (v - (b * n_rb + r) * w) * n_band;
+}
 template <class Tile>
 __device__ __forceinline__ void rein_xh_dense(const uint8_t* __restrict__ w, const uint8_t* __restrict__ img, float* __restrict__ y, float* __restrict__ parts,
                                               unsigned in_dim, unsigned out_dim, unsigned p_rows, unsigned n_grp, unsigned n_whole, unsigned split)
 {
     extern __shared__ __attribute__((aligned(16))) unsigned char rein_xh_lds[];
-    const unsigned n_unit = ((out_dim + 127u) / 128u) * n_grp, n_chunk = in_dim >> 8;
+    const unsigned n_unit = ((out_dim + 127u) / 128u) * n_grp, n_chunk = in_dim >> 8, rb_whole = n_whole / n_grp;
     unsigned u, c0 = 0u, c1 = n_chunk, k = 0u;
     if (blockIdx.x < n_whole) {
         u = blockIdx.x / Tile::kSlots * Tile::kSlots + rein_xh_deal(blockIdx.x % Tile::kSlots, Tile::kSlots);
+        if (u < rb_whole * n_grp) u = rein_xh_banded(u, rb_whole, n_grp);
     } else {
         const unsigned n_seg = (n_unit - n_whole) * split, seg = rein_xh_deal(blockIdx.x - n_whole, n_seg);
         if (seg >= n_seg) return;
@@ -641,6 +656,7 @@ __device__ __forceinline__ void rein_xh_dense(const uint8_t* __restrict__ w, con
         c0 = n_chunk * k / split; c1 = n_chunk * (k + 1u) / split;       // split <= n_chunk: no range is empty
     }
     if (u >= n_unit) return;
+    u = __builtin_amdgcn_readfirstlane(u);           // (the divisions above left it in a vector register)
     const unsigned rb = u / n_grp;
     const XhGroup g = rein_xh_group(p_rows, n_grp, u - rb * n_grp);
     float* const part = u >= n_whole && split > 1u ? parts + rein_xh_part(p_rows, n_grp, n_whole, rb, g, split) + (size_t)k * g.n * 4096u : nullptr;

@@ -192,3 +192,16 @@ def test_infinities_and_nan_stay_where_they_are(fmt, split):
     assert np.array_equal(got[rest].view(np.uint32), clean[rest].view(np.uint32))
     nan_row = got[40][np.isfinite(got[40])]
     assert_close_f32(nan_row, tile[40][np.isfinite(got[40])], what="row with a NaN")
+
+
+@pytest.mark.parametrize("fmt, rows, out_dim", [
+    (rein.Q4_K, 520, 16384),                          # five groups of 17 tiles: bands of three and two; 512 of 640 units whole, the last row block in part
+    (rein.Q6_K, 1100, 7424),                          # nine groups of 35 tiles: three bands of three; 56 row blocks and eight units of the next
+    (rein.Q5_K, 1030, 8192),                          # 576 units, the last tile almost empty
+])
+def test_every_unit_of_a_banded_round_once(fmt, rows, out_dim):
+    in_dim = 256
+    packed = weights(fmt, in_dim, out_dim, rows)
+    x = np.random.default_rng(rows).standard_normal((rows, in_dim)).astype(np.float32)
+    got = matmul(fmt, packed, x, out_dim, 2)
+    assert_close_f32(got, orc.matvec_q8(fmt, packed, in_dim, out_dim, orc.quantize_q8(x), rows), what=f"fmt {fmt}")
