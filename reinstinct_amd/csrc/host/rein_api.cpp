@@ -2245,7 +2245,7 @@ int rein_matmul_ws(int fmt, const void* w, const float* x, float* y, unsigned in
             if (int rc = check_ptr("rein_matmul_ws", w, 16, "w")) return rc;
             if (int rc = check_ptr("rein_matmul_ws", y, 4, "y")) return rc;
             void* pa[] = {(void*)&x, (void*)&img, (void*)&scratch, (void*)&in_dim, (void*)&n_rows, (void*)&with_xsum};          // rein_x8_quantize: the first five
-            if (int rc = launch(KName("rein_", kind->tag, "_quantize"), (n_rows + 31) / 32, in_dim / 256, 1, 256, 0, s, pa)) return rc;
+            if (int rc = launch(KName("rein_", kind->tag, "_quantize"), (n_rows + 31) / 32 * 4, in_dim / 256, 1, 256, 0, s, pa)) return rc;
             void* a[] = {(void*)&w, (void*)&img, (void*)&y, (void*)&parts, (void*)&in_dim, (void*)&out_dim, (void*)&n_rows, (void*)&p.n_grp, (void*)&p.n_whole, (void*)&p.split};
             if (int rc = launch(KName("rein_", kind->tag, "_", fmt_tag(fmt)), (unsigned)grid, 1, 1, 256, wide_lds_bytes(*kind, fmt), s, a)) return rc;
             if (p.split == 1) return 0;

@@ -64,96 +64,99 @@ __host__ __device__ constexpr int rein_xh_slot_weight(int kh, int h, int e)
 #define REIN_XH_REC 4352u
 #define REIN_XH_XS  2048u
 
-// One block of 32 values of row `tok` (zeros past p_rows, with d = 0) with the numbers that quantize_q8_f32 gives: the same sum tree
-// (halves of 16, 8, 4, 2, 1), divisions and rounding, by one thread.  The block itself goes to xq.
-struct XhBlock { float d, sum; int q[32]; };
+// A block of 32 values of row `tok` (zeros past p_rows, with d = 0) with the numbers that quantize_q8_f32 gives, by four lanes: lane q of
+// the four holds values 4 q .. 4 q + 3 and those 16 further on, which are the two dwords of quants that it writes to xq and one 16-byte
+// piece of the operand order.  The sum tree is halves of 16 (inside the lane), 8 and 4 (between lanes), 2 and 1.
+struct XhBlock { float d, sum; int q[8]; };
 __device__ __forceinline__ void rein_xh_quantize_block(XhBlock& b, const float* __restrict__ x, BlockQ8* __restrict__ xq, unsigned in_dim, unsigned p_rows,
-                                                       unsigned tok, unsigned sb)
+                                                       unsigned tok, unsigned sb, unsigned q)
 {
 #pragma clang fp contract(off)
-    float v[32];
-    float inv = 0.0f;
-    b.d = b.sum = 0.0f;
-    if (tok < p_rows) {
-        const float* p = x + (size_t)tok * in_dim + sb * 32u;
-        if (((size_t)x & 15u) == 0u) {
+    float v[8], t[4];
 #pragma unroll
-            for (int i = 0; i < 8; i++) {
-                const float4 f = reinterpret_cast<const float4*>(p)[i];
-                v[4 * i] = f.x; v[4 * i + 1] = f.y; v[4 * i + 2] = f.z; v[4 * i + 3] = f.w;
-            }
+    for (int i = 0; i < 8; i++) v[i] = 0.0f;
+    if (tok < p_rows) {
+        const float* p = x + (size_t)tok * in_dim + sb * 32u + 4u * q;
+        if (((size_t)x & 15u) == 0u) {
+            const float4 lo = reinterpret_cast<const float4*>(p)[0], hi = reinterpret_cast<const float4*>(p)[4];
+            v[0] = lo.x; v[1] = lo.y; v[2] = lo.z; v[3] = lo.w;
+            v[4] = hi.x; v[5] = hi.y; v[6] = hi.z; v[7] = hi.w;
         } else {
 #pragma unroll
-            for (int i = 0; i < 32; i++) v[i] = p[i];
+            for (int i = 0; i < 4; i++) { v[i] = p[i]; v[4 + i] = p[16 + i]; }
         }
-        float amax = 0.0f, t[16];
-#pragma unroll
-        for (int i = 0; i < 32; i++) amax = fmaxf(amax, fabsf(v[i]));
-#pragma unroll
-        for (int i = 0; i < 16; i++) t[i] = v[i] + v[i + 16];
-#pragma unroll
-        for (int m = 8; m >= 1; m >>= 1)
-#pragma unroll
-            for (int i = 0; i < m; i++) t[i] = t[i] + t[i + m];
-        b.sum = t[0];
-        b.d   = amax > 0.0f ? amax / 127.0f : 1.0f;
-        inv   = amax > 0.0f ? 127.0f / amax : 0.0f;
-    } else {
-#pragma unroll
-        for (int i = 0; i < 32; i++) v[i] = 0.0f;
     }
+    float amax = 0.0f;
 #pragma unroll
-    for (int i = 0; i < 32; i++) b.q[i] = max(-127, min(127, (int)rintf(v[i] * inv)));
+    for (int i = 0; i < 8; i++) amax = fmaxf(amax, fabsf(v[i]));
+    amax = fmaxf(amax, rein_dpp_f32<0x4E>(amax, amax));                  // lane ^ 2
+    amax = fmaxf(amax, rein_dpp_f32<0xB1>(amax, amax));                  // lane ^ 1
+#pragma unroll
+    for (int i = 0; i < 4; i++) t[i] = v[i] + v[i + 4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) t[i] = t[i] + rein_dpp_f32<0x4E>(t[i], t[i]);
+#pragma unroll
+    for (int i = 0; i < 4; i++) t[i] = t[i] + rein_dpp_f32<0xB1>(t[i], t[i]);
+    b.sum = (t[0] + t[2]) + (t[1] + t[3]);
+    b.d   = tok >= p_rows ? 0.0f : amax > 0.0f ? amax / 127.0f : 1.0f;
+    const float inv = amax > 0.0f ? 127.0f / amax : 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; i++) b.q[i] = max(-127, min(127, (int)rintf(v[i] * inv)));
     if (tok < p_rows) {
-        BlockQ8 o;
-        o.d = b.d;
-        o.xsum = b.sum;
+        BlockQ8* const o = xq + (size_t)tok * (in_dim >> 5) + sb;
+        if (q == 0u) { o->d = b.d; o->xsum = b.sum; }
 #pragma unroll
-        for (int i = 0; i < 8; i++) o.qs[i] = (b.q[4 * i] & 0xFF) | (b.q[4 * i + 1] & 0xFF) << 8 | (b.q[4 * i + 2] & 0xFF) << 16 | b.q[4 * i + 3] << 24;
-        xq[(size_t)tok * (in_dim >> 5) + sb] = o;
+        for (int k = 0; k < 2; k++)
+            o->qs[4 * k + q] = (b.q[4 * k] & 0xFF) | (b.q[4 * k + 1] & 0xFF) << 8 | (b.q[4 * k + 2] & 0xFF) << 16 | b.q[4 * k + 3] << 24;
     }
 }
 
 // x [p_rows][in_dim] fp32 -> image, and the blocks themselves to xq [p_rows][in_dim / 32] (the caller of rein_matmul_ws may read
-// them there).  blockIdx.x = token tile, blockIdx.y = superblock, 256 threads: thread 8 j + s handles token j,
-// sub-block s: eight threads read a kilobyte of a row and write runs of 128 bytes to the image and 320 to xq.
-// Bound by memory: 4 bytes in, 3.4 out per value (777 x 17408: 54 + 46 MB).
+// them there).  blockIdx.x = eight tokens, blockIdx.y = superblock, 256 threads, four to a block of 32: a wavefront reads 512 bytes of
+// four rows and writes runs of 64 bytes to the image and 160 to xq (eight rows of 256 bytes, or two of 1024: 2048 x 5120 17.2 -> 17.7 us).
+// Bound by memory from a few hundred rows on: 4 bytes in, 3.4 out per value (777 x 17408: 54 + 46 MB); below, by the latency of a load and of
+// what a thread does with it, which is why a block has four (a thread a block: 30 x 5120 4.0 us instead of 2.9).
+struct XhQuantize { unsigned q, j, tok, sb; };
+__device__ __forceinline__ XhQuantize rein_xh_quantize_who()             // j: the token in its tile
+{
+    const unsigned l = threadIdx.x & 63u, w = threadIdx.x >> 6, tok = blockIdx.x * 8u + (w >> 1) * 4u + (l >> 4);
+    return XhQuantize{l & 3u, tok & 31u, tok, blockIdx.y * 8u + (w & 1u) * 4u + ((l >> 2) & 3u)};
+}
 __device__ __forceinline__ void rein_xh_quantize_body(const float* __restrict__ x, uint8_t* __restrict__ img, BlockQ8* __restrict__ xq, unsigned in_dim,
                                                       unsigned p_rows, unsigned with_xsum)
 {
-    __shared__ float xsum[8][33];
-    const unsigned n_tt = (p_rows + 31u) / 32u, n_sub = in_dim >> 5, tt = blockIdx.x, c = blockIdx.y;
-    const unsigned j = threadIdx.x >> 3, s = threadIdx.x & 7u, sb = c * 8u + s;
+    __shared__ float xsum[8][9];
+    const XhQuantize w = rein_xh_quantize_who();
+    const unsigned n_tt = (p_rows + 31u) / 32u, n_sub = in_dim >> 5, tt = w.tok >> 5;
     XhBlock b;
-    rein_xh_quantize_block(b, x, xq, in_dim, p_rows, tt * 32u + j, sb);
-    uint8_t* rec = img + ((size_t)(sb >> 1) * n_tt + tt) * REIN_XH_REC;
-    reinterpret_cast<float*>(rec + REIN_XH_X)[(sb & 1u) * 32u + j] = b.d;
+    rein_xh_quantize_block(b, x, xq, in_dim, p_rows, w.tok, w.sb, w.q);
+    uint8_t* rec = img + ((size_t)(w.sb >> 1) * n_tt + tt) * REIN_XH_REC;
+    if (w.q == 0u) reinterpret_cast<float*>(rec + REIN_XH_X)[(w.sb & 1u) * 32u + w.j] = b.d;
+    const unsigned kh = w.q & 1u, h = w.q >> 1;          // words 2 h + kh
+    rein_v8h o;
 #pragma unroll
-    for (int kh = 0; kh < 2; kh++)
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-            rein_v8h o;
-#pragma unroll
-            for (int e = 0; e < 8; e++) o[e] = (_Float16)b.q[rein_xh_slot_weight(kh, h, e)];
-            *reinterpret_cast<rein_v8h*>(rec + (sb & 1u) * 2048u + kh * 1024u + (32u * h + j) * 16u) = o;
-        }
+    for (int e = 0; e < 8; e++) {
+        constexpr int half[8] = {0, 0, 4, 4, 0, 0, 4, 4};
+        o[e] = (_Float16)b.q[half[e] + (rein_xh_slot_weight(0, 0, e) & 3)];
+    }
+    *reinterpret_cast<rein_v8h*>(rec + (w.sb & 1u) * 2048u + kh * 1024u + (32u * h + w.j) * 16u) = o;
     if (!with_xsum) return;                          // the image of a format without minimums has no xsum part
-    xsum[s][j] = b.sum;
+    if (w.q == 0u) xsum[w.sb & 7u][w.tok & 7u] = b.sum;
     __syncthreads();
-    if (threadIdx.x < 128u) {                        // op = threadIdx.x / 64, lane = threadIdx.x % 64
-        const unsigned op = threadIdx.x >> 6, h = (threadIdx.x >> 5) & 1u;
-        uint32_t o[4] = {0u, 0u, 0u, 0u};
-        if (op == 0u || h == 0u) {
+    if (threadIdx.x < 32u) {                         // [op][lane half][token]
+        const unsigned op = threadIdx.x >> 4, hh = (threadIdx.x >> 3) & 1u, j = (blockIdx.x * 8u + (threadIdx.x & 7u)) & 31u;
+        uint32_t o3[4] = {0u, 0u, 0u, 0u};
+        if (op == 0u || hh == 0u) {
 #pragma unroll
             for (int k = 0; k < 8; k++) {
                 uint16_t p3[3];
-                rein_mmq_split_xsum(xsum[k][threadIdx.x & 31u], p3);
-                const uint32_t x3 = op ? p3[2] : (h ? p3[1] : p3[0]);
-                o[k >> 1] |= x3 << (16 * (k & 1));
+                rein_mmq_split_xsum(xsum[k][threadIdx.x & 7u], p3);
+                const uint32_t x3 = op ? p3[2] : (hh ? p3[1] : p3[0]);
+                o3[k >> 1] |= x3 << (16 * (k & 1));
             }
         }
-        uint8_t* dst = img + (size_t)(n_sub >> 1) * n_tt * REIN_XH_REC + ((size_t)c * n_tt + tt) * REIN_XH_XS;
-        *reinterpret_cast<uint4*>(dst + threadIdx.x * 16u) = make_uint4(o[0], o[1], o[2], o[3]);
+        uint8_t* dst = img + (size_t)(n_sub >> 1) * n_tt * REIN_XH_REC + ((size_t)blockIdx.y * n_tt + tt) * REIN_XH_XS;
+        *reinterpret_cast<uint4*>(dst + op * 1024u + (32u * hh + j) * 16u) = make_uint4(o3[0], o3[1], o3[2], o3[3]);
     }
 }
 

@@ -32,20 +32,16 @@
 __device__ __forceinline__ void rein_x8_quantize_body(const float* __restrict__ x, uint8_t* __restrict__ img, BlockQ8* __restrict__ xq, unsigned in_dim,
                                                       unsigned p_rows)
 {
-    const unsigned n_tt = (p_rows + 31u) / 32u, tt = blockIdx.x, j = threadIdx.x >> 3, sb = blockIdx.y * 8u + (threadIdx.x & 7u);
+    const XhQuantize w = rein_xh_quantize_who();
+    const unsigned n_tt = (p_rows + 31u) / 32u;
     XhBlock b;
-    rein_xh_quantize_block(b, x, xq, in_dim, p_rows, tt * 32u + j, sb);
-    uint8_t* rec = img + ((size_t)(sb >> 1) * n_tt + tt) * REIN_X8_REC;
-    reinterpret_cast<float*>(rec + REIN_X8_X)[(sb & 1u) * 32u + j] = b.d;
+    rein_xh_quantize_block(b, x, xq, in_dim, p_rows, w.tok, w.sb, w.q);
+    uint8_t* rec = img + ((size_t)(w.sb >> 1) * n_tt + (w.tok >> 5)) * REIN_X8_REC;
+    if (w.q == 0u) reinterpret_cast<float*>(rec + REIN_X8_X)[(w.sb & 1u) * 32u + w.j] = b.d;
 #pragma unroll
     for (int h = 0; h < 2; h++) {
-        uint32_t o[4];
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int* q = b.q + 16 * h + 4 * i;
-            o[i] = (q[0] & 0xFF) | (q[1] & 0xFF) << 8 | (q[2] & 0xFF) << 16 | (uint32_t)q[3] << 24;
-        }
-        *reinterpret_cast<uint4*>(rec + (sb & 1u) * 1024u + (32u * h + j) * 16u) = make_uint4(o[0], o[1], o[2], o[3]);
+        const int* q = b.q + 4 * h;
+        *reinterpret_cast<uint32_t*>(rec + (w.sb & 1u) * 1024u + (32u * h + w.j) * 16u + 4u * w.q) = (q[0] & 0xFF) | (q[1] & 0xFF) << 8 | (q[2] & 0xFF) << 16 | (uint32_t)q[3] << 24;
     }
 }
 
