@@ -2045,7 +2045,8 @@ size_t wide_image_bytes(int fmt, unsigned in_dim, unsigned p_rows)
 unsigned wide_lds_bytes(const WideKind& kind, int fmt)
 {
     if (!wide_k_quant(fmt)) return 2 * 18432 + 4 * (fmt == REIN_TYPE_Q8_0 ? 8192 : 4096) + 4 * 2048;         // X8Lds
-    return 2 * kind.most * 4352 + 4 * 4096 + 4 * 3584 + (wide_has_min(fmt) ? kind.most * 2048 : 0);          // rein_xh_lds_bytes
+    const unsigned extra = fmt == REIN_TYPE_Q6_K ? 2048 : fmt == REIN_TYPE_Q5_K ? 1024 : 0;                     // XhLds
+    return 2 * kind.most * (4096 + 1024) + 4 * 4096 + 4 * (extra + 1536 + 512) + (wide_has_min(fmt) ? kind.most * 2048 : 0);
 }
 // Where they are taken, from sweeps through rein_matmul_ws, every cell beside the launches of rein_mmq_xq8_ws (their time / this one's),
 // the weights of two to six matrices in turn:

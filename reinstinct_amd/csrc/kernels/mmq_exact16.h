@@ -56,37 +56,28 @@ __host__ __device__ constexpr int rein_xh_slot_weight(int kh, int h, int e)
 }
 
 // ---- activation image -----------------------------------------------------------------
-//   records  [sub-block pair][32-token tile] of 4352 bytes:
-//              [q: sub-block of the pair][kh][lane = 32 h + token][8 x fp16], then dx [q][32] fp32
+//   records  [superblock][32-token tile] of 17408 bytes: [sub-block][kh][lane = 32 h + token][8 x fp16], then dx [sub-block][token] fp32
 //   xsum     [superblock][32-token tile] of 2048 bytes: [op][lane][8 x bf16]: lane halves 0 / 1 of op 0 the first and second
 //            bf16 of the 8 sub-blocks' xsum, half 0 of op 1 the third, half 1 zeros
-#define REIN_XH_X   4096u
-#define REIN_XH_REC 4352u
-#define REIN_XH_XS  2048u
+#define REIN_XH_PAIR 4096u
+#define REIN_XH_X    16384u
+#define REIN_XH_REC  17408u
+#define REIN_XH_DX   1024u
+#define REIN_XH_XS   2048u
+struct XhImage {
+    uint8_t *rec, *xs;
+    unsigned n_tt;
+    __device__ __forceinline__ XhImage(uint8_t* img, unsigned in_dim, unsigned n_tt) : rec(img), xs(img + (size_t)(in_dim >> 8) * n_tt * REIN_XH_REC), n_tt(n_tt) {}
+};
 
 // A block of 32 values of row `tok` (zeros past p_rows, with d = 0) with the numbers that quantize_q8_f32 gives, by four lanes: lane q of
 // the four holds values 4 q .. 4 q + 3 and those 16 further on, which are the two dwords of quants that it writes to xq and one 16-byte
 // piece of the operand order.  The sum tree is halves of 16 (inside the lane), 8 and 4 (between lanes), 2 and 1.
 struct XhBlock { float d, sum; int q[8]; };
-__device__ __forceinline__ void rein_xh_quantize_block(XhBlock& b, const float* __restrict__ x, BlockQ8* __restrict__ xq, unsigned in_dim, unsigned p_rows,
-                                                       unsigned tok, unsigned sb, unsigned q)
+__device__ __forceinline__ void rein_xh_quantize_values(XhBlock& b, const float (&v)[8])
 {
 #pragma clang fp contract(off)
-    float v[8], t[4];
-#pragma unroll
-    for (int i = 0; i < 8; i++) v[i] = 0.0f;
-    if (tok < p_rows) {
-        const float* p = x + (size_t)tok * in_dim + sb * 32u + 4u * q;
-        if (((size_t)x & 15u) == 0u) {
-            const float4 lo = reinterpret_cast<const float4*>(p)[0], hi = reinterpret_cast<const float4*>(p)[4];
-            v[0] = lo.x; v[1] = lo.y; v[2] = lo.z; v[3] = lo.w;
-            v[4] = hi.x; v[5] = hi.y; v[6] = hi.z; v[7] = hi.w;
-        } else {
-#pragma unroll
-            for (int i = 0; i < 4; i++) { v[i] = p[i]; v[4 + i] = p[16 + i]; }
-        }
-    }
-    float amax = 0.0f;
+    float t[4], amax = 0.0f;
 #pragma unroll
     for (int i = 0; i < 8; i++) amax = fmaxf(amax, fabsf(v[i]));
     amax = fmaxf(amax, rein_dpp_f32<0x4E>(amax, amax));                  // lane ^ 2
@@ -98,17 +89,69 @@ __device__ __forceinline__ void rein_xh_quantize_block(XhBlock& b, const float* 
 #pragma unroll
     for (int i = 0; i < 4; i++) t[i] = t[i] + rein_dpp_f32<0xB1>(t[i], t[i]);
     b.sum = (t[0] + t[2]) + (t[1] + t[3]);
-    b.d   = tok >= p_rows ? 0.0f : amax > 0.0f ? amax / 127.0f : 1.0f;
+    b.d   = amax > 0.0f ? amax / 127.0f : 1.0f;
     const float inv = amax > 0.0f ? 127.0f / amax : 0.0f;
 #pragma unroll
     for (int i = 0; i < 8; i++) b.q[i] = max(-127, min(127, (int)rintf(v[i] * inv)));
+}
+// values 4 q .. 4 q + 3 and 16 further on of block sb of a row
+__device__ __forceinline__ void rein_xh_load_values(float (&v)[8], const float* __restrict__ row, unsigned sb, unsigned q, bool aligned)
+{
+    const float* p = row + sb * 32u + 4u * q;
+    if (aligned) {
+        const float4 lo = reinterpret_cast<const float4*>(p)[0], hi = reinterpret_cast<const float4*>(p)[4];
+        v[0] = lo.x; v[1] = lo.y; v[2] = lo.z; v[3] = lo.w;
+        v[4] = hi.x; v[5] = hi.y; v[6] = hi.z; v[7] = hi.w;
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; i++) { v[i] = p[i]; v[4 + i] = p[16 + i]; }
+    }
+}
+// a lane's dword of the first (k = 0) or second sixteen quants
+__device__ __forceinline__ uint32_t rein_xh_word(const XhBlock& b, int k)
+{
+    return (b.q[4 * k] & 0xFF) | (b.q[4 * k + 1] & 0xFF) << 8 | (b.q[4 * k + 2] & 0xFF) << 16 | (uint32_t)b.q[4 * k + 3] << 24;
+}
+__device__ __forceinline__ void rein_xh_quantize_block(XhBlock& b, const float* __restrict__ x, BlockQ8* __restrict__ xq, unsigned in_dim, unsigned p_rows,
+                                                       unsigned tok, unsigned sb, unsigned q)
+{
+    float v[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) v[i] = 0.0f;
+    if (tok < p_rows) rein_xh_load_values(v, x + (size_t)tok * in_dim, sb, q, ((size_t)x & 15u) == 0u);
+    rein_xh_quantize_values(b, v);
+    if (tok >= p_rows) b.d = 0.0f;
     if (tok < p_rows) {
         BlockQ8* const o = xq + (size_t)tok * (in_dim >> 5) + sb;
         if (q == 0u) { o->d = b.d; o->xsum = b.sum; }
 #pragma unroll
-        for (int k = 0; k < 2; k++)
-            o->qs[4 * k + q] = (b.q[4 * k] & 0xFF) | (b.q[4 * k + 1] & 0xFF) << 8 | (b.q[4 * k + 2] & 0xFF) << 16 | b.q[4 * k + 3] << 24;
+        for (int k = 0; k < 2; k++) o->qs[4 * k + q] = rein_xh_word(b, k);
     }
+}
+
+// A block's piece of the image: sub-block sb of token j of a tile
+__device__ __forceinline__ void rein_xh_store_block(const XhImage& img, const XhBlock& b, unsigned tile, unsigned sb, unsigned j, unsigned q)
+{
+    uint8_t* const rec = img.rec + ((size_t)(sb >> 3) * img.n_tt + tile) * REIN_XH_REC;
+    if (q == 0u) reinterpret_cast<float*>(rec + REIN_XH_X)[(sb & 7u) * 32u + j] = b.d;
+    const unsigned kh = q & 1u, h = q >> 1;          // words 2 h + kh
+    rein_v8h o;
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        constexpr int part[8] = {0, 0, 4, 4, 0, 0, 4, 4};
+        o[e] = (_Float16)b.q[part[e] + (rein_xh_slot_weight(0, 0, e) & 3)];
+    }
+    *reinterpret_cast<rein_v8h*>(rec + (sb & 7u) * 2048u + kh * 1024u + (32u * h + j) * 16u) = o;
+}
+// The first to third bf16 of two sub-blocks' xsum as the word of operand `op` for lane half hh
+__device__ __forceinline__ uint32_t rein_xh_xsum_word(float s0, float s1, unsigned op, unsigned hh)
+{
+    uint16_t a[3], b[3];
+    rein_mmq_split_xsum(s0, a);
+    rein_mmq_split_xsum(s1, b);
+    const unsigned k = op ? 2u : hh;
+    const uint32_t x0 = k == 2u ? a[2] : k ? a[1] : a[0], x1 = k == 2u ? b[2] : k ? b[1] : b[0];
+    return op && hh ? 0u : x0 | x1 << 16;
 }
 
 // x [p_rows][in_dim] fp32 -> image, and the blocks themselves to xq [p_rows][in_dim / 32] (the caller of rein_matmul_ws may read
@@ -127,35 +170,20 @@ __device__ __forceinline__ void rein_xh_quantize_body(const float* __restrict__ 
 {
     __shared__ float xsum[8][9];
     const XhQuantize w = rein_xh_quantize_who();
-    const unsigned n_tt = (p_rows + 31u) / 32u, n_sub = in_dim >> 5, tt = w.tok >> 5;
+    const XhImage image(img, in_dim, (p_rows + 31u) / 32u);
+    const unsigned tt = w.tok >> 5;
     XhBlock b;
     rein_xh_quantize_block(b, x, xq, in_dim, p_rows, w.tok, w.sb, w.q);
-    uint8_t* rec = img + ((size_t)(w.sb >> 1) * n_tt + tt) * REIN_XH_REC;
-    if (w.q == 0u) reinterpret_cast<float*>(rec + REIN_XH_X)[(w.sb & 1u) * 32u + w.j] = b.d;
-    const unsigned kh = w.q & 1u, h = w.q >> 1;          // words 2 h + kh
-    rein_v8h o;
-#pragma unroll
-    for (int e = 0; e < 8; e++) {
-        constexpr int half[8] = {0, 0, 4, 4, 0, 0, 4, 4};
-        o[e] = (_Float16)b.q[half[e] + (rein_xh_slot_weight(0, 0, e) & 3)];
-    }
-    *reinterpret_cast<rein_v8h*>(rec + (w.sb & 1u) * 2048u + kh * 1024u + (32u * h + w.j) * 16u) = o;
+    rein_xh_store_block(image, b, tt, w.sb, w.j, w.q);
     if (!with_xsum) return;                          // the image of a format without minimums has no xsum part
     if (w.q == 0u) xsum[w.sb & 7u][w.tok & 7u] = b.sum;
     __syncthreads();
     if (threadIdx.x < 32u) {                         // [op][lane half][token]
         const unsigned op = threadIdx.x >> 4, hh = (threadIdx.x >> 3) & 1u, j = (blockIdx.x * 8u + (threadIdx.x & 7u)) & 31u;
-        uint32_t o3[4] = {0u, 0u, 0u, 0u};
-        if (op == 0u || hh == 0u) {
+        uint32_t o3[4];
 #pragma unroll
-            for (int k = 0; k < 8; k++) {
-                uint16_t p3[3];
-                rein_mmq_split_xsum(xsum[k][threadIdx.x & 7u], p3);
-                const uint32_t x3 = op ? p3[2] : (hh ? p3[1] : p3[0]);
-                o3[k >> 1] |= x3 << (16 * (k & 1));
-            }
-        }
-        uint8_t* dst = img + (size_t)(n_sub >> 1) * n_tt * REIN_XH_REC + ((size_t)blockIdx.y * n_tt + tt) * REIN_XH_XS;
+        for (int k = 0; k < 4; k++) o3[k] = rein_xh_xsum_word(xsum[2 * k][threadIdx.x & 7u], xsum[2 * k + 1][threadIdx.x & 7u], op, hh);
+        uint8_t* dst = image.xs + ((size_t)blockIdx.y * image.n_tt + tt) * REIN_XH_XS;
         *reinterpret_cast<uint4*>(dst + op * 1024u + (32u * hh + j) * 16u) = make_uint4(o3[0], o3[1], o3[2], o3[3]);
     }
 }
@@ -297,42 +325,51 @@ __device__ __forceinline__ void rein_xh_pin(float (&s)[16])
 
 // ---- the tile -------------------------------------------------------------------------
 // LDS of one workgroup:
-//   acts  2 x MOST x 4352  records of two consecutive sub-block pairs
+//   acts  2 x MOST x 4096  records of two consecutive sub-block pairs
+//   dx    2 x MOST x 1024  activation scales of two superblocks
 //   ring  4 x 2 x 2048     per wavefront: two slots of 4 sub-blocks x 32 rows x 16 B
-//   small 4 x 3584         per wavefront: extra bits of a superblock [row][sub-block] in granules of 16 bytes, rotated; (sc, m) or
-//                          both group scales [row][sub-block], in two bytes each or (padded rows) four; the scale words of two
-//                          superblocks [row]
-//   xs    MOST x 2048          xsum operands of a superblock (formats with minimums)
-// MOST: tiles of the launch's largest group, 4 or (rein_xf_*) 2.
-template <int FMT, unsigned MOST> constexpr unsigned rein_xh_lds_bytes()
-{
-    return 2u * MOST * REIN_XH_REC + 4u * 2u * 2048u + 4u * 3584u + (XhWeights<FMT>::kHasMin ? MOST * REIN_XH_XS : 0u);
-}
+//   small 4 x              per wavefront: extra bits of a superblock [row][sub-block] in granules of 16 bytes, rotated; (sc, m) or both
+//                          group scales of two superblocks, 48 bytes a row; the scale words of four [row][superblock] in a dword each
+//   xs    MOST x 2048      xsum operands of a superblock (formats with minimums)
+// MOST: tiles of the launch's largest group, 4 (80 KB: two workgroups to a CU) or (rein_xf_*) 2 (52 KB: three).
+template <int FMT, unsigned MOST> struct XhLds {
+    static constexpr unsigned kAct = MOST * REIN_XH_PAIR, kDx = 2u * kAct, kRing = kDx + 2u * MOST * REIN_XH_DX, kSmall = kRing + 4u * 4096u;
+    static constexpr unsigned kSm = 256u * XhWeights<FMT>::kHiBytes, kD = kSm + 1536u, kWave = kD + 512u, kXs = kSmall + 4u * kWave;
+    static constexpr unsigned kBytes = kXs + (XhWeights<FMT>::kHasMin ? MOST * REIN_XH_XS : 0u);
+    static_assert(kBytes <= (MOST == 2u ? 54272u : 81920u), "LDS for three workgroups to a CU, or two");
+};
 
-// Superblocks [c0, c1) of rows 128 rb .. and the NT token tiles from `tile` on, into acc.  One barrier per sub-block
+// Superblocks [c0, c1) of the wavefront's 32 rows from row_base on and the NT token tiles from `tile` on, into acc.  One barrier per sub-block
 // pair: at its top everything in flight has landed (it was issued a whole pair earlier: 8 NT or 16 NT matrix instructions per
 // wavefront), behind it the next pair's transfers go out.
 template <int FMT, int NT, unsigned MOST>
 __device__ __forceinline__ void rein_xh_acc(const uint8_t* __restrict__ w, const uint8_t* __restrict__ img, unsigned in_dim, unsigned out_dim,
-                                            unsigned n_tt, unsigned rb, unsigned tile, unsigned c0, unsigned c1, unsigned char* const raw, float (&acc)[NT][16])
+                                            unsigned n_tt, unsigned row_base, unsigned tile, unsigned c0, unsigned c1, unsigned char* const raw, float (&acc)[NT][16])
 {
     using W = XhWeights<FMT>;
     typedef __attribute__((address_space(3))) const void* lptr_t;
-    constexpr unsigned kRing = 2u * MOST * REIN_XH_REC, kSmall = kRing + 4u * 4096u, kXs = kSmall + 4u * 3584u;
+    using L = XhLds<FMT, MOST>;
     const unsigned lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), j = lane & 31u, h = lane >> 5;
     const unsigned n_sub = in_dim >> 5;
     const Fmt<FMT> fmt(w, n_sub, out_dim);
-    const unsigned row_base = rb * 128u + wave * 32u, first = min(row_base, out_dim - 1u);
+    const unsigned first = min(row_base, out_dim - 1u);
     // rows past the matrix read its last one; offsets from the wavefront's first row
     const unsigned row = min(row_base + j, out_dim - 1u) - first;
-    const unsigned d_off = row * fmt.n_super * W::kDBytes;
-    // Extra bits and scales come sixteen bytes a lane, one to three transfers a superblock (by dword and 16-bit word they were
-    // thirteen, each as long as a kilobyte's: 2048 x 5120 -> 17408 Q6_K 749 -> 699 us, Q5_K 633 -> 569, Q5_K 45 x 17408 -> 5120 43 -> 38).
-    // A row's superblock of extra bits is four granules (Q6_K) or two (Q5_K), rotated so that the reads of one granule of every row
-    // meet every bank; its scales are one, unless the slab's rows are padded (a power of two of sub-blocks), which leaves them at
-    // two-byte alignment: then they come by 16-bit words.
-    const bool padded = (fmt.nsp & 1u) != 0u;
+    // Transfers of a step go out one by one between the matrix instructions of three and four tiles; with one or two tiles there are
+    // too few instructions for that, and they go out at the step's top (spread: Q4_K 60 x 5120 -> 5120 19.9 -> 20.9 us).
+    constexpr bool kSpread = NT > 2;
+    // Small planes come in long pieces: a transfer occupies a CU's address path for 16 cycles if its 64 lanes are one run, for 23 if they are
+    // 16 runs, for 64 if they are 32, however few bytes those are.  A row's superblock of extra bits is four granules (Q6_K) or two
+    // (Q5_K), rotated so that the reads of one granule of every row meet every bank.  With one and two tiles, where a weight is used least:
+    //   (sc, m)      of two superblocks, three granules from the dword boundary below them on (rows start at two bytes where the slab pads
+    //                them): two transfers of 64 granules, the middle third in both.  What that reads behind a row's end is the next row or,
+    //                behind the last, up to 32 bytes of the plane of scale words; a matrix that has fewer of those takes its scales word by word.
+    //   scale words  of four superblocks, a lane each.
+    // (a superblock at a time and by 16-bit words in padded rows: 45 x 17408 -> 5120 Q5_K 35.5 -> 33.8 us, 512 tokens of 128 experts of 2048 x 768,
+    // gate + up 105 -> 100).  With three and four tiles the scales of a superblock are one transfer (padded: four) and its scale words another: the
+    // branches that the longer pieces need cost more between the matrix instructions (777 x 17408 -> 5120 Q6_K 318 -> 326 us).
     auto row_at = [&](unsigned n) { return min(row_base + n, out_dim - 1u) - first; };
+    const unsigned odd = ((first + row) * fmt.nsp * 2u) & 2u;            // of this lane's row
     unsigned hi_off[2] = {0u, 0u}, sm_off[4];
     if constexpr (W::kHiBytes == 8) {
 #pragma unroll
@@ -343,62 +380,87 @@ __device__ __forceinline__ void rein_xh_acc(const uint8_t* __restrict__ w, const
     } else if constexpr (W::kHiBytes == 4) {
         hi_off[0] = row_at(lane >> 1) * fmt.nsp * 4u + ((lane ^ (lane >> 3)) & 1u) * 16u;
     }
+    const bool padded = (fmt.nsp & 1u) != 0u;
 #pragma unroll
-    for (unsigned k = 0; k < 4; k++)                 // (unpadded: the upper lanes fetch the rows again)
-        sm_off[k] = padded ? (row_at(8u * k + (lane >> 3)) * fmt.nsp + (lane & 7u)) * 2u : row * fmt.nsp * 2u;
-    const unsigned sm_step = padded ? 4u : 2u;
+    for (unsigned k = 0; k < (kSpread ? 4u : 2u); k++) {
+        if constexpr (kSpread) {                     // (unpadded: the upper lanes fetch the rows again)
+            sm_off[k] = padded ? (row_at(8u * k + (lane >> 3)) * fmt.nsp + (lane & 7u)) * 2u : row * fmt.nsp * 2u;
+        } else {
+            const unsigned i = 32u * k + lane, n = i / 3u, r = row_at(n);
+            sm_off[k] = r * fmt.nsp * 2u - (((first + r) * fmt.nsp * 2u) & 2u) + (i - 3u * n) * 16u + 2u;      // from two bytes below the plane's place
+        }
+    }
+    const unsigned sm_step = kSpread && padded ? 4u : 2u;
 
-    const uint4* const ring = reinterpret_cast<const uint4*>(raw + kRing + wave * 4096u);
-    const unsigned char* const small = raw + kSmall + wave * 3584u;
+
+    const uint4* const ring = reinterpret_cast<const uint4*>(raw + L::kRing + wave * 4096u);
+    const unsigned char* const small = raw + L::kSmall + wave * L::kWave;
     const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(lptr_t)raw);
     MmqWSrc<FMT> wsrc;
     wsrc.init(*reinterpret_cast<const MmqWLds<FMT>*>(ring), fmt, row_base, out_dim, lane);
-    const uint8_t* const xsimg = img + (size_t)(n_sub >> 1) * n_tt * REIN_XH_REC;
+    const XhImage image(const_cast<uint8_t*>(img), in_dim, n_tt);
 
     // src: a pair's record of the first tile.  It runs along with the pairs: addresses worked out of the pair's number for each transfer
     // cost as much scalar issue as the transfers do (777 x 17408 -> 5120 Q6_K 328 -> 320 us).
     auto issue_act = [&](const uint8_t* src, unsigned buf, unsigned t) {
-        const unsigned off = t * REIN_XH_REC + wave * 1024u;
-        rein_lds_dma16_s(lane * 16u, src + off, lds0 + buf * (MOST * REIN_XH_REC) + off);
+        const unsigned at = wave * 1024u;
+        rein_lds_dma16_s(lane * 16u, src + t * REIN_XH_REC + at, lds0 + buf * L::kAct + t * REIN_XH_PAIR + at);
     };
-    auto issue_dx = [&](const uint8_t* src, unsigned buf) {              // (the wavefronts past the last tile fetch its scales again)
-        const unsigned off = min(wave, (unsigned)NT - 1u) * REIN_XH_REC + REIN_XH_X;
-        rein_xh_dma_u32(lane * 4u, src + off, lds0 + buf * (MOST * REIN_XH_REC) + off);
+    auto issue_dx = [&](unsigned c) {
+        if (NT == 4 || wave < (unsigned)NT) rein_lds_dma16_s(lane * 16u, img + ((size_t)c * n_tt + tile + wave) * REIN_XH_REC + REIN_XH_X, lds0 + L::kDx + ((c & 1u) * MOST + wave) * REIN_XH_DX);
     };
     auto issue_xs = [&](unsigned c) {
         if constexpr (W::kHasMin) {
-            const uint8_t* src = xsimg + ((size_t)c * n_tt + tile) * REIN_XH_XS;
+            const uint8_t* src = image.xs + ((size_t)c * n_tt + tile) * REIN_XH_XS;
 #pragma unroll
             for (unsigned k = 0; k < 2; k++) {
                 const unsigned off = (k * 4u + wave) * 1024u;
-                if (k * 4u + wave < 2u * NT) rein_lds_dma16_s(lane * 16u, src + off, lds0 + kXs + off);
+                if (k * 4u + wave < 2u * NT) rein_lds_dma16_s(lane * 16u, src + off, lds0 + L::kXs + off);
             }
         }
     };
-    auto issue_small = [&](unsigned c) {
-        const unsigned dst = lds0 + kSmall + wave * 3584u;
+    const unsigned small_at = lds0 + L::kSmall + wave * L::kWave;
+    auto issue_hi = [&](unsigned c) {
         if constexpr (W::kHiBytes != 0) {
             const char* hp = W::hi(fmt) + ((size_t)first * fmt.nsp + c * 8u) * W::kHiBytes;
-            rein_lds_dma16_s(hi_off[0], hp, dst);
-            if constexpr (W::kHiBytes == 8) rein_lds_dma16_s(hi_off[1], hp, dst + 1024u);
+            rein_lds_dma16_s(hi_off[0], hp, small_at);
+            if constexpr (W::kHiBytes == 8) rein_lds_dma16_s(hi_off[1], hp, small_at + 1024u);
         }
+    };
+    auto issue_sm = [&](unsigned c) {                // of c (and c + 1)
         const char* sp = reinterpret_cast<const char*>(fmt.smp) + ((size_t)first * fmt.nsp + c * 8u) * 2u;
-        if (padded) {
+        if constexpr (kSpread) {
+            if (padded) {
 #pragma unroll
-            for (unsigned k = 0; k < 4; k++) rein_xh_dma_u16(sm_off[k], sp, dst + 2048u + k * 256u);
-        } else {
-            rein_lds_dma16_s(sm_off[0], sp, dst + 2048u);
+                for (unsigned k = 0; k < 4; k++) rein_xh_dma_u16(sm_off[k], sp, small_at + L::kSm + k * 256u);
+            } else {
+                rein_lds_dma16_s(sm_off[0], sp, small_at + L::kSm);
+            }
+        } else if (out_dim * fmt.n_super >= 16u) {
+#pragma unroll
+            for (unsigned k = 0; k < 2; k++) rein_lds_dma16_s(sm_off[k], sp - 2, small_at + L::kSm + k * 512u);
+        } else if (lane < 32u) {
+            uint16_t* const to = reinterpret_cast<uint16_t*>(raw + L::kSmall + wave * L::kWave + L::kSm + j * 48u + odd);
+            for (unsigned k = 0; k < 16u && c * 8u + k < n_sub; k++) to[k] = fmt.smp[(size_t)(first + row) * fmt.nsp + c * 8u + k];
         }
+    };
+    // Scale words: of one superblock (in two places, odd and even) where a step has room for a transfer of 32 runs; of four, a lane each, with
+    // one and two tiles
+    constexpr unsigned kD4 = kSpread ? 1u : 4u;
+    const unsigned d_off = row * fmt.n_super * W::kDBytes;
+    auto issue_d = [&](unsigned c) {
         const char* dp = W::d(fmt) + ((size_t)first * fmt.n_super + c) * W::kDBytes;
-        if constexpr (W::kDBytes == 4) rein_xh_dma_u32(d_off, dp, dst + 3072u + (c & 1u) * 256u);
-        else rein_xh_dma_u16(d_off, dp, dst + 3072u + (c & 1u) * 256u);
+#pragma unroll
+        for (unsigned k = 0; k < (kSpread ? 1u : 2u); k++) {
+            const unsigned off = kSpread ? d_off : (row_at(16u * k + (lane >> 2)) * fmt.n_super + min(lane & 3u, fmt.n_super - 1u - c)) * W::kDBytes;
+            const unsigned to = small_at + L::kD + (kSpread ? c & 1u : k) * 256u;
+            if constexpr (W::kDBytes == 4) rein_xh_dma_u32(off, dp, to);
+            else rein_xh_dma_u16(off, dp, to);
+        }
     };
     // Dots are multiplied by their dx one stage after their instructions went out, two where a stage has two instructions and registers
     // are left: nothing waits for the matrix unit then (Q4_K 2048 x 5120 -> 17408 540 -> 530 us).
     constexpr int kLag = W::kOps == 1 && NT > 2 ? 2 : 1, kBuf = kLag + 1;
-    // Transfers of a step go out one by one between the matrix instructions of three and four tiles; with one or two tiles there are
-    // too few instructions for that, and they go out at the step's top (spread: Q4_K 60 x 5120 -> 5120 19.9 -> 20.9 us).
-    constexpr bool kSpread = NT > 2;
     rein_v16f dot[kBuf], z16;
     float s1[NT][16];
     float dx[kBuf];
@@ -411,13 +473,15 @@ __device__ __forceinline__ void rein_xh_acc(const uint8_t* __restrict__ w, const
 #pragma unroll
     for (int b = 0; b < kBuf; b++) { dot[b] = z16; dx[b] = 0.0f; }
 
-    const size_t src_step = (size_t)n_tt * REIN_XH_REC;
-    const uint8_t* src = img + (c0 * 4u) * src_step + tile * REIN_XH_REC;
+    const size_t src_next = (size_t)n_tt * REIN_XH_REC - 3u * REIN_XH_PAIR;
+    const uint8_t* src = img + ((size_t)c0 * n_tt + tile) * REIN_XH_REC;
     __syncthreads();                                 // the LDS may still be read by the caller's previous tile
 #pragma unroll
     for (unsigned t = 0; t < (unsigned)NT; t++) issue_act(src, 0u, t);
-    issue_dx(src, 0u);
-    issue_small(c0);
+    issue_dx(c0);
+    if (kSpread) issue_d(c0);
+    issue_hi(c0);
+    issue_sm(c0);
     rein_mmq_wload<FMT>(wsrc, 0u, fmt, c0 * 8u, n_sub);
     const unsigned rot = j >> 1;
     const XhMasks mk;
@@ -428,10 +492,11 @@ __device__ __forceinline__ void rein_xh_acc(const uint8_t* __restrict__ w, const
         for (unsigned u = 0; u < 4; u++) {
             const unsigned pair = c * 4u + u;
             const bool more = c + 1u < c1;
-            if (u < 3u || more) src += src_step;     // (past the last pair: it again, read by nobody)
+            if (u < 3u) src += REIN_XH_PAIR;
+            else if (more) src += src_next;          // (past the last pair: it again, read by nobody)
             REIN_WAIT_VMCNT(0);
             __syncthreads();
-            const unsigned char* const sms = small + 2048u + (8u * j + 2u * u) * sm_step;
+            const unsigned char* const sms = small + L::kSm + (kSpread ? (8u * j + 2u * u) * sm_step : j * 48u + odd + ((c - c0) & 1u) * 16u + 4u * u);
             const uint32_t sm2[2] = {*reinterpret_cast<const uint16_t*>(sms), *reinterpret_cast<const uint16_t*>(sms + sm_step)};
             uint32_t hi2[2] = {0u, 0u};
             if constexpr (W::kHiBytes == 8) {
@@ -443,23 +508,33 @@ __device__ __forceinline__ void rein_xh_acc(const uint8_t* __restrict__ w, const
             }
             const unsigned buf = (pair & 1u) ^ 1u;
             auto issue_other = [&]() {
-                if (u == 0u) rein_mmq_wload<FMT>(wsrc, 1u, fmt, c * 8u + 4u, n_sub);
-                if (u == 1u) issue_xs(c);            // read at the superblock's end; the barrier of u = 0 freed it
+                if (u == 0u) {
+                    rein_mmq_wload<FMT>(wsrc, 1u, fmt, c * 8u + 4u, n_sub);
+                    if (!kSpread && ((c - c0) & 3u) == 0u) issue_d(c);   // read at the end of this superblock and the next three
+                }
+                if (u == 1u) {
+                    issue_xs(c);                     // read at the superblock's end; the barrier of u = 0 freed it
+                    if (!kSpread && more) issue_dx(c + 1u);
+                }
                 if (u == 2u && more) rein_mmq_wload<FMT>(wsrc, 0u, fmt, c * 8u + 8u, n_sub);
                 if (u == 3u && more) {
                     if constexpr (!kSpread) __builtin_amdgcn_s_waitcnt(0xC07F);          // lgkmcnt(0): the reads above have left the buffer
-                    issue_small(c + 1u);
+                    if constexpr (kSpread) {         // (any earlier step: 777 x 17408 -> 5120 Q6_K 325 -> 333 us)
+                        issue_dx(c + 1u);
+                        issue_d(c + 1u);
+                    }
+                    issue_hi(c + 1u);
+                    if (kSpread || ((c - c0) & 1u)) issue_sm(c + 1u);
                 }
             };
             if constexpr (!kSpread) {
                 if (u < 3u || more) {
 #pragma unroll
                     for (unsigned t = 0; t < (unsigned)NT; t++) issue_act(src, buf, t);
-                    if (wave < (unsigned)NT) issue_dx(src, buf);
                 }
                 issue_other();
             }
-            const unsigned char* const act = raw + (pair & 1u) * (MOST * REIN_XH_REC);
+            const unsigned char* const act = raw + (pair & 1u) * L::kAct;
 #pragma unroll
             for (unsigned q = 0; q < 2; q++) {
                 const unsigned sb = 2u * u + q, s4 = sb & 3u;
@@ -471,7 +546,7 @@ __device__ __forceinline__ void rein_xh_acc(const uint8_t* __restrict__ w, const
                     const uint32_t m = rein_bf16_of_u8(sm >> 8);
                     if (q == 0u) mpk[u] = m; else mpk[u] |= m << 16;
                 }
-                const float* const dxp = reinterpret_cast<const float*>(act + REIN_XH_X) + q * 32u + j;
+                const float* const dxp = reinterpret_cast<const float*>(raw + L::kDx + (c & 1u) * (MOST * REIN_XH_DX)) + sb * 32u + j;
                 const unsigned char* const x = act + q * 2048u + lane * 16u;
                 rein_v8h xa[2][2];
                 xa[0][0] = *reinterpret_cast<const rein_v8h*>(x);
@@ -487,12 +562,11 @@ __device__ __forceinline__ void rein_xh_acc(const uint8_t* __restrict__ w, const
                 for (int t = 0; t < NT; t++) {
                     const int i = (int)(sb * NT) + t, now = i % kBuf;
                     if (t + 1 < NT) {
-                        xa[(t + 1) & 1][0] = *reinterpret_cast<const rein_v8h*>(x + (t + 1) * REIN_XH_REC);
-                        xa[(t + 1) & 1][1] = *reinterpret_cast<const rein_v8h*>(x + (t + 1) * REIN_XH_REC + 1024u);
+                        xa[(t + 1) & 1][0] = *reinterpret_cast<const rein_v8h*>(x + (t + 1) * REIN_XH_PAIR);
+                        xa[(t + 1) & 1][1] = *reinterpret_cast<const rein_v8h*>(x + (t + 1) * REIN_XH_PAIR + 1024u);
                     }
                     if constexpr (kSpread) {
                         if (q == 0u) issue_act(src, buf, (unsigned)t);
-                        if (q == 0u && t == NT - 1) issue_dx(src, buf);
                         if (q == 1u && t == 0) issue_other();
                     }
                     dot[now] = z16;
@@ -501,7 +575,7 @@ __device__ __forceinline__ void rein_xh_acc(const uint8_t* __restrict__ w, const
                         dot[now] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[0][k], xa[t & 1][0], dot[now], 0, 0, 0);
                         dot[now] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[1][k], xa[t & 1][1], dot[now], 0, 0, 0);
                     }
-                    dx[now] = dxp[t * (REIN_XH_REC / 4u)];
+                    dx[now] = dxp[t * (REIN_XH_DX / 4u)];
                     if (i >= kLag) {
                         const int tp = (i - kLag) % NT, old = (i - kLag) % kBuf;
                         const bool first = i - kLag < NT;                            // the sums' first term of this superblock
@@ -537,14 +611,13 @@ __device__ __forceinline__ void rein_xh_acc(const uint8_t* __restrict__ w, const
 #pragma unroll
             for (int v = 0; v < 16; v++) s1[i % NT][v] = fmaf(dx[i % kBuf], dot[i % kBuf][v], s1[i % NT][v]);
         // acc += d s1 - dmin (m . xsum): register v is weight row 8 (v / 4) + 4 h + v % 4
-        const unsigned char* const xb = raw + kXs + lane * 16u;
+        const unsigned char* const xb = raw + L::kXs + lane * 16u;
         float dv[16], nv[16];
 #pragma unroll
         for (int g = 0; g < 4; g++) {
-            const uint4 d4 = *reinterpret_cast<const uint4*>(small + 3072u + (c & 1u) * 256u + (8 * g + 4u * h) * 4u);
-            const uint32_t dw[4] = {d4.x, d4.y, d4.z, d4.w};
+            const uint32_t* const dw = reinterpret_cast<const uint32_t*>(small + L::kD + (kSpread ? (c & 1u) * 256u : 0u) + (8 * g + 4u * h) * (4u * kD4)) + ((c - c0) & (kD4 - 1u));
 #pragma unroll
-            for (int v = 0; v < 4; v++) { dv[4 * g + v] = W::scale(dw[v]); nv[4 * g + v] = W::min_scale(dw[v]); }
+            for (int v = 0; v < 4; v++) { dv[4 * g + v] = W::scale(dw[kD4 * v]); nv[4 * g + v] = W::min_scale(dw[kD4 * v]); }
         }
 #pragma unroll
         for (int t = 0; t < NT; t++) {
@@ -573,9 +646,9 @@ template <int FMT, unsigned MOST> struct XhTile {
     static constexpr unsigned kMost = MOST, kLeast = MOST == 2u ? 1u : 2u, kSlots = MOST == 2u ? 768u : 512u;
     template <int NT>
     static __device__ __forceinline__ void run(const uint8_t* __restrict__ w, const uint8_t* __restrict__ img, unsigned in_dim, unsigned out_dim, unsigned n_tt,
-                                               unsigned rb, unsigned tile, unsigned c0, unsigned c1, unsigned char* const raw, float (&acc)[NT][16])
+                                               unsigned row_base, unsigned tile, unsigned c0, unsigned c1, unsigned char* const raw, float (&acc)[NT][16])
     {
-        rein_xh_acc<FMT, NT, MOST>(w, img, in_dim, out_dim, n_tt, rb, tile, c0, c1, raw, acc);
+        rein_xh_acc<FMT, NT, MOST>(w, img, in_dim, out_dim, n_tt, row_base, tile, c0, c1, raw, acc);
     }
 };
 
@@ -587,8 +660,8 @@ __device__ __forceinline__ void rein_xh_piece(const uint8_t* __restrict__ w, con
                                               unsigned char* raw)
 {
     float acc[NT][16];
-    Tile::template run<NT>(w, img, in_dim, out_dim, (p_rows + 31u) / 32u, rb, tile, c0, c1, raw, acc);
-    const unsigned lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, j = lane & 31u, h = lane >> 5;
+    const unsigned lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), j = lane & 31u, h = lane >> 5;
+    Tile::template run<NT>(w, img, in_dim, out_dim, (p_rows + 31u) / 32u, rb * 128u + wave * 32u, tile, c0, c1, raw, acc);
     if (part) {
 #pragma unroll
         for (int t = 0; t < NT; t++)

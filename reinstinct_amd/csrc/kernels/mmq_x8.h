@@ -28,6 +28,19 @@
 #define REIN_X8_X   2048u
 #define REIN_X8_REC 2304u
 
+// a block's piece of a record, as rein_xh_store_block: lane q's words of the first and second sixteen quants
+__device__ __forceinline__ void rein_x8_store_words(uint8_t* __restrict__ rec, float d, const int (&word)[2], unsigned half, unsigned j, unsigned q)
+{
+    if (q == 0u) reinterpret_cast<float*>(rec + REIN_X8_X)[half * 32u + j] = d;
+#pragma unroll
+    for (unsigned h = 0; h < 2; h++) *reinterpret_cast<int*>(rec + half * 1024u + (32u * h + j) * 16u + 4u * q) = word[h];
+}
+__device__ __forceinline__ void rein_x8_store_block(uint8_t* __restrict__ rec, const XhBlock& b, unsigned half, unsigned j, unsigned q)
+{
+    const int word[2] = {(int)rein_xh_word(b, 0), (int)rein_xh_word(b, 1)};
+    rein_x8_store_words(rec, b.d, word, half, j, q);
+}
+
 // x -> image and blocks, as rein_xh_quantize_body.  Bound by memory: 4 bytes in, 2.4 out per value.
 __device__ __forceinline__ void rein_x8_quantize_body(const float* __restrict__ x, uint8_t* __restrict__ img, BlockQ8* __restrict__ xq, unsigned in_dim,
                                                       unsigned p_rows)
@@ -36,13 +49,7 @@ __device__ __forceinline__ void rein_x8_quantize_body(const float* __restrict__ 
     const unsigned n_tt = (p_rows + 31u) / 32u;
     XhBlock b;
     rein_xh_quantize_block(b, x, xq, in_dim, p_rows, w.tok, w.sb, w.q);
-    uint8_t* rec = img + ((size_t)(w.sb >> 1) * n_tt + (w.tok >> 5)) * REIN_X8_REC;
-    if (w.q == 0u) reinterpret_cast<float*>(rec + REIN_X8_X)[(w.sb & 1u) * 32u + w.j] = b.d;
-#pragma unroll
-    for (int h = 0; h < 2; h++) {
-        const int* q = b.q + 4 * h;
-        *reinterpret_cast<uint32_t*>(rec + (w.sb & 1u) * 1024u + (32u * h + w.j) * 16u + 4u * w.q) = (q[0] & 0xFF) | (q[1] & 0xFF) << 8 | (q[2] & 0xFF) << 16 | (uint32_t)q[3] << 24;
-    }
+    rein_x8_store_block(img + ((size_t)(w.sb >> 1) * n_tt + (w.tok >> 5)) * REIN_X8_REC, b, w.sb & 1u, w.j, w.q);
 }
 
 // LDS of one workgroup:
@@ -69,13 +76,13 @@ __device__ __forceinline__ void rein_x8_step(float (&acc)[16], const rein_v16i& 
         __builtin_amdgcn_sched_barrier(0);                       \
     } while (0)
 
-// Superblocks [c0, c1) of rows 128 rb .. and the NT token tiles from `tile` on, into acc.  One barrier per step of four
+// Superblocks [c0, c1) of the wavefront's 32 rows from row_base on and the NT token tiles from `tile` on, into acc.  One barrier per step of four
 // sub-blocks: at its top everything that the step reads has landed (issued a whole step earlier: 4 NT matrix instructions of dots and
 // NT of scales per wavefront), behind it the next step's transfers go out.  Padded rows of the slab (a power of two of sub-blocks)
 // leave a row's scales at two-byte alignment: then they come by 16-bit words.
 template <int FMT, int NT>
 __device__ __forceinline__ void rein_x8_acc(const uint8_t* __restrict__ w, const uint8_t* __restrict__ img, unsigned in_dim, unsigned out_dim,
-                                            unsigned n_tt, unsigned rb, unsigned tile, unsigned c0, unsigned c1, unsigned char* const raw, float (&acc)[NT][16])
+                                            unsigned n_tt, unsigned row_base, unsigned tile, unsigned c0, unsigned c1, unsigned char* const raw, float (&acc)[NT][16])
 {
     using L = X8Lds<FMT>;
     using C = MmqChunk<FMT>;
@@ -84,7 +91,7 @@ __device__ __forceinline__ void rein_x8_acc(const uint8_t* __restrict__ w, const
     const unsigned n_sub = in_dim >> 5;
     const Fmt<FMT> fmt(w, n_sub, out_dim);
     // rows past the matrix read its last one; offsets from the wavefront's first row
-    const unsigned row_base = rb * 128u + wave * 32u, first = min(row_base, out_dim - 1u);
+    const unsigned first = min(row_base, out_dim - 1u);
     auto row_at = [&](unsigned n) { return min(row_base + n, out_dim - 1u) - first; };
     const bool padded = (fmt.nsp & 1u) != 0u;
     unsigned w_off[2], sc_off[4];
@@ -217,8 +224,8 @@ template <int FMT> struct X8Tile {
     static constexpr unsigned kMost = 4, kLeast = 1, kSlots = 512;
     template <int NT>
     static __device__ __forceinline__ void run(const uint8_t* __restrict__ w, const uint8_t* __restrict__ img, unsigned in_dim, unsigned out_dim, unsigned n_tt,
-                                               unsigned rb, unsigned tile, unsigned c0, unsigned c1, unsigned char* const raw, float (&acc)[NT][16])
+                                               unsigned row_base, unsigned tile, unsigned c0, unsigned c1, unsigned char* const raw, float (&acc)[NT][16])
     {
-        rein_x8_acc<FMT, NT>(w, img, in_dim, out_dim, n_tt, rb, tile, c0, c1, raw, acc);
+        rein_x8_acc<FMT, NT>(w, img, in_dim, out_dim, n_tt, row_base, tile, c0, c1, raw, acc);
     }
 };

@@ -65,6 +65,23 @@ def test_against_the_oracle(fmt, rows, in_dim, out_dim, split):
     assert_close_f32(got / scale, want / scale, what=f"fmt {fmt}")
 
 
+@pytest.mark.parametrize("fmt", [rein.Q4_K, rein.Q5_K, rein.Q6_K])
+@pytest.mark.parametrize("rows, in_dim, out_dim, split", [
+    (9, 256, 1, None),           # scales come word by word: fewer than sixteen scale words behind them
+    (40, 256, 15, None),
+    (33, 256, 16, None),         # and by sixteen bytes, up to the last scale word
+    (64, 1280, 3, 2),
+    (20, 1024, 129, None),       # rows of the slab padded to an odd number of sub-blocks: odd rows start between two dwords
+    (45, 2048, 257, 3),          # ranges of an odd and an even number of superblocks
+    (64, 2304, 100, 4),
+    (96, 768, 130, 1),
+])
+def test_groups_of_one_and_two_tiles(fmt, rows, in_dim, out_dim, split):
+    packed = weights(fmt, in_dim, out_dim, rows)
+    x = np.random.default_rng(out_dim).standard_normal((rows, in_dim)).astype(np.float32)
+    assert_close_f32(matmul(fmt, packed, x, out_dim, 3, split), orc.matvec_q8(fmt, packed, in_dim, out_dim, orc.quantize_q8(x), rows), what=f"fmt {fmt}")
+
+
 @pytest.mark.parametrize("fmt", [rein.Q4_K, rein.Q6_K])
 @pytest.mark.parametrize("rows, in_dim, skip", [(33, 256, 0), (129, 1280, 0), (77, 768, 1)])          # skip: x not 16-byte aligned
 def test_the_scratch_holds_the_quantized_rows(fmt, rows, in_dim, skip):
