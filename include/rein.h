@@ -110,10 +110,11 @@ int rein_is_loaded(void);
  * REIN_MMQ16 (1: the fp16 formulation where the code object holds it), REIN_MMQXH (0 / 2 / 3: the GEMMs of
  * rein_matmul_ws on 32 x 128 wavefront tiles, exact-dot fp16 and int8, off / wherever they can run / the K-quants' in groups of one and two token tiles), REIN_MMQXH_SPLIT,
  * REIN_MMQXH_GROUPS (their ranges per unit, their groups of token tiles), REIN_TOPK_WAVE,
- * REIN_MOE_SORT_SPLIT, REIN_MOE_CHAIN, REIN_MOE_FUSED, REIN_MOE_FEW, REIN_MOE_GU_ROWS, REIN_MOE_DC_ROWS
+ * REIN_MOE_SORT_SPLIT, REIN_MOE_CHAIN, REIN_MOE_FUSED, REIN_MOE_FEW, REIN_MOE_WIDE, REIN_MOE_GU_ROWS, REIN_MOE_DC_ROWS
  * (MoE glue: 0 = the workgroup router, 1 = the four-launch sort, 0 = no decode chain for few
  * tokens, 0 = unfused gate/up, 0 never / 1 wherever the shape allows the launches that read every touched
- * expert once, rows per workgroup of the two decode launches).
+ * expert once, 0 never / 2 / 4 wherever the shape allows the wide tiles in groups of two / four, rows per
+ * workgroup of the two decode launches).
  * Unknown name: REIN_E_NOT_FOUND; a value that is not an unsigned 32-bit decimal:
  * REIN_E_BAD_SHAPE. */
 int rein_set_option(const char *name, const char *value);   /* value NULL or "": unset */
@@ -564,6 +565,8 @@ size_t rein_moe_workspace_bytes(const rein_moe_shape *shape);
  * From about 0.8 to 5.5 entries per expert a third form reads every expert that the router touched once
  * for all of its tokens (four launches: router + quantizer, gate + up, down, combine); it needs hidden and
  * expert_ff to be multiples of 64.
+ * From about 30 entries per expert (18 of Q8_0) the pipeline's GEMMs run on wider tiles (hidden and expert_ff
+ * multiples of 256, expert_ff 512 and more).
  * The forms add the terms inside an expert's row in different orders: the fp32 bits of a token's output row
  * therefore depend on how many tokens share the call, within the path's 1e-3 / 1e-4 tolerance of any
  * order.  The option REIN_MOE_CHAIN = 0 (with REIN_MOE_FEW unset) keeps every call on the pipeline. */

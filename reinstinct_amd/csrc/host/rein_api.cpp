@@ -192,8 +192,8 @@ int check_ptr(const char* who, const void* p, size_t align, const char* what)
 // rein_set_option changes an entry, so the launch an entry point chooses depends on its arguments
 // and on this table alone.  Entries are single atomic words: setting one while another thread
 // launches is safe, the launch sees the old or the new value.
-enum Opt : int { O_MV_ROWS, O_MV_WPB, O_MV_LOADS, O_MV_LDS, O_QUAD_LDS, O_QUAD_SLICES, O_QUAD_DEPTH, O_QUAD_WIDE32, O_SKINNY_KS, O_SKINNY_FROM, O_QUAD_FROM, O_GROUPED_STRIDED, O_MMQ_TM, O_MMQ_N64, O_MMQ6, O_MMQ6_N4, O_MMQ6_N2, O_MMQ6_SK_GRID, O_MMQ6_SK_SPLIT, O_MMQ6_SK, O_MMQ6_FROM, O_MMQ_SK, O_MMQ_SK_GRID, O_MMQ_SK_SPLIT, O_MMQ_SK_TM, O_MMQ16, O_MMQXH, O_MMQXH_SPLIT, O_MMQXH_GROUPS, O_TOPK_WAVE, O_MOE_SORT_SPLIT, O_MOE_GU_ROWS, O_MOE_DC_ROWS, O_MOE_CHAIN, O_MOE_FUSED, O_MOE_FEW, O_COUNT };
-const char* const kOptNames[O_COUNT] = {"REIN_MV_ROWS", "REIN_MV_WPB", "REIN_MV_LOADS", "REIN_MV_LDS", "REIN_QUAD_LDS", "REIN_QUAD_SLICES", "REIN_QUAD_DEPTH", "REIN_QUAD_WIDE32", "REIN_SKINNY_KS", "REIN_SKINNY_FROM", "REIN_QUAD_FROM", "REIN_GROUPED_STRIDED", "REIN_MMQ_TM", "REIN_MMQ_N64", "REIN_MMQ6", "REIN_MMQ6_N4", "REIN_MMQ6_N2", "REIN_MMQ6_SK_GRID", "REIN_MMQ6_SK_SPLIT", "REIN_MMQ6_SK", "REIN_MMQ6_FROM", "REIN_MMQ_SK", "REIN_MMQ_SK_GRID", "REIN_MMQ_SK_SPLIT", "REIN_MMQ_SK_TM", "REIN_MMQ16", "REIN_MMQXH", "REIN_MMQXH_SPLIT", "REIN_MMQXH_GROUPS", "REIN_TOPK_WAVE", "REIN_MOE_SORT_SPLIT", "REIN_MOE_GU_ROWS", "REIN_MOE_DC_ROWS", "REIN_MOE_CHAIN", "REIN_MOE_FUSED", "REIN_MOE_FEW"};
+enum Opt : int { O_MV_ROWS, O_MV_WPB, O_MV_LOADS, O_MV_LDS, O_QUAD_LDS, O_QUAD_SLICES, O_QUAD_DEPTH, O_QUAD_WIDE32, O_SKINNY_KS, O_SKINNY_FROM, O_QUAD_FROM, O_GROUPED_STRIDED, O_MMQ_TM, O_MMQ_N64, O_MMQ6, O_MMQ6_N4, O_MMQ6_N2, O_MMQ6_SK_GRID, O_MMQ6_SK_SPLIT, O_MMQ6_SK, O_MMQ6_FROM, O_MMQ_SK, O_MMQ_SK_GRID, O_MMQ_SK_SPLIT, O_MMQ_SK_TM, O_MMQ16, O_MMQXH, O_MMQXH_SPLIT, O_MMQXH_GROUPS, O_TOPK_WAVE, O_MOE_SORT_SPLIT, O_MOE_GU_ROWS, O_MOE_DC_ROWS, O_MOE_CHAIN, O_MOE_FUSED, O_MOE_FEW, O_MOE_WIDE, O_COUNT };
+const char* const kOptNames[O_COUNT] = {"REIN_MV_ROWS", "REIN_MV_WPB", "REIN_MV_LOADS", "REIN_MV_LDS", "REIN_QUAD_LDS", "REIN_QUAD_SLICES", "REIN_QUAD_DEPTH", "REIN_QUAD_WIDE32", "REIN_SKINNY_KS", "REIN_SKINNY_FROM", "REIN_QUAD_FROM", "REIN_GROUPED_STRIDED", "REIN_MMQ_TM", "REIN_MMQ_N64", "REIN_MMQ6", "REIN_MMQ6_N4", "REIN_MMQ6_N2", "REIN_MMQ6_SK_GRID", "REIN_MMQ6_SK_SPLIT", "REIN_MMQ6_SK", "REIN_MMQ6_FROM", "REIN_MMQ_SK", "REIN_MMQ_SK_GRID", "REIN_MMQ_SK_SPLIT", "REIN_MMQ_SK_TM", "REIN_MMQ16", "REIN_MMQXH", "REIN_MMQXH_SPLIT", "REIN_MMQXH_GROUPS", "REIN_TOPK_WAVE", "REIN_MOE_SORT_SPLIT", "REIN_MOE_GU_ROWS", "REIN_MOE_DC_ROWS", "REIN_MOE_CHAIN", "REIN_MOE_FUSED", "REIN_MOE_FEW", "REIN_MOE_WIDE"};
 constexpr uint64_t kOptSet = 1ull << 63;
 std::atomic<uint64_t> g_opts[O_COUNT];          // zero = unset
 std::once_flag g_opts_env_once;
@@ -2330,9 +2330,11 @@ int rein_moe_sort(const int32_t* ids, unsigned n_entries, unsigned n_expert, uns
         if (int rc = check_ptr("rein_moe_sort", p, 4, "buffer")) return rc;
     if (moe_sort_in_one_block(n_entries, n_expert)) {
         // cursor is left as it is: the rank counters of the one-workgroup sort live in LDS
-        int32_t* inv = nullptr;
-        void* a[] = {(void*)&ids, (void*)&count, (void*)&expert_off, (void*)&tile_off, (void*)&perm, (void*)&inv,
-                     (void*)&n_entries, (void*)&n_expert, (void*)&bn};
+        int32_t *inv = nullptr, *place = nullptr;
+        void* units = nullptr;
+        unsigned per_xcd = 0;
+        void* a[] = {(void*)&ids, (void*)&count, (void*)&expert_off, (void*)&tile_off, (void*)&perm, (void*)&inv, (void*)&n_entries,
+                     (void*)&n_expert, (void*)&bn, (void*)&place, (void*)&units, (void*)&per_xcd, (void*)&units, (void*)&per_xcd};
         return launch("rein_moe_sort_one_block", 1, 1, 1, 1024, 0, s, a);
     }
     const unsigned ge = (n_expert + 255) / 256, gn = (n_entries + 255) / 256;
@@ -2605,9 +2607,28 @@ int rein_moe_combine(const float* experts, const int32_t* ids, const float* weig
 // Workspace carve-up for rein_moe_ffn (all offsets 256-byte aligned).
 namespace {
 struct MoeWs {
-    size_t ids, weights, count, cursor, perm, inv, eoff, toff, xq_in, g_in, e_gate, e_up, xq_exp, g_out, total;
+    size_t ids, weights, count, cursor, perm, inv, eoff, toff, xq_in, g_in, e_gate, e_up, xq_exp, g_out, img_in, img_exp, place, units2, units4, total;
 };
 size_t up256(size_t v) { return (v + 255) & ~(size_t)255; }
+// the pipeline on the wide tiles (kernels/moe_wide.h): contractions of whole superblocks
+bool moe_wide_fmt(int fmt) { return wide_k_quant(fmt) || fmt == REIN_TYPE_Q8_0; }
+bool moe_wide_fits(const rein_moe_shape& sh)
+{
+    return moe_wide_fmt(sh.gate_up_fmt) && moe_wide_fmt(sh.down_fmt) && sh.hidden % 256 == 0 && sh.expert_ff % 256 == 0 &&
+           (unsigned long long)sh.n_tok * sh.n_used <= 0x3FFFFFFull && sh.n_expert <= 65535;
+}
+// no routing has more tiles of 32 entries of one expert
+size_t moe_most_tiles(const rein_moe_shape& sh)
+{
+    const size_t ne = (size_t)sh.n_tok * sh.n_used;
+    return (ne + 31 * std::min<size_t>(ne, sh.n_expert)) / 32;
+}
+// groups of `most` tiles on an XCD at most, with one to spare for either kind (rein_moe_list_units)
+unsigned moe_units_per_xcd(const rein_moe_shape& sh, unsigned most)
+{
+    const size_t ne = (size_t)sh.n_tok * sh.n_used, bn = 32 * most;
+    return (unsigned)(((ne + (bn - 1) * std::min<size_t>(ne, sh.n_expert)) / bn + 7) / 8 + 2);
+}
 MoeWs moe_ws(const rein_moe_shape& sh)
 {
     const size_t ne = (size_t)sh.n_tok * sh.n_used;
@@ -2623,11 +2644,28 @@ MoeWs moe_ws(const rein_moe_shape& sh)
     w.eoff    = take(((size_t)sh.n_expert + 1) * 4);
     w.toff    = take(((size_t)sh.n_expert + 1) * 4);
     w.xq_in   = take((size_t)sh.n_tok * (sh.hidden / 32) * 40);
+    const size_t shared = o;
     w.g_in    = take(ne * (sh.hidden / 32) * 40);
     w.e_gate  = take(ne * sh.expert_ff * 4);
     w.e_up    = take(ne * sh.expert_ff * 4);
     w.xq_exp  = take(ne * (sh.expert_ff / 32) * 40);
+    w.img_in = w.img_exp = w.place = w.units2 = w.units4 = shared;
+    size_t end = o;
+    if (moe_wide_fits(sh)) {
+        // instead of the four above: the wide pipeline's lists and its two images.  That of the tokens lies last and may reach into the rows of the
+        // down projection, whose launch is behind the one that reads it.
+        const size_t tiles = moe_most_tiles(sh);
+        o = shared;
+        w.place   = take(ne * 4);
+        w.units2  = take((size_t)8 * moe_units_per_xcd(sh, 2) * 16);
+        w.units4  = take((size_t)8 * moe_units_per_xcd(sh, 4) * 16);
+        w.img_exp = take(wide_image_bytes(sh.down_fmt, sh.expert_ff, (unsigned)(tiles * 32)));
+        w.img_in  = o;
+        end = std::max(end, o);
+        o = end;
+    }
     w.g_out   = take(ne * sh.hidden * 4);
+    if (moe_wide_fits(sh)) o = std::max(o, up256(w.img_in + wide_image_bytes(sh.gate_up_fmt, sh.hidden, (unsigned)(moe_most_tiles(sh) * 32))));
     w.total   = o;
     return w;
 }
@@ -2687,6 +2725,32 @@ bool moe_few_pays(const rein_moe_shape& sh)
     const double touched = sh.n_expert * (1.0 - std::pow(1.0 - (double)sh.n_used / sh.n_expert, (double)sh.n_tok));
     return (entries - touched) * bytes + entries * 0.2e6 >= 30e6 + (sh.gate_up_fmt == REIN_TYPE_Q8_0 ? 0.45 : 0.3) * touched * bytes;
 }
+}  // namespace
+
+namespace {
+// Tiles of a group of the pipeline on the wide tiles (kernels/moe_wide.h), 0: the pipeline of 32-token tiles.  From 4543 cells -- 32 to 256 experts, hidden
+// 1024-4096, ff 256-1536, top 2-8, 5 to 256 entries per expert, five pairs of formats, the weights of several layers in turn -- the time of
+// the 32-token tiles over that of groups of two / of four, geometric means by entries per expert:
+//   up to 6 0.95 / 0.93, 17 0.98 / 0.95, 30 1.03 / 0.99, 36 1.07 / 1.02, 60 1.12 / 1.06, 110 1.13 / 1.10, 220 1.21 / 1.19, more 1.23 / 1.22
+// A tile that fills its 32 tokens needs the unpack shared with a second one; Q8_0, whose unpack is nothing, gains from 18 entries on.  Not
+// below 320 units of the gate + up launch (128 of them, half of the CUs: 0.82-0.95) nor with one superblock to the down projection (ff 256:
+// 0.99 in the mean, 0.82 at worst); up to 512 and with two superblocks from 36 entries, with a Q5_K down, which has both extra bits and minimums, from
+// six more.  Where it is taken it is ahead by 1.18 in the mean of 1098 cells and nowhere behind by more than 1 %: 128 experts top-8, 2048 x 768
+// Q4_K / Q6_K, 512 tokens 228 / 191 us, 640 268 / 214; 256 top-8, 2048 x 1024, 1000 tokens 508 / 461; 64 top-4 of Q8_0, 300 tokens 122 / 115.
+// Groups of four are never ahead by enough to choose them: 0.91-1.03 of groups of two.  An option that pins a form of the other pipeline keeps it.
+unsigned moe_wide_most(const rein_moe_shape& sh)
+{
+    if (!moe_wide_fits(sh)) return 0;
+    if (opt_is_set(O_MOE_WIDE)) return opt_u(O_MOE_WIDE, 0) == 0 ? 0 : opt_u(O_MOE_WIDE, 0) == 2 ? 2 : 4;
+    if (opt_is_set(O_MOE_FUSED) || opt_is_set(O_GROUPED_STRIDED)) return 0;
+    const unsigned long long entries = (unsigned long long)sh.n_tok * sh.n_used, experts = sh.n_expert, blocks = experts * (sh.expert_ff / 64);
+    const unsigned long long groups = std::max(1ull, (entries + 64 * experts - 1) / (64 * experts));
+    if (sh.expert_ff < 512 || blocks * groups < 320) return 0;
+    if (sh.gate_up_fmt == REIN_TYPE_Q8_0) return entries >= 18 * experts ? 2 : 0;
+    const unsigned least = (sh.expert_ff > 512 && blocks >= 512 ? 30u : 36u) + (sh.down_fmt == REIN_TYPE_Q5_K ? 6u : 0u);
+    return entries >= least * experts ? 2 : 0;
+}
+const WideKind& moe_wide_kind(int fmt, unsigned most) { return fmt == REIN_TYPE_Q8_0 ? kWideInt8 : most == 2 ? kWideFew : wide_exact(fmt); }
 }  // namespace
 
 size_t rein_moe_workspace_bytes(const rein_moe_shape* sh)
@@ -2799,15 +2863,28 @@ int rein_moe_ffn(const rein_moe_shape* shp, const float* x, const float* logits,
         return rein_moe_down_combine(sh.down_fmt, down_exps, ids, weights, down_exps_s, base + w.xq_exp, out, sh.expert_ff, sh.hidden,
                                      (unsigned)bpe_dn, sh.n_used * ns_f, ns_f, sh.n_used, sh.n_tok, s);
     }
-    if (int rc = rein_moe_topk(logits, sh.n_tok, sh.n_expert, sh.n_used, ids, weights, s)) return rc;
+    const unsigned most = moe_wide_most(sh);
+    if (most && wave) {
+        if (int rc = route_quantize()) return rc;
+    } else {
+        if (int rc = rein_moe_topk(logits, sh.n_tok, sh.n_expert, sh.n_used, ids, weights, s)) return rc;
+        if (most)
+            if (int rc = rein_quantize_q8(x, base + w.xq_in, sh.hidden, sh.n_tok, s)) return rc;
+    }
     // counting sort by expert (moe_expert_sort.hip), with the inverse permutation kept so
     // that the combine can read the sorted expert outputs in place
     int32_t* count = (int32_t*)(base + w.count);
     int32_t* inv = (int32_t*)(base + w.inv);
     const unsigned bn = rein_moe_gemm_bn();
+    // of the wide pipeline: the place of an entry in the tiles, the groups of two and of four tiles that its two launches go by
+    const unsigned most_g = most ? moe_wide_kind(sh.gate_up_fmt, most).most : 0, most_d = most ? moe_wide_kind(sh.down_fmt, most).most : 0;
+    const unsigned per_xcd2 = moe_units_per_xcd(sh, 2), per_xcd4 = moe_units_per_xcd(sh, 4);
+    int32_t* const place = most ? (int32_t*)(base + w.place) : nullptr;
+    char* const units2 = most_g == 2 || most_d == 2 ? base + w.units2 : nullptr;
+    char* const units4 = most_g == 4 || most_d == 4 ? base + w.units4 : nullptr;
     if (moe_sort_in_one_block(ne, sh.n_expert)) {
         void* a[] = {(void*)&ids, (void*)&count, (void*)&eoff, (void*)&toff, (void*)&perm, (void*)&inv, (void*)&ne,
-                     (void*)&sh.n_expert, (void*)&bn};
+                     (void*)&sh.n_expert, (void*)&bn, (void*)&place, (void*)&units2, (void*)&per_xcd2, (void*)&units4, (void*)&per_xcd4};
         if (int rc = launch("rein_moe_sort_one_block", 1, 1, 1, 1024, 0, s, a)) return rc;
     } else {
         int32_t* cursor = (int32_t*)(base + w.cursor);
@@ -2819,8 +2896,48 @@ int rein_moe_ffn(const rein_moe_shape* shp, const float* x, const float* logits,
         if (int rc = launch("moe_sort_histogram", gn, 1, 1, 256, 0, s, a1)) return rc;
         void* a2[] = {(void*)&count, (void*)&eoff, (void*)&toff, (void*)&sh.n_expert, (void*)&bn};
         if (int rc = launch("moe_sort_scan", 1, 1, 1, 64, 0, s, a2)) return rc;
-        void* a3[] = {(void*)&ids, (void*)&eoff, (void*)&cursor, (void*)&perm, (void*)&inv, (void*)&ne, (void*)&sh.n_expert};
+        void* a3[] = {(void*)&ids, (void*)&eoff, (void*)&cursor, (void*)&perm, (void*)&inv, (void*)&ne, (void*)&sh.n_expert,
+                      (void*)&toff, (void*)&place};
         if (int rc = launch("rein_moe_sort_scatter_inv", gn, 1, 1, 256, 0, s, a3)) return rc;
+        if (most) {
+            void* a4[] = {(void*)&eoff, (void*)&toff, (void*)&sh.n_expert, (void*)&units2, (void*)&per_xcd2, (void*)&units4, (void*)&per_xcd4};
+            if (int rc = launch("rein_moe_units", 1, 1, 1, 128, 0, s, a4)) return rc;
+        }
+    }
+    // scatter + weighted combine in one pass over the sorted rows
+    const auto combine = [&]() -> int {
+        const float* sorted = (const float*)(base + w.g_out);
+        void* a[] = {(void*)&sorted, (void*)&inv, (void*)&ids, (void*)&weights, (void*)&down_exps_s, (void*)&out,
+                     (void*)&sh.hidden, (void*)&sh.n_used};
+        // four columns per thread where the rows allow 128-bit accesses (the same bits)
+        if (sh.hidden % 4 == 0 && ((uintptr_t)out & 15) == 0 && ((uintptr_t)sorted & 15) == 0)
+            return launch("rein_moe_combine_sorted4_f32", (sh.hidden / 4 + 127) / 128, sh.n_tok, 1, 128, 0, s, a);
+        return launch("rein_moe_combine_sorted_f32", (sh.hidden + 255) / 256, sh.n_tok, 1, 256, 0, s, a);
+    };
+    if (most) {
+        const WideKind &kind = moe_wide_kind(sh.gate_up_fmt, most), &kind_d = moe_wide_kind(sh.down_fmt, most);
+        const unsigned n_tt = (unsigned)moe_most_tiles(sh), bpe_g = (unsigned)bpe_gu, bpe_d = (unsigned)bpe_dn, with_min = wide_has_min(sh.gate_up_fmt);
+        const unsigned out_kind = sh.down_fmt == REIN_TYPE_Q8_0 ? 0u : wide_has_min(sh.down_fmt) ? 2u : 1u;          // XgOut
+        const unsigned per_g = most_g == 2 ? per_xcd2 : per_xcd4, per_d = most_d == 2 ? per_xcd2 : per_xcd4;
+        const char *const units_g = most_g == 2 ? units2 : units4, *const units_d = most_d == 2 ? units2 : units4;
+        const unsigned long long grid = 8ull * per_g * (sh.expert_ff / 64), grid_d = 8ull * per_d * ((sh.hidden + 127) / 128);
+        const char* const xq_in = base + w.xq_in;
+        char* const img = base + w.img_in;
+        char* const img_exp = base + w.img_exp;
+        float* const rows = (float*)(base + w.g_out);
+        const int32_t* const n_sorted = eoff + sh.n_expert;
+        if (grid <= 0x7FFFFFFFull && grid_d <= 0x7FFFFFFFull) {
+            void* a[] = {(void*)&xq_in, (void*)&perm, (void*)&place, (void*)&n_sorted, (void*)&img, (void*)&sh.hidden, (void*)&sh.n_used, (void*)&ne,
+                         (void*)&n_tt, (void*)&with_min};
+            if (int rc = launch(KName("rein_moe_gather_", sh.gate_up_fmt == REIN_TYPE_Q8_0 ? "x8" : "xh"), (ne + 7) / 8, (sh.hidden / 256 + 1) / 2, 1, 256, 0, s, a)) return rc;
+            void* b[] = {(void*)&gate_exps, (void*)&up_exps, (void*)&bpe_g, (void*)&units_g, (void*)&per_g, (void*)&img, (void*)&img_exp,
+                         (void*)&sh.hidden, (void*)&sh.expert_ff, (void*)&n_tt, (void*)&out_kind};
+            if (int rc = launch(KName("rein_mmq_", fmt_tag(sh.gate_up_fmt), "_xg", most_g, "_swiglu"), (unsigned)grid, 1, 1, 256, wide_lds_bytes(kind, sh.gate_up_fmt), s, b)) return rc;
+            void* c[] = {(void*)&down_exps, (void*)&bpe_d, (void*)&units_d, (void*)&per_d, (void*)&img_exp, (void*)&rows,
+                         (void*)&sh.expert_ff, (void*)&sh.hidden, (void*)&n_tt};
+            if (int rc = launch(KName("rein_mmq_", fmt_tag(sh.down_fmt), "_xg", most_d, "_rows"), (unsigned)grid_d, 1, 1, 256, wide_lds_bytes(kind_d, sh.down_fmt), s, c)) return rc;
+            return combine();
+        }
     }
     // the expert-sorted BlockQ8 rows straight from x (quantize_q8 + moe_gather_xq in one launch)
     if (int rc = rein_moe_quantize_scatter(x, inv, base + w.g_in, sh.hidden, sh.n_used, sh.n_tok, s)) return rc;
@@ -2845,17 +2962,7 @@ int rein_moe_ffn(const rein_moe_shape* shp, const float* x, const float* logits,
     }
     if (int rc = rein_moe_grouped_gemm(sh.down_fmt, down_exps, (unsigned)bpe_dn, eoff, toff, sh.n_expert,
                                        base + w.xq_exp, (float*)(base + w.g_out), sh.expert_ff, sh.hidden, ne, s)) return rc;
-    // scatter + weighted combine in one pass over the sorted rows
-    {
-        const float* sorted = (const float*)(base + w.g_out);
-        const int32_t* inv = (const int32_t*)(base + w.inv);
-        void* a[] = {(void*)&sorted, (void*)&inv, (void*)&ids, (void*)&weights, (void*)&down_exps_s, (void*)&out,
-                     (void*)&sh.hidden, (void*)&sh.n_used};
-        // four columns per thread where the rows allow 128-bit accesses (the same bits)
-        if (sh.hidden % 4 == 0 && ((uintptr_t)out & 15) == 0 && ((uintptr_t)sorted & 15) == 0)
-            return launch("rein_moe_combine_sorted4_f32", (sh.hidden / 4 + 127) / 128, sh.n_tok, 1, 128, 0, s, a);
-        return launch("rein_moe_combine_sorted_f32", (sh.hidden + 255) / 256, sh.n_tok, 1, 256, 0, s, a);
-    }
+    return combine();
 }
 
 }  // extern "C"
