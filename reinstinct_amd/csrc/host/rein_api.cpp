@@ -2728,29 +2728,29 @@ bool moe_few_pays(const rein_moe_shape& sh)
 }  // namespace
 
 namespace {
-// Tiles of a group of the pipeline on the wide tiles (kernels/moe_wide.h), 0: the pipeline of 32-token tiles.  From 4543 cells -- 32 to 256 experts, hidden
-// 1024-4096, ff 256-1536, top 2-8, 5 to 256 entries per expert, five pairs of formats, the weights of several layers in turn -- the time of
-// the 32-token tiles over that of groups of two / of four, geometric means by entries per expert:
-//   up to 6 0.95 / 0.93, 17 0.98 / 0.95, 30 1.03 / 0.99, 36 1.07 / 1.02, 60 1.12 / 1.06, 110 1.13 / 1.10, 220 1.21 / 1.19, more 1.23 / 1.22
+// The pipeline on the wide tiles (kernels/moe_wide.h), K-quants in groups of two 32-token tiles, Q8_0 of four, or that of single 32-token tiles.  From
+// 4543 cells -- 32 to 256 experts, hidden 1024-4096, ff 256-1536, top 2-8, 5 to 256 entries per expert, five pairs of formats, the weights of several
+// layers in turn -- the time of the single tiles over that of the wide ones, geometric means by entries per expert:
+//   up to 6 0.95, 17 0.98, 30 1.03, 36 1.07, 60 1.12, 110 1.13, 220 1.21, more 1.23
 // A tile that fills its 32 tokens needs the unpack shared with a second one; Q8_0, whose unpack is nothing, gains from 18 entries on.  Not
 // below 320 units of the gate + up launch (128 of them, half of the CUs: 0.82-0.95) nor with one superblock to the down projection (ff 256:
 // 0.99 in the mean, 0.82 at worst); up to 512 and with two superblocks from 36 entries, with a Q5_K down, which has both extra bits and minimums, from
 // six more.  Where it is taken it is ahead by 1.18 in the mean of 1098 cells and nowhere behind by more than 1 %: 128 experts top-8, 2048 x 768
 // Q4_K / Q6_K, 512 tokens 228 / 191 us, 640 268 / 214; 256 top-8, 2048 x 1024, 1000 tokens 508 / 461; 64 top-4 of Q8_0, 300 tokens 122 / 115.
-// Groups of four are never ahead by enough to choose them: 0.91-1.03 of groups of two.  An option that pins a form of the other pipeline keeps it.
-unsigned moe_wide_most(const rein_moe_shape& sh)
+// K-quants in groups of four were 0.91-1.03 of groups of two, never ahead by enough to have them.  An option that pins a form of the other pipeline keeps it.
+bool moe_wide_pays(const rein_moe_shape& sh)
 {
-    if (!moe_wide_fits(sh)) return 0;
-    if (opt_is_set(O_MOE_WIDE)) return opt_u(O_MOE_WIDE, 0) == 0 ? 0 : opt_u(O_MOE_WIDE, 0) == 2 ? 2 : 4;
-    if (opt_is_set(O_MOE_FUSED) || opt_is_set(O_GROUPED_STRIDED)) return 0;
+    if (!moe_wide_fits(sh)) return false;
+    if (opt_is_set(O_MOE_WIDE)) return opt_u(O_MOE_WIDE, 0) != 0;
+    if (opt_is_set(O_MOE_FUSED) || opt_is_set(O_GROUPED_STRIDED)) return false;
     const unsigned long long entries = (unsigned long long)sh.n_tok * sh.n_used, experts = sh.n_expert, blocks = experts * (sh.expert_ff / 64);
     const unsigned long long groups = std::max(1ull, (entries + 64 * experts - 1) / (64 * experts));
-    if (sh.expert_ff < 512 || blocks * groups < 320) return 0;
-    if (sh.gate_up_fmt == REIN_TYPE_Q8_0) return entries >= 18 * experts ? 2 : 0;
+    if (sh.expert_ff < 512 || blocks * groups < 320) return false;
+    if (sh.gate_up_fmt == REIN_TYPE_Q8_0) return entries >= 18 * experts;
     const unsigned least = (sh.expert_ff > 512 && blocks >= 512 ? 30u : 36u) + (sh.down_fmt == REIN_TYPE_Q5_K ? 6u : 0u);
-    return entries >= least * experts ? 2 : 0;
+    return entries >= least * experts;
 }
-const WideKind& moe_wide_kind(int fmt, unsigned most) { return fmt == REIN_TYPE_Q8_0 ? kWideInt8 : most == 2 ? kWideFew : wide_exact(fmt); }
+const WideKind& moe_wide_kind(int fmt) { return fmt == REIN_TYPE_Q8_0 ? kWideInt8 : kWideFew; }
 }  // namespace
 
 size_t rein_moe_workspace_bytes(const rein_moe_shape* sh)
@@ -2863,12 +2863,12 @@ int rein_moe_ffn(const rein_moe_shape* shp, const float* x, const float* logits,
         return rein_moe_down_combine(sh.down_fmt, down_exps, ids, weights, down_exps_s, base + w.xq_exp, out, sh.expert_ff, sh.hidden,
                                      (unsigned)bpe_dn, sh.n_used * ns_f, ns_f, sh.n_used, sh.n_tok, s);
     }
-    const unsigned most = moe_wide_most(sh);
-    if (most && wave) {
+    const bool wide = moe_wide_pays(sh);
+    if (wide && wave) {
         if (int rc = route_quantize()) return rc;
     } else {
         if (int rc = rein_moe_topk(logits, sh.n_tok, sh.n_expert, sh.n_used, ids, weights, s)) return rc;
-        if (most)
+        if (wide)
             if (int rc = rein_quantize_q8(x, base + w.xq_in, sh.hidden, sh.n_tok, s)) return rc;
     }
     // counting sort by expert (moe_expert_sort.hip), with the inverse permutation kept so
@@ -2877,9 +2877,10 @@ int rein_moe_ffn(const rein_moe_shape* shp, const float* x, const float* logits,
     int32_t* inv = (int32_t*)(base + w.inv);
     const unsigned bn = rein_moe_gemm_bn();
     // of the wide pipeline: the place of an entry in the tiles, the groups of two and of four tiles that its two launches go by
-    const unsigned most_g = most ? moe_wide_kind(sh.gate_up_fmt, most).most : 0, most_d = most ? moe_wide_kind(sh.down_fmt, most).most : 0;
+    const WideKind &kind = moe_wide_kind(sh.gate_up_fmt), &kind_d = moe_wide_kind(sh.down_fmt);
+    const unsigned most_g = wide ? kind.most : 0, most_d = wide ? kind_d.most : 0;
     const unsigned per_xcd2 = moe_units_per_xcd(sh, 2), per_xcd4 = moe_units_per_xcd(sh, 4);
-    int32_t* const place = most ? (int32_t*)(base + w.place) : nullptr;
+    int32_t* const place = wide ? (int32_t*)(base + w.place) : nullptr;
     char* const units2 = most_g == 2 || most_d == 2 ? base + w.units2 : nullptr;
     char* const units4 = most_g == 4 || most_d == 4 ? base + w.units4 : nullptr;
     if (moe_sort_in_one_block(ne, sh.n_expert)) {
@@ -2899,7 +2900,7 @@ int rein_moe_ffn(const rein_moe_shape* shp, const float* x, const float* logits,
         void* a3[] = {(void*)&ids, (void*)&eoff, (void*)&cursor, (void*)&perm, (void*)&inv, (void*)&ne, (void*)&sh.n_expert,
                       (void*)&toff, (void*)&place};
         if (int rc = launch("rein_moe_sort_scatter_inv", gn, 1, 1, 256, 0, s, a3)) return rc;
-        if (most) {
+        if (wide) {
             void* a4[] = {(void*)&eoff, (void*)&toff, (void*)&sh.n_expert, (void*)&units2, (void*)&per_xcd2, (void*)&units4, (void*)&per_xcd4};
             if (int rc = launch("rein_moe_units", 1, 1, 1, 128, 0, s, a4)) return rc;
         }
@@ -2914,8 +2915,7 @@ int rein_moe_ffn(const rein_moe_shape* shp, const float* x, const float* logits,
             return launch("rein_moe_combine_sorted4_f32", (sh.hidden / 4 + 127) / 128, sh.n_tok, 1, 128, 0, s, a);
         return launch("rein_moe_combine_sorted_f32", (sh.hidden + 255) / 256, sh.n_tok, 1, 256, 0, s, a);
     };
-    if (most) {
-        const WideKind &kind = moe_wide_kind(sh.gate_up_fmt, most), &kind_d = moe_wide_kind(sh.down_fmt, most);
+    if (wide) {
         const unsigned n_tt = (unsigned)moe_most_tiles(sh), bpe_g = (unsigned)bpe_gu, bpe_d = (unsigned)bpe_dn, with_min = wide_has_min(sh.gate_up_fmt);
         const unsigned out_kind = sh.down_fmt == REIN_TYPE_Q8_0 ? 0u : wide_has_min(sh.down_fmt) ? 2u : 1u;          // XgOut
         const unsigned per_g = most_g == 2 ? per_xcd2 : per_xcd4, per_d = most_d == 2 ? per_xcd2 : per_xcd4;

@@ -16,22 +16,18 @@ REIN_DEFINE_XG_GATHER(rein_moe_gather_x8, true)
     extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES))) void rein_mmq_##tag##_swiglu(      \
         const unsigned char* __restrict__ gate, const unsigned char* __restrict__ up, unsigned int bytes_per_expert,            \
         const ReinMoeUnit* __restrict__ units, unsigned int per_xcd, const unsigned char* __restrict__ img,                     \
-        unsigned char* __restrict__ out, unsigned int in_dim, unsigned int out_dim, unsigned int n_tt, unsigned int out_kind)                                                                               \
+        unsigned char* __restrict__ out, unsigned int in_dim, unsigned int out_dim, unsigned int n_tt, unsigned int out_kind)                      \
     {                                                                                                                           \
         rein_xg_swiglu<TILE>(gate, up, bytes_per_expert, units, per_xcd, img, out, in_dim, out_dim, n_tt, out_kind); \
     }                                                                                                                           \
     extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES))) void rein_mmq_##tag##_rows(        \
         const unsigned char* __restrict__ slab, unsigned int bytes_per_expert, const ReinMoeUnit* __restrict__ units,           \
-        unsigned int per_xcd, const unsigned char* __restrict__ img, float* __restrict__ y, unsigned int in_dim, unsigned int out_dim, unsigned int n_tt)                                                           \
+        unsigned int per_xcd, const unsigned char* __restrict__ img, float* __restrict__ y, unsigned int in_dim, unsigned int out_dim, unsigned int n_tt)  \
     {                                                                                                                           \
         rein_xg_rows<TILE>(slab, bytes_per_expert, units, per_xcd, img, y, in_dim, out_dim, n_tt);             \
     }
-typedef XhTile<REIN_Q4_K, 2> XgQ4Few; typedef XhTile<REIN_Q5_K, 2> XgQ5Few; typedef XhTile<REIN_Q6_K, 2> XgQ6Few;
-typedef XhTile<REIN_Q4_K, 4> XgQ4; typedef XhTile<REIN_Q5_K, 4> XgQ5; typedef XhTile<REIN_Q6_K, 4> XgQ6;
-REIN_DEFINE_XG(q4k_xg2, XgQ4Few, 3)
-REIN_DEFINE_XG(q5k_xg2, XgQ5Few, 3)
-REIN_DEFINE_XG(q6k_xg2, XgQ6Few, 3)
-REIN_DEFINE_XG(q4k_xg4, XgQ4, 2)
-REIN_DEFINE_XG(q5k_xg4, XgQ5, 2)
-REIN_DEFINE_XG(q6k_xg4, XgQ6, 2)
+typedef XhTile<REIN_Q4_K, 2> XgQ4; typedef XhTile<REIN_Q5_K, 2> XgQ5; typedef XhTile<REIN_Q6_K, 2> XgQ6;
+REIN_DEFINE_XG(q4k_xg2, XgQ4, 3)
+REIN_DEFINE_XG(q5k_xg2, XgQ5, 3)
+REIN_DEFINE_XG(q6k_xg2, XgQ6, 3)
 REIN_DEFINE_XG(q8_0_xg4, X8Tile<REIN_Q8_0>, 2)

@@ -1,5 +1,5 @@
 """rein_moe_ffn on the wide tiles (kernels/moe_wide.h) against the CPU chain: experts of no, one, 31 to 33, 63 to 65 and more entries, groups of two
-and of four tiles, every pair of image kinds, rows of the slab with and without padding (a power of two of sub-blocks), superblocks in odd and even
+(K-quants) and of four tiles (Q8_0), every pair of image kinds, rows of the slab with and without padding (a power of two of sub-blocks), superblocks in odd and even
 number, the one-launch and the four-launch sort, ids that leave experts out."""
 import numpy as np
 import pytest
@@ -59,10 +59,9 @@ def one_each(rng):
     return logits
 
 
-@pytest.mark.parametrize("most", [2, 4])
 @pytest.mark.parametrize("gu,dn,hidden,ff", [(rein.Q4_K, rein.Q6_K, 1024, 768), (rein.Q6_K, rein.Q4_K, 768, 256), (rein.Q5_K, rein.Q5_K, 256, 1024),
                                              (rein.Q8_0, rein.Q5_K, 512, 256), (rein.Q4_K, rein.Q8_0, 1280, 512), (rein.Q8_0, rein.Q8_0, 256, 768)])
-def test_experts_of_every_number_of_tiles(gu, dn, hidden, ff, most, options):
+def test_experts_of_every_number_of_tiles(gu, dn, hidden, ff, options):
     rng = np.random.default_rng(hidden + ff)
     logits = one_each(rng)
     x = rng.standard_normal((len(logits), hidden)).astype(np.float32)
@@ -71,7 +70,7 @@ def test_experts_of_every_number_of_tiles(gu, dn, hidden, ff, most, options):
     want = reference(gu, dn, hidden, ff, x, logits, 1, weights, scale)
     options.set("REIN_MOE_FEW", "0")
     options.set("REIN_MOE_CHAIN", "0")
-    options.set("REIN_MOE_WIDE", str(most))
+    options.set("REIN_MOE_WIDE", "1")
     got = ffn(gu, dn, hidden, ff, x, logits, 1, weights, scale)
     check(got, want, "wide tiles")
     options.set("REIN_MOE_SORT_SPLIT", "1")
@@ -89,7 +88,7 @@ def test_many_experts(n_expert, n_used, options):
     scale = np.ones(n_expert, np.float32)
     options.set("REIN_MOE_FEW", "0")
     options.set("REIN_MOE_CHAIN", "0")
-    options.set("REIN_MOE_WIDE", "2")
+    options.set("REIN_MOE_WIDE", "1")
     check(ffn(gu, dn, hidden, ff, x, logits, n_used, weights, scale), reference(gu, dn, hidden, ff, x, logits, n_used, weights, scale), "many experts")
 
 
@@ -102,6 +101,6 @@ def test_the_default_choice_equals_the_pinned_one(n_tok, n_used, options):
     weights = [slab(f, k, n, 8, s) for f, k, n, s in ((gu, hidden, ff, 1), (gu, hidden, ff, 2), (dn, ff, hidden, 3))]
     scale = np.ones(8, np.float32)
     default = ffn(gu, dn, hidden, ff, x, logits, n_used, weights, scale)
-    options.set("REIN_MOE_WIDE", "2")
+    options.set("REIN_MOE_WIDE", "1")
     assert np.array_equal(ffn(gu, dn, hidden, ff, x, logits, n_used, weights, scale).view(np.uint32), default.view(np.uint32))
     check(default, reference(gu, dn, hidden, ff, x, logits, n_used, weights, scale), "default")
