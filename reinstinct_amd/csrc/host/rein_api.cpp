@@ -2061,8 +2061,7 @@ unsigned wide_lds_bytes(const WideKind& kind, int fmt)
 //         0.84, 6144 -> 2048 0.91) -- and the 4-bit formats from 56M weights with a contraction of 6144 or against more than 16384 rows
 //         (5120 -> 18432 1.07, 6144 -> 12288 1.08, 11008 -> 12288 1.45; 4096 and 5120 -> 14336 0.87-0.97; Q8_0 there 0.75-1.0).
 //   exact, 13 shapes (those and 3584 -> 18944) x 17 row counts from 33:
-//     Q6_K  1.07-3.0 in all 221 cells (17408 -> 5120, 200 rows 220 / 72 us; 5120 -> 17408, 512 rows 311 / 182); below 2.5e8 operations
-//           nothing was measured.
+//     Q6_K  1.07-3.0 in all 221 cells (17408 -> 5120, 200 rows 220 / 72 us; 5120 -> 17408, 512 rows 311 / 182).
 //     Q4_K  33-64 rows contractions of 3072 and more 0.98-1.27 in 27 cells (2048 1.05-1.14, but 1536 -> 32000 0.85); 65-95 rows those of 4096
 //           and more against matrices of 48M weights (1.09-1.36; 5120 -> 5120 0.90: three tiles at the cost of a whole group's unpack);
 //           from 96 rows contractions of 4096 and more, 0.86-1.85, median 1.10 (below, 0.70-1.22: ranges of few superblocks do not
@@ -2083,32 +2082,40 @@ unsigned wide_lds_bytes(const WideKind& kind, int fmt)
 //           deal evenly (8192 -> 8192 0.95, 4096 -> 16384 0.89, 14336 -> 8192 1.08); Q4_K
 //           contractions of 10752 and more up to 6144 rows and from 8193 to 18432 (60M: 1.01-1.33; 11008 -> 7168 and 8192 0.91-0.93), shorter ones
 //           and Q5_K's below 8192 against more than 16384 rows (85M: 1.06-1.21; 8192 -> 14336 0.93, 6144 -> 16384 0.96, Q5_K 11008 -> 8192 0.91).
+//   both again from 33 rows, since the tiles became faster, over 6600 shapes drawn at random (contractions 768-18432, 512-49152 weight rows) that were on the
+//   launches of rein_mmq_xq8_ws.  Of the 1224 that changed over, 1.30 in the mean, two are 3 % behind and none more:
+//     few   Q6_K to 128 rows from contractions of 768 (421 shapes, 1.27-1.81; 1280 -> 1632, 40 rows 16.9 / 9.7 us); Q4_K up to 64 pieces of 128 x 32 from 1024,
+//           128 from 1536 to 2048 (1.16-1.25 in the mean; with more of them 0.82-1.0: the plain launch holds them at once); Q5_K up to 64 pieces from 768
+//           (1.01-1.48), from 65 rows to 128 and, below 2560, 256 or 512 (1.16; three tiles of more than 256 pieces 0.90-0.97).
+//     exact Q6_K from 129 rows below 2.5e8 operations (1.19-1.52); Q5_K at 65-128 rows from contractions of 2560 against 161 to 512 pieces (1.18).
 bool wide_exact_shape(int fmt, unsigned in_dim, unsigned p_rows)          // for any number of weight rows
 {
     const unsigned mode = opt_u(O_MMQXH, 1);
     if (mode == 0 || mode == 3 || p_rows <= 32) return false;             // the kernel is built for groups of at least two tiles
     if (mode == 2 || fmt == REIN_TYPE_Q6_K) return true;
     if (fmt == REIN_TYPE_Q4_K) return in_dim >= (p_rows <= 64 ? 3072u : 4096u);
-    return p_rows > 64 && in_dim >= (p_rows >= 1024 ? 1536u : 3072u);
+    return p_rows > 64 && in_dim >= (p_rows >= 1024 ? 1536u : p_rows <= 128 ? 2560u : 3072u);
 }
+unsigned long long wide_pieces(unsigned out_dim, unsigned p_rows) { return ((unsigned long long)out_dim + 127) / 128 * ((p_rows + 31) / 32); }
 bool wide_exact_take(int fmt, unsigned in_dim, unsigned out_dim, unsigned p_rows)
 {
     if (!wide_exact_shape(fmt, in_dim, p_rows)) return false;
     if (opt_u(O_MMQXH, 1) == 2) return true;
     const unsigned long long weights = (unsigned long long)in_dim * out_dim;
-    if (fmt == REIN_TYPE_Q6_K) return 2.0 * p_rows * (double)weights >= 2.5e8;
+    if (fmt == REIN_TYPE_Q6_K) return 2.0 * p_rows * (double)weights >= (p_rows > 128 && in_dim >= 768 ? 1e8 : 2.5e8);
     if (fmt == REIN_TYPE_Q4_K) return p_rows <= 64 || p_rows >= 96 || weights >= 48ull << 20;
     if (p_rows >= 384) return in_dim >= 4096 || out_dim >= 16384 || (p_rows >= 1024 && (in_dim >= 3072 || out_dim >= 4096));
-    const unsigned long long pieces = ((unsigned long long)out_dim + 127) / 128 * ((p_rows + 31) / 32);
+    const unsigned long long pieces = wide_pieces(out_dim, p_rows);
+    if (p_rows <= 128 && pieces > 160 && pieces <= 512) return true;
     if (in_dim < 4096 && pieces > 640 && pieces <= 768) return false;                 // the plain launch's three workgroups on every CU
-    return weights >= (p_rows > 100 ? 24ull << 20 : 48ull << 20) ||
-           (2ull * in_dim >= 5ull * out_dim && weights >= 5ull << 20 && (p_rows > 100 || in_dim <= 20ull * out_dim));
+    return in_dim >= 3072 && (weights >= (p_rows > 100 ? 24ull << 20 : 48ull << 20) ||
+                              (2ull * in_dim >= 5ull * out_dim && weights >= 5ull << 20 && (p_rows > 100 || in_dim <= 20ull * out_dim)));
 }
 bool wide_few_shape(int fmt, unsigned in_dim, unsigned p_rows)
 {
     const unsigned mode = opt_u(O_MMQXH, 1);
     if (mode == 3) return p_rows > 8;
-    return mode == 1 && p_rows > 8 && p_rows <= (fmt == REIN_TYPE_Q5_K ? 64u : 32u) && in_dim >= (fmt == REIN_TYPE_Q6_K ? 512u : 1024u);
+    return mode == 1 && p_rows > 8 && p_rows <= 128 && in_dim >= (fmt == REIN_TYPE_Q6_K && p_rows <= 32 ? 512u : p_rows <= 32 || fmt == REIN_TYPE_Q4_K ? 1024u : 768u);
 }
 bool wide_few_take(int fmt, unsigned in_dim, unsigned out_dim, unsigned p_rows)
 {
@@ -2121,9 +2128,15 @@ bool wide_few_take(int fmt, unsigned in_dim, unsigned out_dim, unsigned p_rows)
         if (fmt == REIN_TYPE_Q4_K && in_dim >= 10752) return weights >= 60ull << 20 && (out_dim <= 6144 || out_dim > 8192);
         return weights >= 85ull << 20 && out_dim > 16384 && (fmt == REIN_TYPE_Q4_K || in_dim < 8192);
     }
-    if (weights < 4ull << 20) return false;
-    if (p_rows > 32) return in_dim >= 3072 || out_dim <= 32768 || out_dim > 49152;          // 513 to 768 workgroups of the plain launch
-    return fmt == REIN_TYPE_Q6_K || out_dim <= (in_dim < 1280 ? 8192u : in_dim < 10240 ? 12288u : 5120u);
+    if (p_rows <= 32) return weights >= 4ull << 20 && (fmt == REIN_TYPE_Q6_K || out_dim <= (in_dim < 1280 ? 8192u : in_dim < 10240 ? 12288u : 5120u));
+    if (weights < 4ull << 20 && (out_dim <= 512 || in_dim < 768)) return false;       // up to 512 rows rein_matmul_ws has the bits of quantize_q8 + rein_mmq_xq8_ws
+    if (fmt == REIN_TYPE_Q6_K) return true;
+    const unsigned long long pieces = wide_pieces(out_dim, p_rows);
+    if (fmt == REIN_TYPE_Q4_K) return pieces <= (in_dim < 1536 ? 64u : p_rows > 64 ? (in_dim < 2048 || in_dim >= 4096 ? 64u : 128u) : in_dim < 2560 ? 128u : 256u);
+    if (in_dim < 1024) return pieces <= 64;
+    if (p_rows <= 64) return pieces <= 64 || in_dim >= 3072 || out_dim <= 32768 || out_dim > 49152;          // 513 to 768 workgroups of the plain launch
+    if (p_rows <= 100 && in_dim > 20ull * out_dim) return false;
+    return pieces <= 128 || (in_dim < 2560 && pieces <= (p_rows <= 96 || (in_dim >= 1536 && in_dim < 2048) ? 256u : 512u));
 }
 bool wide_int8_shape(unsigned in_dim) { return in_dim >= 768 || opt_u(O_MMQXH, 1) >= 2; }          // for any number of weight rows
 bool wide_int8_take(int fmt, unsigned in_dim, unsigned out_dim, unsigned p_rows)
@@ -2134,7 +2147,7 @@ bool wide_int8_take(int fmt, unsigned in_dim, unsigned out_dim, unsigned p_rows)
         if (in_dim >= 8192 && in_dim >= (in_dim >= 11008 ? 3ull : 4ull) * out_dim) return true;
         return fmt != REIN_TYPE_Q8_0 && (in_dim >= 6144 || out_dim >= 16384) && out_dim <= 18432 && (unsigned long long)in_dim * out_dim >= 56ull << 20;
     }
-    const unsigned long long pieces = ((unsigned long long)out_dim + 127) / 128 * ((p_rows + 31) / 32);
+    const unsigned long long pieces = wide_pieces(out_dim, p_rows);
     if (in_dim < 1536) return in_dim >= 768 && (pieces <= 64 || (pieces > 1024 && in_dim >= 1024));
     return in_dim != 2048 || pieces <= 256 || pieces > 512;
 }

@@ -222,3 +222,23 @@ def test_every_unit_of_a_banded_round_once(fmt, rows, out_dim):
     x = np.random.default_rng(rows).standard_normal((rows, in_dim)).astype(np.float32)
     got = matmul(fmt, packed, x, out_dim, 2)
     assert_close_f32(got, orc.matvec_q8(fmt, packed, in_dim, out_dim, orc.quantize_q8(x), rows), what=f"fmt {fmt}")
+
+
+@pytest.mark.parametrize("fmt, mode, rows, in_dim, out_dim", [
+    (rein.Q6_K, 3, 33, 768, 513),                     # few operations: groups of one and two tiles to 128 rows, above groups of four
+    (rein.Q6_K, 3, 128, 768, 520),
+    (rein.Q6_K, 2, 129, 768, 1030),
+    (rein.Q4_K, 3, 33, 1024, 513),                    # below four million weights
+    (rein.Q4_K, 3, 33, 1024, 4095),                   # 64 pieces of 128 x 32
+    (rein.Q4_K, 3, 65, 4096, 2560),                   # 60
+    (rein.Q4_K, 3, 128, 2048, 4096),                  # 128
+    (rein.Q5_K, 3, 33, 768, 4000),                    # 64
+    (rein.Q5_K, 3, 97, 1024, 6001),                   # 188
+    (rein.Q5_K, 2, 128, 2560, 5200),                  # 164
+])
+def test_the_rule_takes_the_tiles_and_the_scratch_holds_their_plan(fmt, mode, rows, in_dim, out_dim):
+    packed = weights(fmt, in_dim, out_dim, rows)
+    x = np.random.default_rng(rows).standard_normal((rows, in_dim)).astype(np.float32)
+    got = matmul(fmt, packed, x, out_dim, 1)
+    assert np.array_equal(got.view(np.uint32), matmul(fmt, packed, x, out_dim, mode).view(np.uint32))
+    assert_close_f32(got, orc.matvec_q8(fmt, packed, in_dim, out_dim, orc.quantize_q8(x), rows), what=f"fmt {fmt}")
