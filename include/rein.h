@@ -113,7 +113,7 @@ int rein_is_loaded(void);
  * REIN_MOE_SORT_SPLIT, REIN_MOE_CHAIN, REIN_MOE_FUSED, REIN_MOE_FEW, REIN_MOE_WIDE, REIN_MOE_GU_ROWS, REIN_MOE_DC_ROWS
  * (MoE glue: 0 = the workgroup router, 1 = the four-launch sort, 0 = no decode chain for few
  * tokens, 0 = unfused gate/up, 0 never / 1 wherever the shape allows the launches that read every touched
- * expert once, 0 never / 2 / 4 wherever the shape allows the wide tiles in groups of two / four, rows per
+ * expert once, 0 never / 1 wherever the shape allows the wide tiles, rows per
  * workgroup of the two decode launches).
  * Unknown name: REIN_E_NOT_FOUND; a value that is not an unsigned 32-bit decimal:
  * REIN_E_BAD_SHAPE. */
