@@ -2083,7 +2083,7 @@ unsigned wide_lds_bytes(const WideKind& kind, int fmt)
 //           contractions of 10752 and more up to 6144 rows and from 8193 to 18432 (60M: 1.01-1.33; 11008 -> 7168 and 8192 0.91-0.93), shorter ones
 //           and Q5_K's below 8192 against more than 16384 rows (85M: 1.06-1.21; 8192 -> 14336 0.93, 6144 -> 16384 0.96, Q5_K 11008 -> 8192 0.91).
 //   both again from 33 rows, since the tiles became faster, over 6600 shapes drawn at random (contractions 768-18432, 512-49152 weight rows) that were on the
-//   launches of rein_mmq_xq8_ws.  Of the 1224 that changed over, 1.30 in the mean, two are 3 % behind and none more:
+//   launches of rein_mmq_xq8_ws.  Of the 1224 that changed over, 1.30 in the mean, two are 3 % behind and none more (a second draw, 890 changed: 1.33, Q4_K 2304 -> 3488, 62 rows 15.3 / 16.2 us and 15616 -> 2592, 68 rows 29.4 / 30.4):
 //     few   Q6_K to 128 rows from contractions of 768 (421 shapes, 1.27-1.81; 1280 -> 1632, 40 rows 16.9 / 9.7 us); Q4_K up to 64 pieces of 128 x 32 from 1024,
 //           128 from 1536 to 2048 (1.16-1.25 in the mean; with more of them 0.82-1.0: the plain launch holds them at once); Q5_K up to 64 pieces from 768
 //           (1.01-1.48), from 65 rows to 128 and, below 2560, 256 or 512 (1.16; three tiles of more than 256 pieces 0.90-0.97).
