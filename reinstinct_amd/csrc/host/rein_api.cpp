@@ -2620,12 +2620,14 @@ int rein_moe_combine(const float* experts, const int32_t* ids, const float* weig
 // Workspace carve-up for rein_moe_ffn (all offsets 256-byte aligned).
 namespace {
 struct MoeWs {
-    size_t ids, weights, count, cursor, perm, inv, eoff, toff, xq_in, g_in, e_gate, e_up, xq_exp, g_out, img_in, img_exp, place, units2, units4, total;
+    size_t ids, weights, count, cursor, perm, inv, eoff, toff, xq_in, g_in, e_gate, e_up, xq_exp, g_out, total;
+    size_t img_in, img_exp, place, units2, units4;
+    bool wide;                                       // whether those five have room
 };
 size_t up256(size_t v) { return (v + 255) & ~(size_t)255; }
 // the pipeline on the wide tiles (kernels/moe_wide.h): contractions of whole superblocks
 bool moe_wide_fmt(int fmt) { return wide_k_quant(fmt) || fmt == REIN_TYPE_Q8_0; }
-bool moe_wide_fits(const rein_moe_shape& sh)
+bool moe_wide_shape(const rein_moe_shape& sh)
 {
     return moe_wide_fmt(sh.gate_up_fmt) && moe_wide_fmt(sh.down_fmt) && sh.hidden % 256 == 0 && sh.expert_ff % 256 == 0 &&
            (unsigned long long)sh.n_tok * sh.n_used <= 0x3FFFFFFull && sh.n_expert <= 65535;
@@ -2645,7 +2647,7 @@ unsigned moe_units_per_xcd(const rein_moe_shape& sh, unsigned most)
 MoeWs moe_ws(const rein_moe_shape& sh)
 {
     const size_t ne = (size_t)sh.n_tok * sh.n_used;
-    MoeWs w;
+    MoeWs w{};
     size_t o = 0;
     auto take = [&](size_t bytes) { const size_t at = o; o += up256(bytes); return at; };
     w.ids     = take(ne * 4);
@@ -2662,11 +2664,13 @@ MoeWs moe_ws(const rein_moe_shape& sh)
     w.e_gate  = take(ne * sh.expert_ff * 4);
     w.e_up    = take(ne * sh.expert_ff * 4);
     w.xq_exp  = take(ne * (sh.expert_ff / 32) * 40);
-    w.img_in = w.img_exp = w.place = w.units2 = w.units4 = shared;
-    size_t end = o;
-    if (moe_wide_fits(sh)) {
-        // instead of the four above: the wide pipeline's lists and its two images.  That of the tokens lies last and may reach into the rows of the
-        // down projection, whose launch is behind the one that reads it.
+    w.g_out   = take(ne * sh.hidden * 4);
+    w.total   = o;
+    if (moe_wide_shape(sh)) {
+        // Instead of the four behind the tokens' blocks: the wide pipeline's lists and its two images.  That of the tokens lies last and may reach into
+        // the rows of the down projection, whose launch is behind the one that reads it.  An image has whole tiles, in the worst routing almost
+        // one for each expert more than the entries fill: there is room for it from 7 (Q8_0) to 24 entries per expert on, and wherever the wide tiles are
+        // the default.  The workspace stays that of the other pipeline, whatever the options say.
         const size_t tiles = moe_most_tiles(sh);
         o = shared;
         w.place   = take(ne * 4);
@@ -2674,12 +2678,8 @@ MoeWs moe_ws(const rein_moe_shape& sh)
         w.units4  = take((size_t)8 * moe_units_per_xcd(sh, 4) * 16);
         w.img_exp = take(wide_image_bytes(sh.down_fmt, sh.expert_ff, (unsigned)(tiles * 32)));
         w.img_in  = o;
-        end = std::max(end, o);
-        o = end;
+        w.wide    = o <= w.g_out && o + wide_image_bytes(sh.gate_up_fmt, sh.hidden, (unsigned)(tiles * 32)) <= w.total;
     }
-    w.g_out   = take(ne * sh.hidden * 4);
-    if (moe_wide_fits(sh)) o = std::max(o, up256(w.img_in + wide_image_bytes(sh.gate_up_fmt, sh.hidden, (unsigned)(moe_most_tiles(sh) * 32))));
-    w.total   = o;
     return w;
 }
 }  // namespace
@@ -2751,9 +2751,9 @@ namespace {
 // six more.  Where it is taken it is ahead by 1.18 in the mean of 1098 cells and nowhere behind by more than 1 %: 128 experts top-8, 2048 x 768
 // Q4_K / Q6_K, 512 tokens 228 / 191 us, 640 268 / 214; 256 top-8, 2048 x 1024, 1000 tokens 508 / 461; 64 top-4 of Q8_0, 300 tokens 122 / 115.
 // K-quants in groups of four were 0.91-1.03 of groups of two, never ahead by enough to have them.  An option that pins a form of the other pipeline keeps it.
-bool moe_wide_pays(const rein_moe_shape& sh)
+bool moe_wide_pays(const rein_moe_shape& sh, const MoeWs& w)
 {
-    if (!moe_wide_fits(sh)) return false;
+    if (!w.wide) return false;
     if (opt_is_set(O_MOE_WIDE)) return opt_u(O_MOE_WIDE, 0) != 0;
     if (opt_is_set(O_MOE_FUSED) || opt_is_set(O_GROUPED_STRIDED)) return false;
     const unsigned long long entries = (unsigned long long)sh.n_tok * sh.n_used, experts = sh.n_expert, blocks = experts * (sh.expert_ff / 64);
@@ -2876,7 +2876,7 @@ int rein_moe_ffn(const rein_moe_shape* shp, const float* x, const float* logits,
         return rein_moe_down_combine(sh.down_fmt, down_exps, ids, weights, down_exps_s, base + w.xq_exp, out, sh.expert_ff, sh.hidden,
                                      (unsigned)bpe_dn, sh.n_used * ns_f, ns_f, sh.n_used, sh.n_tok, s);
     }
-    const bool wide = moe_wide_pays(sh);
+    const bool wide = moe_wide_pays(sh, w);
     if (wide && wave) {
         if (int rc = route_quantize()) return rc;
     } else {

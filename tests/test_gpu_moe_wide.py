@@ -78,11 +78,12 @@ def test_experts_of_every_number_of_tiles(gu, dn, hidden, ff, options):
     assert np.array_equal(ffn(gu, dn, hidden, ff, x, logits, 1, weights, scale).view(np.uint32), got.view(np.uint32))
 
 
-@pytest.mark.parametrize("n_expert,n_used", [(300, 3), (70, 4)])               # more experts than the one-wavefront router and a scan of 64 hold
-def test_many_experts(n_expert, n_used, options):
+# more experts than the one-wavefront router and a scan of 64 hold (at 150 tokens the workspace has no room for the wide tiles)
+@pytest.mark.parametrize("n_expert,n_used,n_tok", [(300, 3, 150), (70, 4, 150), (300, 3, 1800), (70, 4, 400)])
+def test_many_experts(n_expert, n_used, n_tok, options):
     gu, dn, hidden, ff = rein.Q4_K, rein.Q6_K, 512, 256
     rng = np.random.default_rng(n_expert)
-    logits, x = rng.standard_normal((150, n_expert)).astype(np.float32), rng.standard_normal((150, hidden)).astype(np.float32)
+    logits, x = rng.standard_normal((n_tok, n_expert)).astype(np.float32), rng.standard_normal((n_tok, hidden)).astype(np.float32)
     logits[:, 1] += 2.0                                                         # an expert of many tiles
     weights = [slab(f, k, n, n_expert, s) for f, k, n, s in ((gu, hidden, ff, 1), (gu, hidden, ff, 2), (dn, ff, hidden, 3))]
     scale = np.ones(n_expert, np.float32)

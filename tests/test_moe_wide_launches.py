@@ -1,0 +1,49 @@
+"""rein_moe_ffn on the wide tiles, without a GPU (tests/launches.py records the launches): what workspace it has, and where it is taken."""
+import random
+
+import pytest
+
+import reinstinct_amd as rein
+from launches import record
+from reinstinct_amd import runtime
+
+FORMATS = (rein.Q4_K, rein.Q5_K, rein.Q6_K, rein.Q8_0)
+
+
+def kernels(calls, tmp_path):
+    return [[r[0] for r in d["launches"]] for d in record(calls, tmp_path)]
+
+
+def wide(names):
+    return any("_swiglu" in n and "_xg" in n for n in names)
+
+
+def pipeline_bytes(n_tok, hidden, n_expert, n_used, ff, gu=0, dn=0):
+    """the pipeline of 32-token tiles: routing, lists of the sort, BlockQ8 rows of the tokens and the entries, gate, up, their rows, down"""
+    ne = n_tok * n_used
+    parts = [4 * ne, 4 * ne, 4 * n_expert, 4 * n_expert, 4 * ne, 4 * ne, 4 * n_expert + 4, 4 * n_expert + 4, n_tok * hidden // 32 * 40,
+             ne * hidden // 32 * 40, 4 * ne * ff, 4 * ne * ff, ne * ff // 32 * 40, 4 * ne * hidden]
+    return sum((p + 255) // 256 * 256 for p in parts)
+
+
+@pytest.mark.parametrize("option", [None, "REIN_MOE_WIDE"])
+def test_the_workspace_is_that_of_the_pipeline(option, options):
+    """what a call may take instead of the pipeline lives inside the pipeline's own room, so no option changes the size"""
+    if option:
+        options.set(option, "1")
+    rng = random.Random(3)
+    shapes = [(1, 2048, 128, 8, 768), (16, 2048, 128, 8, 768), (48, 2048, 128, 8, 768), (32, 4096, 256, 8, 1536), (512, 2048, 128, 8, 768), (1, 256, 1, 1, 256)]
+    shapes += [(int(2 ** rng.uniform(0, 12)), 256 * rng.randint(1, 16), e, rng.randint(1, min(8, e)), 256 * rng.randint(1, 8)) for e in (2, 8, 60, 128, 300) for _ in range(40)]
+    for s in shapes:
+        gu, dn = rng.choice(FORMATS), rng.choice(FORMATS)
+        assert runtime.moe_workspace_bytes(runtime.moe_shape(*s, gu, dn)) == pipeline_bytes(*s), (s, gu, dn)
+
+
+def test_wide_tiles_that_have_no_room_are_not_taken(tmp_path):
+    """one entry of an expert would be charged a whole tile: however it is asked for, the workspace does not hold that"""
+    q4, q6, q8 = rein.Q4_K, rein.Q6_K, rein.Q8_0
+    pins = [("option", [n, v]) for n, v in (("REIN_MOE_FEW", 0), ("REIN_MOE_CHAIN", 0), ("REIN_MOE_WIDE", 1))]
+    cases = [((48, 2048, 128, 8, 768, q4, q6), 0), ((96, 2048, 128, 8, 768, q8, q8), 0), ((256, 2048, 128, 8, 768, q8, q8), 1), ((272, 2048, 128, 8, 768, q4, q6), 0),
+             ((512, 2048, 128, 8, 768, q4, q6), 1), ((512, 4096, 128, 8, 256, q4, q4), 1), ((1, 256, 1, 1, 256, q4, q6), 0)]
+    for (shape, want), names in zip(cases, kernels(pins + [("moe_ffn", list(s)) for s, _ in cases], tmp_path)[len(pins):]):
+        assert wide(names) == bool(want), (shape, names)
