@@ -569,7 +569,8 @@ size_t rein_moe_workspace_bytes(const rein_moe_shape *shape);
  * multiples of 256, expert_ff 512 and more).
  * The forms add the terms inside an expert's row in different orders: the fp32 bits of a token's output row
  * therefore depend on how many tokens share the call, within the path's 1e-3 / 1e-4 tolerance of any
- * order.  The option REIN_MOE_CHAIN = 0 (with REIN_MOE_FEW unset) keeps every call on the pipeline. */
+ * order.  The option REIN_MOE_CHAIN = 0 (with REIN_MOE_FEW and REIN_MOE_WIDE unset) keeps every call on the pipeline's
+ * 32-token tiles, whose bits do not. */
 int rein_moe_ffn(const rein_moe_shape *shape, const float *x, const float *logits,
                  const void *gate_exps, const void *up_exps, const void *down_exps,
                  const float *down_exps_s, void *workspace, float *out, rein_stream_t s);

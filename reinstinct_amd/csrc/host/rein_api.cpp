@@ -2750,12 +2750,13 @@ namespace {
 // 0.99 in the mean, 0.82 at worst); up to 512 and with two superblocks from 36 entries, with a Q5_K down, which has both extra bits and minimums, from
 // six more.  Where it is taken it is ahead by 1.18 in the mean of 1098 cells and nowhere behind by more than 1 %: 128 experts top-8, 2048 x 768
 // Q4_K / Q6_K, 512 tokens 228 / 191 us, 640 268 / 214; 256 top-8, 2048 x 1024, 1000 tokens 508 / 461; 64 top-4 of Q8_0, 300 tokens 122 / 115.
-// K-quants in groups of four were 0.91-1.03 of groups of two, never ahead by enough to have them.  An option that pins a form of the other pipeline keeps it.
+// K-quants in groups of four were 0.91-1.03 of groups of two, never ahead by enough to have them.  An option that pins a form of the other pipeline
+// keeps it; REIN_MOE_CHAIN does too, with which a token's result is the same however many share its call.
 bool moe_wide_pays(const rein_moe_shape& sh, const MoeWs& w)
 {
     if (!w.wide) return false;
     if (opt_is_set(O_MOE_WIDE)) return opt_u(O_MOE_WIDE, 0) != 0;
-    if (opt_is_set(O_MOE_FUSED) || opt_is_set(O_GROUPED_STRIDED)) return false;
+    if (opt_is_set(O_MOE_CHAIN) || opt_is_set(O_MOE_FUSED) || opt_is_set(O_GROUPED_STRIDED)) return false;
     const unsigned long long entries = (unsigned long long)sh.n_tok * sh.n_used, experts = sh.n_expert, blocks = experts * (sh.expert_ff / 64);
     const unsigned long long groups = std::max(1ull, (entries + 64 * experts - 1) / (64 * experts));
     if (sh.expert_ff < 512 || blocks * groups < 320) return false;

@@ -105,3 +105,15 @@ def test_the_default_choice_equals_the_pinned_one(n_tok, n_used, options):
     options.set("REIN_MOE_WIDE", "1")
     assert np.array_equal(ffn(gu, dn, hidden, ff, x, logits, n_used, weights, scale).view(np.uint32), default.view(np.uint32))
     check(default, reference(gu, dn, hidden, ff, x, logits, n_used, weights, scale), "default")
+
+
+def test_on_the_pinned_pipeline_a_token_has_the_same_bits_in_every_call(options):
+    gu, dn, hidden, ff = rein.Q4_K, rein.Q6_K, 256, 2560
+    rng = np.random.default_rng(7)
+    logits, x = rng.standard_normal((64, 8)).astype(np.float32), rng.standard_normal((64, hidden)).astype(np.float32)
+    weights = [slab(f, k, n, 8, s) for f, k, n, s in ((gu, hidden, ff, 1), (gu, hidden, ff, 2), (dn, ff, hidden, 3))]
+    scale = np.ones(8, np.float32)
+    options.set("REIN_MOE_CHAIN", "0")
+    together = ffn(gu, dn, hidden, ff, x, logits, 5, weights, scale)               # 40 entries per expert
+    for some in (slice(0, 1), slice(20, 33)):
+        assert np.array_equal(ffn(gu, dn, hidden, ff, x[some], logits[some], 5, weights, scale).view(np.uint32), together[some].view(np.uint32))

@@ -47,3 +47,14 @@ def test_wide_tiles_that_have_no_room_are_not_taken(tmp_path):
              ((512, 2048, 128, 8, 768, q4, q6), 1), ((512, 4096, 128, 8, 256, q4, q4), 1), ((1, 256, 1, 1, 256, q4, q6), 0)]
     for (shape, want), names in zip(cases, kernels(pins + [("moe_ffn", list(s)) for s, _ in cases], tmp_path)[len(pins):]):
         assert wide(names) == bool(want), (shape, names)
+
+
+def test_a_pinned_pipeline_has_one_form(tmp_path):
+    """REIN_MOE_CHAIN and the options of the 32-token tiles keep them at every number of tokens; only REIN_MOE_WIDE = 1 is asked for by name"""
+    calls = [("moe_ffn", [n, 2048, 128, 8, 768, rein.Q4_K, rein.Q6_K]) for n in (1, 48, 479, 480, 2048)]
+    for pins, want in ([], [0, 0, 0, 1, 1]), ([("REIN_MOE_CHAIN", 0)], [0] * 5), ([("REIN_MOE_FUSED", 1)], [0] * 5), ([("REIN_GROUPED_STRIDED", 1)], [0] * 5), \
+            ([("REIN_MOE_WIDE", 0)], [0] * 5), ([("REIN_MOE_CHAIN", 0), ("REIN_MOE_WIDE", 1)], [0, 0, 1, 1, 1]):
+        done = kernels([("option", list(p)) for p in pins] + calls, tmp_path)[len(pins):]
+        assert [wide(names) for names in done] == [bool(w) for w in want], pins
+        if pins == [("REIN_MOE_CHAIN", 0)]:
+            assert all("rein_mmq_q4k_grouped_swiglu_q8" in names and "rein_mmq_q6k_grouped_t32" in names for names in done)
