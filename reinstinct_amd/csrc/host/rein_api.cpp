@@ -2084,9 +2084,15 @@ unsigned wide_lds_bytes(const WideKind& kind, int fmt)
 //           and Q5_K's below 8192 against more than 16384 rows (85M: 1.06-1.21; 8192 -> 14336 0.93, 6144 -> 16384 0.96, Q5_K 11008 -> 8192 0.91).
 //   both again from 33 rows, since the tiles became faster, over 6600 shapes drawn at random (contractions 768-18432, 512-49152 weight rows) that were on the
 //   launches of rein_mmq_xq8_ws.  Of the 1224 that changed over, 1.30 in the mean, two are 3 % behind and none more (a second draw, 890 changed: 1.33, Q4_K 2304 -> 3488, 62 rows 15.3 / 16.2 us and 15616 -> 2592, 68 rows 29.4 / 30.4):
-//     few   Q6_K to 128 rows from contractions of 768 (421 shapes, 1.27-1.81; 1280 -> 1632, 40 rows 16.9 / 9.7 us); Q4_K up to 64 pieces of 128 x 32 from 1024,
-//           128 from 1536 to 2048 (1.16-1.25 in the mean; with more of them 0.82-1.0: the plain launch holds them at once); Q5_K up to 64 pieces from 768
-//           (1.01-1.48), from 65 rows to 128 and, below 2560, 256 or 512 (1.16; three tiles of more than 256 pieces 0.90-0.97).
+//     few   Q6_K to 128 rows from contractions of 768 (421 shapes, 1.27-1.81; 1280 -> 1632, 40 rows 16.9 / 9.7 us).  Q4_K and Q5_K by pieces of 128 x 32, of which the
+//           plain launch holds up to 256 and more at once:
+//           Q4_K 33-64 rows up to 64 from contractions of 1024 (1.02-1.56), 128 from 1536 (1.06-1.24; 1024 and 1280 0.96-1.13), 256 from 2560 (1.03-1.35; shorter ones
+//           0.88-1.23).  65-128 rows up to 64 from 1024 (1.01-1.51), 128 from 2048 to below 4096 (1.02-1.32; 1536 and 1792 0.99-1.24; from 4096 at 65-95 rows 0.95-1.12,
+//           1.02 in the mean of 56), not 129 and more (0.95-1.18 below 2560, 0.98-1.28 from there).
+//           Q5_K up to 64 from 768 (1.02-1.37); at 33-64 rows as above; at 65-128 rows 128 from 1024 (1.01-1.51) and, below 2560, 512 (1.12-1.41) or, with three tiles
+//           and with contractions of 1536 and 1792, 256 (1.01-1.39; beyond 0.86-0.99 and 0.86-1.21).
+//           Down to one row of weights: up to 512 of them, 1470 cells, 1.01-1.72 (Q4_K), 1.05-1.50 (Q5_K), 1.24-1.86 (Q6_K; 2048 -> 512, 40 rows 14.3 / 9.1 us), and
+//           6245 shapes drawn at random, 1.05 at least.
 //     exact Q6_K from 129 rows below 2.5e8 operations (1.19-1.52); Q5_K at 65-128 rows from contractions of 2560 against 161 to 512 pieces (1.18).
 bool wide_exact_shape(int fmt, unsigned in_dim, unsigned p_rows)          // for any number of weight rows
 {
@@ -2129,13 +2135,11 @@ bool wide_few_take(int fmt, unsigned in_dim, unsigned out_dim, unsigned p_rows)
         return weights >= 85ull << 20 && out_dim > 16384 && (fmt == REIN_TYPE_Q4_K || in_dim < 8192);
     }
     if (p_rows <= 32) return weights >= 4ull << 20 && (fmt == REIN_TYPE_Q6_K || out_dim <= (in_dim < 1280 ? 8192u : in_dim < 10240 ? 12288u : 5120u));
-    if (weights < 4ull << 20 && (out_dim <= 512 || in_dim < 768)) return false;       // up to 512 rows rein_matmul_ws has the bits of quantize_q8 + rein_mmq_xq8_ws
     if (fmt == REIN_TYPE_Q6_K) return true;
     const unsigned long long pieces = wide_pieces(out_dim, p_rows);
     if (fmt == REIN_TYPE_Q4_K) return pieces <= (in_dim < 1536 ? 64u : p_rows > 64 ? (in_dim < 2048 || in_dim >= 4096 ? 64u : 128u) : in_dim < 2560 ? 128u : 256u);
     if (in_dim < 1024) return pieces <= 64;
     if (p_rows <= 64) return pieces <= 64 || in_dim >= 3072 || out_dim <= 32768 || out_dim > 49152;          // 513 to 768 workgroups of the plain launch
-    if (p_rows <= 100 && in_dim > 20ull * out_dim) return false;
     return pieces <= 128 || (in_dim < 2560 && pieces <= (p_rows <= 96 || (in_dim >= 1536 && in_dim < 2048) ? 256u : 512u));
 }
 bool wide_int8_shape(unsigned in_dim) { return in_dim >= 768 || opt_u(O_MMQXH, 1) >= 2; }          // for any number of weight rows

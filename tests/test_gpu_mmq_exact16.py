@@ -235,6 +235,9 @@ def test_every_unit_of_a_banded_round_once(fmt, rows, out_dim):
     (rein.Q5_K, 3, 33, 768, 4000),                    # 64
     (rein.Q5_K, 3, 97, 1024, 6001),                   # 188
     (rein.Q5_K, 2, 128, 2560, 5200),                  # 164
+    (rein.Q6_K, 3, 40, 2048, 512),                    # narrow matrices
+    (rein.Q4_K, 3, 33, 1024, 1),
+    (rein.Q5_K, 3, 65, 17408, 640),                   # less than a twentieth of the contraction
 ])
 def test_the_rule_takes_the_tiles_and_the_scratch_holds_their_plan(fmt, mode, rows, in_dim, out_dim):
     packed = weights(fmt, in_dim, out_dim, rows)

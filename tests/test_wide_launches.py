@@ -78,10 +78,21 @@ def test_where_the_small_groups_are_taken(tmp_path):
            (q4, 5120, 17408, 9, "xf_q4k"), (q5, 6144, 18432, 16, "xf_q5k"), (q5, 11008, 8192, 9, 0), (q5, 17408, 5120, 12, 0)], tmp_path)
 
 
+def test_narrow_matrices_of_the_k_quants(tmp_path):
+    """33 to 128 rows: the small groups down to one row of weights"""
+    tags = {f: "xf_" + t for f, t in K_QUANTS.items()}
+    taken([(f, k, n, rows, tags[f]) for f in tags for k, n, rows in [(1024, 1, 33), (2048, 512, 40), (2048, 513, 40), (2048, 512, 64), (1280, 96, 128), (3072, 32, 33 if f == rein.Q6_K else 65)]] +
+          [(rein.Q5_K, 17408, n, 65, "xf_q5k") for n in (32, 512, 513, 640, 832)] + [(rein.Q4_K, 768, 512, 40, 0), (rein.Q5_K, 512, 512, 40, 0), (rein.Q6_K, 512, 512, 40, 0)] +
+          # Q4_K by pieces of 128 x 32: 64, 128 and 256
+          [(rein.Q4_K, k, n, rows, tags[rein.Q4_K] if yes else 0) for k, n, rows, yes in
+           [(1280, 4096, 64, 1), (1280, 4224, 64, 0), (1536, 8192, 64, 1), (1536, 8320, 64, 0), (2304, 8320, 64, 0), (2560, 16384, 64, 1), (2560, 16512, 64, 0),
+            (1792, 2048, 128, 1), (1792, 2176, 128, 0), (2048, 4096, 128, 1), (2048, 4224, 128, 0), (3840, 4096, 128, 1), (4096, 2688, 95, 1), (4096, 2816, 95, 0)]], tmp_path)
+
+
 def test_where_the_exact_dot_gemm_of_q5_k_is_taken(tmp_path):
     q5, kernel = rein.Q5_K, "xh_q5k"
     taken([(q5, 1536, 4064, 1024, 0), (q5, 1536, 4096, 1024, kernel), (q5, 2816, 3072, 1024, 0), (q5, 3072, 512, 1024, kernel), (q5, 2816, 18944, 1023, 0),
-           (q5, 3072, 17408, 160, 0), (q5, 3072, 17408, 161, kernel), (q5, 4096, 17408, 160, kernel), (q5, 17408, 832, 65, 0), (q5, 17408, 1024, 65, kernel),
+           (q5, 3072, 17408, 160, 0), (q5, 3072, 17408, 161, kernel), (q5, 4096, 17408, 160, kernel), (q5, 17408, 832, 65, "xf_q5k"), (q5, 17408, 1024, 65, kernel),
            (q5, 17408, 640, 101, kernel), (q5, 8192, 640, 100, kernel)], tmp_path)
 
 
