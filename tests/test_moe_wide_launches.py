@@ -58,3 +58,30 @@ def test_a_pinned_pipeline_has_one_form(tmp_path):
         assert [wide(names) for names in done] == [bool(w) for w in want], pins
         if pins == [("REIN_MOE_CHAIN", 0)]:
             assert all("rein_mmq_q4k_grouped_swiglu_q8" in names and "rein_mmq_q6k_grouped_t32" in names for names in done)
+
+
+def test_where_the_wide_tiles_are_taken(tmp_path):
+    """both sides of every line: entries per expert by formats, units of the gate + up launch, superblocks of the down projection"""
+    q4, q5, q6, q8 = FORMATS
+    k2, k4, tiles = ("rein_mmq_{}_xg2_swiglu", "rein_mmq_{}_xg2_rows"), ("rein_mmq_{}_xg4_swiglu", "rein_mmq_{}_xg4_rows"), None
+    # tokens, hidden, experts, used, width, formats
+    cases = [((480, 2048, 128, 8, 768, q4, q6), ("q4k", k2, "q6k", k2)), ((479, 2048, 128, 8, 768, q4, q6), tiles),           # 30 entries per expert
+             ((480, 1024, 128, 8, 768, q5, q4), ("q5k", k2, "q4k", k2)), ((480, 1024, 128, 8, 768, q6, q8), ("q6k", k2, "q8_0", k4)),
+             ((576, 2048, 128, 8, 768, q4, q5), ("q4k", k2, "q5k", k2)), ((575, 2048, 128, 8, 768, q4, q5), tiles),           # 36 with a Q5_K down
+             ((576, 2048, 128, 8, 512, q4, q6), ("q4k", k2, "q6k", k2)), ((575, 2048, 128, 8, 512, q4, q6), tiles),           # and with two superblocks to it
+             ((672, 2048, 128, 8, 512, q4, q5), ("q4k", k2, "q5k", k2)), ((671, 2048, 128, 8, 512, q4, q5), tiles),           # 42 with both
+             ((2048, 2048, 128, 8, 256, q4, q6), tiles), ((2048, 2048, 128, 8, 256, q8, q8), tiles),                          # one superblock
+             ((288, 2048, 32, 4, 768, q4, q6), ("q4k", k2, "q6k", k2)), ((287, 2048, 32, 4, 768, q4, q6), tiles),             # 384 units: 36
+             ((480, 2048, 64, 4, 512, q4, q6), tiles), ((384, 2048, 43, 4, 768, q4, q6), ("q4k", k2, "q6k", k2)), ((323, 2048, 43, 4, 768, q4, q6), ("q4k", k2, "q6k", k2)),
+             ((322, 2048, 43, 4, 768, q4, q6), tiles), ((384, 2048, 42, 4, 768, q4, q6), ("q4k", k2, "q6k", k2)), ((377, 2048, 42, 4, 768, q4, q6), tiles),          # 516 units and 504
+             ((72, 256, 8, 4, 2560, q4, q6), ("q4k", k2, "q6k", k2)), ((71, 256, 8, 4, 2560, q4, q6), tiles),                 # 320 units
+             ((128, 256, 8, 4, 2304, q4, q6), tiles), ((129, 256, 8, 4, 2304, q4, q6), ("q4k", k2, "q6k", k2)),               # 288, and twice as many
+             ((288, 2048, 128, 8, 768, q8, q8), ("q8_0", k4, "q8_0", k4)), ((287, 2048, 128, 8, 768, q8, q8), tiles),         # 18 of Q8_0
+             ((288, 2048, 128, 8, 768, q8, q5), ("q8_0", k4, "q5k", k2)), ((288, 2048, 128, 8, 512, q8, q6), ("q8_0", k4, "q6k", k2)),
+             ((512, 2080, 128, 8, 768, q8, q8), tiles), ((512, 2048, 128, 8, 800, q8, q8), tiles)]                            # contractions of whole superblocks
+    for (shape, want), names in zip(cases, kernels([("moe_ffn", list(s)) for s, _ in cases], tmp_path)):
+        if want is tiles:
+            assert any("_grouped_swiglu_q8" in n for n in names) and not wide(names), (shape, names)
+        else:
+            gu, (first, _), dn, (_, second) = want
+            assert first.format(gu) in names and second.format(dn) in names, (shape, names)
