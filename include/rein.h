@@ -113,7 +113,7 @@ int rein_is_loaded(void);
  * REIN_MOE_SORT_SPLIT, REIN_MOE_CHAIN, REIN_MOE_FUSED, REIN_MOE_FEW, REIN_MOE_WIDE, REIN_MOE_GU_ROWS, REIN_MOE_DC_ROWS
  * (MoE glue: 0 = the workgroup router, 1 = the four-launch sort, 0 = no decode chain for few
  * tokens, 0 = unfused gate/up, 0 never / 1 wherever the shape allows the launches that read every touched
- * expert once, 0 never / 1 wherever the shape allows the wide tiles, rows per
+ * expert once, 0 never / 1 wherever the workspace has room for the wide tiles, rows per
  * workgroup of the two decode launches).
  * Unknown name: REIN_E_NOT_FOUND; a value that is not an unsigned 32-bit decimal:
  * REIN_E_BAD_SHAPE. */
@@ -568,9 +568,10 @@ size_t rein_moe_workspace_bytes(const rein_moe_shape *shape);
  * From about 30 entries per expert (18 of Q8_0) the pipeline's GEMMs run on wider tiles (hidden and expert_ff
  * multiples of 256, expert_ff 512 and more).
  * The forms add the terms inside an expert's row in different orders: the fp32 bits of a token's output row
- * therefore depend on how many tokens share the call, within the path's 1e-3 / 1e-4 tolerance of any
- * order.  The option REIN_MOE_CHAIN = 0 (with REIN_MOE_FEW and REIN_MOE_WIDE unset) keeps every call on the pipeline's
- * 32-token tiles, whose bits do not. */
+ * therefore depend on how many tokens share the call -- by the last bits of those sums and, where such a bit moves a
+ * quant of the intermediate by one step, by what that step is worth (below 5e-4 of a result in the norm).
+ * The option REIN_MOE_CHAIN = 0 (with REIN_MOE_FEW and REIN_MOE_WIDE unset) keeps every call on the pipeline's
+ * 32-token tiles, on which they do not. */
 int rein_moe_ffn(const rein_moe_shape *shape, const float *x, const float *logits,
                  const void *gate_exps, const void *up_exps, const void *down_exps,
                  const float *down_exps_s, void *workspace, float *out, rein_stream_t s);

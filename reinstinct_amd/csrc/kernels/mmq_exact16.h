@@ -24,8 +24,10 @@
 // 2.4 GHz under this load; the kernel takes 88 and 118.  Without its transfers it is 14 % faster (Q4_K 17 %), with the activations
 // always from one place in cache 3-7 %: what is left is the way from L2 to LDS and the scalar issue around it.  Waits, barriers and
 // the operand reads from LDS cost nothing measurable.  Whole calls of rein_matmul_ws against the launches of rein_mmq_xq8_ws (fp6 for
-// Q4_K, else int8), us, Q4_K / Q5_K / Q6_K: 2048 x 5120 -> 17408 633 / 809 / 1268 -> 512 / 557 / 670; 512 x 5120 -> 17408 169 / 203 /
-// 347 -> 138 / 149 / 184; 777 x 17408 -> 5120 Q6_K 569 -> 320; 45 x 17408 -> 5120 (one group of two tiles) Q5_K 42.1 -> 36.3.
+// Q4_K, else int8), both on one card, three inputs and the weights of several matrices in turn, us, Q4_K / Q5_K / Q6_K: 2048 x 5120 -> 17408 569 / 715 /
+// 1066 -> 511 / 552 / 676; 512 x 5120 -> 17408 148 / 192 / 292 -> 138 / 150 / 183; 777 x 17408 -> 5120 Q6_K 492 -> 325; 45 x 17408 -> 5120 (one group of
+// two tiles) Q5_K 44.5 -> 38.0.  Other cards are up to 7 % off (777 rows 328 to 343).  The figures beside single choices below have both sides from one
+// card and one session each; they do not add up over sessions.
 //
 // Replaces, from nine rows, kernels/mmq_gemm_{q4k,q5k,q6k}_repacked.cpp of the reference behind rein_matmul_ws.
 #pragma once
@@ -701,8 +703,8 @@ __device__ __forceinline__ unsigned rein_xh_deal(unsigned i, unsigned n)
 }
 // Unit `v` of n_rb x n_grp in the order of the launch: bands of up to four token groups, in a band row block by row block.  An XCD's
 // 64 resident workgroups are then 16 row blocks x 4 groups instead of 4 x 16: they share the activations sixteen ways in their L2, and what
-// it fetches is halved (a group's activations are 272 bytes a value of the contraction, a row block's weights 72 to 136).  2048 x 5120
-// -> 17408 Q4_K 548 -> 522 us, Q8_0 523 -> 500, Q8_0 1000 x 4096 -> 4096 75 -> 68; bands of eight 532 and 503.  Band b has the groups b,
+// it fetches is halved (a group's activations are 272 bytes a value of the contraction, a row block's weights 72 to 136).  Whole calls of 2048 x 5120
+// -> 17408 Q4_K 527 -> 511 us, Q5_K 568 -> 552, Q8_0 506 -> 490, Q6_K 678 -> 676; bands of eight are 2 and 1 % slower (Q4_K, Q8_0).  Band b has the groups b,
 // b + n_band, ..., so that the longer groups, which come first, are in all of them.  Units that are cut keep their order, the ranges of
 // one side by side: banded, or range by range, 777 x 17408 -> 5120 takes 345 to 360 us instead of 333.
 __device__ __forceinline__ unsigned rein_xh_banded(unsigned v, unsigned n_rb, unsigned n_grp)

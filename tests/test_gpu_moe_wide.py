@@ -50,9 +50,11 @@ def reference(gu, dn, hidden, ff, x, logits, n_used, weights, scale):
 
 
 def check(got, want, what):
-    # the intermediate is quantized again after SwiGLU: fp32 noise in gate / up can move a quant by one step
+    # The intermediate is quantized again after SwiGLU: fp32 noise in gate / up can move a quant by one step, 1/127 of its block's largest value.
+    # With 256 columns and a largest value of 5 times their rms that is 5 / 127 / 16 = 0.0025 of a token's row in the norm: 5e-4 over all is
+    # such a step in one row of 25 (seen: 1.6e-4).
     assert not np.isnan(got).any(), what
-    assert rel_l2(got, want) < 2e-3, what
+    assert rel_l2(got, want) < 5e-4, what
     assert_close_f32(got, want, rel=2e-2, abs_=2e-3, what=what)
 
 
